@@ -166,6 +166,7 @@ TESTING_SIGNATURES = {
 }
 
 _lib = None
+_host = None
 _testing_lib = None
 _lock = threading.Lock()
 
@@ -189,6 +190,22 @@ def lib() -> ctypes.CDLL:
                 fn.argtypes = argtypes
             _lib = handle
     return _lib
+
+
+def host():
+    """The ``_launch`` module (``csrc/host/``), loaded once: the launches that
+    check and fill their arguments in native code."""
+    global _host
+    if _host is None:
+        lib()  # what the module is linked against; raises its own message when missing
+        try:
+            from . import _launch
+        except ImportError as e:
+            raise RuntimeError(
+                f"iris_amd native launch module not usable ({e}). Build it with `python -m iris_amd.build`."
+            ) from e
+        _host = _launch
+    return _host
 
 
 def testing_lib() -> ctypes.CDLL:

@@ -7,6 +7,9 @@
 this file, ``libfinegrained_allocator.so`` to ``csrc/finegrained_alloc/`` --
 the place the reference's package looks for it (iris/__init__.py:29-38; built
 there by setup.py:22-84 / csrc/finegrained_alloc/build.sh).
+``_launch.so`` (``csrc/host/``) is the CPython module through which the Python
+launchers call the former: host code, compiled by the host compiler against
+torch's headers.
 ``libiris_amd_testing.so`` (``csrc/testing/``: measurement probes and unit-test
 kernels that only the tests and bench.py call) is a library of its own, so
 that the product library exports nothing but the product's entry points.
@@ -20,6 +23,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
@@ -28,6 +32,8 @@ OBJ = CSRC / "build"
 LIB = PKG / "libiris_amd.so"
 ALLOC_LIB = CSRC / "finegrained_alloc" / "libfinegrained_allocator.so"
 TESTING_LIB = PKG / "libiris_amd_testing.so"
+HOST_SRC = CSRC / "host" / "launch_module.cpp"
+HOST_EXT = PKG / "_launch.so"
 
 ARCH = "gfx950"
 # packed-fp32 instructions are kept out of all device code
@@ -76,6 +82,20 @@ def _run(cmd):
     return proc
 
 
+def _build_host_module() -> None:
+    import torch
+
+    cxx = os.environ.get("CXX") or shutil.which("g++") or "c++"
+    torch_dir = Path(torch.__file__).resolve().parent
+    includes = [torch_dir / "include", torch_dir / "include" / "torch" / "csrc" / "api" / "include",
+                sysconfig.get_paths()["include"]]
+    _run([cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-D__HIP_PLATFORM_AMD__=1",
+          "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+          *(f"-isystem{d}" for d in includes), f"-isystem{Path(hipcc()).resolve().parent.parent / 'include'}",
+          str(HOST_SRC), "-o", str(HOST_EXT), f"-L{PKG}", f"-l:{LIB.name}", f"-L{torch_dir / 'lib'}",
+          "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN"])
+
+
 def build(force: bool = False, jobs: int | None = None, verbose: bool = True) -> None:
     cc = hipcc()
     OBJ.mkdir(parents=True, exist_ok=True)
@@ -109,6 +129,11 @@ def build(force: bool = False, jobs: int | None = None, verbose: bool = True) ->
         _run([cc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(TESTING_LIB), *map(str, testing_objs)])
         if verbose:
             print(f"[iris_amd.build] linked {TESTING_LIB.name}", flush=True)
+
+    if force or _stale(HOST_EXT, [HOST_SRC, PKG.parent / "include" / "iris_amd.h"]):
+        _build_host_module()
+        if verbose:
+            print(f"[iris_amd.build] linked {HOST_EXT.name}", flush=True)
 
     alloc_src = CSRC / "finegrained_alloc" / "finegrained_allocator.hip"
     if force or _stale(ALLOC_LIB, [alloc_src]):

@@ -268,6 +268,16 @@ def gemm_launch(a, b, c, c_global, tile_completed, heap_bases, rank, world_size,
 
     The kernel launch of the reference wrappers (matmul_wrapper.py:109-150).
     """
+    if not noalloc:
+        err = _native.host().gemm(a, b, c, c_global, tile_completed, heap_bases, mm_begin_timestamp, mm_end_timestamp,
+                                  status, partials, locks, rank, world_size, num_sms, BLK_M, BLK_N, BLK_K, gsize_m,
+                                  epilogue, phase, notify, num_xcds, scope, variant, spin_timeout_ticks, split_k,
+                                  split_handover, flag_sem, touch_ahead)
+        if err == 0:
+            return
+        if err > 0:
+            _gemm_launch_failed(err)
+    # what the native code declines: the full checks, which say what is wrong, and the launch
     if noalloc:
         if partials is not None or locks is not None:
             raise ValueError("the no-allocation launch takes no workspace")
@@ -293,6 +303,11 @@ def gemm_launch(a, b, c, c_global, tile_completed, heap_bases, rank, world_size,
     stream = torch.cuda.current_stream(a.device).cuda_stream
     with torch.cuda.device(a.device):
         err = launch(ctypes.byref(args), stream)
+    _gemm_launch_failed(err)
+
+
+def _gemm_launch_failed(err):
+    """Raise for a launch status other than success."""
     if err == _native.HIP_ERROR_INVALID_VALUE:
         raise ValueError(
             "iris_gemm_launch rejected the arguments (shape, strides, dtypes, grid or rank layout it does not take)"
@@ -376,6 +391,11 @@ def one_shot_reduce(c, c_global, tile_completed, heap_bases, rank, world_size, B
     every flag wait (:220-234); by default the loads are coherent at the
     flags' scope by themselves.
     """
+    err = _native.host().one_shot_reduce(c, c_global, tile_completed, heap_bases, status, rank, world_size, BLK_M, BLK_N,
+                                         gsize_m, num_sms, num_xcds, scope, wait_flags, variant, spin_timeout_ticks,
+                                         flag_sem)
+    if err >= 0:
+        return _reduce_launch_failed(err)
     if c.dim() != 2 or c_global.dim() != 2:
         raise ValueError("c and c_global must be matrices")
     M, N = c.shape
@@ -411,6 +431,10 @@ def one_shot_reduce(c, c_global, tile_completed, heap_bases, rank, world_size, B
     stream = torch.cuda.current_stream(device).cuda_stream
     with torch.cuda.device(device):
         err = _native.lib().iris_one_shot_reduce_launch(ctypes.byref(args), stream)
+    _reduce_launch_failed(err)
+
+
+def _reduce_launch_failed(err):
     if err == _native.HIP_ERROR_INVALID_VALUE:
         raise ValueError("iris_one_shot_reduce_launch rejected the arguments")
     _native.hip_try(err)

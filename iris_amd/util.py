@@ -88,6 +88,11 @@ def do_bench(fn, barrier_fn=lambda: None, preamble_fn=lambda: None, n_warmup=25,
 
 def memset_tensor(tensor, value):
     """Fill a contiguous int32 tensor on the current stream (iris/util.py:117-128)."""
+    err = _native.host().memset_i32(tensor, value)
+    if err == 0:
+        return
+    if err > 0:
+        _native.hip_try(err)
     assert tensor.is_contiguous(), "Tensor must be contiguous"
     assert tensor.dtype == torch.int32, "Only torch.int32 tensors are supported"
     if not tensor.is_cuda:
