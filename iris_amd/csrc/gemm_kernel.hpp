@@ -149,6 +149,8 @@ struct GemmKArgs {
   // the whole launch (they all do the same work): two groups 2 us apart take 3 % off the headline launch on zeros
   // and 1.5 % on data, the 2 us that the later group ends after the first included.
   int stagger_groups, stagger_sleeps;
+  // (LOAD_GATHER tiles) the operand's rows (A) / columns (B) are contiguous in memory rather than its k
+  int a_across, b_across;
 };
 
 template <int DT>
@@ -190,16 +192,21 @@ struct Mfma<IRIS_DTYPE_F32> {
 // of fetch and multiply time.  LW_ = 4 adds one wave per SIMD that does
 // nothing but issue the stage loads and wait for them; the WM x WN waves then
 // issue no memory instruction in the K loop.
-template <int DT_, int CM_, int CN_, int BK_, int WM_, int WN_, int S_, bool DMA_, int LW_ = 0, bool TOUCH_ = false>
+// LOAD_: how the slabs get into LDS.  LOAD_DMA: see the top of the file.  LOAD_GATHER: through the fetching waves'
+// registers, for operands with any alignment that are contiguous along k or across it (see Gather).  LOAD_GENERIC:
+// element by element, for what is contiguous along neither.
+enum SlabLoad { LOAD_GENERIC = 0, LOAD_DMA = 1, LOAD_GATHER = 2 };
+template <int DT_, int CM_, int CN_, int BK_, int WM_, int WN_, int S_, int LOAD_, int LW_ = 0, bool TOUCH_ = false>
 struct GemmCfg {
   static constexpr int DT = DT_, CM = CM_, CN = CN_, BK = BK_, WM = WM_, WN = WN_, S = S_;
-  static constexpr bool DMA = DMA_;
+  static constexpr bool DMA = LOAD_ == LOAD_DMA, GATHER = LOAD_ == LOAD_GATHER;
+  static constexpr bool PIPE = LOAD_ != LOAD_GENERIC;  // the K loop runs as a pipeline across tiles
   static constexpr int NW = WM * WN, NT = NW * 64;  // the waves (threads) that multiply and store
   static constexpr int LW = LW_;
   static constexpr int NL = LW ? LW : NW;           // the waves that fetch
   // TOUCH_: a build of the eight-wave 256 x 256 tile that touches lines of K-steps to come (see Loader::touch)
   static constexpr bool TOUCH = TOUCH_;
-  static_assert(!TOUCH_ || (DMA_ && LW_ == 0 && WM_ * WN_ == 8 && CM_ == 256 && CN_ == 256), "the touching build's tile");
+  static_assert(!TOUCH_ || (LOAD_ == LOAD_DMA && LW_ == 0 && WM_ * WN_ == 8 && CM_ == 256 && CN_ == 256), "the touching build's tile");
   static constexpr int THREADS = (NW + LW) * 64;    // launch size
   static constexpr int TM = CM / WM, TN = CN / WN;
   static constexpr int IM = TM / 16, IN = TN / 16;  // 16x16 MFMA blocks of the wave tile
@@ -217,7 +224,7 @@ struct GemmCfg {
   // stream-K runs hand over); the 128x64 wave tiles have no registers to spare
   // for that exchange and only take the sliced hand-over, in which a part's
   // accumulators are dead once its partial is written.
-  static constexpr bool SPLITK = DMA_ && KSUB % 2 == 0 && IM * IN * 4 <= 128;
+  static constexpr bool SPLITK = PIPE && KSUB % 2 == 0 && IM * IN * 4 <= 128;
   static constexpr bool SPLIT_OWNER = SPLITK && IM * IN * 4 <= 64;
   // Waves per SIMD the register budget is sized for: 256 registers a wave.
   static constexpr int WPE = 2;
@@ -230,11 +237,12 @@ struct GemmCfg {
   static_assert(CM % (WM * 32) == 0 && CN % (WN * 32) == 0, "wave tile must be a multiple of 32x32");
   static_assert(BK == 32 || BK == 64 || BK == 128, "BK");
   static_assert((CM * CPR) % (NL * 64) == 0 && (CN * CPR) % (NL * 64) == 0, "slab must split evenly over lanes");
-  static_assert(LW == 0 || (DMA && NW + LW <= 8), "fetching waves: LDS-DMA tiles of at most eight waves in all");
+  static_assert(LW == 0 || (PIPE && NW + LW <= 8), "fetching waves: pipelined tiles of at most eight waves in all");
+  static_assert(!GATHER || (LW == 4 && S == 2 && BK >= 64), "the gathering tiles: two fetching waves an operand, two stages");
   static_assert(A_LOADS >= 1 && B_LOADS >= 1, "too many waves for this slab");
   static constexpr bool S_POW2 = (S & (S - 1)) == 0;  // (else the ring slot is counted along instead of masked out of g)
   static_assert(S >= 1, "ring depth");
-  static_assert(!DMA || S >= 2, "the DMA ring needs a stage being read and one in flight");
+  static_assert(!PIPE || S >= 2, "the ring needs a stage being read and one in flight");
   static_assert(L * (S - 1) <= 63, "vmcnt immediate");
   static_assert(IM * IN * 4 <= 128, "accumulators of a wave tile: at most 128 registers (two waves a SIMD)");
   static_assert(TN == 32 || TN == 64 || TN == 128, "wave tile width");
@@ -454,6 +462,205 @@ struct Loader {
     if constexpr (I < Cfg::L) {
       issue_at(p, stage, k, wave, I);
       issue<I + 1>(p, stage, k, wave);
+    }
+  }
+};
+
+// Gathering loader: operands contiguous along k at any alignment, or across it (a row-major B, a column-major A).
+// The LDS-DMA cannot take either (it moves aligned 16-byte chunks that lie along k), so the slabs pass through the
+// fetching waves' registers: waves 0 and 1 fetch A, 2 and 3 fetch B, 16 bytes a lane and load, and write the same
+// swizzled slab the DMA would.  Two register sets: the loads of a K-step are issued three steps before it is
+// multiplied and written into its stage one step before, so a load has two steps to arrive.
+//   * along k: a lane's 16 bytes are a chunk of the slab, at whatever byte they start (the memory pipeline takes
+//     16-byte loads at any address).
+//   * across k: a lane takes blocks of 8 k x 8 rows: eight 16-byte loads, one per k, eight lanes of a wave side by
+//     side (whole 128-byte lines), transposed in registers (32 v_perm_b32 a block) into eight chunks.  The eight
+//     lanes that differ in k write the chunks of one row together: no bank conflict.
+// Edges never read outside the operand: rows past the edge are clamped to the last one (their results are not
+// stored); a 16-byte load that would cross the end of its line is moved back to end there and shifted into place;
+// k past K is zeroed, in the one K-step that can hold any.
+// Bound by the fetching waves' issue and LDS writes, a step of 128 x 128 x 64 takes as long as the DMA's.
+template <class Cfg, bool IS_A>
+struct Gather {
+  static constexpr int ROWS = IS_A ? Cfg::CM : Cfg::CN;
+  static constexpr bool F32 = Cfg::DT == IRIS_DTYPE_F32;
+  static constexpr int ES = F32 ? 4 : 2;         // bytes of an element
+  static constexpr int EPC = 16 / ES;            // elements of a 16-byte chunk
+  static constexpr int SETS = 2;
+  // chunks a lane fetches per step, contiguous along k: the operand's slab over two waves
+  static constexpr int ALONG = ROWS * Cfg::CPR / 128;
+  // blocks of EPC k x 8 rows over two waves (a slab of fewer than 128 blocks leaves the second wave idle)
+  static constexpr int BLOCKS = (ROWS / 8 * Cfg::CPR + 127) / 128;
+  static constexpr bool HALF_IDLE = ROWS / 8 * Cfg::CPR < 128;
+  static constexpr int NV = ALONG > 8 * BLOCKS ? ALONG : 8 * BLOCKS;
+
+  const IRIS_GLOBAL char* base;  // the tile's rows of the operand at k = 0
+  int64_t ld;                    // bytes from one row (along k) or one k (across) to the next
+  uint32_t off[ALONG];           // along k: byte offset of each chunk at k0 = 0; across: of each block
+  int back[BLOCKS];              // across: elements the block's loads are moved back from the operand's edge
+  bool edge;                     // some block of the tile is (wave-uniform)
+  bool across;
+
+  u32x4 v[SETS][NV];
+  // `back` and `edge` of the tile a set's loads belong to: the load cursor may be in the next tile when it is stored
+  int set_back[SETS][BLOCKS];
+  bool set_edge[SETS];
+
+  typedef u32x4 __attribute__((aligned(2))) u32x4_any;
+  __device__ static inline u32x4 load16(const IRIS_GLOBAL char* p) { return *(const IRIS_GLOBAL u32x4_any*)p; }
+  // A scalar address that the compiler takes as it is: base in scalar registers, a 32-bit lane offset per load.  (Left
+  // to itself it turns the loads of a K loop into 64-bit pointers per lane, two registers each and an addition a step.)
+  __device__ static inline const IRIS_GLOBAL char* scalar(const IRIS_GLOBAL char* p) {
+    asm volatile("" : "+s"(p));
+    return p;
+  }
+  // 128-bit right shift by n 16-bit units, 0 <= n; zero from eight on
+  __device__ static inline u32x4 shift_right(u32x4 x, int n) {
+    if (n & 4) x = u32x4{x[2], x[3], 0u, 0u};
+    if (n & 2) x = u32x4{x[1], x[2], x[3], 0u};
+    if (n & 1)
+      x = u32x4{(x[0] >> 16) | (x[1] << 16), (x[1] >> 16) | (x[2] << 16), (x[2] >> 16) | (x[3] << 16), x[3] >> 16};
+    if (n >= 8) x = u32x4{0u, 0u, 0u, 0u};
+    return x;
+  }
+  // block `i` of this lane across k: k block kb and rows 8 nb ..
+  __device__ static inline void block_of(int i, int half, int lane, int* kb, int* nb) {
+    const int b = (i * 2 + half) * 64 + lane;
+    // eight lanes side by side hold eight k blocks of one row block (their chunks of a row are written together)
+    const int q = b >> 3;
+    *nb = q % (ROWS / 8);
+    *kb = (b & 7) + 8 * (q / (ROWS / 8));
+  }
+
+  __device__ inline void setup(const GemmKArgs& p, const Item& it, int fwave, int lane) {
+    const int half = fwave & 1;
+    across = (IS_A ? p.a_across : p.b_across) != 0;
+    edge = false;
+    ld = (across ? (IS_A ? p.sak : p.sbk) : (IS_A ? p.sam : p.sbn)) * 2;
+    const int row0 = IS_A ? it.m0 : it.n0, extent = IS_A ? p.M : p.N;
+    base = (const IRIS_GLOBAL char*)(IS_A ? p.a : p.b) + (across ? 0 : (int64_t)min(row0, extent - 1) * ld);
+    if (!across) {
+#pragma unroll
+      for (int i = 0; i < ALONG; ++i) {
+        const int row = (i * 2 + half) * Cfg::RPB + lane / Cfg::CPR;
+        const int ch = (lane % Cfg::CPR) ^ ((row / Cfg::RP) % Cfg::CPR);
+        off[i] = (uint32_t)((int64_t)(min(row0 + row, extent - 1) - min(row0, extent - 1)) * ld) + ch * 16;
+      }
+    } else {
+      edge = row0 + ROWS > extent;
+#pragma unroll
+      for (int i = 0; i < BLOCKS; ++i) {
+        int kb, nb;
+        block_of(i, half, lane, &kb, &nb);
+        const int n = row0 + nb * 8, at = min(n, extent - 8);
+        back[i] = n - at;
+        off[i] = (uint32_t)(kb * EPC) * (uint32_t)ld + (uint32_t)at * ES;
+      }
+    }
+  }
+
+  // Fetch K-step `k` into register set SET.  TAIL: it may hold k past K (or nothing, `live` false).
+  template <int SET, bool TAIL>
+  __device__ inline void load(int K, int k, bool live, int fwave, int lane) {
+    const int half = fwave & 1;
+    if (TAIL && !live) {
+      set_edge[SET] = false;
+#pragma unroll
+      for (int i = 0; i < NV; ++i) v[SET][i] = u32x4{0u, 0u, 0u, 0u};
+      return;
+    }
+    if (!across) {
+      const IRIS_GLOBAL char* src = scalar(base + (int64_t)k * (Cfg::BK * 2));
+#pragma unroll
+      for (int i = 0; i < ALONG; ++i) {
+        if constexpr (TAIL) {
+          const int row = (i * 2 + half) * Cfg::RPB + lane / Cfg::CPR;
+          const int ch = (lane % Cfg::CPR) ^ ((row / Cfg::RP) % Cfg::CPR);
+          const int over = max(0, k * Cfg::BK + ch * 8 + 8 - K);  // 16-bit units past K
+          v[SET][i] = shift_right(load16(src + ((int64_t)off[i] - over * 2)), over);  // (stays inside the row: K >= 8)
+        } else {
+          v[SET][i] = load16(src + off[i]);
+        }
+      }
+    } else {
+      set_edge[SET] = edge;
+#pragma unroll
+      for (int i = 0; i < BLOCKS; ++i) set_back[SET][i] = back[i];
+      // (a slab smaller than two waves' blocks: the second wave has nothing to fetch)
+      if (HALF_IDLE && half != 0) return;
+      constexpr int KE = F32 ? Cfg::BK / 2 : Cfg::BK;  // elements of K a step covers
+      const int Ke = F32 ? K / 2 : K;
+      const IRIS_GLOBAL char* src = base + (int64_t)k * KE * ld;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        // 16-bit: load j is k j of the block, its 8 rows.  fp32: k j / 2, rows 4 (j % 2) ..
+        const int kj = F32 ? j >> 1 : j;
+        const IRIS_GLOBAL char* line = scalar(src + (int64_t)kj * ld + (F32 ? (j & 1) * 16 : 0));
+#pragma unroll
+        for (int i = 0; i < BLOCKS; ++i) {
+          if constexpr (TAIL) {
+            int kb, nb;
+            block_of(i, half, lane, &kb, &nb);
+            const int past = k * KE + kb * EPC + kj - (Ke - 1);  // > 0: k past the last
+            const u32x4 x = load16(line + ((int64_t)off[i] - (int64_t)max(0, past) * ld));
+            v[SET][i * 8 + j] = past > 0 ? u32x4{0u, 0u, 0u, 0u} : x;
+          } else {
+            v[SET][i * 8 + j] = load16(line + off[i]);
+          }
+        }
+      }
+    }
+  }
+  // Write register set SET into the stage.
+  template <int SET>
+  __device__ inline void store(IRIS_LDS char* stage, int fwave, int lane) {
+    IRIS_LDS char* slab = stage + (IS_A ? 0 : Cfg::A_BYTES);
+    const int half = fwave & 1;
+    if (!across) {
+#pragma unroll
+      for (int i = 0; i < ALONG; ++i)
+        *reinterpret_cast<IRIS_LDS u32x4*>(slab + (i * 2 + half) * 1024 + lane * 16) = v[SET][i];
+      return;
+    }
+    if (HALF_IDLE && half != 0) return;
+#pragma unroll
+    for (int i = 0; i < BLOCKS; ++i) {
+      int kb, nb;
+      block_of(i, half, lane, &kb, &nb);
+      u32x4 x[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[j] = v[SET][i * 8 + j];
+      if (set_edge[SET]) {
+        // (moved back by `back` elements; what lies past the operand's edge is never stored)
+        if constexpr (F32) {
+          // the block's 8 rows as two loads: shift them together, 32 bytes, by whole elements
+#pragma unroll
+          for (int j = 0; j < 8; j += 2)
+#pragma unroll
+            for (int b = 1; b < 8; b *= 2) {
+              const unsigned int w[8] = {x[j][0], x[j][1], x[j][2], x[j][3], x[j + 1][0], x[j + 1][1], x[j + 1][2], x[j + 1][3]};
+              if (set_back[SET][i] & b)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) x[j + e / 4][e % 4] = e + b < 8 ? w[e + b] : 0u;
+            }
+        } else {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) x[j] = shift_right(x[j], set_back[SET][i]);
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < 8; ++r) {
+        const int row = nb * 8 + r;
+        u32x4 y;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          if constexpr (F32)
+            y[q] = x[2 * q + r / 4][r % 4];
+          else  // k 2q and 2q + 1 of row r: the low or the high halves of two dwords
+            y[q] = __builtin_amdgcn_perm(x[2 * q + 1][r / 2], x[2 * q][r / 2], r & 1 ? 0x07060302u : 0x05040100u);
+        }
+        *reinterpret_cast<IRIS_LDS u32x4*>(slab + row * (Cfg::BK * 2) + (kb ^ ((row / Cfg::RP) % Cfg::CPR)) * 16) = y;
+      }
     }
   }
 };
@@ -1140,9 +1347,12 @@ __device__ inline void fused_reduce_tile(const GemmKArgs& p, const Item& it, int
 // (gemm_one_shot_all_reduce.py:197-271): store the partial tile, signal the
 // other ranks, wait for the tile's own flag, reduce it over all ranks and
 // store the result, tile by tile, while other programs are in their K loops.
-template <class Cfg, int OP, int ODT, bool SPLIT = false, bool FUSED = false, bool MERGED = false>
-__global__ __launch_bounds__(Cfg::THREADS) __attribute__((amdgpu_waves_per_eu(Cfg::WPE, Cfg::WPE))) void
-gemm_persistent_kernel(const GemmKArgs p) {
+// ROLE: which waves the code is for.  The gathering tiles compile it three times, for the multiplying waves and for the
+// two that fetch either operand, so that none holds registers for another's state (the accumulators here, two register sets of a slab
+// there); the control flow is the same, so every barrier is still met by all.
+enum WaveRole { ROLE_ANY = 0, ROLE_WORKER = 1, ROLE_FETCH_A = 2, ROLE_FETCH_B = 3 };
+template <class Cfg, int OP, int ODT, bool SPLIT, bool FUSED, bool MERGED, int ROLE>
+__device__ __attribute__((always_inline)) inline void gemm_program(const GemmKArgs& p) {
   static_assert(!MERGED || !FUSED, "blocks of the caller's tiles: no build with the reduce inside");
   extern __shared__ __attribute__((aligned(1024))) char lds_raw[];
   IRIS_LDS char* lds = (IRIS_LDS char*)lds_raw;
@@ -1153,8 +1363,8 @@ gemm_persistent_kernel(const GemmKArgs p) {
   // barrier below is met by all of them; only the work is told apart: the
   // first NW waves multiply and store, the fetching waves (if the tile has
   // any; otherwise every wave does both) issue the stage loads.
-  const bool worker = Cfg::LW == 0 || wave < Cfg::NW;
-  const bool fetcher = Cfg::LW == 0 || wave >= Cfg::NW;
+  const bool worker = ROLE == ROLE_ANY ? Cfg::LW == 0 || wave < Cfg::NW : ROLE == ROLE_WORKER;
+  const bool fetcher = ROLE == ROLE_ANY ? Cfg::LW == 0 || wave >= Cfg::NW : ROLE != ROLE_WORKER;
   const int fwave = Cfg::LW == 0 ? wave : wave - Cfg::NW;  // index among the fetching waves
   int pid;
   if (p.xcd_per > 0) {
@@ -1226,7 +1436,7 @@ gemm_persistent_kernel(const GemmKArgs p) {
   // have completed.  Waiting for that right after issuing them would stall
   // the matrix cores, so the publication is deferred to the top of the next
   // K-step, where the whole group waits on its memory counter anyway.
-  const bool defer_publish = !FUSED && Cfg::DMA && nk > 0 && p.flag_mode != 0;
+  const bool defer_publish = !FUSED && Cfg::PIPE && nk > 0 && p.flag_mode != 0;
   int pending_tile = -1;
   // 1: the pending tile's stores are exactly the FAST_STORES youngest memory
   // operations of this wave, so the next hand-over can wait for the loads
@@ -1246,7 +1456,7 @@ gemm_persistent_kernel(const GemmKArgs p) {
   constexpr bool PF = Cfg::LW != 0 && Cfg::DMA && !FUSED && Cfg::CM == 256 && Cfg::CN == 64;
   // a third build of the K-step, without the hand-over's tests (see `step`; not with the reduce inside the program,
   // where the K loop is the smaller part and a third copy of the step adds to what the 128-accumulator tiles spill)
-  constexpr bool LEAN_STEPS = Cfg::DMA && !FUSED;
+  constexpr bool LEAN_STEPS = Cfg::PIPE && !FUSED;
   // the lean steps of the eight-wave 256 x 256 tile each end with the two touches of Loader::touch, which the
   // next lean step's hand-over leaves in flight
   constexpr bool PF8 = Cfg::TOUCH && LEAN_STEPS;
@@ -1484,7 +1694,7 @@ gemm_persistent_kernel(const GemmKArgs p) {
   if (nk == 0) {
     // K == 0 leaves every tile all zeros: one epilogue per item, no loads
     for (int it = 0; it < n_items; ++it) epilogue();
-  } else if constexpr (Cfg::DMA) {
+  } else if constexpr (Cfg::PIPE) {
     // ---- the (item, k) pipeline -------------------------------------------
     // Ring of S stages.  A step's last fragment fetch happens one substep
     // before its last MFMAs, so at the hand-over in step g every wave is done
@@ -1492,41 +1702,81 @@ gemm_persistent_kernel(const GemmKArgs p) {
     // tail of step g is multiplied, stage g+1 has landed and stages
     // g+2..g+S are in flight.  The load cursor runs S steps ahead of the
     // compute cursor and crosses into the next item on its own.
-    Loader<Cfg> ld;
+    // (LOAD_GATHER: a tile's steps are walked in pairs, one register set each; an odd number of steps gets one more
+    // that holds nothing.  The load cursor runs three steps ahead: two in registers, one on its way into a stage.)
+    constexpr int AHEAD = Cfg::GATHER ? 1 + 2 : Cfg::S;
+    std::conditional_t<Cfg::GATHER, Gather<Cfg, ROLE == ROLE_FETCH_A>, Loader<Cfg>> ld;
     int l_item = 0, l_k = 0, l_kend = nk;  // load cursor
+    int l_klive = 0;                       // (LOAD_GATHER) end of the cursor's real steps
     Item l_it;
+    auto cursor_to = [&](const KRange& kr) __attribute__((always_inline)) {
+      l_k = kr.k_begin;
+      l_kend = kr.k_end;
+      if constexpr (Cfg::GATHER) {
+        l_klive = l_kend;
+        l_kend += (l_kend - l_k) & 1;
+        ld.setup(p, l_it, fwave, lane);
+      } else {
+        ld.setup(p, l_it, fwave, lane, l_k);
+      }
+    };
     auto advance_load_cursor = [&]() __attribute__((always_inline)) {
       if (++l_k == l_kend) {
         if (!ONE_ITEM && ++l_item < n_items) {
           l_it = decode_item<Cfg, SPLIT>(p, sr, pid, l_item);
-          const KRange kr = k_range<Cfg, SPLIT>(p, sr, pid, l_item, nk);
-          l_k = kr.k_begin;
-          l_kend = kr.k_end;
-          ld.setup(p, l_it, fwave, lane, l_k);
+          cursor_to(k_range<Cfg, SPLIT>(p, sr, pid, l_item, nk));
         } else {
+          // nothing left to load
           l_k = 0;
-          l_kend = nk;
-          ld.park();  // nothing left to load
+          if constexpr (Cfg::GATHER) {
+            l_kend = 0x7FFFFFFF;
+            l_klive = 0;
+          } else {
+            l_kend = nk;
+            ld.park();
+          }
         }
-      } else {
+      } else if constexpr (!Cfg::GATHER) {
         ld.before_step(l_k, fwave, lane);
+      }
+    };
+    // (LOAD_GATHER) fetch the cursor's step into register set SET; LEAN: a whole step, inside the tile
+    auto gather = [&](auto set_tag, auto lean_tag) __attribute__((always_inline)) {
+      if constexpr (Cfg::GATHER) {
+        constexpr int SET = decltype(set_tag)::value;
+        if constexpr (decltype(lean_tag)::value) {
+          ld.template load<SET, false>(p.K, l_k, true, fwave, lane);
+        } else if (l_k < l_klive && (l_k + 1) * Cfg::BK <= p.K) {
+          ld.template load<SET, false>(p.K, l_k, true, fwave, lane);
+        } else {
+          ld.template load<SET, true>(p.K, l_k, l_k < l_klive, fwave, lane);
+        }
       }
     };
     Frags<Cfg> fr;
     if (total_steps > 0) {
       if (fetcher) {
         l_it = c_it;  // (item 0, decoded above for the compute cursor)
-        const KRange kr = k_range<Cfg, SPLIT>(p, sr, pid, 0, nk);
-        l_k = kr.k_begin;
-        l_kend = kr.k_end;
-        ld.setup(p, l_it, fwave, lane, l_k);
-#pragma unroll
-        for (int s = 0; s < Cfg::S; ++s) {
-          ld.issue(p, lds + s * Cfg::STAGE, l_k, fwave);
+        cursor_to(k_range<Cfg, SPLIT>(p, sr, pid, 0, nk));
+        if constexpr (Cfg::GATHER) {
+          using Set0 = std::integral_constant<int, 0>;
+          gather(Set0{}, std::false_type{});
           advance_load_cursor();
+          gather(std::integral_constant<int, 1>{}, std::false_type{});
+          advance_load_cursor();
+          ld.template store<0>(lds, fwave, lane);
+          gather(Set0{}, std::false_type{});
+          advance_load_cursor();
+          IRIS_WAIT_LGKMCNT0();
+        } else {
+#pragma unroll
+          for (int s = 0; s < Cfg::S; ++s) {
+            ld.issue(p, lds + s * Cfg::STAGE, l_k, fwave);
+            advance_load_cursor();
+          }
+          // stage 0 has landed once at most S-1 younger slabs are outstanding
+          IRIS_WAIT_VMCNT(Cfg::L * (Cfg::S - 1));
         }
-        // stage 0 has landed once at most S-1 younger slabs are outstanding
-        IRIS_WAIT_VMCNT(Cfg::L * (Cfg::S - 1));
       }
       block_barrier_raw();
       if (worker) {
@@ -1553,7 +1803,8 @@ gemm_persistent_kernel(const GemmKArgs p) {
     // previous tile's flag went up at this tile's second hand-over) and the load cursor's next step lies inside
     // the tile and is a full one, so the hand-over is a wait, the barrier and the refill, with no test between
     // them: the waves all pass it at the same time, and what it costs, every SIMD's matrix core waits out.
-    auto step = [&](int g, auto first_tag, auto par_tag, auto lean_tag) __attribute__((always_inline)) {
+    // SET: (LOAD_GATHER) the register set that holds step g+1.
+    auto step = [&](int g, auto first_tag, auto par_tag, auto lean_tag, auto set_tag) __attribute__((always_inline)) {
       constexpr bool FIRST = decltype(first_tag)::value;
       constexpr int PAR = decltype(par_tag)::value;
       constexpr bool LEAN = decltype(lean_tag)::value;
@@ -1600,7 +1851,15 @@ gemm_persistent_kernel(const GemmKArgs p) {
         // (S-2 younger slabs may stay in flight), then meet the other waves
         const int pend = LEAN ? -1 : __builtin_amdgcn_readfirstlane(pending_tile);
         const int skip = LEAN ? 0 : __builtin_amdgcn_readfirstlane(pending_skip);
-        if constexpr (LEAN) {
+        if constexpr (Cfg::GATHER) {
+          // stage g+1's slot has been free since the last hand-over: write it, then hand it over
+          if (fetcher) {
+            ld.template store<decltype(set_tag)::value>(lds + slot_n * Cfg::STAGE, fwave, lane);
+            IRIS_WAIT_LGKMCNT0();
+          } else if (!LEAN && pend >= 0 && skip == 0) {
+            IRIS_WAIT_VMCNT(0);  // the previous tile's stores (all this wave has in flight)
+          }
+        } else if constexpr (LEAN) {
           if (Cfg::LW == 0 || fetcher) IRIS_WAIT_VMCNT(Cfg::L * (Cfg::S - 2) + TOUCHES);
         } else if constexpr (Cfg::LW != 0) {
           if (fetcher) {
@@ -1652,7 +1911,10 @@ gemm_persistent_kernel(const GemmKArgs p) {
         if constexpr (Cfg::LW != 0) {
           // every wave is past its reads of stage g: refill it with step g+S
           if (fetcher) {
-            ld.issue(p, rstage, l_k, fwave);
+            if constexpr (Cfg::GATHER)
+              gather(set_tag, lean_tag);
+            else
+              ld.issue(p, rstage, l_k, fwave);
             if constexpr (LEAN)
               ++l_k;
             else
@@ -1668,16 +1930,41 @@ gemm_persistent_kernel(const GemmKArgs p) {
     // B buffer a step starts with: substeps alternate, so with an odd KSUB
     // it flips from step to step
     auto run_step = [&](int g, auto first_tag, auto lean_tag) __attribute__((always_inline)) {
+      using Set0 = std::integral_constant<int, 0>;
       if constexpr (Cfg::KSUB % 2 == 0) {
-        step(g, first_tag, std::integral_constant<int, 0>{}, lean_tag);
+        step(g, first_tag, std::integral_constant<int, 0>{}, lean_tag, Set0{});
       } else {
         if (g & 1)
-          step(g, first_tag, std::integral_constant<int, 1>{}, lean_tag);
+          step(g, first_tag, std::integral_constant<int, 1>{}, lean_tag, Set0{});
         else
-          step(g, first_tag, std::integral_constant<int, 0>{}, lean_tag);
+          step(g, first_tag, std::integral_constant<int, 0>{}, lean_tag, Set0{});
       }
     };
     int g = 0;
+    // (LOAD_GATHER) a tile in pairs of steps: every pair begins with an even step of the program, so that the set
+    // a step's successor waits in is known at compile time
+    auto run_pair = [&](auto first_tag, auto lean_tag) __attribute__((always_inline)) {
+      using I0 = std::integral_constant<int, 0>;
+      using I1 = std::integral_constant<int, 1>;
+      step(g, first_tag, I0{}, lean_tag, I1{});
+      step(g + 1, std::false_type{}, I0{}, lean_tag, I0{});
+      g += 2;
+    };
+    auto run_item_gathered = [&](int it) __attribute__((always_inline)) {
+      stamp_begin();
+      const KRange kr = k_range<Cfg, SPLIT>(p, sr, pid, it, nk);
+      const int steps = kr.k_end - kr.k_begin, pairs_end = (steps + 1) & ~1;
+      run_pair(std::true_type{}, std::false_type{});
+      int k = 2;
+      if constexpr (LEAN_STEPS) {
+        // lean: the cursor, three steps ahead, stays on whole steps of this tile and does not cross into the next
+        const int whole = min(steps - 1, p.K / Cfg::BK - kr.k_begin);
+        for (; k + 1 + AHEAD < whole; k += 2) run_pair(std::false_type{}, std::true_type{});
+      }
+      for (; k < pairs_end; k += 2) run_pair(std::false_type{}, std::false_type{});
+      if constexpr (ONE_ITEM) IRIS_WAIT_VMCNT(0);
+      epilogue();
+    };
     auto run_item = [&](int it) __attribute__((always_inline)) {
       stamp_begin();
       const KRange kr = k_range<Cfg, SPLIT>(p, sr, pid, it, nk);
@@ -1742,10 +2029,16 @@ gemm_persistent_kernel(const GemmKArgs p) {
       if constexpr (ONE_ITEM) IRIS_WAIT_VMCNT(0);  // (the loads past the last step fetch nothing, and nothing follows)
       epilogue();
     };
+    auto run = [&](int it) __attribute__((always_inline)) {
+      if constexpr (Cfg::GATHER)
+        run_item_gathered(it);
+      else
+        run_item(it);
+    };
     if constexpr (ONE_ITEM) {
-      if (n_items > 0) run_item(0);
+      if (n_items > 0) run(0);
     } else {
-      for (int it = 0; it < n_items; ++it) run_item(it);
+      for (int it = 0; it < n_items; ++it) run(it);
     }
     IRIS_WAIT_VMCNT(0);  // no load may still be writing this group's LDS when it exits
   } else {
@@ -1778,6 +2071,22 @@ gemm_persistent_kernel(const GemmKArgs p) {
     IRIS_WAIT_VMCNT(0);
     __syncthreads();
     if (wave == 0) publish_tile<MERGED>(p, pending_tile, lane);
+  }
+}
+
+template <class Cfg, int OP, int ODT, bool SPLIT = false, bool FUSED = false, bool MERGED = false>
+__global__ __launch_bounds__(Cfg::THREADS) __attribute__((amdgpu_waves_per_eu(Cfg::WPE, Cfg::WPE))) void
+gemm_persistent_kernel(const GemmKArgs p) {
+  if constexpr (Cfg::GATHER) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (wave < Cfg::NW)
+      gemm_program<Cfg, OP, ODT, SPLIT, FUSED, MERGED, ROLE_WORKER>(p);
+    else if (wave < Cfg::NW + 2)
+      gemm_program<Cfg, OP, ODT, SPLIT, FUSED, MERGED, ROLE_FETCH_A>(p);
+    else
+      gemm_program<Cfg, OP, ODT, SPLIT, FUSED, MERGED, ROLE_FETCH_B>(p);
+  } else {
+    gemm_program<Cfg, OP, ODT, SPLIT, FUSED, MERGED, ROLE_ANY>(p);
   }
 }
 

@@ -41,7 +41,7 @@ const GemmKernelEntry* entries_for(int dt, int op, int* count) {
 // The plain build (every wave fetches its share) of the tile shape of `e`, an
 // entry with fetching waves; null if `e` has none or the list holds no such build.
 const GemmKernelEntry* plain_twin(const GemmKernelEntry* list, int count, const GemmKernelEntry& e) {
-  if (e.fetch_waves == 0) return nullptr;
+  if (e.fetch_waves == 0 || !e.dma) return nullptr;
   for (int i = 0; i < count; ++i)
     if (list[i].dma && list[i].fetch_waves == 0 && list[i].cm == e.cm && list[i].cn == e.cn && list[i].wm == e.wm &&
         list[i].wn == e.wn)
@@ -644,7 +644,22 @@ hipError_t make_plan_body(const iris_gemm_args& a, Plan* plan) {
   const int unit = a.ab_dtype == IRIS_DTYPE_F32 ? 2 : 1;
   const bool dma_ok = a.stride_ak == unit && a.stride_bk == unit && (a.stride_am % 8) == 0 && (a.stride_bn % 8) == 0 &&
                       aligned16(a.a) && aligned16(a.b) && (a.K % 8) == 0 && a.stride_am > 0 && a.stride_bn > 0;
+  // The gathering loader takes operands that are contiguous in one direction, with at least one 16-byte load of them
+  // in it (a load at the edge is moved back inside), a block of eight rows when that direction is across K, and
+  // 32-bit offsets inside a tile.
+  const bool a_along = a.stride_ak == unit && a.K >= 8, b_along = a.stride_bk == unit && a.K >= 8;
+  const bool a_across = !a_along && a.stride_am == unit && a.M >= 8, b_across = !b_along && a.stride_bn == unit && a.N >= 8;
+  k.a_across = a_across;
+  k.b_across = b_across;
+  auto gatherable = [&](bool along, bool across, int rows, int bk, int64_t ld_row, int64_t ld_k, int64_t extent) {
+    const int64_t lim = (int64_t)1 << 30;  // 16-bit units
+    return (along && ld_row >= 0 && rows * ld_row + a.K < lim) ||
+           (across && ld_k >= 0 && bk * ld_k + extent * unit < lim);
+  };
   auto fits = [&](const GemmKernelEntry& e) {
+    if (e.gather)
+      return gatherable(a_along, a_across, e.cm, e.bk, a.stride_am, a.stride_ak, a.M) &&
+             gatherable(b_along, b_across, e.cn, e.bk, a.stride_bn, a.stride_bk, a.N);
     if (!e.dma) return true;
     if (!dma_ok) return false;
     const int64_t lim = (int64_t)1 << 31;
@@ -670,7 +685,8 @@ hipError_t make_plan_body(const iris_gemm_args& a, Plan* plan) {
     // columns a small matrix cannot fill are not worth a tall compute tile
     for (int i = 0; i < count && !pick; ++i) {
       const GemmKernelEntry& e = list[i];
-      if (!fits(e)) continue;
+      // (the gathering tiles are for what the DMA does not take)
+      if (!fits(e) || (e.gather && dma_ok)) continue;
       if (plan->in_program && !e.fn_fused) continue;
       // (a caller's split needs a K-step per part: a tile with a deeper step may not have them)
       if (a.split_k > 1 && a.split_k > (a.K + e.bk - 1) / e.bk && e.bk > 64) continue;
@@ -686,9 +702,9 @@ hipError_t make_plan_body(const iris_gemm_args& a, Plan* plan) {
       if ((op == OP_ATOMIC32 || op == OP_ATOMIC16) && e.cm * e.cn > 256 * 128) continue;
       pick = &e;
     }
-    // otherwise the generic tile, with masked sub-tiles
-    for (int i = count - 1; i >= 0 && !pick; --i)
-      if (!list[i].dma && list[i].cm == 64 && list[i].cn == 64) pick = &list[i];
+    // otherwise 64 x 64, with masked sub-tiles: gathered if the operands allow it, else element by element
+    for (int i = 0; i < count && !pick; ++i)
+      if (!list[i].dma && list[i].cm == 64 && list[i].cn == 64 && fits(list[i])) pick = &list[i];
   }
   if (!pick) return hipErrorInvalidValue;
   if (plan->in_program && !pick->fn_fused) return hipErrorInvalidValue;

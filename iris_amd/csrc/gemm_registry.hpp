@@ -15,6 +15,7 @@ struct GemmKernelEntry {
   int cm, cn;  // compute tile
   int bk, wm, wn, stages;  // (bk in 16-bit units: half as many elements of fp32 operands)
   bool dma;    // LDS-DMA loader (needs K-contiguous, 16-byte aligned operands)
+  bool gather;  // gathering loader (operands contiguous along K or across it, at any alignment); neither: generic
   bool splitk;  // the kernel can share a tile's K range with other programs
   bool split_owner;  // ... and its first part can add the others' partials itself (needed for stream-K runs)
   int threads;        // launch size: the multiplying waves and the fetching waves (if any)
@@ -40,9 +41,10 @@ constexpr GemmKernelFn split_fn() {
 
 template <class Cfg, int OP, int ODT>
 constexpr GemmKernelFn fused_fn() {
-  // (the tiles with fetching waves have no such build: the reduce wants the registers their
-  // fetch state takes, and the launcher takes the plain tile of the same shape instead)
-  if constexpr ((OP == OP_STORE16 || OP == OP_STORE32) && Cfg::LW == 0)
+  // (the DMA tiles with fetching waves have no such build: the reduce wants the registers their
+  // fetch state takes, and the launcher takes the plain tile of the same shape instead; the gathering tiles, which
+  // have no plain twin, have one where the accumulators leave room)
+  if constexpr ((OP == OP_STORE16 || OP == OP_STORE32) && (Cfg::LW == 0 || (Cfg::GATHER && Cfg::IM * Cfg::IN * 4 <= 64)))
     return &gemm_persistent_kernel<Cfg, OP, ODT, false, true>;
   else
     return nullptr;
@@ -89,7 +91,7 @@ template <class Cfg, int OP>
 constexpr GemmKernelEntry make_entry(const char* name) {
   constexpr int ODT = (OP == OP_STORE32 || OP == OP_ATOMIC32) ? IRIS_DTYPE_F32 : Cfg::DT;
   return GemmKernelEntry{Cfg::DT, OP,      Cfg::CM, Cfg::CN, Cfg::BK,        Cfg::WM,
-                         Cfg::WN, Cfg::S,  Cfg::DMA, Cfg::SPLITK, Cfg::SPLIT_OWNER, Cfg::THREADS, Cfg::LW, Cfg::LDS_BYTES,
+                         Cfg::WN, Cfg::S,  Cfg::DMA, Cfg::GATHER, Cfg::SPLITK, Cfg::SPLIT_OWNER, Cfg::THREADS, Cfg::LW, Cfg::LDS_BYTES,
                          &gemm_persistent_kernel<Cfg, OP, ODT, false>, split_fn<Cfg, OP, ODT>(), fused_fn<Cfg, OP, ODT>(),
                          merged_fn<Cfg, OP, ODT>(), split_merged_fn<Cfg, OP, ODT>(), touch_fn<Cfg, OP, ODT, false>(),
                          touch_fn<Cfg, OP, ODT, true>(), name};
@@ -98,7 +100,7 @@ constexpr GemmKernelEntry make_entry(const char* name) {
 // The variants, in the launcher's order of preference: the first entry whose
 // compute tile divides the logical tile (and whose loader fits the operands)
 // wins.  `variant` k > 0 in iris_gemm_args forces entry k-1 (tuning runs).
-// Columns: compute tile CM, CN, BK; waves WM x WN; stages; LDS-DMA loader;
+// Columns: compute tile CM, CN, BK; waves WM x WN; stages; loader (SlabLoad);
 // fetching waves; whether the tile also has a split-K build (must equal
 // GemmCfg::SPLITK); name.
 //
@@ -110,31 +112,39 @@ constexpr GemmKernelEntry make_entry(const char* name) {
 // two: 57 -> 42 us on the same shape); and plain, which the launcher takes
 // where the first loses: with the reduce inside the program (no such build)
 // and for two programs per CU.
+//
+// The `_gather` tiles take what the DMA cannot: operands that lie along K at any alignment, or across it (a row-major
+// B, a column-major A).  The generic tile is left for operands that are contiguous in neither direction.
 #define IRIS_GEMM_VARIANTS(X, DT, OP)                                     \
-  X(DT, OP, 256, 256, 64, 2, 4, 2, true, 0, 1, "256x256x64_w2x4_s2")         \
-  X(DT, OP, 256, 128, 64, 2, 2, 3, true, 4, 1, "256x128x64_w2x2_s3_f4")      \
-  X(DT, OP, 128, 256, 64, 1, 4, 3, true, 4, 1, "128x256x64_w1x4_s3_f4")      \
-  X(DT, OP, 128, 128, 64, 2, 2, 4, true, 4, 1, "128x128x64_w2x2_s4_f4")      \
-  X(DT, OP, 256, 64, 64, 4, 1, 3, true, 4, 1, "256x64x64_w4x1_s3_f4")        \
-  X(DT, OP, 128, 64, 64, 2, 2, 4, true, 4, 1, "128x64x64_w2x2_s4_f4")        \
-  X(DT, OP, 64, 128, 64, 2, 2, 4, true, 4, 1, "64x128x64_w2x2_s4_f4")        \
-  X(DT, OP, 64, 64, 128, 2, 2, 4, true, 4, 1, "64x64x128_w2x2_s4_f4")        \
-  X(DT, OP, 256, 128, 64, 2, 2, 2, true, 0, 1, "256x128x64_w2x2_s2")         \
-  X(DT, OP, 128, 256, 64, 1, 4, 2, true, 0, 1, "128x256x64_w1x4_s2")         \
-  X(DT, OP, 128, 128, 64, 2, 2, 4, true, 0, 1, "128x128x64_w2x2_s4")         \
-  X(DT, OP, 256, 64, 64, 4, 1, 2, true, 0, 1, "256x64x64_w4x1_s2")           \
-  X(DT, OP, 64, 64, 64, 2, 2, 4, true, 0, 1, "64x64x64_w2x2_s4")             \
-  X(DT, OP, 64, 64, 32, 2, 2, 1, false, 0, 0, "64x64x32_w2x2_generic")
+  X(DT, OP, 256, 256, 64, 2, 4, 2, LOAD_DMA, 0, 1, "256x256x64_w2x4_s2")         \
+  X(DT, OP, 256, 128, 64, 2, 2, 3, LOAD_DMA, 4, 1, "256x128x64_w2x2_s3_f4")      \
+  X(DT, OP, 128, 256, 64, 1, 4, 3, LOAD_DMA, 4, 1, "128x256x64_w1x4_s3_f4")      \
+  X(DT, OP, 128, 128, 64, 2, 2, 4, LOAD_DMA, 4, 1, "128x128x64_w2x2_s4_f4")      \
+  X(DT, OP, 256, 64, 64, 4, 1, 3, LOAD_DMA, 4, 1, "256x64x64_w4x1_s3_f4")        \
+  X(DT, OP, 128, 64, 64, 2, 2, 4, LOAD_DMA, 4, 1, "128x64x64_w2x2_s4_f4")        \
+  X(DT, OP, 64, 128, 64, 2, 2, 4, LOAD_DMA, 4, 1, "64x128x64_w2x2_s4_f4")        \
+  X(DT, OP, 64, 64, 128, 2, 2, 4, LOAD_DMA, 4, 1, "64x64x128_w2x2_s4_f4")        \
+  X(DT, OP, 256, 128, 64, 2, 2, 2, LOAD_DMA, 0, 1, "256x128x64_w2x2_s2")         \
+  X(DT, OP, 128, 256, 64, 1, 4, 2, LOAD_DMA, 0, 1, "128x256x64_w1x4_s2")         \
+  X(DT, OP, 128, 128, 64, 2, 2, 4, LOAD_DMA, 0, 1, "128x128x64_w2x2_s4")         \
+  X(DT, OP, 256, 64, 64, 4, 1, 2, LOAD_DMA, 0, 1, "256x64x64_w4x1_s2")           \
+  X(DT, OP, 64, 64, 64, 2, 2, 4, LOAD_DMA, 0, 1, "64x64x64_w2x2_s4")             \
+  X(DT, OP, 256, 128, 64, 2, 2, 2, LOAD_GATHER, 4, 1, "256x128x64_w2x2_gather") \
+  X(DT, OP, 128, 128, 64, 2, 2, 2, LOAD_GATHER, 4, 1, "128x128x64_w2x2_gather") \
+  X(DT, OP, 256, 64, 64, 4, 1, 2, LOAD_GATHER, 4, 1, "256x64x64_w4x1_gather")   \
+  X(DT, OP, 64, 128, 64, 2, 2, 2, LOAD_GATHER, 4, 1, "64x128x64_w2x2_gather")   \
+  X(DT, OP, 64, 64, 128, 2, 2, 2, LOAD_GATHER, 4, 1, "64x64x128_w2x2_gather")   \
+  X(DT, OP, 64, 64, 32, 2, 2, 1, LOAD_GENERIC, 0, 0, "64x64x32_w2x2_generic")
 
 // extra variants, compiled for the bf16 store op only (tuning runs, and the
 // one-substep stage whose fragment buffers alternate from step to step)
 #define IRIS_GEMM_TUNING_VARIANTS(X, DT, OP)                              \
-  X(DT, OP, 256, 128, 32, 2, 4, 4, true, 0, 0, "256x128x32_w2x4_s4")         \
-  X(DT, OP, 256, 128, 64, 2, 4, 2, true, 0, 1, "256x128x64_w2x4_s2")         \
-  X(DT, OP, 128, 256, 64, 2, 4, 2, true, 0, 1, "128x256x64_w2x4_s2")         \
-  X(DT, OP, 128, 128, 32, 2, 2, 4, true, 0, 0, "128x128x32_w2x2_s4")         \
-  X(DT, OP, 64, 64, 64, 2, 2, 4, true, 4, 1, "64x64x64_w2x2_s4_f4")          \
-  X(DT, OP, 256, 64, 64, 4, 1, 2, true, 4, 1, "256x64x64_w4x1_s2_f4")
+  X(DT, OP, 256, 128, 32, 2, 4, 4, LOAD_DMA, 0, 0, "256x128x32_w2x4_s4")         \
+  X(DT, OP, 256, 128, 64, 2, 4, 2, LOAD_DMA, 0, 1, "256x128x64_w2x4_s2")         \
+  X(DT, OP, 128, 256, 64, 2, 4, 2, LOAD_DMA, 0, 1, "128x256x64_w2x4_s2")         \
+  X(DT, OP, 128, 128, 32, 2, 2, 4, LOAD_DMA, 0, 0, "128x128x32_w2x2_s4")         \
+  X(DT, OP, 64, 64, 64, 2, 2, 4, LOAD_DMA, 4, 1, "64x64x64_w2x2_s4_f4")          \
+  X(DT, OP, 256, 64, 64, 4, 1, 2, LOAD_DMA, 4, 1, "256x64x64_w4x1_s2_f4")
 
 #define IRIS_GEMM_ENTRY(DT, OP, CM, CN, BK, WM, WN, S, DMA, LW, SPLIT, NAME) \
   make_entry<GemmCfg<DT, CM, CN, BK, WM, WN, S, DMA, LW>, OP>(NAME),
@@ -157,6 +167,7 @@ constexpr GemmKernelEntry make_entry(const char* name) {
 // the store epilogues' build with the one-shot reduce inside the program
 #define IRIS_GEMM_INSTANTIATE_FUSED(DT, OP, CM, CN, BK, WM, WN, S, DMA, LW, SPLIT, NAME) \
   IRIS_GEMM_INSTANTIATE_FUSED_##LW(DT, OP, CM, CN, BK, WM, WN, S, DMA)
+// (the gathering tiles' fused builds are instantiated by the table entries)
 #define IRIS_GEMM_INSTANTIATE_FUSED_0(DT, OP, CM, CN, BK, WM, WN, S, DMA)                     \
   template __global__ void gemm_persistent_kernel<GemmCfg<DT, CM, CN, BK, WM, WN, S, DMA>, OP, \
                                                   IRIS_GEMM_ODT(DT, OP), false, true>(const GemmKArgs);
@@ -187,15 +198,15 @@ constexpr GemmKernelEntry make_entry(const char* name) {
 template <class Cfg, int OP>
 constexpr GemmKernelEntry make_entry_f32(const char* name) {
   static_assert(Cfg::DT == IRIS_DTYPE_F32 && (OP == OP_STORE32 || OP == OP_ATOMIC32), "fp32 operands, fp32 output");
-  return GemmKernelEntry{Cfg::DT, OP, Cfg::CM, Cfg::CN, Cfg::BK, Cfg::WM, Cfg::WN, Cfg::S, Cfg::DMA, false, false,
+  return GemmKernelEntry{Cfg::DT, OP, Cfg::CM, Cfg::CN, Cfg::BK, Cfg::WM, Cfg::WN, Cfg::S, Cfg::DMA, Cfg::GATHER, false, false,
                          Cfg::THREADS, Cfg::LW, Cfg::LDS_BYTES, &gemm_persistent_kernel<Cfg, OP, IRIS_DTYPE_F32, false>,
                          nullptr, fused_fn<Cfg, OP, IRIS_DTYPE_F32>(), nullptr, nullptr, nullptr, nullptr, name};
 }
 #define IRIS_GEMM_F32_VARIANTS(X, OP)                                                   \
-  X(IRIS_DTYPE_F32, OP, 128, 128, 64, 2, 2, 4, true, 4, "128x128x32_w2x2_s4_f4_fp32")  \
-  X(IRIS_DTYPE_F32, OP, 128, 128, 64, 2, 2, 4, true, 0, "128x128x32_w2x2_s4_fp32")     \
-  X(IRIS_DTYPE_F32, OP, 64, 64, 64, 2, 2, 4, true, 0, "64x64x32_w2x2_s4_fp32")         \
-  X(IRIS_DTYPE_F32, OP, 64, 64, 32, 2, 2, 1, false, 0, "64x64x16_w2x2_generic_fp32")
+  X(IRIS_DTYPE_F32, OP, 128, 128, 64, 2, 2, 4, LOAD_DMA, 4, "128x128x32_w2x2_s4_f4_fp32")  \
+  X(IRIS_DTYPE_F32, OP, 128, 128, 64, 2, 2, 4, LOAD_DMA, 0, "128x128x32_w2x2_s4_fp32")     \
+  X(IRIS_DTYPE_F32, OP, 64, 64, 64, 2, 2, 4, LOAD_DMA, 0, "64x64x32_w2x2_s4_fp32")         \
+  X(IRIS_DTYPE_F32, OP, 64, 64, 32, 2, 2, 1, LOAD_GENERIC, 0, "64x64x16_w2x2_generic_fp32")
 #define IRIS_GEMM_F32_ENTRY(DT, OP, CM, CN, BK, WM, WN, S, DMA, LW, NAME) \
   make_entry_f32<GemmCfg<DT, CM, CN, BK, WM, WN, S, DMA, LW>, OP>(NAME),
 #define IRIS_GEMM_F32_INSTANTIATE(DT, OP, CM, CN, BK, WM, WN, S, DMA, LW, NAME)                    \
