@@ -284,6 +284,26 @@ __device__ inline void store_through(IRIS_GLOBAL T* p, T v, bool sys) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// 16 (8) bytes written through at any address, 2-byte aligned ones included (the memory pipeline takes them).  AUX:
+// AUX_SC1 (agent) or AUX_SC0 | AUX_SC1 (system).  The compiler has no such store with a cache policy; s_nop is the
+// wait state it would leave before the data registers may be written again.
+template <int AUX>
+__device__ inline void store16_any(IRIS_GLOBAL char* p, u32x4 v) {
+  static_assert(AUX == AUX_SC1 || AUX == (AUX_SC0 | AUX_SC1), "written through");
+  if constexpr (AUX == AUX_SC1)
+    asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 0" ::"v"(p), "v"(v) : "memory");
+  else
+    asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 0" ::"v"(p), "v"(v) : "memory");
+}
+template <int AUX>
+__device__ inline void store8_any(IRIS_GLOBAL char* p, u32x2 v) {
+  static_assert(AUX == AUX_SC1 || AUX == (AUX_SC0 | AUX_SC1), "written through");
+  if constexpr (AUX == AUX_SC1)
+    asm volatile("global_store_dwordx2 %0, %1, off sc1\n\ts_nop 0" ::"v"(p), "v"(v) : "memory");
+  else
+    asm volatile("global_store_dwordx2 %0, %1, off sc0 sc1\n\ts_nop 0" ::"v"(p), "v"(v) : "memory");
+}
+
 // CAS(expected -> desired) with acquire; returns the old value
 // (tl.atomic_cas semantics, iris/iris.py:476-497).
 __device__ inline int flag_cas_acquire(IRIS_GLOBAL int32_t* p, int expected, int desired, bool sys) {

@@ -151,6 +151,8 @@ struct GemmKArgs {
   int stagger_groups, stagger_sleeps;
   // (LOAD_GATHER tiles) the operand's rows (A) / columns (B) are contiguous in memory rather than its k
   int a_across, b_across;
+  // rows of `out` are contiguous, at whatever alignment (vec_out: and 16-byte aligned)
+  int row_out;
 };
 
 template <int DT>
@@ -480,7 +482,9 @@ struct Loader {
 // stored); a 16-byte load that would cross the end of its line is moved back to end there and shifted into place;
 // k past K is zeroed, in the one K-step that can hold any.
 // Bound by the fetching waves' issue and LDS writes, a step of 128 x 128 x 64 takes as long as the DMA's.
-template <class Cfg, bool IS_A>
+// (Which operand and which direction are template parameters: with both directions' loads in one program, the
+// compiler, which must count the loads in flight on either path, waits for all of them at every join.)
+template <class Cfg, bool IS_A, bool ACROSS>
 struct Gather {
   static constexpr int ROWS = IS_A ? Cfg::CM : Cfg::CN;
   static constexpr bool F32 = Cfg::DT == IRIS_DTYPE_F32;
@@ -492,14 +496,13 @@ struct Gather {
   // blocks of EPC k x 8 rows over two waves (a slab of fewer than 128 blocks leaves the second wave idle)
   static constexpr int BLOCKS = (ROWS / 8 * Cfg::CPR + 127) / 128;
   static constexpr bool HALF_IDLE = ROWS / 8 * Cfg::CPR < 128;
-  static constexpr int NV = ALONG > 8 * BLOCKS ? ALONG : 8 * BLOCKS;
+  static constexpr int NV = ACROSS ? 8 * BLOCKS : ALONG;
 
   const IRIS_GLOBAL char* base;  // the tile's rows of the operand at k = 0
   int64_t ld;                    // bytes from one row (along k) or one k (across) to the next
-  uint32_t off[ALONG];           // along k: byte offset of each chunk at k0 = 0; across: of each block
+  uint32_t off[ACROSS ? BLOCKS : ALONG];  // along k: byte offset of each chunk at k0 = 0; across: of each block
   int back[BLOCKS];              // across: elements the block's loads are moved back from the operand's edge
   bool edge;                     // some block of the tile is (wave-uniform)
-  bool across;
 
   u32x4 v[SETS][NV];
   // `back` and `edge` of the tile a set's loads belong to: the load cursor may be in the next tile when it is stored
@@ -511,17 +514,19 @@ struct Gather {
   // A scalar address that the compiler takes as it is: base in scalar registers, a 32-bit lane offset per load.  (Left
   // to itself it turns the loads of a K loop into 64-bit pointers per lane, two registers each and an addition a step.)
   __device__ static inline const IRIS_GLOBAL char* scalar(const IRIS_GLOBAL char* p) {
-    asm volatile("" : "+s"(p));
-    return p;
+    uint64_t u = uniform_u64((uint64_t)p);
+    asm volatile("" : "+s"(u));
+    return (const IRIS_GLOBAL char*)u;
   }
   // 128-bit right shift by n 16-bit units, 0 <= n; zero from eight on
   __device__ static inline u32x4 shift_right(u32x4 x, int n) {
-    if (n & 4) x = u32x4{x[2], x[3], 0u, 0u};
-    if (n & 2) x = u32x4{x[1], x[2], x[3], 0u};
-    if (n & 1)
-      x = u32x4{(x[0] >> 16) | (x[1] << 16), (x[1] >> 16) | (x[2] << 16), (x[2] >> 16) | (x[3] << 16), x[3] >> 16};
-    if (n >= 8) x = u32x4{0u, 0u, 0u, 0u};
-    return x;
+    const u32x4 zero = {0u, 0u, 0u, 0u};
+    x = n & 4 ? u32x4{x[2], x[3], 0u, 0u} : x;
+    x = n & 2 ? u32x4{x[1], x[2], x[3], 0u} : x;
+    const unsigned int sh = n & 1 ? 16 : 0;  // (v_alignbit_b32: 32 bits of a pair of words from bit `sh` on)
+    x = u32x4{__builtin_amdgcn_alignbit(x[1], x[0], sh), __builtin_amdgcn_alignbit(x[2], x[1], sh),
+              __builtin_amdgcn_alignbit(x[3], x[2], sh), x[3] >> sh};
+    return n >= 8 ? zero : x;
   }
   // block `i` of this lane across k: k block kb and rows 8 nb ..
   __device__ static inline void block_of(int i, int half, int lane, int* kb, int* nb) {
@@ -534,12 +539,11 @@ struct Gather {
 
   __device__ inline void setup(const GemmKArgs& p, const Item& it, int fwave, int lane) {
     const int half = fwave & 1;
-    across = (IS_A ? p.a_across : p.b_across) != 0;
     edge = false;
-    ld = (across ? (IS_A ? p.sak : p.sbk) : (IS_A ? p.sam : p.sbn)) * 2;
+    ld = (ACROSS ? (IS_A ? p.sak : p.sbk) : (IS_A ? p.sam : p.sbn)) * 2;
     const int row0 = IS_A ? it.m0 : it.n0, extent = IS_A ? p.M : p.N;
-    base = (const IRIS_GLOBAL char*)(IS_A ? p.a : p.b) + (across ? 0 : (int64_t)min(row0, extent - 1) * ld);
-    if (!across) {
+    base = (const IRIS_GLOBAL char*)(IS_A ? p.a : p.b) + (ACROSS ? 0 : (int64_t)min(row0, extent - 1) * ld);
+    if constexpr (!ACROSS) {
 #pragma unroll
       for (int i = 0; i < ALONG; ++i) {
         const int row = (i * 2 + half) * Cfg::RPB + lane / Cfg::CPR;
@@ -569,18 +573,25 @@ struct Gather {
       for (int i = 0; i < NV; ++i) v[SET][i] = u32x4{0u, 0u, 0u, 0u};
       return;
     }
-    if (!across) {
+    if constexpr (!ACROSS) {
       const IRIS_GLOBAL char* src = scalar(base + (int64_t)k * (Cfg::BK * 2));
-#pragma unroll
-      for (int i = 0; i < ALONG; ++i) {
-        if constexpr (TAIL) {
+      if constexpr (TAIL) {
+        // (all loads first, then the shifts: a load at a time, a K of a few steps waits longer for this one than for
+        // all the others)
+        auto over = [&](int i) {  // 16-bit units of chunk i past K
           const int row = (i * 2 + half) * Cfg::RPB + lane / Cfg::CPR;
           const int ch = (lane % Cfg::CPR) ^ ((row / Cfg::RP) % Cfg::CPR);
-          const int over = max(0, k * Cfg::BK + ch * 8 + 8 - K);  // 16-bit units past K
-          v[SET][i] = shift_right(load16(src + ((int64_t)off[i] - over * 2)), over);  // (stays inside the row: K >= 8)
-        } else {
-          v[SET][i] = load16(src + off[i]);
-        }
+          return max(0, k * Cfg::BK + ch * 8 + 8 - K);
+        };
+        u32x4 x[ALONG];
+#pragma unroll
+        for (int i = 0; i < ALONG; ++i) x[i] = load16(src + ((int64_t)off[i] - over(i) * 2));  // (inside the row: K >= 8)
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < ALONG; ++i) v[SET][i] = shift_right(x[i], over(i));
+      } else {
+#pragma unroll
+        for (int i = 0; i < ALONG; ++i) v[SET][i] = load16(src + off[i]);
       }
     } else {
       set_edge[SET] = edge;
@@ -616,51 +627,51 @@ struct Gather {
   __device__ inline void store(IRIS_LDS char* stage, int fwave, int lane) {
     IRIS_LDS char* slab = stage + (IS_A ? 0 : Cfg::A_BYTES);
     const int half = fwave & 1;
-    if (!across) {
+    if constexpr (!ACROSS) {
 #pragma unroll
       for (int i = 0; i < ALONG; ++i)
         *reinterpret_cast<IRIS_LDS u32x4*>(slab + (i * 2 + half) * 1024 + lane * 16) = v[SET][i];
-      return;
+    } else {
+      if (HALF_IDLE && half != 0) return;
+#pragma unroll
+      for (int i = 0; i < BLOCKS; ++i) {
+        int kb, nb;
+        block_of(i, half, lane, &kb, &nb);
+        u32x4 x[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) x[j] = v[SET][i * 8 + j];
+        if (set_edge[SET]) {
+          // (moved back by `back` elements; what lies past the operand's edge is never stored)
+          if constexpr (F32) {
+            // the block's 8 rows as two loads: shift them together, 32 bytes, by whole elements
+#pragma unroll
+            for (int j = 0; j < 8; j += 2)
+#pragma unroll
+              for (int b = 1; b < 8; b *= 2) {
+                const unsigned int w[8] = {x[j][0], x[j][1], x[j][2], x[j][3], x[j + 1][0], x[j + 1][1], x[j + 1][2], x[j + 1][3]};
+                if (set_back[SET][i] & b)
+#pragma unroll
+                  for (int e = 0; e < 8; ++e) x[j + e / 4][e % 4] = e + b < 8 ? w[e + b] : 0u;
+              }
+          } else {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) x[j] = shift_right(x[j], set_back[SET][i]);
+          }
+        }
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+          const int row = nb * 8 + r;
+          u32x4 y;
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            if constexpr (F32)
+              y[q] = x[2 * q + r / 4][r % 4];
+            else  // k 2q and 2q + 1 of row r: the low or the high halves of two dwords
+              y[q] = __builtin_amdgcn_perm(x[2 * q + 1][r / 2], x[2 * q][r / 2], r & 1 ? 0x07060302u : 0x05040100u);
+          }
+          *reinterpret_cast<IRIS_LDS u32x4*>(slab + row * (Cfg::BK * 2) + (kb ^ ((row / Cfg::RP) % Cfg::CPR)) * 16) = y;
+        }
     }
-    if (HALF_IDLE && half != 0) return;
-#pragma unroll
-    for (int i = 0; i < BLOCKS; ++i) {
-      int kb, nb;
-      block_of(i, half, lane, &kb, &nb);
-      u32x4 x[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) x[j] = v[SET][i * 8 + j];
-      if (set_edge[SET]) {
-        // (moved back by `back` elements; what lies past the operand's edge is never stored)
-        if constexpr (F32) {
-          // the block's 8 rows as two loads: shift them together, 32 bytes, by whole elements
-#pragma unroll
-          for (int j = 0; j < 8; j += 2)
-#pragma unroll
-            for (int b = 1; b < 8; b *= 2) {
-              const unsigned int w[8] = {x[j][0], x[j][1], x[j][2], x[j][3], x[j + 1][0], x[j + 1][1], x[j + 1][2], x[j + 1][3]};
-              if (set_back[SET][i] & b)
-#pragma unroll
-                for (int e = 0; e < 8; ++e) x[j + e / 4][e % 4] = e + b < 8 ? w[e + b] : 0u;
-            }
-        } else {
-#pragma unroll
-          for (int j = 0; j < 8; ++j) x[j] = shift_right(x[j], set_back[SET][i]);
-        }
-      }
-#pragma unroll
-      for (int r = 0; r < 8; ++r) {
-        const int row = nb * 8 + r;
-        u32x4 y;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          if constexpr (F32)
-            y[q] = x[2 * q + r / 4][r % 4];
-          else  // k 2q and 2q + 1 of row r: the low or the high halves of two dwords
-            y[q] = __builtin_amdgcn_perm(x[2 * q + 1][r / 2], x[2 * q][r / 2], r & 1 ? 0x07060302u : 0x05040100u);
-        }
-        *reinterpret_cast<IRIS_LDS u32x4*>(slab + row * (Cfg::BK * 2) + (kb ^ ((row / Cfg::RP) % Cfg::CPR)) * 16) = y;
-      }
     }
   }
 };
@@ -925,6 +936,33 @@ __device__ __attribute__((always_inline)) inline bool store_acc(const GemmKArgs&
               }
 #pragma unroll
               for (int t = 0; t < NV; ++t) __builtin_amdgcn_raw_buffer_store_b128(v[t], rs, off[t], 0, AUX);
+            }
+          } else if ((OP == OP_STORE16 || OP == OP_STORE32) && p.row_out) {
+            // ragged edge or unaligned rows: 16 bytes a lane at any address, what is left of a row by elements.
+            // (element by element throughout, 32 round trips to LDS instead of 4 a block and rank, the epilogue of
+            // [1000,1500] x [1500,999] in 256 x 64 tiles on two ranks took half of the launch's 47 us)
+            if constexpr (OP == OP_STORE16 || OP == OP_STORE32) {
+#pragma nounroll
+              for (int t = 0; t < 32 * Cfg::U16 / 64; ++t) {
+                const int row = t * (64 / Cfg::U16) + lane / Cfg::U16, u = lane % Cfg::U16;
+                const int m = row0 + row, n = col0 + u * EPV;
+                if (m >= m_end || n >= n_end) continue;
+                const IRIS_LDS char* src = ws + row * Cfg::WS_PITCH + (u ^ ((row / Cfg::ERPB) % Cfg::U16)) * 16;
+                IRIS_GLOBAL char* d = dst + ((int64_t)m * p.som + n) * ES;
+                if (n + EPV <= n_end) {
+                  store16_any<AUX>(d, *reinterpret_cast<const IRIS_LDS u32x4*>(src));
+                } else {
+#pragma nounroll
+                  for (int e = 0; e < n_end - n; ++e) {
+                    if constexpr (OP == OP_STORE32)
+                      store_through((IRIS_GLOBAL unsigned int*)(d + e * 4),
+                                    *reinterpret_cast<const IRIS_LDS unsigned int*>(src + e * 4), p.sys != 0);
+                    else
+                      store_through((IRIS_GLOBAL unsigned short*)(d + e * 2),
+                                    *reinterpret_cast<const IRIS_LDS unsigned short*>(src + e * 2), p.sys != 0);
+                  }
+                }
+              }
             }
           } else {
             // ragged edge or unaligned destination: element by element
@@ -1208,6 +1246,23 @@ __device__ inline void slice_epilogue(const GemmKArgs& p, const Item& it, int sl
 #pragma unroll
         for (int u = 0; u < UN; ++u) {
           if (ooff[u] != DEAD_OFFSET) continue;
+          if constexpr (OP == OP_STORE32 || OP == OP_STORE16) {
+            if (p.row_out && ncols[u] == 4) {  // a whole strip of an unaligned row
+              IRIS_GLOBAL char* d = dst + ((int64_t)row[u] * p.som + col[u]) * ES;
+              auto whole = [&](auto aux_tag) __attribute__((always_inline)) {
+                constexpr int AUX = decltype(aux_tag)::value;
+                if constexpr (OP == OP_STORE32)
+                  store16_any<AUX>(d, __builtin_bit_cast(u32x4, sum[u]));
+                else
+                  store8_any<AUX>(d, u32x2{pack2<ODT>(sum[u][0], sum[u][1]), pack2<ODT>(sum[u][2], sum[u][3])});
+              };
+              if (p.sys)
+                whole(std::integral_constant<int, 17>{});
+              else
+                whole(std::integral_constant<int, 16>{});
+              continue;
+            }
+          }
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             if (e >= ncols[u]) continue;
@@ -1347,10 +1402,10 @@ __device__ inline void fused_reduce_tile(const GemmKArgs& p, const Item& it, int
 // (gemm_one_shot_all_reduce.py:197-271): store the partial tile, signal the
 // other ranks, wait for the tile's own flag, reduce it over all ranks and
 // store the result, tile by tile, while other programs are in their K loops.
-// ROLE: which waves the code is for.  The gathering tiles compile it three times, for the multiplying waves and for the
-// two that fetch either operand, so that none holds registers for another's state (the accumulators here, two register sets of a slab
+// ROLE: which waves the code is for.  The gathering tiles compile it for the multiplying waves and for those that
+// fetch either operand in either direction, so that none holds registers for another's state (the accumulators here, two register sets of a slab
 // there); the control flow is the same, so every barrier is still met by all.
-enum WaveRole { ROLE_ANY = 0, ROLE_WORKER = 1, ROLE_FETCH_A = 2, ROLE_FETCH_B = 3 };
+enum WaveRole { ROLE_ANY, ROLE_WORKER, ROLE_FETCH_A, ROLE_FETCH_A_ACROSS, ROLE_FETCH_B, ROLE_FETCH_B_ACROSS };
 template <class Cfg, int OP, int ODT, bool SPLIT, bool FUSED, bool MERGED, int ROLE>
 __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKArgs& p) {
   static_assert(!MERGED || !FUSED, "blocks of the caller's tiles: no build with the reduce inside");
@@ -1705,7 +1760,9 @@ __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKAr
     // (LOAD_GATHER: a tile's steps are walked in pairs, one register set each; an odd number of steps gets one more
     // that holds nothing.  The load cursor runs three steps ahead: two in registers, one on its way into a stage.)
     constexpr int AHEAD = Cfg::GATHER ? 1 + 2 : Cfg::S;
-    std::conditional_t<Cfg::GATHER, Gather<Cfg, ROLE == ROLE_FETCH_A>, Loader<Cfg>> ld;
+    std::conditional_t<Cfg::GATHER, Gather<Cfg, ROLE == ROLE_FETCH_A || ROLE == ROLE_FETCH_A_ACROSS,
+                                             ROLE == ROLE_FETCH_A_ACROSS || ROLE == ROLE_FETCH_B_ACROSS>,
+                       Loader<Cfg>> ld;
     int l_item = 0, l_k = 0, l_kend = nk;  // load cursor
     int l_klive = 0;                       // (LOAD_GATHER) end of the cursor's real steps
     Item l_it;
@@ -1911,9 +1968,11 @@ __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKAr
         if constexpr (Cfg::LW != 0) {
           // every wave is past its reads of stage g: refill it with step g+S
           if (fetcher) {
-            if constexpr (Cfg::GATHER)
+            if constexpr (Cfg::GATHER) {
               gather(set_tag, lean_tag);
-            else
+              // (the other set's stores, which wait for their own loads, stay behind these)
+              __builtin_amdgcn_sched_barrier(0);
+            } else
               ld.issue(p, rstage, l_k, fwave);
             if constexpr (LEAN)
               ++l_k;
@@ -2079,12 +2138,19 @@ __global__ __launch_bounds__(Cfg::THREADS) __attribute__((amdgpu_waves_per_eu(Cf
 gemm_persistent_kernel(const GemmKArgs p) {
   if constexpr (Cfg::GATHER) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (wave < Cfg::NW)
+    if (wave < Cfg::NW) {
       gemm_program<Cfg, OP, ODT, SPLIT, FUSED, MERGED, ROLE_WORKER>(p);
-    else if (wave < Cfg::NW + 2)
-      gemm_program<Cfg, OP, ODT, SPLIT, FUSED, MERGED, ROLE_FETCH_A>(p);
-    else
-      gemm_program<Cfg, OP, ODT, SPLIT, FUSED, MERGED, ROLE_FETCH_B>(p);
+    } else if (wave < Cfg::NW + 2) {
+      if (p.a_across)
+        gemm_program<Cfg, OP, ODT, SPLIT, FUSED, MERGED, ROLE_FETCH_A_ACROSS>(p);
+      else
+        gemm_program<Cfg, OP, ODT, SPLIT, FUSED, MERGED, ROLE_FETCH_A>(p);
+    } else {
+      if (p.b_across)
+        gemm_program<Cfg, OP, ODT, SPLIT, FUSED, MERGED, ROLE_FETCH_B_ACROSS>(p);
+      else
+        gemm_program<Cfg, OP, ODT, SPLIT, FUSED, MERGED, ROLE_FETCH_B>(p);
+    }
   } else {
     gemm_program<Cfg, OP, ODT, SPLIT, FUSED, MERGED, ROLE_ANY>(p);
   }

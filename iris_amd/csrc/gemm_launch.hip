@@ -622,6 +622,7 @@ hipError_t make_plan_body(const iris_gemm_args& a, Plan* plan) {
   k.num_pid_n = (a.N + a.block_n - 1) / a.block_n;
   k.total_tiles = k.num_pid_m * k.num_pid_n;
   k.sys = a.scope == IRIS_SCOPE_SYSTEM;
+  k.row_out = k.son == 1;
   k.vec_out = vec_ok(k.out, k.som, k.son, dtype_size(out_dt)) ? 1 : 0;
   if (plan->in_program) {
     // 16-byte strips in the in-program reduce: aligned rows on both sides, tile
