@@ -68,11 +68,20 @@ def _headers():
     return list(CSRC.glob("*.hpp")) + [inc / "iris_amd.h", inc / "iris_amd_testing.h", inc / "iris_device.hpp"]
 
 
+def _included(obj: Path):
+    """The files an object was compiled from, as the compiler listed them beside it; every header where it has not."""
+    listed = obj.with_suffix(".d")
+    if not listed.exists():
+        return _headers()
+    words = listed.read_text().replace("\\\n", " ").split()
+    return [p for p in map(Path, words[1:]) if not str(p).startswith("/opt/")]
+
+
 def _stale(target: Path, deps) -> bool:
     if not target.exists():
         return True
     t = target.stat().st_mtime
-    return any(d.stat().st_mtime > t for d in deps)
+    return any(not d.exists() or d.stat().st_mtime > t for d in deps)
 
 
 def _run(cmd):
@@ -99,7 +108,6 @@ def _build_host_module() -> None:
 def build(force: bool = False, jobs: int | None = None, verbose: bool = True) -> None:
     cc = hipcc()
     OBJ.mkdir(parents=True, exist_ok=True)
-    hdrs = _headers()
     jobs = jobs or min(8, os.cpu_count() or 1)
 
     todo = []
@@ -108,12 +116,12 @@ def build(force: bool = False, jobs: int | None = None, verbose: bool = True) ->
         for src in sources:
             obj = OBJ / (src.stem + ".o")
             into.append(obj)
-            if force or _stale(obj, [src] + hdrs):
+            if force or _stale(obj, [src] + _included(obj)):
                 todo.append((src, obj))
 
     def compile_one(item):
         src, obj = item
-        _run([cc, *COMMON, "-c", str(src), "-o", str(obj)])
+        _run([cc, *COMMON, "-MMD", "-MF", str(obj.with_suffix(".d")), "-c", str(src), "-o", str(obj)])
         return src.name
 
     if todo:

@@ -207,9 +207,8 @@ __device__ inline __amdgpu_buffer_rsrc_t tile_rsrc(const IRIS_GLOBAL char* base,
   return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, (int)bytes, 0x00020000);
 }
 
-template <int DT, int AUX>
-__device__ inline void load_vec(__amdgpu_buffer_rsrc_t rs, uint32_t off, float (&v)[Vec<DT>::N]) {
-  const u32x4 x = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off, 0, AUX);
+template <int DT>
+__device__ inline void unpack_vec(u32x4 x, float (&v)[Vec<DT>::N]) {
   if constexpr (DT == IRIS_DTYPE_F32) {
     // cast the whole vector: a bit_cast of one element reads element 0
     const f32x4 f = __builtin_bit_cast(f32x4, x);
@@ -219,6 +218,19 @@ __device__ inline void load_vec(__amdgpu_buffer_rsrc_t rs, uint32_t off, float (
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] = from16<DT>((unsigned short)(x[e / 2] >> (16 * (e & 1))));
   }
+}
+
+template <int DT, int AUX>
+__device__ inline void load_vec(__amdgpu_buffer_rsrc_t rs, uint32_t off, float (&v)[Vec<DT>::N]) {
+  unpack_vec<DT>(__builtin_amdgcn_raw_buffer_load_b128(rs, (int)off, 0, AUX), v);
+}
+// acc (+)= the 16 bytes `x` as elements of type DT; `first`: acc starts at +0
+template <int DT>
+__device__ inline void add_vec(bool first, u32x4 x, float (&acc)[Vec<DT>::N]) {
+  float v[Vec<DT>::N];
+  unpack_vec<DT>(x, v);
+#pragma unroll
+  for (int e = 0; e < Vec<DT>::N; ++e) acc[e] = (first ? 0.f : acc[e]) + v[e];
 }
 
 // store NE fp32 values as elements of type DT

@@ -37,11 +37,14 @@ struct ReduceKArgs {
   // an acquire fence at the flags' scope after every flag wait, as the reference's sem="acquire" (the loads are
   // coherent at that scope by themselves and need none)
   int acquire;
+  // flat kernel: items of the matrix taken as one array (band_items counts them), and the division of an element's
+  // index by N
+  FastDiv div_n;
 };
 
-// The row-band kernel counts its finished groups in the upper half of the
-// first tile's flag (a producer's +1 only ever touches the lower half), so a
-// flag's value is its lower half.
+// The row-band and flat kernels count their finished groups in the upper half
+// of the first tile's flag (a producer's +1 only ever touches the lower half),
+// so a flag's value is its lower half.
 constexpr int FLAG_COUNT_SHIFT = 16, FLAG_VALUE_MASK = 0xFFFF;
 
 // Block-wide wait for one tile's flag.  One lane polls; the outcome is
@@ -154,6 +157,222 @@ __global__ __launch_bounds__(256) void reduce_tiles_vec_kernel(const ReduceKArgs
       }
     }
   }
+}
+
+// This group is past all its waits.  Groups count themselves on the upper half of flags[0]; the one that counts last
+// knows that nobody polls any more and takes every flag that reached ws-1 back to 0, which is what the consumer's
+// CAS(ws-1 -> 0) leaves (gemm_one_shot_all_reduce.py:228-234).  The count comes off with one atomic per flag, so a
+// +1 of the next round that lands meanwhile is kept.  (Spread over sixteen flags, the count takes as long.)
+__device__ inline void reset_by_last_group(const ReduceKArgs& p, IRIS_LDS int* last) {
+  const int tid = threadIdx.x;
+  if (tid == 0) {
+    // (at the flags' scope, like the producers' increments of the same word)
+    const int before = p.sys ? __hip_atomic_fetch_add((IRIS_GLOBAL int32_t*)p.flags, 1 << FLAG_COUNT_SHIFT,
+                                                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM)
+                             : __hip_atomic_fetch_add((IRIS_GLOBAL int32_t*)p.flags, 1 << FLAG_COUNT_SHIFT,
+                                                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    *last = (before >> FLAG_COUNT_SHIFT) == (int)gridDim.x - 1 ? 1 : 0;
+  }
+  __syncthreads();
+  if (!*last) return;
+  const int consumed = p.ws - 1;
+  for (int t = tid; t < p.total_tiles; t += 256) {
+    IRIS_GLOBAL int32_t* f = (IRIS_GLOBAL int32_t*)(p.flags + t);
+    const int v = p.sys ? __hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM)
+                        : __hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    int take = (v & FLAG_VALUE_MASK) >= consumed ? consumed : 0;
+    if (t == 0) take += (int)gridDim.x << FLAG_COUNT_SHIFT;  // the groups' count, too
+    if (take) flag_add_relaxed(f, -take, p.sys != 0);
+  }
+}
+
+// Flat kernel, for matrices without gaps between their rows (what the wrappers allocate): the partials and the result
+// are arrays, a lane's strip is 16 bytes of an array wherever its rows begin, and an item is 256 K consecutive
+// strips.  Rows of any length, odd ones included, are read as one wide stream, and the items can be made as small as
+// a small matrix needs to occupy the chip (K = 1: one strip a lane, all ranks' in flight together).
+// Bound by HBM at K = 8, by the chain of latencies (flag, bases, partials, result, reset) at K = 1.  Measured against
+// the tile walk, fill of the flags included: 4 x bf16 [8192,4096] 88 -> 55 us (6.1 TB/s), 8 x fp32 [2048,4096] 60 -> 45,
+// 4 x fp32 [2314,128] in 256 x 256 tiles 34 -> 7.3; against the element-wise kernel: 8 x fp32 [777,1111] 212 -> 10.
+//
+// Flags: an item waits for every tile its rows cross (its columns only, when it lies inside one row) without
+// consuming them; the flags go back to 0 as in the row-band kernel.  When one does not arrive within the timeout the
+// item goes element by element and leaves that tile's elements alone.
+//
+// STREAM, for launches of many items: a lane keeps two loads in flight where it could keep dozens.  HBM likes that
+// better: 8 x fp32 [8192,8192] with 1 / 2 / 3 / 4 / 8 / 12 loads ahead 382 / 359 / 366 / 375 / 386 / 388 us, two groups a
+// CU (477, 376 and 382 with one, three and four); 8 x bf16 213 -> 190.  A launch of one or two items a group has
+// latencies to cover instead: 8 x fp32 [512,4096] 21.0 us two ahead, 17.6 eight ahead.
+template <int IN_DT, int OUT_DT, int LAUX, int WS, int K, bool STREAM = false>
+__global__ __launch_bounds__(256) void reduce_flat_kernel(const ReduceKArgs p) {
+  static_assert(!STREAM || K % 4 == 0, "the ring of strips in flight");
+  constexpr int IES = Vec<IN_DT>::ES, VE = Vec<IN_DT>::N, OES = Vec<OUT_DT>::ES;
+  constexpr int SAUX = (LAUX & AUX_SC0) ? (AUX_SC0 | AUX_SC1) : AUX_SC1;
+  constexpr uint32_t ITEM = 256u * K * VE;  // elements
+  __shared__ int slot;
+  const int tid = threadIdx.x;
+  const uint64_t cur_base = p.heap_bases ? uniform_u64(heap_base_at(p.heap_bases, p.cur_rank)) : 0;
+  const bool wait = p.wait_flags && p.ws > 1;
+  const uint32_t total = (uint32_t)p.M * (uint32_t)p.N;  // (the launcher keeps it below 2^31)
+  auto rank_c = [&](int rk) __attribute__((always_inline)) {
+    return (rk == p.cur_rank || !p.heap_bases) ? (const IRIS_GLOBAL char*)p.c
+                                               : translate(p.c, cur_base, uniform_u64(heap_base_at(p.heap_bases, rk)));
+  };
+  const IRIS_GLOBAL char* src[WS > 0 ? WS : 1];
+  if constexpr (WS > 0) {
+#pragma unroll
+    for (int rk = 0; rk < WS; ++rk) src[rk] = rank_c(rk);
+  }
+  auto sum_element = [&](uint32_t e) __attribute__((always_inline)) {
+    float acc = 0.f;
+    for (int rk = 0; rk < p.ws; ++rk) {
+      const IRIS_GLOBAL char* s = rank_c(rk) + (int64_t)e * IES;
+      if constexpr (IN_DT == IRIS_DTYPE_F32) {
+        const unsigned int w =
+            p.sys ? __hip_atomic_load((const IRIS_GLOBAL unsigned int*)s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM)
+                  : __hip_atomic_load((const IRIS_GLOBAL unsigned int*)s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        acc += __builtin_bit_cast(float, w);
+      } else {
+        const unsigned short h =
+            p.sys ? __hip_atomic_load((const IRIS_GLOBAL unsigned short*)s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM)
+                  : __hip_atomic_load((const IRIS_GLOBAL unsigned short*)s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        acc += from16<IN_DT>(h);
+      }
+    }
+    IRIS_GLOBAL char* d = (IRIS_GLOBAL char*)p.cg + (int64_t)e * OES;
+    if constexpr (OUT_DT == IRIS_DTYPE_F32)
+      store_through((IRIS_GLOBAL unsigned int*)d, __builtin_bit_cast(unsigned int, acc), p.sys != 0);
+    else
+      store_through((IRIS_GLOBAL unsigned short*)d, to16<OUT_DT>(acc), p.sys != 0);
+  };
+
+  for (int item = blockIdx.x; item < p.band_items; item += gridDim.x) {
+    const uint32_t e0 = (uint32_t)item * ITEM, e1 = min(e0 + ITEM, total);
+    bool all = true;
+    if (wait) {
+      const int r0 = (int)fast_div(e0, p.div_n), r1 = (int)fast_div(e1 - 1, p.div_n);
+      const bool one_row = r0 == r1;
+      const int t0 = one_row ? (int)(e0 - (uint32_t)r0 * p.N) / p.BN : 0;
+      const int t1 = one_row ? (int)(e1 - 1 - (uint32_t)r0 * p.N) / p.BN : p.num_pid_n - 1;
+      const int m0 = r0 / p.BM, width = t1 - t0 + 1, count = width * (r1 / p.BM - m0 + 1);
+      int ok = 1;
+      for (int i = tid; i < count; i += 256) {
+        const int dm = i / width;
+        const int t = tile_id_of(m0 + dm, t0 + i - dm * width, p.num_pid_m, p.num_pid_n, p.G);
+        ok &= wait_tile_ready((IRIS_GLOBAL int32_t*)(p.flags + t), p.ws - 1, p.sys != 0, p.timeout, p.status, FLAG_VALUE_MASK)
+                  ? 1
+                  : 0;
+      }
+      all = __syncthreads_and(ok) != 0;
+      if (p.acquire) {
+        if (p.sys)
+          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "");
+        else
+          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+      }
+    }
+    if (!all) {
+      for (uint32_t e = e0 + tid; e < e1; e += 256) {
+        const int r = (int)(e / (uint32_t)p.N), t = tile_id_of(r / p.BM, (int)(e - (uint32_t)r * p.N) / p.BN, p.num_pid_m,
+                                                               p.num_pid_n, p.G);
+        const IRIS_GLOBAL int32_t* f = (const IRIS_GLOBAL int32_t*)(p.flags + t);
+        const int v = p.sys ? __hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM)
+                            : __hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if ((v & FLAG_VALUE_MASK) >= p.ws - 1) sum_element(e);
+      }
+      continue;
+    }
+    // whole strips through descriptors that end with the last one; what is left of the array by elements
+    const uint32_t strips = (e1 - e0) / VE;
+    auto rsrc = [&](const IRIS_GLOBAL char* base) __attribute__((always_inline)) {
+      return tile_rsrc(base + (int64_t)e0 * IES, strips * 16);
+    };
+    uint32_t off[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) off[k] = (uint32_t)(k * 256 + tid) * 16;  // (past the last strip: reads zero, stores nothing)
+    float acc[K][VE];
+    if constexpr (STREAM) {
+      // strip after strip, rank after rank, each lane two loads ahead of its additions and not more
+      u32x4 v[4];
+      auto fetch = [&](const IRIS_GLOBAL char* base, int t) __attribute__((always_inline)) {
+        v[t % 4] = __builtin_amdgcn_raw_buffer_load_b128(rsrc(base), (int)off[t % K], 0, LAUX);
+      };
+      const int ranks = WS > 0 ? WS : p.ws;
+      const IRIS_GLOBAL char* next = WS > 0 ? src[0] : rank_c(0);
+      fetch(next, 0);
+      fetch(next, 1);
+#pragma unroll
+      for (int rk = 0; rk < (WS > 0 ? WS : 1 << 30); ++rk) {
+        if (WS == 0 && rk >= ranks) break;
+        const IRIS_GLOBAL char* cur = next;
+        if constexpr (WS > 0)
+          next = src[rk + 1 < WS ? rk + 1 : rk];
+        else
+          next = rk + 1 < ranks ? rank_c(rk + 1) : cur;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+          if (k + 2 < K)
+            fetch(cur, k + 2);
+          else if (rk + 1 < ranks)
+            fetch(next, k + 2);
+          __builtin_amdgcn_sched_barrier(0);
+          add_vec<IN_DT>(rk == 0, v[k % 4], acc[k]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    } else if constexpr (WS > 0 && WS * K <= 32) {
+      u32x4 v[WS][K];
+#pragma unroll
+      for (int rk = 0; rk < WS; ++rk) {
+        const __amdgpu_buffer_rsrc_t rs = rsrc(src[rk]);
+#pragma unroll
+        for (int k = 0; k < K; ++k) v[rk][k] = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off[k], 0, LAUX);
+      }
+#pragma unroll
+      for (int rk = 0; rk < WS; ++rk)
+#pragma unroll
+        for (int k = 0; k < K; ++k) add_vec<IN_DT>(rk == 0, v[rk][k], acc[k]);
+    } else {
+      // ranks two at a time, the next one's strips in flight while one's are added
+      u32x4 v[2][K];
+      auto base = [&](int rk) __attribute__((always_inline)) {
+        if constexpr (WS > 0)
+          return src[rk];
+        else
+          return rank_c(rk);
+      };
+      auto fetch = [&](int rk, u32x4 (&to)[K]) __attribute__((always_inline)) {
+        const __amdgpu_buffer_rsrc_t rs = rsrc(base(rk));
+#pragma unroll
+        for (int k = 0; k < K; ++k) to[k] = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off[k], 0, LAUX);
+      };
+      auto add = [&](bool first, const u32x4 (&from)[K]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < K; ++k) add_vec<IN_DT>(first, from[k], acc[k]);
+      };
+      fetch(0, v[0]);
+      if constexpr (WS > 0) {
+#pragma unroll
+        for (int rk = 0; rk < WS; ++rk) {
+          if (rk + 1 < WS) fetch(rk + 1, v[(rk + 1) & 1]);
+          add(rk == 0, v[rk & 1]);
+        }
+      } else {
+        for (int rk = 0; rk < p.ws; rk += 2) {
+          if (rk + 1 < p.ws) fetch(rk + 1, v[1]);
+          add(rk == 0, v[0]);
+          if (rk + 1 < p.ws) {
+            if (rk + 2 < p.ws) fetch(rk + 2, v[0]);
+            add(false, v[1]);
+          }
+        }
+      }
+    }
+    const __amdgpu_buffer_rsrc_t out_rs = tile_rsrc((const IRIS_GLOBAL char*)p.cg + (int64_t)e0 * OES, strips * VE * OES);
+#pragma unroll
+    for (int k = 0; k < K; ++k) store_vec<OUT_DT, VE, SAUX>(out_rs, off[k] / 16 * (VE * OES), acc[k]);
+    for (uint32_t e = e0 + strips * VE + tid; e < e1; e += 256) sum_element(e);
+  }
+  if (wait && p.reset_in_kernel) reset_by_last_group(p, (IRIS_LDS int*)&slot);
 }
 
 // Row-band kernel, for matrices whose rows are long.  The tile kernel above
@@ -302,34 +521,7 @@ __global__ __launch_bounds__(256) void reduce_rows_kernel(const ReduceKArgs p) {
     for (int k = 0; k < K; ++k) store_vec<OUT_DT, VE, SAUX>(out_rs, ooff[k], acc[k]);
     if (wait) __syncthreads();  // `ready` is rewritten for the next item
   }
-  if (wait && p.reset_in_kernel) {
-    // This group is past all its waits.  Groups count themselves on the upper
-    // half of flags[0]; the one that counts last knows that nobody polls any
-    // more and takes every flag that reached ws-1 back to 0, which is what the
-    // consumer's CAS(ws-1 -> 0) leaves (gemm_one_shot_all_reduce.py:228-234).
-    // The count comes off with one atomic per flag, so a +1 of the next round
-    // that lands meanwhile is kept.
-    if (tid == 0) {
-      // (at the flags' scope, like the producers' increments of the same word)
-      const int before = p.sys ? __hip_atomic_fetch_add((IRIS_GLOBAL int32_t*)p.flags, 1 << FLAG_COUNT_SHIFT,
-                                                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM)
-                               : __hip_atomic_fetch_add((IRIS_GLOBAL int32_t*)p.flags, 1 << FLAG_COUNT_SHIFT,
-                                                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      ready[0] = (before >> FLAG_COUNT_SHIFT) == (int)gridDim.x - 1 ? 1 : 0;
-    }
-    __syncthreads();
-    if (ready[0]) {
-      const int consumed = p.ws - 1;
-      for (int t = tid; t < p.total_tiles; t += 256) {
-        IRIS_GLOBAL int32_t* f = (IRIS_GLOBAL int32_t*)(p.flags + t);
-        const int v = p.sys ? __hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM)
-                            : __hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        int take = (v & FLAG_VALUE_MASK) >= consumed ? consumed : 0;
-        if (t == 0) take += (int)gridDim.x << FLAG_COUNT_SHIFT;  // the groups' count, too
-        if (take) flag_add_relaxed(f, -take, p.sys != 0);
-      }
-    }
-  }
+  if (wait && p.reset_in_kernel) reset_by_last_group(p, (IRIS_LDS int*)ready);
 }
 
 // Flags that the row-band kernel has consumed (value ws-1) back to 0, as the

@@ -57,6 +57,42 @@ ReduceFn pick(int in_dt, int out_dt, int ws, int variant, bool sys, bool rows) {
   return nullptr;
 }
 
+// The flat kernel for (element types, ranks, strips a lane, streaming).
+template <int IN_DT, int OUT_DT, int LAUX, int K, bool STREAM>
+ReduceFn pick_flat_ranks(int ws) {
+  switch (ws) {
+    case 2: return &reduce_flat_kernel<IN_DT, OUT_DT, LAUX, 2, K, STREAM>;
+    case 4: return &reduce_flat_kernel<IN_DT, OUT_DT, LAUX, 4, K, STREAM>;
+    case 8: return &reduce_flat_kernel<IN_DT, OUT_DT, LAUX, 8, K, STREAM>;
+    default: return &reduce_flat_kernel<IN_DT, OUT_DT, LAUX, 0, K, STREAM>;
+  }
+}
+template <int IN_DT, int OUT_DT>
+ReduceFn pick_flat(int ws, bool sys, int strips, bool stream) {
+  constexpr int AGENT = AUX_NT | AUX_SC1, SYSTEM = AUX_NT | AUX_SC1 | AUX_SC0;
+  if (sys)  // (partials of other devices: bound by the links)
+    return strips == 1 ? &reduce_flat_kernel<IN_DT, OUT_DT, SYSTEM, 0, 1> : &reduce_flat_kernel<IN_DT, OUT_DT, SYSTEM, 0, 8>;
+  return stream        ? pick_flat_ranks<IN_DT, OUT_DT, AGENT, 8, true>(ws)
+         : strips == 1 ? pick_flat_ranks<IN_DT, OUT_DT, AGENT, 1, false>(ws)
+         : strips == 4 ? pick_flat_ranks<IN_DT, OUT_DT, AGENT, 4, false>(ws)
+                       : pick_flat_ranks<IN_DT, OUT_DT, AGENT, 8, false>(ws);
+}
+ReduceFn pick_flat(int in_dt, int out_dt, int ws, bool sys, int strips, bool stream) {
+  if (in_dt == IRIS_DTYPE_F32) {
+    if (out_dt == IRIS_DTYPE_BF16) return pick_flat<IRIS_DTYPE_F32, IRIS_DTYPE_BF16>(ws, sys, strips, stream);
+    if (out_dt == IRIS_DTYPE_F16) return pick_flat<IRIS_DTYPE_F32, IRIS_DTYPE_F16>(ws, sys, strips, stream);
+    return pick_flat<IRIS_DTYPE_F32, IRIS_DTYPE_F32>(ws, sys, strips, stream);
+  }
+  if (in_dt == IRIS_DTYPE_BF16) {
+    if (out_dt == IRIS_DTYPE_BF16) return pick_flat<IRIS_DTYPE_BF16, IRIS_DTYPE_BF16>(ws, sys, strips, stream);
+    if (out_dt == IRIS_DTYPE_F32) return pick_flat<IRIS_DTYPE_BF16, IRIS_DTYPE_F32>(ws, sys, strips, stream);
+    return nullptr;
+  }
+  if (out_dt == IRIS_DTYPE_F16) return pick_flat<IRIS_DTYPE_F16, IRIS_DTYPE_F16>(ws, sys, strips, stream);
+  if (out_dt == IRIS_DTYPE_F32) return pick_flat<IRIS_DTYPE_F16, IRIS_DTYPE_F32>(ws, sys, strips, stream);
+  return nullptr;
+}
+
 bool valid_dtype(int dt) { return dt == IRIS_DTYPE_F32 || dt == IRIS_DTYPE_F16 || dt == IRIS_DTYPE_BF16; }
 
 }  // namespace
@@ -139,15 +175,39 @@ extern "C" int iris_one_shot_reduce_launch(const iris_reduce_args* a, void* stre
     rows = fits && (a->variant == 7 ||
                     (a->variant == 0 && (int64_t)k.N * ies >= 16384 && k.band_items >= current_cu_count()));
   }
+  // Without gaps between the rows: the matrices as arrays.  In items of eight strips a lane where they give one to
+  // every CU (8 x fp32 [512,4096]: 16.7 us, 18.2 in items of four, the fill of the flags included), of four down to a
+  // quarter of that (128 rows: 11.9, 8.9, 11.9 in items of eight, four, one), else of one, for the sake of the loads
+  // in flight (16 rows: 10.7, 8.4, 7.0).  With so few, and a tile for each of them, the tile walk has no count of
+  // finished groups to wait for (6.8).  Partials that are
+  // three times what the last-level cache (256 MB) holds come from HBM and are streamed; smaller ones may just have
+  // been produced, and a cache gives more to who asks for more (4 ranks' reduces of 4 x bf16 [8192,4096] behind their
+  // producers: 55 us each with all ranks' loads in flight, 66 streamed).
+  ReduceFn flat = nullptr;
+  const int64_t elems = (int64_t)k.M * k.N, groups = (elems + 256 * ve - 1) / (256 * ve);
+  const int cus = current_cu_count();
+  if (a->variant == 0 && k.scn == 1 && k.sgn == 1 && k.scm == k.N && k.sgm == k.N && aligned16(k.c) && aligned16(k.cg) &&
+      elems < ((int64_t)1 << 31) && !(vec && groups < cus && groups <= k.total_tiles)) {
+    int strips = groups >= 8 * cus ? 8 : groups >= cus ? 4 : 1;
+    if (k.sys && strips == 4) strips = 8;
+    flat = pick_flat(k.c_dt, k.cg_dt, k.ws, k.sys != 0, strips,
+                     groups * 4096 * k.ws >= ((int64_t)768 << 20));
+    if (flat) {
+      rows = false;
+      k.band_items = (int)((groups + strips - 1) / strips);
+      k.div_n = make_fast_div((uint32_t)k.N, (uint64_t)elems + 1);
+    }
+  }
   // (the tile kernel paces its walk only when a program has several tiles)
   k.pace = k.total_tiles > grid ? 1 : 0;
-  ReduceFn fn = vec ? pick(k.c_dt, k.cg_dt, k.ws, a->variant, k.sys != 0, rows) : nullptr;
+  ReduceFn fn = flat ? flat : vec ? pick(k.c_dt, k.cg_dt, k.ws, a->variant, k.sys != 0, rows) : nullptr;
   if (!fn) {
     fn = &reduce_tiles_generic_kernel;
     rows = false;
   }
+  if (flat) rows = true;  // (flags are reset as the row bands' are)
   if (rows) {
-    grid = a->num_sms > 0 ? a->num_sms : 2 * current_cu_count();
+    grid = a->num_sms > 0 ? a->num_sms : 2 * cus;
     if (grid > k.band_items) grid = k.band_items;
   }
   // (the groups' count shares a 32-bit flag with a value below 2^16)

@@ -153,3 +153,42 @@ def test_signal_include_self_and_memset(shmem):
     iris_amd.memset_tensor(big[3:4999], -2)
     torch.cuda.synchronize()
     assert big.cpu().tolist() == [0, 0, 0] + [-2] * 4996 + [0]
+
+
+@pytest.mark.parametrize("in_dt,out_dt,ws,M,N,BM,BN,grid", [
+    (torch.float32, torch.bfloat16, 8, 3, 11, 64, 64, 0),           # fewer elements than a group has lanes
+    (torch.bfloat16, torch.bfloat16, 4, 17, 268, 16, 64, 0),        # items of one strip that cross rows and tile rows
+    (torch.float16, torch.float16, 2, 1001, 999, 256, 64, 0),       # odd rows, items of four strips, a tail of 7 elements
+    (torch.float32, torch.float32, 3, 1030, 1021, 128, 128, 0),     # a rank count without a kernel of its own
+    (torch.bfloat16, torch.bfloat16, 8, 4099, 1024, 256, 256, 0),   # items of eight strips, ranks streamed
+    (torch.float32, torch.float16, 4, 2051, 1028, 256, 128, 7),     # ... all ranks in flight, several items a group
+    (torch.bfloat16, torch.float32, 2, 64, 16640, 64, 64, 0),       # items inside a row: its columns' flags only
+])
+@pytest.mark.parametrize("scope", [ops.SCOPE_AGENT, ops.SCOPE_SYSTEM])
+def test_matrices_without_gaps_are_reduced_as_arrays(shmem, in_dt, out_dt, ws, M, N, BM, BN, grid, scope):
+    """Bit-exact, nothing past the result's end, every flag consumed; then with
+    one tile's flag missing: its elements alone are left as they were."""
+    c = shmem.zeros((M, N), dtype=in_dt)
+    flat = shmem.full((M * N + 64,), 3, dtype=out_dt)
+    cg = flat[:M * N].view(M, N)
+    total = ops.cdiv(M, BM) * ops.cdiv(N, BN)
+    flags = shmem.zeros((total,), dtype=torch.int32)
+    status = torch.zeros(1, dtype=torch.int32, device="cuda")
+    host = fill_partials(shmem, c, ws, seed=M * 5 + N)
+    want = O.one_shot_reduce(host, out_dt)
+    args = (c, cg, flags, shmem.get_heap_bases(), 0, ws, BM, BN, 4)
+    flags.fill_(ws - 1)
+    ops.one_shot_reduce(*args, num_sms=grid, scope=scope, status=status)
+    torch.cuda.synchronize()
+    assert torch.equal(cg.cpu(), want) and bool((flat[M * N:] == 3).all())
+    assert not flags.any() and int(status.item()) == 0
+    cg.fill_(3)
+    flags.fill_(ws - 1)
+    missing = total // 2
+    flags[missing] = 0
+    ops.one_shot_reduce(*args, num_sms=grid, scope=scope, status=status, spin_timeout_ticks=1000)
+    torch.cuda.synchronize()
+    pm, pn = ops.tile_map_host(missing, M, N, BM, BN, 4)
+    want = want.clone()
+    want[pm * BM:(pm + 1) * BM, pn * BN:(pn + 1) * BN] = 3
+    assert torch.equal(cg.cpu(), want) and not flags.any() and int(status.item()) == 1
