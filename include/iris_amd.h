@@ -88,8 +88,10 @@ int iris_hip_arch_name(int device, char* buf, size_t len);
 /* phases of IRIS_EPI_ONE_SHOT (bit mask) */
 #define IRIS_PHASE_PRODUCE 1 /* store partial tile + signal the other ranks  (:197-218) */
 #define IRIS_PHASE_CONSUME 2 /* wait for the tile's flag, reduce, store       (:220-271) */
-#define IRIS_PHASE_FUSED 3   /* both, in one program and tile by tile, as the reference kernel: every rank's
-                              * launch must be on its device at the same time (a program waits for its peers) */
+#define IRIS_PHASE_FUSED 3   /* both: every rank's launch must be on its device at the same time (it waits for its
+                              * peers).  In one program and tile by tile, as the reference kernel, where that is the
+                              * faster form or the launch has fewer programs than the device has CUs; else as
+                              * IRIS_PHASE_TWO_KERNELS.  Results and flags are the same. */
 #define IRIS_PHASE_TWO_KERNELS 7 /* both, as two kernels on the stream: the producer GEMM, then the reduce kernel
                                   * (iris_one_shot_reduce_launch) behind it */
 
@@ -258,7 +260,8 @@ int iris_gemm_split_k(const iris_gemm_args* args, int* split_k);
  * caller's tiles as one (each tile keeps its own id and flag), and by
  * "+last_round_in_N_parts" where a second launch shares K of the last round's
  * tiles out over the programs that round would leave idle (needs partials and
- * locks). */
+ * locks), and by "+kernel+reduce" where an IRIS_PHASE_FUSED launch reduces in
+ * a kernel behind the producer rather than inside it. */
 int iris_gemm_plan_name(const iris_gemm_args* args, char* buf, size_t len);
 
 /* Name of tuning variant `variant` (1-based) of the kernel list used for

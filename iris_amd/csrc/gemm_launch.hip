@@ -61,6 +61,7 @@ struct Plan {
   GemmKArgs k{};
   int fused_reduce = 0;  // ONE_SHOT, CONSUME on its own or IRIS_PHASE_TWO_KERNELS: follow with the reduce kernel
   int in_program = 0;    // ONE_SHOT, IRIS_PHASE_FUSED: the build of the kernel that reduces each tile itself
+  int two_kernels = 0;   // ... or, for such a launch too, producer and reduce as two kernels (reduce_in_program)
   // the few-rows kernel instead of a table entry, one workgroup per 16 columns
   GemmKernelFn skinny = nullptr;
   int skinny_grid = 0, skinny_grid_y = 1, skinny_lds = 0;
@@ -476,7 +477,37 @@ hipError_t make_plan(const iris_gemm_args& a, Plan* plan) {
   return make_plan_units(b, plan);
 }
 
+// Whether a launch of IRIS_PHASE_FUSED is better off reducing inside the program than behind it, `producer` being the
+// plan of the same launch without the reduce.  Inside, a tile is one program's from its first K-step to its last
+// strip: K is not shared out, the caller's tiles are not blocked, the fetching waves' registers are not there, and
+// CUs whose tiles are done do not help with the others' reduces.  Behind, a kernel boundary is paid, 4 us.  So inside
+// for one round of small tiles with a short K, whose producer would run the same way (K-shard [785,216] x [216,2752],
+// 8 fp32 partials, 256 x 64 tiles: 27.8 against 30.7 us; 64^3 10 against 13); behind otherwise ([1999,1376] x
+// [1376,4096] in 256 x 128 tiles 68 against 55 us, in two rounds of 256 x 256 tiles 200 against 175, 25 tiles of
+// K = 29408 838 against 106).  A launch that shares the device with its peers' (fewer programs than CUs) stays inside:
+// every program's CU is counted there.
+bool reduce_in_program(const iris_gemm_args& a, const Plan& producer) {
+  if (a.num_sms < current_cu_count() || a.variant != 0 || a.split_k != 0 || a.mm_begin_timestamp || a.mm_end_timestamp) return true;
+  if (!producer.entry && !producer.skinny) return true;  // (nothing to compute)
+  if (producer.skinny || producer.last_round || producer.rest) return false;
+  const GemmKArgs& k = producer.k;
+  if (k.split_k > 1 || k.merge_m * k.merge_n > 1 || k.total_tiles > a.num_sms || !k.vec_out) return false;
+  const int steps = (a.K + 63) / 64;
+  return steps <= 8 || (steps <= 24 && a.block_m * a.block_n <= 128 * 128);
+}
+
 hipError_t make_plan_units(const iris_gemm_args& a, Plan* plan) {
+  if (a.epilogue == IRIS_EPI_ONE_SHOT && a.phase == IRIS_PHASE_FUSED) {
+    iris_gemm_args b = a;
+    b.phase = IRIS_PHASE_TWO_KERNELS;
+    Plan behind;
+    if (a.split_k <= 1 && a.split_k != IRIS_GEMM_SPLIT_STREAM_K && make_plan_units(b, &behind) == hipSuccess &&
+        !reduce_in_program(a, behind)) {
+      *plan = behind;
+      plan->two_kernels = 1;
+      return hipSuccess;
+    }
+  }
   const bool plain = a.variant == 0 && a.split_k == 0 && !a.mm_begin_timestamp && !a.mm_end_timestamp &&
                      !(a.epilogue == IRIS_EPI_ONE_SHOT && a.phase != IRIS_PHASE_PRODUCE) &&
                      a.epilogue != IRIS_EPI_ATOMIC_ADD && a.num_sms > 0 && (a.block_m == 128 || a.block_m == 256) &&
@@ -776,7 +807,9 @@ iris_reduce_args reduce_args_from(const iris_gemm_args& a) {
   r.block_m = a.block_m;
   r.block_n = a.block_n;
   r.group_size_m = a.group_size_m;
-  r.num_sms = a.num_sms;
+  // A launch that owns the device leaves the reduce its own grid, two groups a CU: with one (num_sms programs) HBM is
+  // not kept busy (8 x fp32 [8192,8192] 477 us instead of 359).
+  r.num_sms = a.num_sms >= current_cu_count() ? 0 : a.num_sms;
   r.num_xcds = a.num_xcds;
   r.cur_rank = a.cur_rank;
   r.world_size = a.world_size;
@@ -1036,6 +1069,10 @@ extern "C" int iris_gemm_plan_name(const iris_gemm_args* args, char* buf, size_t
   if (plan.rest) {
     const size_t n = std::strlen(buf);
     std::snprintf(buf + n, len > n ? len - n : 0, "+last_%d_columns_apart", plan.rest->k.N);
+  }
+  if (plan.two_kernels) {
+    const size_t n = std::strlen(buf);
+    std::snprintf(buf + n, len > n ? len - n : 0, "+kernel+reduce");
   }
   return hipSuccess;
 }
