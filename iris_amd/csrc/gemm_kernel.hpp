@@ -183,8 +183,11 @@ struct Mfma<IRIS_DTYPE_F32> {
   using vec8 = f32x4;
   __device__ static inline f32x4 run(vec8 a, vec8 b, f32x4 c) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], c, 0, 0, 0);
+    for (int e = 0; e < 4; ++e) c = part(a, b, c, e);
     return c;
+  }
+  __device__ static inline f32x4 part(vec8 a, vec8 b, f32x4 c, int e) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], c, 0, 0, 0);
   }
 };
 
@@ -760,6 +763,17 @@ __device__ inline void load_all(const IRIS_LDS char* sA, const IRIS_LDS char* sB
 // FIRST: the block's first product of a tile, which defines the accumulator.
 template <class Cfg, bool FIRST>
 __device__ inline void mma_row(f32x4 (&acc)[Cfg::IM][Cfg::IN], const Frags<Cfg>& f, int cb, int i) {
+  if constexpr (Cfg::DT == IRIS_DTYPE_F32) {
+    // the four products of a block add to one accumulator: the row's blocks in turn, so that none waits for its last
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int j = 0; j < Cfg::IN; ++j) {
+        const f32x4 z = {0, 0, 0, 0};
+        acc[i][j] = Mfma<Cfg::DT>::part(f.b[cb][j], f.a[i], FIRST && e == 0 ? z : acc[i][j], e);
+      }
+    return;
+  }
 #pragma unroll
   for (int j = 0; j < Cfg::IN; ++j) {
     if constexpr (FIRST) {
@@ -1267,8 +1281,9 @@ __device__ inline void slice_epilogue(const GemmKArgs& p, const Item& it, int sl
           for (int e = 0; e < 4; ++e) {
             if (e >= ncols[u]) continue;
             IRIS_GLOBAL char* d = dst + ((int64_t)row[u] * p.som + (int64_t)(col[u] + e) * p.son) * ES;
+            const float f = sum[u][e];  // (a bit cast of the element itself reads element 0)
             if constexpr (OP == OP_STORE32)
-              store_through((IRIS_GLOBAL unsigned int*)d, __builtin_bit_cast(unsigned int, sum[u][e]), p.sys != 0);
+              store_through((IRIS_GLOBAL unsigned int*)d, __builtin_bit_cast(unsigned int, f), p.sys != 0);
             else if constexpr (OP == OP_STORE16)
               store_through((IRIS_GLOBAL unsigned short*)d, to16<ODT>(sum[u][e]), p.sys != 0);
             else if constexpr (OP == OP_ATOMIC32)

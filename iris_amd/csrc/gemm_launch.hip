@@ -38,6 +38,28 @@ const GemmKernelEntry* entries_for(int dt, int op, int* count) {
   return nullptr;
 }
 
+// Tiles behind the table (`variant` does not number them): the fp32 ones for a K of at least LONG_STEPS of their
+// K-steps, the gathering ones.
+constexpr int LONG_STEPS = 8;
+const GemmKernelEntry* more_entries_for(int dt, int op, int* count) {
+  *count = 0;
+  switch (op) {
+    case OP_STORE16:
+      return dt == IRIS_DTYPE_BF16 ? gemm_entries_bf16_store16_gather(count) : gemm_entries_f16_store16_gather(count);
+    case OP_STORE32:
+      return dt == IRIS_DTYPE_F32    ? gemm_entries_f32_store32_long(count)
+             : dt == IRIS_DTYPE_BF16 ? gemm_entries_bf16_store32_gather(count)
+                                     : gemm_entries_f16_store32_gather(count);
+    case OP_ATOMIC32:
+      return dt == IRIS_DTYPE_F32    ? gemm_entries_f32_atomic32_long(count)
+             : dt == IRIS_DTYPE_BF16 ? gemm_entries_bf16_atomic32_gather(count)
+                                     : gemm_entries_f16_atomic32_gather(count);
+    case OP_ATOMIC16:
+      return dt == IRIS_DTYPE_BF16 ? gemm_entries_bf16_atomic16_gather(count) : gemm_entries_f16_atomic16_gather(count);
+  }
+  return nullptr;
+}
+
 // The plain build (every wave fetches its share) of the tile shape of `e`, an
 // entry with fetching waves; null if `e` has none or the list holds no such build.
 const GemmKernelEntry* plain_twin(const GemmKernelEntry* list, int count, const GemmKernelEntry& e) {
@@ -715,8 +737,11 @@ hipError_t make_plan_body(const iris_gemm_args& a, Plan* plan) {
   if (!pick) {
     // first entry whose compute tile divides the logical tile; the rows and
     // columns a small matrix cannot fill are not worth a tall compute tile
-    for (int i = 0; i < count && !pick; ++i) {
-      const GemmKernelEntry& e = list[i];
+    int more = 0;
+    const GemmKernelEntry* more_list = more_entries_for(a.ab_dtype, op, &more);
+    for (int i = 0; i < more + count && !pick; ++i) {
+      const GemmKernelEntry& e = i < more ? more_list[i] : list[i - more];
+      if (i < more && a.ab_dtype == IRIS_DTYPE_F32 && a.K < LONG_STEPS * e.bk) continue;
       // (the gathering tiles are for what the DMA does not take)
       if (!fits(e) || (e.gather && dma_ok)) continue;
       if (plan->in_program && !e.fn_fused) continue;
@@ -735,8 +760,11 @@ hipError_t make_plan_body(const iris_gemm_args& a, Plan* plan) {
       pick = &e;
     }
     // otherwise 64 x 64, with masked sub-tiles: gathered if the operands allow it, else element by element
-    for (int i = 0; i < count && !pick; ++i)
-      if (!list[i].dma && list[i].cm == 64 && list[i].cn == 64 && fits(list[i])) pick = &list[i];
+    for (int i = 0; i < more + count && !pick; ++i) {
+      const GemmKernelEntry& e = i < more ? more_list[i] : list[i - more];
+      if (i < more && a.ab_dtype == IRIS_DTYPE_F32) continue;
+      if (!e.dma && e.cm == 64 && e.cn == 64 && fits(e) && !(plan->in_program && !e.fn_fused)) pick = &e;
+    }
   }
   if (!pick) return hipErrorInvalidValue;
   if (plan->in_program && !pick->fn_fused) return hipErrorInvalidValue;

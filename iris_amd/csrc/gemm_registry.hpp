@@ -113,8 +113,7 @@ constexpr GemmKernelEntry make_entry(const char* name) {
 // where the first loses: with the reduce inside the program (no such build)
 // and for two programs per CU.
 //
-// The `_gather` tiles take what the DMA cannot: operands that lie along K at any alignment, or across it (a row-major
-// B, a column-major A).  The generic tile is left for operands that are contiguous in neither direction.
+// The generic tile is left for operands that are contiguous neither along K nor across it.
 #define IRIS_GEMM_VARIANTS(X, DT, OP)                                     \
   X(DT, OP, 256, 256, 64, 2, 4, 2, LOAD_DMA, 0, 1, "256x256x64_w2x4_s2")         \
   X(DT, OP, 256, 128, 64, 2, 2, 3, LOAD_DMA, 4, 1, "256x128x64_w2x2_s3_f4")      \
@@ -129,12 +128,16 @@ constexpr GemmKernelEntry make_entry(const char* name) {
   X(DT, OP, 128, 128, 64, 2, 2, 4, LOAD_DMA, 0, 1, "128x128x64_w2x2_s4")         \
   X(DT, OP, 256, 64, 64, 4, 1, 2, LOAD_DMA, 0, 1, "256x64x64_w4x1_s2")           \
   X(DT, OP, 64, 64, 64, 2, 2, 4, LOAD_DMA, 0, 1, "64x64x64_w2x2_s4")             \
+  X(DT, OP, 64, 64, 32, 2, 2, 1, LOAD_GENERIC, 0, 0, "64x64x32_w2x2_generic")
+
+// Tiles behind the table, which `variant` does not number.  The `_gather` tiles take what the DMA cannot: operands that
+// lie along K at any alignment, or across it (a row-major B, a column-major A).
+#define IRIS_GEMM_GATHER_VARIANTS(X, DT, OP)                                \
   X(DT, OP, 256, 128, 64, 2, 2, 2, LOAD_GATHER, 4, 1, "256x128x64_w2x2_gather") \
   X(DT, OP, 128, 128, 64, 2, 2, 2, LOAD_GATHER, 4, 1, "128x128x64_w2x2_gather") \
   X(DT, OP, 256, 64, 64, 4, 1, 2, LOAD_GATHER, 4, 1, "256x64x64_w4x1_gather")   \
   X(DT, OP, 64, 128, 64, 2, 2, 2, LOAD_GATHER, 4, 1, "64x128x64_w2x2_gather")   \
-  X(DT, OP, 64, 64, 128, 2, 2, 2, LOAD_GATHER, 4, 1, "64x64x128_w2x2_gather")   \
-  X(DT, OP, 64, 64, 32, 2, 2, 1, LOAD_GENERIC, 0, 0, "64x64x32_w2x2_generic")
+  X(DT, OP, 64, 64, 128, 2, 2, 2, LOAD_GATHER, 4, 1, "64x64x128_w2x2_gather")
 
 // extra variants, compiled for the bf16 store op only (tuning runs, and the
 // one-substep stage whose fragment buffers alternate from step to step)
@@ -167,7 +170,6 @@ constexpr GemmKernelEntry make_entry(const char* name) {
 // the store epilogues' build with the one-shot reduce inside the program
 #define IRIS_GEMM_INSTANTIATE_FUSED(DT, OP, CM, CN, BK, WM, WN, S, DMA, LW, SPLIT, NAME) \
   IRIS_GEMM_INSTANTIATE_FUSED_##LW(DT, OP, CM, CN, BK, WM, WN, S, DMA)
-// (the gathering tiles' fused builds are instantiated by the table entries)
 #define IRIS_GEMM_INSTANTIATE_FUSED_0(DT, OP, CM, CN, BK, WM, WN, S, DMA)                     \
   template __global__ void gemm_persistent_kernel<GemmCfg<DT, CM, CN, BK, WM, WN, S, DMA>, OP, \
                                                   IRIS_GEMM_ODT(DT, OP), false, true>(const GemmKArgs);
@@ -195,18 +197,34 @@ constexpr GemmKernelEntry make_entry(const char* name) {
 // fp32 operands (fp32 output only): a short table.  The tiles are the 16-bit ones' (a stage of BK 16-bit units holds
 // BK / 2 elements of K; the names count elements); the matrix cores run fp32 at a sixteenth of the 16-bit rate, so any
 // tile that keeps them fed will do, and none is split along K or merged.
-template <class Cfg, int OP>
+// (SPLIT: with a split-K build, which only the tiles behind the table have)
+template <class Cfg, int OP, bool SPLIT = false>
 constexpr GemmKernelEntry make_entry_f32(const char* name) {
   static_assert(Cfg::DT == IRIS_DTYPE_F32 && (OP == OP_STORE32 || OP == OP_ATOMIC32), "fp32 operands, fp32 output");
-  return GemmKernelEntry{Cfg::DT, OP, Cfg::CM, Cfg::CN, Cfg::BK, Cfg::WM, Cfg::WN, Cfg::S, Cfg::DMA, Cfg::GATHER, false, false,
+  GemmKernelFn split = nullptr;
+  if constexpr (SPLIT) split = split_fn<Cfg, OP, IRIS_DTYPE_F32>();
+  return GemmKernelEntry{Cfg::DT, OP, Cfg::CM, Cfg::CN, Cfg::BK, Cfg::WM, Cfg::WN, Cfg::S, Cfg::DMA, Cfg::GATHER, SPLIT, SPLIT && Cfg::SPLIT_OWNER,
                          Cfg::THREADS, Cfg::LW, Cfg::LDS_BYTES, &gemm_persistent_kernel<Cfg, OP, IRIS_DTYPE_F32, false>,
-                         nullptr, fused_fn<Cfg, OP, IRIS_DTYPE_F32>(), nullptr, nullptr, nullptr, nullptr, name};
+                         split, fused_fn<Cfg, OP, IRIS_DTYPE_F32>(), nullptr, nullptr, nullptr, nullptr, name};
 }
 #define IRIS_GEMM_F32_VARIANTS(X, OP)                                                   \
   X(IRIS_DTYPE_F32, OP, 128, 128, 64, 2, 2, 4, LOAD_DMA, 4, "128x128x32_w2x2_s4_f4_fp32")  \
   X(IRIS_DTYPE_F32, OP, 128, 128, 64, 2, 2, 4, LOAD_DMA, 0, "128x128x32_w2x2_s4_fp32")     \
   X(IRIS_DTYPE_F32, OP, 64, 64, 64, 2, 2, 4, LOAD_DMA, 0, "64x64x32_w2x2_s4_fp32")         \
   X(IRIS_DTYPE_F32, OP, 64, 64, 32, 2, 2, 1, LOAD_GENERIC, 0, "64x64x16_w2x2_generic_fp32")
+// Tiles behind the fp32 table: the launcher takes them for a K of eight K-steps or more.
+// The scripts' 256 x 64 tile as one compute tile ([2048,1024] x [1024,2048]: as four of 64 x 64, fetch-bound, 131 us;
+// 66 so), split-K builds, and the gathering loader.
+#define IRIS_GEMM_F32_LONG_VARIANTS(X, OP)                                                        \
+  X(IRIS_DTYPE_F32, OP, 128, 128, 64, 2, 2, 4, LOAD_DMA, 4, "128x128x32_w2x2_s4_f4_fp32")        \
+  X(IRIS_DTYPE_F32, OP, 256, 64, 64, 4, 1, 3, LOAD_DMA, 4, "256x64x32_w4x1_s3_f4_fp32")          \
+  X(IRIS_DTYPE_F32, OP, 64, 128, 64, 2, 2, 4, LOAD_DMA, 4, "64x128x32_w2x2_s4_f4_fp32")          \
+  X(IRIS_DTYPE_F32, OP, 64, 64, 128, 2, 2, 4, LOAD_DMA, 4, "64x64x64_w2x2_s4_f4_fp32")           \
+  X(IRIS_DTYPE_F32, OP, 128, 128, 64, 2, 2, 2, LOAD_GATHER, 4, "128x128x32_w2x2_gather_fp32")    \
+  X(IRIS_DTYPE_F32, OP, 256, 64, 64, 4, 1, 2, LOAD_GATHER, 4, "256x64x32_w4x1_gather_fp32")      \
+  X(IRIS_DTYPE_F32, OP, 64, 64, 128, 2, 2, 2, LOAD_GATHER, 4, "64x64x64_w2x2_gather_fp32")
+#define IRIS_GEMM_F32_LONG_ENTRY(DT, OP, CM, CN, BK, WM, WN, S, DMA, LW, NAME) \
+  make_entry_f32<GemmCfg<DT, CM, CN, BK, WM, WN, S, DMA, LW>, OP, true>(NAME),
 #define IRIS_GEMM_F32_ENTRY(DT, OP, CM, CN, BK, WM, WN, S, DMA, LW, NAME) \
   make_entry_f32<GemmCfg<DT, CM, CN, BK, WM, WN, S, DMA, LW>, OP>(NAME),
 #define IRIS_GEMM_F32_INSTANTIATE(DT, OP, CM, CN, BK, WM, WN, S, DMA, LW, NAME)                    \
@@ -218,6 +236,16 @@ constexpr GemmKernelEntry make_entry_f32(const char* name) {
 #define IRIS_GEMM_DECLARE(TAG) const GemmKernelEntry* gemm_entries_##TAG(int* count);
 IRIS_GEMM_DECLARE(f32_store32)
 IRIS_GEMM_DECLARE(f32_atomic32)
+IRIS_GEMM_DECLARE(f32_store32_long)
+IRIS_GEMM_DECLARE(f32_atomic32_long)
+IRIS_GEMM_DECLARE(bf16_store16_gather)
+IRIS_GEMM_DECLARE(bf16_store32_gather)
+IRIS_GEMM_DECLARE(bf16_atomic32_gather)
+IRIS_GEMM_DECLARE(bf16_atomic16_gather)
+IRIS_GEMM_DECLARE(f16_store16_gather)
+IRIS_GEMM_DECLARE(f16_store32_gather)
+IRIS_GEMM_DECLARE(f16_atomic32_gather)
+IRIS_GEMM_DECLARE(f16_atomic16_gather)
 IRIS_GEMM_DECLARE(bf16_store16)
 IRIS_GEMM_DECLARE(bf16_store32)
 IRIS_GEMM_DECLARE(bf16_atomic32)
