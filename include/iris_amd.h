@@ -260,7 +260,8 @@ int iris_gemm_split_k(const iris_gemm_args* args, int* split_k);
  * caller's tiles as one (each tile keeps its own id and flag), and by
  * "+last_round_in_N_parts" where a second launch shares K of the last round's
  * tiles out over the programs that round would leave idle (needs partials and
- * locks), and by "+kernel+reduce" where an IRIS_PHASE_FUSED launch reduces in
+ * locks), by "+parts_of_tiles" where the caller's tiles are computed as several
+ * smaller ones, and by "+kernel+reduce" where an IRIS_PHASE_FUSED launch reduces in
  * a kernel behind the producer rather than inside it. */
 int iris_gemm_plan_name(const iris_gemm_args* args, char* buf, size_t len);
 

@@ -153,6 +153,11 @@ struct GemmKArgs {
   int a_across, b_across;
   // rows of `out` are contiguous, at whatever alignment (vec_out: and 16-byte aligned)
   int row_out;
+  // part_m * part_n > 1 (tiles of up to 128 x 128): the launch's tiles are parts of the caller's, part_m x part_n to
+  // one, numbered over num_pid_m x num_pid_n; the parts of a caller's tile count their arrivals in
+  // tile_arrivals[its id] (all zero between launches), and the last one raises its flag
+  int part_m, part_n;
+  int32_t* tile_arrivals;
 };
 
 template <int DT>
@@ -231,6 +236,8 @@ struct GemmCfg {
   // accumulators are dead once its partial is written.
   static constexpr bool SPLITK = PIPE && KSUB % 2 == 0 && IM * IN * 4 <= 128;
   static constexpr bool SPLIT_OWNER = SPLITK && IM * IN * 4 <= 64;
+  // The launcher may run the tile as a part of the caller's (see GemmKArgs::part_m).
+  static constexpr bool PARTS = CM <= 128 && CN <= 128 && LW != 0;
   // Waves per SIMD the register budget is sized for: 256 registers a wave.
   static constexpr int WPE = 2;
   // wave-private epilogue scratch: 32 rows x TN 16-bit elements
@@ -1024,7 +1031,8 @@ __device__ __attribute__((always_inline)) inline bool store_acc(const GemmKArgs&
 // Lane l takes ranks l, l + 64, ...: the ranks' heap bases come in with one
 // vector load and the increments leave together (one thread walking the ranks
 // waits for a scalar load per rank: 0.8 us for eight).
-template <bool MERGED = false>
+// PARTS: the build may run launches whose tiles are parts of the caller's.
+template <bool MERGED = false, bool PARTS = false>
 __device__ __attribute__((always_inline)) inline void publish_tile(const GemmKArgs& p, int tile_id, int lane) {
   // the caller's tiles the launch's tile covers: itself, or (the MERGED builds, which only run launches whose
   // tiles are blocks of the caller's) merge_m x merge_n of them, fewer at the edges.  A build of its own: the
@@ -1037,6 +1045,22 @@ __device__ __attribute__((always_inline)) inline void publish_tile(const GemmKAr
     pn0 = t.pid_n * p.merge_n + p.flag_pn_base;
     rows = min(p.merge_m, p.flag_num_pid_m - pm0);
     cols = min(p.merge_n, p.flag_num_pid_n - pn0);
+  }
+  if constexpr (PARTS) {
+    if (p.part_m * p.part_n > 1) {
+      const TileCoord t = tile_map_fast(tile_id, p.num_pid_m, p.num_pid_n, p.G, p.tile_divs);
+      const int pm = t.pid_m / p.part_m, pn = t.pid_n / p.part_n;
+      first = tile_id_of(pm, pn, p.flag_num_pid_m, p.flag_num_pid_n, p.G);
+      const int parts = min(p.part_m, p.num_pid_m - pm * p.part_m) * min(p.part_n, p.num_pid_n - pn * p.part_n);
+      // (the group's stores of the part have completed, written through: the part that counts last finds all of them)
+      IRIS_GLOBAL int32_t* cnt = (IRIS_GLOBAL int32_t*)(p.tile_arrivals + first);
+      int last = 0;
+      if (lane == 0) {
+        last = __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == parts - 1;
+        if (last) __hip_atomic_store(cnt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
+      }
+      if (!__builtin_amdgcn_readfirstlane(last)) return;
+    }
   }
   for (int i = 0; i < rows; ++i)
     for (int j = 0; j < cols; ++j) {
@@ -1578,7 +1602,7 @@ __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKAr
       // a one-step tile: the previous tile has not been published yet
       IRIS_WAIT_VMCNT(0);
       __syncthreads();
-      if (wave == 0) publish_tile<MERGED>(p, pending_tile, lane);
+      if (wave == 0) publish_tile<MERGED, Cfg::PARTS>(p, pending_tile, lane);
       pending_tile = -1;
     }
     if constexpr (SPLIT) {
@@ -1653,7 +1677,7 @@ __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKAr
           before = __builtin_amdgcn_readfirstlane(before);
           if (before == parts - 1) {
             // every slice is in memory: publish, and leave both counters at 0
-            if (p.flag_mode != 0) publish_tile<MERGED>(p, c_it.tile_id, lane);
+            if (p.flag_mode != 0) publish_tile<MERGED, Cfg::PARTS>(p, c_it.tile_id, lane);
             if (lane == 0) {
               flag_add_relaxed(done, -parts, false);
               flag_add_relaxed((IRIS_GLOBAL int32_t*)(p.locks + slot0), -parts, false);
@@ -1714,7 +1738,7 @@ __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKAr
         __syncthreads();
         int ok = 1;
         if (p.ws > 1) {
-          if (wave == 0) publish_tile<MERGED>(p, c_it.tile_id, lane);  // +1 on every other rank (:207-218)
+          if (wave == 0) publish_tile<MERGED, Cfg::PARTS>(p, c_it.tile_id, lane);  // +1 on every other rank (:207-218)
           if (tid == 0) {
             *slot = !peers_gone && wait_tile_flag((IRIS_GLOBAL int32_t*)(p.flags + c_it.tile_id), p.ws, p.sys != 0,
                                                   p.timeout, p.status)
@@ -1747,7 +1771,7 @@ __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKAr
       } else if (p.flag_mode != 0) {
         IRIS_WAIT_VMCNT(0);  // this wave's stores of the tile have completed
         __syncthreads();
-        if (wave == 0) publish_tile<MERGED>(p, c_it.tile_id, lane);
+        if (wave == 0) publish_tile<MERGED, Cfg::PARTS>(p, c_it.tile_id, lane);
       }
       if (p.ts_end && tid == 0)
         __hip_atomic_fetch_max((IRIS_GLOBAL unsigned long long*)(p.ts_end + c_it.tile_id),
@@ -1950,7 +1974,7 @@ __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKAr
         if constexpr (!LEAN) {
           if (pend >= 0) {
             if (skip == 0) {
-              if (wave == 0) publish_tile<MERGED>(p, pend, lane);
+              if (wave == 0) publish_tile<MERGED, Cfg::PARTS>(p, pend, lane);
               pending_tile = -1;
             } else {
               pending_skip = 0;
@@ -2144,7 +2168,7 @@ __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKAr
   if (pending_tile >= 0) {
     IRIS_WAIT_VMCNT(0);
     __syncthreads();
-    if (wave == 0) publish_tile<MERGED>(p, pending_tile, lane);
+    if (wave == 0) publish_tile<MERGED, Cfg::PARTS>(p, pending_tile, lane);
   }
 }
 

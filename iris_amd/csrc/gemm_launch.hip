@@ -83,6 +83,7 @@ struct Plan {
   GemmKArgs k{};
   int fused_reduce = 0;  // ONE_SHOT, CONSUME on its own or IRIS_PHASE_TWO_KERNELS: follow with the reduce kernel
   int in_program = 0;    // ONE_SHOT, IRIS_PHASE_FUSED: the build of the kernel that reduces each tile itself
+  int parts = 0;         // the launch's tiles are parts of the caller's (plan_parts)
   int two_kernels = 0;   // ... or, for such a launch too, producer and reduce as two kernels (reduce_in_program)
   // the few-rows kernel instead of a table entry, one workgroup per 16 columns
   GemmKernelFn skinny = nullptr;
@@ -499,6 +500,69 @@ hipError_t make_plan(const iris_gemm_args& a, Plan* plan) {
   return make_plan_units(b, plan);
 }
 
+// A caller's tile is the unit of a flag, not of work: where its tiles are too few for the programs, the launch is
+// planned in parts of them, 64 x 64 or the next larger tile that still gives every part a program of its own in one
+// round.  The parts of a tile count their arrivals in the caller's locks; the last one raises its flag.
+// [1000,1504] x [1504,999] in 256 x 64 tiles: 64 tiles, K in four parts, 21.6 us; 256 parts of 64 x 64, 10.7.
+// [1418,384] x [384,224] in 256 x 256 tiles: 13.9 as 6 tiles, 6.7 as 92 parts.  [627,14528] x [14528,3208] in
+// 128 x 128 tiles: 130 tiles for 256 programs 82.7 us, 255 parts of 128 x 64 69.7.  Only what the few-rows kernel does
+// not take, for a launch that owns the device and leaves tile and split to the launcher.
+bool plan_parts(const iris_gemm_args& a, Plan* plan) {
+  if (a.variant != 0 || a.split_k != 0 || a.mm_begin_timestamp || a.mm_end_timestamp || a.M <= 0 || a.N <= 0 || a.K <= 0) return false;
+  if (a.block_m <= 0 || a.block_n <= 0 || a.num_sms != current_cu_count()) return false;
+  if (a.epilogue == IRIS_EPI_ONE_SHOT && (a.phase == IRIS_PHASE_FUSED || a.phase == IRIS_PHASE_CONSUME)) return false;
+  // (fp32 operands, K in 16-bit units here: the tiles for longer K)
+  if (a.ab_dtype == IRIS_DTYPE_F32 && a.K < 1024) return false;
+  const bool flags = a.epilogue == IRIS_EPI_ALL_SCATTER ? a.notify != 0 : a.epilogue == IRIS_EPI_ONE_SHOT && a.world_size > 1;
+  const int64_t flag_m = (a.M + (int64_t)a.block_m - 1) / a.block_m, flag_n = (a.N + (int64_t)a.block_n - 1) / a.block_n;
+  const int64_t words = flags ? flag_m * flag_n : 0;
+  if (words > 0 && (!a.locks || words > a.num_sms)) return false;
+  static const int shapes[4][2] = {{64, 64}, {128, 64}, {64, 128}, {128, 128}};
+  for (const auto& s : shapes) {
+    const int cm = s[0], cn = s[1];
+    if (a.block_m % cm != 0 || a.block_n % cn != 0) continue;
+    const int64_t tiles = ((a.M + (int64_t)cm - 1) / cm) * ((a.N + (int64_t)cn - 1) / cn);
+    if (tiles > a.num_sms) continue;
+    if (cm == a.block_m && cn == a.block_n) return false;  // (the caller's tile is the smallest that fits)
+    Plan whole;
+    if (make_plan_body(a, &whole) != hipSuccess || whole.skinny) return false;
+    // (a larger part than 64 x 64 only halves or quarters the tile; where K is shared out over as many programs that
+    // has been done)
+    if (cm * cn > 64 * 64 && whole.k.split_k > 1) return false;
+    iris_gemm_args b = a;
+    b.block_m = cm;
+    b.block_n = cn;
+    b.variant = IRIS_GEMM_VARIANT_PERSISTENT;
+    Plan parts;
+    if (make_plan_body(b, &parts) != hipSuccess || !parts.entry) return false;
+    auto fits = [&](const Plan& q) {
+      return q.entry && q.entry->cm == cm && q.entry->cn == cn && q.k.sub_m == 1 && q.k.sub_n == 1 && !q.k.stream_k &&
+             q.entry->fetch_waves > 0 && q.k.num_sms == a.num_sms;
+    };
+    if (!fits(parts)) continue;
+    if (parts.k.split_k > 1 && parts.k.total_tiles * (int64_t)parts.k.split_k + words > a.num_sms) {
+      // (the parts of a part's K use the locks, too)
+      const int64_t sk = (a.num_sms - words) / parts.k.total_tiles;
+      b.split_k = sk >= 2 ? (int)sk : 1;
+      parts = Plan();
+      if (make_plan_body(b, &parts) != hipSuccess || !fits(parts)) continue;
+    }
+    parts.k.merge_m = parts.k.merge_n = 1;
+    parts.k.flag_num_pid_m = (int)flag_m;
+    parts.k.flag_num_pid_n = (int)flag_n;
+    parts.k.flag_pn_base = 0;
+    if (words > 0) {
+      parts.k.part_m = a.block_m / cm;
+      parts.k.part_n = a.block_n / cn;
+      parts.k.tile_arrivals = a.locks + (a.num_sms - words);
+    }
+    parts.parts = 1;
+    *plan = parts;
+    return true;
+  }
+  return false;
+}
+
 // Whether a launch of IRIS_PHASE_FUSED is better off reducing inside the program than behind it, `producer` being the
 // plan of the same launch without the reduce.  Inside, a tile is one program's from its first K-step to its last
 // strip: K is not shared out, the caller's tiles are not blocked, the fetching waves' registers are not there, and
@@ -511,7 +575,7 @@ hipError_t make_plan(const iris_gemm_args& a, Plan* plan) {
 bool reduce_in_program(const iris_gemm_args& a, const Plan& producer) {
   if (a.num_sms < current_cu_count() || a.variant != 0 || a.split_k != 0 || a.mm_begin_timestamp || a.mm_end_timestamp) return true;
   if (!producer.entry && !producer.skinny) return true;  // (nothing to compute)
-  if (producer.skinny || producer.last_round || producer.rest) return false;
+  if (producer.skinny || producer.last_round || producer.rest || producer.parts) return false;
   const GemmKArgs& k = producer.k;
   if (k.split_k > 1 || k.merge_m * k.merge_n > 1 || k.total_tiles > a.num_sms || !k.vec_out) return false;
   const int steps = (a.K + 63) / 64;
@@ -530,6 +594,7 @@ hipError_t make_plan_units(const iris_gemm_args& a, Plan* plan) {
       return hipSuccess;
     }
   }
+  if (plan_parts(a, plan)) return hipSuccess;
   const bool plain = a.variant == 0 && a.split_k == 0 && !a.mm_begin_timestamp && !a.mm_end_timestamp &&
                      !(a.epilogue == IRIS_EPI_ONE_SHOT && a.phase != IRIS_PHASE_PRODUCE) &&
                      a.epilogue != IRIS_EPI_ATOMIC_ADD && a.num_sms > 0 && (a.block_m == 128 || a.block_m == 256) &&
@@ -1024,7 +1089,7 @@ extern "C" int iris_gemm_launch_noalloc(const iris_gemm_args* args, void* stream
   // wait that timed out leaves one raised).  A fill kernel, not a memset, so
   // that the call can be recorded into a HIP graph.
   auto needs_locks = [](const Plan& q) {
-    return (q.skinny && q.k.flag_mode != 0) || (q.entry && (q.k.split_k > 1 || q.k.stream_k || q.last_round));
+    return (q.skinny && q.k.flag_mode != 0) || q.k.part_m * q.k.part_n > 1 || (q.entry && (q.k.split_k > 1 || q.k.stream_k || q.last_round));
   };
   const bool uses_locks = needs_locks(plan) || (plan.rest && needs_locks(*plan.rest));
   if (uses_locks) {
@@ -1097,6 +1162,10 @@ extern "C" int iris_gemm_plan_name(const iris_gemm_args* args, char* buf, size_t
   if (plan.rest) {
     const size_t n = std::strlen(buf);
     std::snprintf(buf + n, len > n ? len - n : 0, "+last_%d_columns_apart", plan.rest->k.N);
+  }
+  if (plan.parts) {
+    const size_t n = std::strlen(buf);
+    std::snprintf(buf + n, len > n ? len - n : 0, "+parts_of_tiles");
   }
   if (plan.two_kernels) {
     const size_t n = std::strlen(buf);

@@ -39,7 +39,7 @@ def test_scatter(shmem, M, N, K, BM, BN, grid, ws, row_major, plan, parts):
     P = shmem.zeros((grid, BM * BN), dtype=F32)
     locks = shmem.zeros((grid,), dtype=torch.int32)
     args = (a, b, None, cg, flags, shmem.get_heap_bases(), 0, ws, grid, BM, BN, 64, 2, ops.EPI_ALL_SCATTER)
-    kw = dict(partials=P, locks=locks)
+    kw = dict(partials=P, locks=locks, split_k=parts if parts > 1 else 0)
     assert ops.gemm_plan_name(*args, **kw) == plan and ops.gemm_split_k(*args, **kw) == parts
     want = O.shard_gemm(A, B, F32)
     for launch in (1, 2):
