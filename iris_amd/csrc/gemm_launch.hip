@@ -85,10 +85,10 @@ struct Plan {
   int in_program = 0;    // ONE_SHOT, IRIS_PHASE_FUSED: the build of the kernel that reduces each tile itself
   int parts = 0;         // the launch's tiles are parts of the caller's (plan_parts)
   int two_kernels = 0;   // ... or, for such a launch too, producer and reduce as two kernels (reduce_in_program)
-  // the few-rows kernel instead of a table entry, one workgroup per 16 columns
+  // the few-rows kernel instead of a table entry: workgroups along the columns, the rows and K
   GemmKernelFn skinny = nullptr;
-  int skinny_grid = 0, skinny_grid_y = 1, skinny_lds = 0;
-  int skinny_rb = 1, skinny_cb = 1;  // blocks of 16 rows / 16 columns a workgroup of the few-rows kernel takes
+  int skinny_grid = 0, skinny_grid_y = 1, skinny_grid_z = 1, skinny_lds = 0;
+  int skinny_rb = 1;  // blocks of 16 rows a workgroup of the few-rows kernel takes
   // a second launch of the entry's split-K build behind the first: the tiles of the last round, K shared out
   // over the programs that round would leave idle
   int last_round = 0;
@@ -104,54 +104,73 @@ int dbg() {
   return v;
 }
 
+// Workgroups that share the K range of each of `cells` blocks of C in the few-rows kernel, from what bounds it: the
+// CU with the most workgroups (`block_us` for a block of K a wave), B at the rate a stream of it reaches (6 TB/s),
+// and for a shared range the hand-over (2 us, 0.1 more for every part).  A part keeps 32 blocks, four a wave.  (us a
+// pass, by parts: [4,8192] x [8192,192] 9.8 / 9.1 / 8.0 / 8.3 with 1 / 2 / 4 / 8, [16,8192] x [8192,1024] 10.0 / 9.6 /
+// 8.9 / 10.2, [6,9344] x [9344,2560] 13.2 unshared and 14.4 in 3.)
+int few_rows_parts(int64_t cells, int64_t nb, double block_us, int64_t b_bytes) {
+  const int64_t cus = current_cu_count();
+  int best = 1;
+  double least = 0;
+  for (int parts = 1; parts <= SKINNY_MAX_SPLIT && (parts == 1 || parts * 32 <= nb); ++parts) {
+    const int64_t share = (nb + parts - 1) / parts;
+    if ((parts - 1) * share >= nb) continue;  // (the last part would be empty)
+    const double busiest = (double)((cells * parts + cus - 1) / cus * ((share + SKINNY_WAVES - 1) / SKINNY_WAVES)) * block_us;
+    const double stream = (double)b_bytes / 6e6;
+    const double cost = (busiest > stream ? busiest : stream) + (parts > 1 ? 2 + 0.1 * parts : 0);
+    if (parts == 1 || cost < least) best = parts, least = cost;
+  }
+  return best;
+}
+
 // A few rows: the product is a stream over B, and the kernel built for that
 // takes it when the operands allow the 16-byte fetches, the logical tile
-// covers every row, the tiles' arrival counters have a home, and (with more
-// than 16 rows: two workgroups per 16 columns) every workgroup finds a place
-// on the device at once, so that B comes from HBM once.  Fills the plan and
-// returns true when the launch qualifies.
+// covers every row and the tiles' arrival counters have a home.  Fills the
+// plan and returns true when the launch qualifies.
 bool plan_few_rows(const iris_gemm_args& a, int op, bool dma_ok, Plan* plan) {
   GemmKArgs& k = plan->k;
   const int64_t lim = (int64_t)1 << 31;
-  // Up to 32 rows: a workgroup per 16 rows x 16 columns.  Up to 64 rows of a long K, where the persistent
-  // kernel would split K and pay for the hand-over: 32 rows x 16 columns a workgroup, as long as one round of
-  // workgroups covers the matrix ([64,4096] x [4096,1376]: 172 workgroups, 11.5 us against 12.7).
-  int rb = 1, cb = 1;
-  if (a.M > SKINNY_MAX_ROWS) rb = 2;
+  // Up to 32 rows: a workgroup per 16 rows x 16 columns, unless B is more than the 16 MB that are as well read
+  // twice ([32,4096] x [4096,4096] 12.5 us in blocks of 16 rows and 11.3 in 32, [32,2560] x [2560,8192] 18.5 and 13.8, but
+  // [17,4096] x [4096,1376] 8.4 and 9.2).  Up to 64 rows of a long K, where the persistent kernel would split K and
+  // pay more for the hand-over: 32 rows x 16 columns a workgroup, as long as one round of workgroups covers the
+  // matrix ([64,4096] x [4096,1376]: 172 workgroups, 11.5 us against 12.7).
+  const int64_t b_bytes = (int64_t)a.N * a.K * 2;
+  const bool mid = a.M > SKINNY_MAX_ROWS;
+  const int rb = mid || (a.M > SKINNY_ROWS && a.K >= SKINNY_MID_MIN_K && b_bytes > (16 << 20)) ? 2 : 1;
   const int m_blocks = (a.M + SKINNY_ROWS * rb - 1) / (SKINNY_ROWS * rb);
-  const int n_blocks = (a.N + SKINNY_COLS * cb - 1) / (SKINNY_COLS * cb);
-  // fetches in flight per wave: enough for the whole K range, 8 blocks at most (4 with two blocks of columns:
-  // LDS holds no more)
-  const int per_wave = ((a.K + 63) / 64 + SKINNY_WAVES - 1) / SKINNY_WAVES;
-  int un = per_wave <= 2 ? 2 : per_wave <= 4 ? 4 : 8;
-  if (cb == 2 && un > 4) un = 4;
-  const int wide = SKINNY_COLS * cb;
-  const bool counters = (m_blocks == 1 && (a.block_n <= wide || a.N <= wide)) || k.flag_mode == 0 ||
+  const int n_blocks = (a.N + SKINNY_COLS - 1) / SKINNY_COLS;
+  const int64_t cells = (int64_t)m_blocks * n_blocks;
+  const bool counters = (m_blocks == 1 && (a.block_n <= SKINNY_COLS || a.N <= SKINNY_COLS)) || k.flag_mode == 0 ||
                         (a.locks && k.total_tiles <= a.num_sms);
-  bool room = true;
-  if (rb > 1) {
-    room = (int64_t)m_blocks * n_blocks <= (int64_t)current_cu_count() && a.M <= SKINNY_MID_MAX_ROWS &&
-           a.K >= SKINNY_MID_MIN_K;
-  } else if (m_blocks > 1) {
-    const int per_cu = 160 * 1024 / skinny_lds_bytes(un) > 4 ? 4 : 160 * 1024 / skinny_lds_bytes(un);
-    room = (int64_t)m_blocks * n_blocks <= (int64_t)current_cu_count() * per_cu;
-  }
-  const bool ok = room && a.K > 0 && dma_ok && !plan->in_program && a.block_m >= a.M && (a.block_n % wide) == 0 &&
+  const bool room = !mid || (cells <= (int64_t)current_cu_count() && a.M <= SKINNY_MID_MAX_ROWS && a.K >= SKINNY_MID_MIN_K);
+  const bool ok = room && a.K > 0 && dma_ok && !plan->in_program && a.block_m >= a.M && (a.block_n % SKINNY_COLS) == 0 &&
                   !a.mm_begin_timestamp && !a.mm_end_timestamp && (a.split_k == 0 || a.split_k == 1) && counters &&
-                  skinny_lds_bytes(un, rb, cb) <= 160 * 1024 &&
                   ((int64_t)SKINNY_ROWS * rb * a.stride_am + a.K) * 2 < lim &&
-                  ((int64_t)wide * a.stride_bn + a.K) * 2 < lim;
+                  ((int64_t)SKINNY_COLS * a.stride_bn + a.K) * 2 < lim;
   if (!ok) return false;
-  const bool a_lds = rb > 1 || (a.M >= SKINNY_A_VIA_LDS_ROWS && a.K >= SKINNY_A_VIA_LDS_K);
-  plan->skinny = gemm_skinny_kernel_for(a.ab_dtype, op, un, a_lds, rb, cb);
+  // K shared out: the blocks of C count their parts' arrivals in the words of `locks` behind the tiles' own
+  int parts = 1;
+  if (a.split_k == 0 && a.partials && aligned16(a.partials) && a.locks && k.total_tiles + cells <= a.num_sms) {
+    // a block of K of a workgroup alone on its CU, by what it fetches; rows that do not start on a cache line
+    // touch half as many lines again ([31,11800] x [11800,1360] 0.85 us, [40,16384] x [16384,512] 0.48)
+    const bool lines = a.stride_am % 64 == 0 && a.stride_bn % 64 == 0;
+    const double block_us = (rb == 2 ? 0.5 : 0.3) * (lines ? 1 : 1.6);
+    parts = few_rows_parts(cells, (a.K + 63) / 64, block_us, b_bytes);
+    const int64_t elems = cells * rb * (SKINNY_ROWS * SKINNY_COLS);  // of one part's sums
+    if (parts * elems > (int64_t)a.num_sms * a.partials_slot_elems) parts = 1;
+  }
+  plan->skinny = gemm_skinny_kernel_for(a.ab_dtype, op, a.M <= 8 ? 8 : 16, rb);
   if (!plan->skinny) return false;
-  plan->skinny_lds = skinny_lds_bytes(un, rb, cb);
+  plan->skinny_lds = skinny_lds_bytes(rb);
   plan->skinny_grid = n_blocks;
   plan->skinny_grid_y = m_blocks;
+  plan->skinny_grid_z = parts;
   plan->skinny_rb = rb;
-  plan->skinny_cb = cb;
   k.split_k = 1;
   k.locks = a.locks;
+  k.partials = a.partials;
   return true;
 }
 
@@ -947,13 +966,13 @@ hipError_t run_plan(const Plan& plan, const iris_gemm_args& args, void* stream) 
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (plan.skinny) {
     if (dbg())
-      std::fprintf(stderr, "[iris_amd] gemm few-rows M=%d N=%d K=%d tiles=%d grid=%dx%d\n", plan.k.M, plan.k.N, plan.k.K,
-                   plan.k.total_tiles, plan.skinny_grid, plan.skinny_grid_y);
+      std::fprintf(stderr, "[iris_amd] gemm few-rows M=%d N=%d K=%d tiles=%d grid=%dx%dx%d\n", plan.k.M, plan.k.N, plan.k.K,
+                   plan.k.total_tiles, plan.skinny_grid, plan.skinny_grid_y, plan.skinny_grid_z);
     if (plan.skinny_lds > 64 * 1024) {
       err = ensure_lds(plan.skinny, plan.skinny_lds);
       if (err != hipSuccess) return err;
     }
-    hipLaunchKernelGGL(plan.skinny, dim3(plan.skinny_grid, plan.skinny_grid_y), dim3(SKINNY_THREADS), plan.skinny_lds, s,
+    hipLaunchKernelGGL(plan.skinny, dim3(plan.skinny_grid, plan.skinny_grid_y, plan.skinny_grid_z), dim3(SKINNY_THREADS), plan.skinny_lds, s,
                        plan.k);
     err = hipGetLastError();
     if (err != hipSuccess) return err;
@@ -1089,7 +1108,7 @@ extern "C" int iris_gemm_launch_noalloc(const iris_gemm_args* args, void* stream
   // wait that timed out leaves one raised).  A fill kernel, not a memset, so
   // that the call can be recorded into a HIP graph.
   auto needs_locks = [](const Plan& q) {
-    return (q.skinny && q.k.flag_mode != 0) || q.k.part_m * q.k.part_n > 1 || (q.entry && (q.k.split_k > 1 || q.k.stream_k || q.last_round));
+    return (q.skinny && (q.k.flag_mode != 0 || q.skinny_grid_z > 1)) || q.k.part_m * q.k.part_n > 1 || (q.entry && (q.k.split_k > 1 || q.k.stream_k || q.last_round));
   };
   const bool uses_locks = needs_locks(plan) || (plan.rest && needs_locks(*plan.rest));
   if (uses_locks) {

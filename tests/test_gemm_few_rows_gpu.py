@@ -365,3 +365,40 @@ def test_persistent_choice_gives_the_same_result(shmem):
     assert got[0][0] == FEW and got[ops.VARIANT_PERSISTENT][0] != FEW
     check_close(got[0][1], got[ops.VARIANT_PERSISTENT][1])
     assert got[0][2] == got[ops.VARIANT_PERSISTENT][2]
+
+
+@pytest.mark.parametrize("M,N,K,odt", [
+    (1, 128, 36864, torch.bfloat16),   # one row, parts of four K blocks a wave
+    (8, 50, 6200, torch.bfloat16),     # A as one instruction a block; N and K no multiples of the blocks
+    (9, 272, 9000, torch.float32),     # ... as two; fp32 partial, rows that start off a cache line
+    (31, 1360, 11800, torch.bfloat16), # 32 rows a workgroup
+    (17, 520, 20480, torch.float32),   # ... the second block with one row
+    (40, 64, 16384, torch.bfloat16),
+])
+def test_shared_k(shmem, M, N, K, odt):
+    """With the workspace, few workgroups and a long K: its range is shared out
+    over workgroups, which add their sums up there.  The words of the
+    workspace's counters are back at zero behind every launch, and the sum
+    does not depend on which part arrives last."""
+    dtype = torch.bfloat16
+    A, B = make_ab(M, N, K, dtype)
+    a, b = to_heap(shmem, A), to_heap(shmem, B)
+    out = shmem.zeros((M, N), dtype=odt)
+    total = ops.cdiv(N, 64)
+    flags = shmem.zeros((total,), dtype=torch.int32)
+    locks = shmem.zeros((256,), dtype=torch.int32)
+    P = shmem.full((256, 64 * 64), float("nan"), dtype=torch.float32)
+    epi = ops.EPI_ALL_SCATTER if odt == dtype else ops.EPI_ONE_SHOT
+    first = None
+    for launch in (1, 2, 3):
+        out.fill_(7)
+        args = (a, b, None, out, flags) if odt == dtype else (a, b, out, shmem.zeros((M, N), dtype=dtype), flags)
+        ops.gemm_launch(*args, shmem.get_heap_bases(), 0, 1, 256, 64, 64, 64, 4, epi, locks=locks, partials=P,
+                        phase=ops.PHASE_PRODUCE)
+        torch.cuda.synchronize()
+        check_close(out, O.shard_gemm(A, B, odt), f"launch {launch}")
+        assert first is None or torch.equal(out, first)
+        first = out.clone()
+        assert not locks.any()
+        assert flags.cpu().tolist() == ([launch] if odt == dtype else [0]) * total
+    assert not torch.isnan(P.view(-1)[:4]).any()  # (the parts did meet there)
