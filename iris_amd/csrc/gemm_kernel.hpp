@@ -829,6 +829,35 @@ __device__ inline void atomic_add16_pair(IRIS_GLOBAL unsigned int* p, unsigned i
   }
 }
 
+// 16-bit atomic add of the two elements of the aligned word at `w`: `lo` / `hi` are the bits to add where have_lo /
+// have_hi.  An element that is not to change takes -0, which leaves every number as it is, where it belongs to the
+// output as well (near_lo / near_hi); a word of which one half is somebody else's goes the way of the CAS.
+template <int DT>
+__device__ inline void atomic_add16_word(IRIS_GLOBAL char* w, unsigned int lo, unsigned int hi, bool have_lo, bool have_hi,
+                                         bool near_lo, bool near_hi) {
+  if (!have_lo && !have_hi) return;
+  if ((have_lo || near_lo) && (have_hi || near_hi))
+    atomic_add16_pair<DT>((IRIS_GLOBAL unsigned int*)w, (have_lo ? lo & 0xFFFFu : 0x8000u) | (have_hi ? hi << 16 : 0x80000000u));
+  else
+    atomic_add16_cas<DT>((IRIS_GLOBAL unsigned short*)(w + (have_lo ? 0 : 2)), from16<DT>((unsigned short)(have_lo ? lo : hi)));
+}
+
+// ... of the first `valid` of four neighbouring elements at `d`, any even address.  before / after: the elements in
+// front of the first and behind the last of them belong to the output too.
+template <int DT>
+__device__ inline void atomic_add16_strip(IRIS_GLOBAL char* d, f32x4 v, int valid, bool before, bool after) {
+  const unsigned int h[2] = {pack2<DT>(v[0], v[1]), pack2<DT>(v[2], v[3])};
+  const bool more[5] = {valid > 0, valid > 1, valid > 2, valid > 3, false};
+  if (((uintptr_t)d & 2) == 0) {
+    atomic_add16_word<DT>(d, h[0], h[0] >> 16, more[0], more[1], before, after);
+    atomic_add16_word<DT>(d + 4, h[1], h[1] >> 16, more[2], more[3], true, after);
+  } else {
+    atomic_add16_word<DT>(d - 2, 0, h[0], false, more[0], before, after);
+    atomic_add16_word<DT>(d + 2, h[0] >> 16, h[1], more[1], more[2], true, after);
+    atomic_add16_word<DT>(d + 6, h[1] >> 16, 0, more[3], false, true, after);
+  }
+}
+
 // Write the wave's TM x TN accumulator block to `out` on the destination
 // ranks, rows < m_end, columns < n_end, through the wave-private LDS scratch.
 //
@@ -983,6 +1012,27 @@ __device__ __attribute__((always_inline)) inline bool store_acc(const GemmKArgs&
                                     *reinterpret_cast<const IRIS_LDS unsigned short*>(src + e * 2), p.sys != 0);
                   }
                 }
+              }
+            }
+          } else if (OP == OP_ATOMIC16 && p.row_out) {
+            // ragged edge or unaligned rows: the aligned words of a row, lanes along it (one more than half the
+            // columns where a row starts on an odd element).  Element by element through a CAS, every tile at an edge
+            // of [1444,4608] x [4608,3776] in 256 x 64 tiles cost as much as the rest of the launch: 98 us -> 32.
+            if constexpr (OP == OP_ATOMIC16) {
+              constexpr int W = CP / 2 + 1;
+#pragma nounroll
+              for (int idx = lane; idx < 32 * W; idx += 64) {
+                const int row = idx / W;
+                if (row >= rows_ok) break;
+                IRIS_GLOBAL char* d = dst + ((int64_t)(row0 + row) * p.som + col0) * ES;
+                const int c = (idx % W) * 2 - (((uintptr_t)d & 2) ? 1 : 0);
+                auto element = [&](int cc) -> unsigned int {
+                  const int u = (cc / EPV) ^ ((row / Cfg::ERPB) % Cfg::U16);
+                  return *reinterpret_cast<const IRIS_LDS unsigned short*>(ws + row * Cfg::WS_PITCH + u * 16 + (cc % EPV) * ES);
+                };
+                const bool lo = c >= 0 && c < cols_ok, hi = c + 1 < cols_ok;
+                atomic_add16_word<ODT>(d + c * ES, lo ? element(c) : 0, hi ? element(c + 1) : 0, lo, hi, col0 + c >= 0,
+                                       col0 + c + 1 < p.N);
               }
             }
           } else {
@@ -1298,6 +1348,13 @@ __device__ inline void slice_epilogue(const GemmKArgs& p, const Item& it, int sl
                 whole(std::integral_constant<int, 17>{});
               else
                 whole(std::integral_constant<int, 16>{});
+              continue;
+            }
+          }
+          if constexpr (OP == OP_ATOMIC16) {
+            if (p.row_out) {
+              const int n = it.n0 + col[u];
+              atomic_add16_strip<ODT>(dst + ((int64_t)row[u] * p.som + col[u]) * ES, sum[u], ncols[u], n > 0, n + ncols[u] < p.N);
               continue;
             }
           }

@@ -279,24 +279,26 @@ gemm_skinny_kernel(const GemmKArgs p) {
         for (int w = 1; w < SKINNY_WAVES; ++w) s += red[w * 64 + lane];  // wave order: the sum does not depend on timing
       }
       constexpr int ES = F32 ? 4 : 2;
-      [[maybe_unused]] const bool whole = p.vec_out && n + 4 <= p.N;
       for (int r = r_begin + wave; r < r_end; r += SKINNY_WAVES) {
         IRIS_GLOBAL char* dst = rank_ptr(p, p.out, r);
         if constexpr (ATOMIC) {
           // 08: add into the destination (gemm_atomics_all_reduce.py:236-248)
+          if constexpr (OP == OP_ATOMIC16) {
+            if (p.row_out) {
+              const int valid = min(4, p.N - n);
+              atomic_add16_strip<ODT>(dst + ((int64_t)m * p.som + n) * ES, s, valid, n > 0, n + valid < p.N);
+              continue;
+            }
+          }
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             if (n + e >= p.N) continue;
             IRIS_GLOBAL char* d = dst + ((int64_t)m * p.som + (int64_t)(n + e) * p.son) * ES;
             const float f = s[e];
-            if constexpr (OP == OP_ATOMIC32) {
+            if constexpr (OP == OP_ATOMIC32)
               __hip_atomic_fetch_add((IRIS_GLOBAL float*)d, f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            } else if (whole && (e & 1) == 0) {
-              atomic_add16_pair<ODT>((IRIS_GLOBAL unsigned int*)d, pack2<ODT>(s[e], s[e + 1]));
-              ++e;  // the pair took the next column too
-            } else {
+            else
               atomic_add16_cas<ODT>((IRIS_GLOBAL unsigned short*)d, from16<ODT>(to16<ODT>(f)));
-            }
           }
         } else if (p.row_out && n + 4 <= p.N) {
           // four columns in one store (at any address: rows of an odd length are no exception)
