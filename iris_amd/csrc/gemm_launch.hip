@@ -126,7 +126,7 @@ int few_rows_parts(int64_t cells, int64_t nb, double block_us, int64_t b_bytes) 
 
 // A few rows: the product is a stream over B, and the kernel built for that
 // takes it when the operands allow the 16-byte fetches, the logical tile
-// covers every row and the tiles' arrival counters have a home.  Fills the
+// covers every row (or whole workgroups of them) and the tiles' arrival counters have a home.  Fills the
 // plan and returns true when the launch qualifies.
 bool plan_few_rows(const iris_gemm_args& a, int op, bool dma_ok, Plan* plan) {
   GemmKArgs& k = plan->k;
@@ -144,8 +144,18 @@ bool plan_few_rows(const iris_gemm_args& a, int op, bool dma_ok, Plan* plan) {
   const int64_t cells = (int64_t)m_blocks * n_blocks;
   const bool counters = (m_blocks == 1 && (a.block_n <= SKINNY_COLS || a.N <= SKINNY_COLS)) || k.flag_mode == 0 ||
                         (a.locks && k.total_tiles <= a.num_sms);
-  const bool room = !mid || (cells <= (int64_t)current_cu_count() && a.M <= SKINNY_MID_MAX_ROWS && a.K >= SKINNY_MID_MIN_K);
-  const bool ok = room && a.K > 0 && dma_ok && !plan->in_program && a.block_m >= a.M && (a.block_n % SKINNY_COLS) == 0 &&
+  // fp32: the matrix cores do a sixteenth of the 16-bit rate and a tile that is half padding costs twice, so it is
+  // taken up to 128 rows, above 64 where the workgroups come in (nearly) whole rounds.  (us a pass: [64,512] x
+  // [512,1024] 13.8 by the persistent kernel, 8.7 here, [96,4096] x [4096,1024] 23.1 and 17.8, [128,2048] x
+  // [2048,2048] 24.2 and 17.3, but [128,4096] x [4096,1376], 344 workgroups, 26.4 and 28.4.)
+  const bool f32 = a.ab_dtype == IRIS_DTYPE_F32;
+  const int64_t cus = current_cu_count();
+  const bool f32_room = a.M <= SKINNY_MID_MAX_ROWS ||
+                        (a.M <= SKINNY_F32_MAX_ROWS && (cells <= cus || cells * 4 >= (cells + cus - 1) / cus * cus * 3));
+  const bool room = !mid || (f32 && f32_room) || (cells <= (int64_t)current_cu_count() && a.M <= SKINNY_MID_MAX_ROWS && a.K >= SKINNY_MID_MIN_K);
+  // (the workgroups' rows belong to one tile)
+  const bool rows_ok = a.block_m >= a.M || (f32 && a.block_m % (SKINNY_ROWS * rb) == 0);
+  const bool ok = room && a.K > 0 && dma_ok && !plan->in_program && rows_ok && (a.block_n % SKINNY_COLS) == 0 &&
                   !a.mm_begin_timestamp && !a.mm_end_timestamp && (a.split_k == 0 || a.split_k == 1) && counters &&
                   ((int64_t)SKINNY_ROWS * rb * a.stride_am + a.K) * 2 < lim &&
                   ((int64_t)SKINNY_COLS * a.stride_bn + a.K) * 2 < lim;

@@ -25,6 +25,9 @@ GemmKernelFn gemm_skinny_kernel_for(int dt, int op, int arows, int rb) {
     if (op == OP_STORE32) return pick<IRIS_DTYPE_F16, OP_STORE32>(arows, rb);
     if (op == OP_ATOMIC32) return pick<IRIS_DTYPE_F16, OP_ATOMIC32>(arows, rb);
     if (op == OP_ATOMIC16) return pick<IRIS_DTYPE_F16, OP_ATOMIC16>(arows, rb);
+  } else if (dt == IRIS_DTYPE_F32) {
+    if (op == OP_STORE32) return pick<IRIS_DTYPE_F32, OP_STORE32>(arows, rb);
+    if (op == OP_ATOMIC32) return pick<IRIS_DTYPE_F32, OP_ATOMIC32>(arows, rb);
   }
   return nullptr;
 }

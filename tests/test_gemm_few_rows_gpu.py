@@ -402,3 +402,32 @@ def test_shared_k(shmem, M, N, K, odt):
         assert not locks.any()
         assert flags.cpu().tolist() == ([launch] if odt == dtype else [0]) * total
     assert not torch.isnan(P.view(-1)[:4]).any()  # (the parts did meet there)
+
+
+@pytest.mark.parametrize("M,N,K,BM,BN", [
+    (1, 128, 7480, 128, 128),  # K shared out
+    (16, 72, 36, 64, 64),      # nine chunks of K
+    (31, 200, 520, 64, 64),
+    (64, 4096, 516, 64, 64),   # more workgroups than CUs
+    (80, 130, 512, 64, 64),    # two tiles of rows
+    (97, 512, 2052, 32, 16),   # four
+    (128, 2048, 100, 128, 128),
+])
+def test_fp32(shmem, M, N, K, BM, BN):
+    """fp32 operands, up to 128 rows, in tiles that need not cover every row."""
+    A, B = make_ab(M, N, K, torch.float32)
+    a, b = to_heap(shmem, A), to_heap(shmem, B)
+    cg = shmem.zeros((M, N), dtype=torch.float32)
+    total = ops.cdiv(M, BM) * ops.cdiv(N, BN)
+    flags = shmem.zeros((total,), dtype=torch.int32)
+    locks = shmem.zeros((256,), dtype=torch.int32)
+    P = shmem.zeros((256, BM * BN), dtype=torch.float32)
+    args = (a, b, None, cg, flags, shmem.get_heap_bases(), 0, 1, 256, BM, BN, 64, 2, ops.EPI_ALL_SCATTER)
+    assert ops.gemm_plan_name(*args, locks=locks, partials=P) in (FEW, MID)
+    for launch in (1, 2):
+        cg.fill_(7)
+        ops.gemm_launch(*args, locks=locks, partials=P)
+        torch.cuda.synchronize()
+        check_close(cg, O.shard_gemm(A, B, torch.float32), f"launch {launch}")
+        assert flags.cpu().tolist() == [launch] * total
+        assert not locks.any()
