@@ -74,6 +74,35 @@ __host__ __device__ inline uint32_t fast_div(uint32_t n, const FastDiv& f) {
   return n / f.d;
 }
 
+// Fetches all lines of a kernel's argument block (its only parameter) into the scalar cache, which every launch finds
+// cold, in one round trip.  The compiler loads arguments where they are first read: a line at a time, 0.24 us each, eight
+// of them one after another before a program's first operand load.
+template <int BYTES>
+__device__ __attribute__((always_inline)) inline void touch_args() {
+  typedef const __attribute__((address_space(4))) uint32_t* ArgPtr;
+  const ArgPtr args = (ArgPtr)__builtin_amdgcn_kernarg_segment_ptr();
+  constexpr int LINES = (BYTES + 63) / 64;
+  static_assert(LINES <= 10 && LINES > 1, "lines touched below");
+  uint32_t t0, t1, t2, t3, t4, t5, t6, t7, t8, t9;
+  // (one that lies past the block's end reads its first line again)
+  asm volatile(
+      "s_load_dword %0, %10, 0x0\n\ts_load_dword %1, %10, %11\n\ts_load_dword %2, %10, %12\n\ts_load_dword %3, %10, %13\n\t"
+      "s_load_dword %4, %10, %14\n\ts_load_dword %5, %10, %15\n\ts_load_dword %6, %10, %16\n\ts_load_dword %7, %10, %17\n\t"
+      "s_load_dword %8, %10, %18\n\ts_load_dword %9, %10, %19\n\ts_waitcnt lgkmcnt(0)"
+      : "=&s"(t0), "=&s"(t1), "=&s"(t2), "=&s"(t3), "=&s"(t4), "=&s"(t5), "=&s"(t6), "=&s"(t7), "=&s"(t8), "=&s"(t9)
+      : "s"(args), "i"(64), "i"(LINES > 2 ? 128 : 0), "i"(LINES > 3 ? 192 : 0), "i"(LINES > 4 ? 256 : 0),
+        "i"(LINES > 5 ? 320 : 0), "i"(LINES > 6 ? 384 : 0), "i"(LINES > 7 ? 448 : 0), "i"(LINES > 8 ? 512 : 0),
+        "i"(LINES > 9 ? 576 : 0));
+}
+
+// ... and the line at `p`, which may be null, into the caches.
+__device__ __attribute__((always_inline)) inline void touch_line(const void* p) {
+  if (p) {
+    uint32_t t;
+    asm volatile("s_load_dword %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=&s"(t) : "s"(p));
+  }
+}
+
 // The divisors of a launch's tile decode.
 struct TileDivs {
   FastDiv in_group;  // G * num_pid_n: tiles per group of G tile rows

@@ -158,6 +158,7 @@ struct GemmKArgs {
   // tile_arrivals[its id] (all zero between launches), and the last one raises its flag
   int part_m, part_n;
   int32_t* tile_arrivals;
+  FastDiv div_xcd;  // num_xcds
 };
 
 template <int DT>
@@ -1505,6 +1506,7 @@ enum WaveRole { ROLE_ANY, ROLE_WORKER, ROLE_FETCH_A, ROLE_FETCH_A_ACROSS, ROLE_F
 template <class Cfg, int OP, int ODT, bool SPLIT, bool FUSED, bool MERGED, int ROLE>
 __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKArgs& p) {
   static_assert(!MERGED || !FUSED, "blocks of the caller's tiles: no build with the reduce inside");
+  touch_args<sizeof(GemmKArgs)>();
   extern __shared__ __attribute__((aligned(1024))) char lds_raw[];
   IRIS_LDS char* lds = (IRIS_LDS char*)lds_raw;
   const int tid = threadIdx.x;
@@ -1520,7 +1522,7 @@ __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKAr
   int pid;
   if (p.xcd_per > 0) {
     // workgroups are dealt to the XCDs round-robin: this one is number j on XCD x
-    const int x = blockIdx.x % p.num_xcds, j = blockIdx.x / p.num_xcds;
+    const int j = (int)fast_div(blockIdx.x, p.div_xcd), x = blockIdx.x - j * p.num_xcds;
     pid = j < p.xcd_per ? x * p.xcd_per + j : p.num_sms * 2;  // (past every item: nothing to do)
   } else {
     pid = xcd_remap(blockIdx.x, p.num_sms, p.num_xcds);
@@ -1547,7 +1549,7 @@ __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKAr
   constexpr bool ONE_ITEM = SPLIT && !Cfg::SPLIT_OWNER;
   const int nk = (p.K + Cfg::BK - 1) / Cfg::BK;
   const int work = split ? p.total_tiles * p.split_k : p.total_tiles;  // tiles, or (tile, part) pairs
-  const int n_mine = pid < work ? (work - pid + p.num_sms - 1) / p.num_sms : 0;
+  const int n_mine = pid >= work ? 0 : work <= p.num_sms ? 1 : (work - pid + p.num_sms - 1) / p.num_sms;
   int n_items = split ? n_mine : n_mine * p.sub_m * p.sub_n;
   StreamRun sr{0, 0, 0};
   if constexpr (SPLIT) {
@@ -1931,6 +1933,7 @@ __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKAr
           IRIS_WAIT_VMCNT(Cfg::L * (Cfg::S - 1));
         }
       }
+      if (worker) touch_line(p.heap_bases);  // (read in the epilogue; the multiplying waves have nothing else to do here)
       block_barrier_raw();
       if (worker) {
         load_all<Cfg>(lds + a_row_off + xoff[0], lds + Cfg::A_BYTES + b_row_off + xoff[0], fr, 0);

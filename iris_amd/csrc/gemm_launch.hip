@@ -303,6 +303,7 @@ void launch_constants(const iris_gemm_args& a, const GemmKernelEntry& pick, Gemm
   k.div_subs = make_fast_div((uint32_t)(k.sub_m * k.sub_n), items);
   k.div_sub_n = make_fast_div((uint32_t)k.sub_n, items);
   k.div_split = make_fast_div((uint32_t)k.split_k, (uint64_t)a.num_sms + 1);
+  k.div_xcd = make_fast_div((uint32_t)a.num_xcds, 2 * (uint64_t)a.num_sms + 1);
   k.div_nk = make_fast_div((uint32_t)(nk > 0 ? nk : 1), (uint64_t)k.total_tiles * (nk > 0 ? nk : 1) + 1);
   // Fewer (tile, part) items than programs: deal them to the XCDs evenly, in
   // consecutive runs, instead of filling the first XCDs and idling the rest.

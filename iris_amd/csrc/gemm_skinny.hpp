@@ -75,6 +75,7 @@ gemm_skinny_kernel(const GemmKArgs p) {
   static_assert(RB == 1 || RB == 2, "blocks of rows per workgroup");
   using vec8 = typename Mfma<DT>::vec8;
   extern __shared__ __attribute__((aligned(1024))) char skinny_lds[];
+  touch_args<sizeof(GemmKArgs)>();
   IRIS_LDS char* lds = (IRIS_LDS char*)skinny_lds;
   // each wave's blocks of A ([SKINNY_WAVES][RB][64] partial accumulators at the end), then each wave's UN blocks of B
   IRIS_LDS f32x4* red = (IRIS_LDS f32x4*)lds;
@@ -166,6 +167,7 @@ gemm_skinny_kernel(const GemmKArgs p) {
     fetch(u, b0 + SKINNY_WAVES * u);
     asm volatile("" ::: "memory");  // (the blocks' loads stay in this order: the waits below count them)
   }
+  touch_line(p.heap_bases);  // (read by the stores)
   // A long range of K: as a block has been read its place takes the one UN further on, so that the fetches in
   // flight never run dry (B has landed in this wave's own region once the wave's counter says so: nobody else
   // reads or writes it).
