@@ -159,6 +159,10 @@ struct GemmKArgs {
   int part_m, part_n;
   int32_t* tile_arrivals;
   FastDiv div_xcd;  // num_xcds
+  // (the few-rows kernel in cells of 32 x 32) `cells` of them, numbered in runs of cells_inner along the rows of C
+  // (cells_by_row) or its columns; xcd_per consecutive ones to an XCD
+  int cells, cells_inner, cells_by_row;
+  FastDiv div_inner;
 };
 
 template <int DT>

@@ -88,7 +88,7 @@ struct Plan {
   // the few-rows kernel instead of a table entry: workgroups along the columns, the rows and K
   GemmKernelFn skinny = nullptr;
   int skinny_grid = 0, skinny_grid_y = 1, skinny_grid_z = 1, skinny_lds = 0;
-  int skinny_rb = 1;  // blocks of 16 rows a workgroup of the few-rows kernel takes
+  int skinny_rb = 1, skinny_cb = 1;  // blocks of 16 rows and of 16 columns a workgroup of the few-rows kernel takes
   // a second launch of the entry's split-K build behind the first: the tiles of the last round, K shared out
   // over the programs that round would leave idle
   int last_round = 0;
@@ -178,6 +178,46 @@ bool plan_few_rows(const iris_gemm_args& a, int op, bool dma_ok, Plan* plan) {
   plan->skinny_grid_y = m_blocks;
   plan->skinny_grid_z = parts;
   plan->skinny_rb = rb;
+  k.split_k = 1;
+  k.locks = a.locks;
+  k.partials = a.partials;
+  return true;
+}
+
+// A small product of more rows in cells of 32 x 32 (gemm_skinny.hpp), where one round of workgroups covers it.  us a pass
+// as 64 x 64 tiles, K shared out where that helps, and as cells: [213,624] x [624,320] 7.7 / 6.4, [475,2560] x [2560,480]
+// 12.3 / 8.6, [128,4096] x [4096,1376] 12.7 / 9.6, [1239,4288] x [4288,192] 13.9 / 10.0, [100,8192] x [8192,256] 12.3 /
+// 9.0; fp32 [475,2560] x [2560,480] 21.7 / 17.6.  In two rounds the second starts from nothing and the tiles are as good
+// or better: [728,3072] x [3072,448] 13.8 / 13.8, [1113,832] x [832,393] 8.9 / 10.3.  Only for a launch that owns the
+// device and says how many XCDs it has: the cells are dealt to them so that each fetches its own part of an operand.
+bool plan_cells(const iris_gemm_args& a, int op, bool dma_ok, Plan* plan) {
+  GemmKArgs& k = plan->k;
+  const int64_t lim = (int64_t)1 << 31, cus = current_cu_count();
+  const int64_t m_cells = (a.M + CELL - 1) / CELL, n_cells = (a.N + CELL - 1) / CELL, cells = m_cells * n_cells;
+  const bool counters = k.flag_mode == 0 || (a.locks && k.total_tiles <= a.num_sms);
+  const bool ok = a.K > 0 && dma_ok && !plan->in_program && cells <= cus && a.num_sms >= cus && a.num_xcds > 1 && (a.block_m >= a.M || a.block_m % CELL == 0) &&
+                  a.block_n % CELL == 0 && !a.mm_begin_timestamp && !a.mm_end_timestamp && (a.split_k == 0 || a.split_k == 1) &&
+                  counters && (CELL * a.stride_am + a.K) * 2 < lim && (CELL * a.stride_bn + a.K) * 2 < lim;
+  if (!ok) return false;
+  int parts = 1;
+  if (a.split_k == 0 && a.partials && aligned16(a.partials) && a.locks && k.total_tiles + cells <= a.num_sms) {
+    parts = few_rows_parts(cells, (a.K + 63) / 64, 0.6, (int64_t)a.N * a.K * 2);
+    if (parts * cells * (CELL * CELL) > (int64_t)a.num_sms * a.partials_slot_elems) parts = 1;
+  }
+  plan->skinny = gemm_skinny_kernel_for(a.ab_dtype, op, 16, 2, 2);
+  if (!plan->skinny) return false;
+  k.cells = (int)cells;
+  k.cells_by_row = a.M > a.N;
+  k.cells_inner = (int)(k.cells_by_row ? n_cells : m_cells);
+  k.xcd_per = (int)((cells + a.num_xcds - 1) / a.num_xcds);
+  k.div_inner = make_fast_div((uint32_t)k.cells_inner, (uint64_t)cells + 1);
+  k.div_xcd = make_fast_div((uint32_t)a.num_xcds, (uint64_t)k.xcd_per * a.num_xcds + 1);
+  plan->skinny_lds = cells_lds_bytes();
+  plan->skinny_grid = k.xcd_per * a.num_xcds;
+  plan->skinny_grid_y = 1;
+  plan->skinny_grid_z = parts;
+  plan->skinny_rb = 2;
+  plan->skinny_cb = 2;
   k.split_k = 1;
   k.locks = a.locks;
   k.partials = a.partials;
@@ -605,8 +645,10 @@ bool plan_parts(const iris_gemm_args& a, Plan* plan) {
 bool reduce_in_program(const iris_gemm_args& a, const Plan& producer) {
   if (a.num_sms < current_cu_count() || a.variant != 0 || a.split_k != 0 || a.mm_begin_timestamp || a.mm_end_timestamp) return true;
   if (!producer.entry && !producer.skinny) return true;  // (nothing to compute)
-  if (producer.skinny || producer.last_round || producer.rest || producer.parts) return false;
+  if ((producer.skinny && producer.skinny_cb == 1) || producer.last_round || producer.rest || producer.parts) return false;
   const GemmKArgs& k = producer.k;
+  // (cells: the caller's tiles inside, when they are as small as the parts they would be run in)
+  if (producer.skinny && a.block_m * a.block_n > 64 * 64) return false;
   if (k.split_k > 1 || k.merge_m * k.merge_n > 1 || k.total_tiles > a.num_sms || !k.vec_out) return false;
   const int steps = (a.K + 63) / 64;
   return steps <= 8 || (steps <= 24 && a.block_m * a.block_n <= 128 * 128);
@@ -817,6 +859,7 @@ hipError_t make_plan_body(const iris_gemm_args& a, Plan* plan) {
 
   if (a.variant == 0 || a.variant == IRIS_GEMM_VARIANT_FEW_ROWS) {
     if (plan_few_rows(a, op, dma_ok, plan)) return hipSuccess;
+    if (a.variant == 0 && plan_cells(a, op, dma_ok, plan)) return hipSuccess;
     if (a.variant == IRIS_GEMM_VARIANT_FEW_ROWS) return hipErrorInvalidValue;
   }
 
@@ -1170,7 +1213,7 @@ extern "C" int iris_gemm_plan_name(const iris_gemm_args* args, char* buf, size_t
   Plan plan;
   hipError_t err = make_plan(*args, &plan);
   if (err != hipSuccess) return err;
-  const char* few = plan.skinny_rb == 2 ? "few_rows_32xN" : "few_rows_16xN";
+  const char* few = plan.skinny_cb == 2 ? "cells_32x32" : plan.skinny_rb == 2 ? "few_rows_32xN" : "few_rows_16xN";
   std::snprintf(buf, len, "%s%s%s", plan.skinny ? few : plan.entry ? plan.entry->name : "",
                 plan.entry && plan.k.stream_k                   ? "+stream_k"
                 : plan.entry && plan.in_program                 ? "+reduce"

@@ -62,10 +62,23 @@ constexpr int SKINNY_MAX_SPLIT = 16;
 constexpr int skinny_a_bytes(int rb) { return SKINNY_WAVES * rb * SKINNY_BLOCK_BYTES; }
 constexpr int skinny_lds_bytes(int rb) { return skinny_a_bytes(rb) + SKINNY_WAVES * SKINNY_UN * SKINNY_BLOCK_BYTES; }
 
+// Blocks of 32 rows x 32 columns a workgroup (CB = 2): shard products of up to a few hundred rows, which in the
+// persistent kernel's tiles are too few to fill the chip or too short to pay for its fixed costs (its prologue, hand-over
+// and flag take 3 us more than this kernel's; sharing K out over programs 4 to 6 us).  Here the eight waves share K
+// inside the workgroup.  A comes in like B, by LDS-DMA, two blocks a wave in flight: 8 KiB a block of K, 128 KiB a
+// workgroup, one workgroup a CU.  It is bound by the CU's L1, 64 bytes a clock: 0.06 us for every 64 of K.
+// A lane's columns are eight in a row: the block j of a row of 32 columns takes columns 8q + 4j .. + 3, so that a row
+// leaves in 16-byte stores.  The cells are dealt to the XCDs in consecutive runs (the shorter direction first), so that
+// each XCD's L2 fetches its share of the longer operand once.
+constexpr int CELL = 32;
+// LDS of a workgroup of RB x CB blocks
+constexpr int cells_lds_bytes() { return SKINNY_WAVES * SKINNY_UN * 4 * SKINNY_BLOCK_BYTES; }
+
 // AROWS: rows of A in a block, 8 or 16.
 // RB: blocks of 16 rows a workgroup computes (1 for up to 32 rows; 2 up to 64
 // rows of a long K, and from 17 rows on where B is large).
-template <int DT, int OP, int ODT, int AROWS, int RB = 1>
+// CB: blocks of 16 columns, 1 or (with RB 2) 2.
+template <int DT, int OP, int ODT, int AROWS, int RB = 1, int CB = 1>
 __global__ __launch_bounds__(SKINNY_THREADS) __attribute__((amdgpu_waves_per_eu(2, 8))) void
 gemm_skinny_kernel(const GemmKArgs p) {
   constexpr bool ATOMIC = OP == OP_ATOMIC32 || OP == OP_ATOMIC16;
@@ -73,6 +86,9 @@ gemm_skinny_kernel(const GemmKArgs p) {
   constexpr int UN = SKINNY_UN, AH = AROWS / 8;  // fetches of a block of A
   static_assert(AROWS == 16 || (AROWS == 8 && RB == 1), "rows of a block of A");
   static_assert(RB == 1 || RB == 2, "blocks of rows per workgroup");
+  static_assert(CB == 1 || (CB == 2 && RB == 2 && AROWS == 16), "blocks of columns per workgroup");
+  constexpr bool A_DMA = CB == 2;  // A in LDS, UN blocks a wave, like B
+  constexpr int NB = RB * CB;
   using vec8 = typename Mfma<DT>::vec8;
   extern __shared__ __attribute__((aligned(1024))) char skinny_lds[];
   touch_args<sizeof(GemmKArgs)>();
@@ -84,14 +100,24 @@ gemm_skinny_kernel(const GemmKArgs p) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
   const int lr = lane & 15, lq = lane >> 4;
-  const int n0 = blockIdx.x * SKINNY_COLS;
-  const int m0 = blockIdx.y * (SKINNY_ROWS * RB);
-  IRIS_LDS char* wb = lds + skinny_a_bytes(RB) + wave * (UN * SKINNY_BLOCK_BYTES);
-  IRIS_LDS char* wa = lds + wave * (RB * SKINNY_BLOCK_BYTES);
+  int bx = blockIdx.x, by = blockIdx.y;  // the workgroup's block of columns and of rows
+  int cell = by * gridDim.x + bx;
+  if constexpr (CB == 2) {
+    const int round = (int)fast_div((uint32_t)bx, p.div_xcd);
+    cell = (bx - round * p.num_xcds) * p.xcd_per + round;
+    if (cell >= p.cells) return;
+    const int outer = (int)fast_div((uint32_t)cell, p.div_inner), inner = cell - outer * p.cells_inner;
+    bx = p.cells_by_row ? inner : outer;
+    by = p.cells_by_row ? outer : inner;
+  }
+  const int n0 = bx * (SKINNY_COLS * CB);
+  const int m0 = by * (SKINNY_ROWS * RB);
+  IRIS_LDS char* wb = lds + (A_DMA ? SKINNY_WAVES * UN * RB * SKINNY_BLOCK_BYTES : skinny_a_bytes(RB)) + wave * (UN * CB * SKINNY_BLOCK_BYTES);
+  IRIS_LDS char* wa = lds + wave * ((A_DMA ? UN : 1) * RB * SKINNY_BLOCK_BYTES);
 
   // Rows past the edge of either operand lie past the end of its buffer
   // descriptor and read as zero; chunks past K are parked out of range.
-  const int rows_b = min(SKINNY_COLS, p.N - n0);
+  const int rows_b = min(SKINNY_COLS * CB, p.N - n0);
   const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(
       (void*)(p.b + (int64_t)n0 * p.sbn * 2), 0, (int)((((int64_t)rows_b - 1) * p.sbn + p.K) * 2), 0x00020000);
   const int rows_a = min(SKINNY_ROWS * RB, p.M - m0);
@@ -100,7 +126,13 @@ gemm_skinny_kernel(const GemmKArgs p) {
   // B: lane l of fetch j of a block brings row 8j + l/8 and lands at byte
   // l*16 of the fetch's 1 KiB, i.e. at physical chunk l%8 of that row; the
   // chunk of the row it must bring there is (l%8) ^ (row/2 % 8).
+  // (CB 2: row 16j + r of the block's 32 holds column 8 (r / 4) + 4j + r % 4)
   const int brow = lane >> 3;  // + 8j
+  auto b_column = [&](int j) {
+    if constexpr (CB == 1) return brow + 8 * j;
+    const int r = brow + 8 * (j & 1);
+    return (r >> 2) * 8 + (j >> 1) * 4 + (r & 3);
+  };
   const int bchunk = (lane & 7) ^ ((brow >> 1) & 7);  // rows 8j + .. : (row/2)%8 = 4j + brow/2, and 4j flips bit 2
   // A comes in the same way, but into registers, and then goes through a 2 KiB
   // region of the wave, laid out like a block of B, on its way to the MFMAs.
@@ -115,19 +147,19 @@ gemm_skinny_kernel(const GemmKArgs p) {
   const int kb0 = blockIdx.z * share;
   const int nb = min(nb_all, kb0 + share);
 
-  f32x4 acc[RB];
+  f32x4 acc[NB];  // [row block][column block]
 #pragma unroll
-  for (int i = 0; i < RB; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < NB; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  u32x4 va[UN][RB][AH];
+  u32x4 va[A_DMA ? 1 : UN][RB][AH];
   // fetches of K block kb into set u (blocks past the end are parked: the number of loads never changes)
   auto fetch = [&](int u, int kb) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int ch = bchunk ^ (j << 2);
+    for (int j = 0; j < 2 * CB; ++j) {
+      const int ch = bchunk ^ ((j & 1) << 2);
       const bool ok = kb < nb && kb * 64 + ch * 8 < p.K;
-      const uint32_t off = (uint32_t)(((int64_t)(brow + 8 * j) * p.sbn) * 2 + kb * 128 + ch * 16);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (IRIS_LDS void*)(wb + u * SKINNY_BLOCK_BYTES + j * 1024), 16,
+      const uint32_t off = (uint32_t)(((int64_t)b_column(j) * p.sbn) * 2 + kb * 128 + ch * 16);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (IRIS_LDS void*)(wb + u * (CB * SKINNY_BLOCK_BYTES) + j * 1024), 16,
                                                ok ? (int)off : (int)0x80000000, 0, 0, 0);
     }
 #pragma unroll
@@ -137,29 +169,40 @@ gemm_skinny_kernel(const GemmKArgs p) {
         const int ch = bchunk ^ (j << 2);
         const bool ok = kb < nb && kb * 64 + ch * 8 < p.K;
         const uint32_t off = (uint32_t)(((int64_t)(i * 16 + brow + 8 * j) * p.sam) * 2 + kb * 128 + ch * 16);
-        va[u][i][j] = __builtin_amdgcn_raw_buffer_load_b128(ra, ok ? (int)off : (int)0x80000000, 0, 0);
+        if constexpr (A_DMA)
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(
+              ra, (IRIS_LDS void*)(wa + (u * RB + i) * SKINNY_BLOCK_BYTES + j * 1024), 16, ok ? (int)off : (int)0x80000000, 0, 0, 0);
+        else
+          va[u][i][j] = __builtin_amdgcn_raw_buffer_load_b128(ra, ok ? (int)off : (int)0x80000000, 0, 0);
       }
   };
   auto multiply = [&](int u) __attribute__((always_inline)) {
     // (the wave's LDS operations execute in order: these writes land after
     // the previous block's reads and before this block's)
+    if constexpr (!A_DMA) {
 #pragma unroll
-    for (int i = 0; i < RB; ++i)
+      for (int i = 0; i < RB; ++i)
 #pragma unroll
-      for (int j = 0; j < AH; ++j)
-        *reinterpret_cast<IRIS_LDS u32x4*>(wa + i * SKINNY_BLOCK_BYTES + j * 1024 + lane * 16) = va[u][i][j];
+        for (int j = 0; j < AH; ++j)
+          *reinterpret_cast<IRIS_LDS u32x4*>(wa + i * SKINNY_BLOCK_BYTES + j * 1024 + lane * 16) = va[u][i][j];
+    }
+    const IRIS_LDS char* sa = wa + (A_DMA ? u * (RB * SKINNY_BLOCK_BYTES) : 0);
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int pc = (lq * 2 + h) ^ ((lr >> 1) & 7);
-      const vec8 fb = *reinterpret_cast<const IRIS_LDS vec8*>(wb + u * SKINNY_BLOCK_BYTES + lr * 128 + pc * 16);
+      vec8 fb[CB];
+#pragma unroll
+      for (int j = 0; j < CB; ++j)
+        fb[j] = *reinterpret_cast<const IRIS_LDS vec8*>(wb + (u * CB + j) * SKINNY_BLOCK_BYTES + lr * 128 + pc * 16);
 #pragma unroll
       for (int i = 0; i < RB; ++i) {
-        const vec8 fa = *reinterpret_cast<const IRIS_LDS vec8*>(wa + i * SKINNY_BLOCK_BYTES + lr * 128 + pc * 16);
-        acc[i] = Mfma<DT>::run(fb, fa, acc[i]);
+        const vec8 fa = *reinterpret_cast<const IRIS_LDS vec8*>(sa + i * SKINNY_BLOCK_BYTES + lr * 128 + pc * 16);
+#pragma unroll
+        for (int j = 0; j < CB; ++j) acc[i * CB + j] = Mfma<DT>::run(fb[j], fa, acc[i * CB + j]);
       }
     }
   };
-  constexpr int LOADS = 2 + AH * RB;  // a block's
+  constexpr int LOADS = 2 * CB + AH * RB;  // a block's
   static_assert(LOADS * (UN - 1) <= 63, "vmcnt immediate");
   int b0 = kb0 + wave;
 #pragma unroll
@@ -194,20 +237,20 @@ gemm_skinny_kernel(const GemmKArgs p) {
   // persistent kernel).  The waves' partial sums meet in LDS, [wave][block][lane].
   __syncthreads();  // every wave is done with its blocks of A: the region becomes `red`
 #pragma unroll
-  for (int i = 0; i < RB; ++i) red[(wave * RB + i) * 64 + lane] = acc[i];
+  for (int i = 0; i < NB; ++i) red[(wave * NB + i) * 64 + lane] = acc[i];
   __syncthreads();
-  if constexpr (RB > 1) {
+  if constexpr (NB > 1) {
     // With several blocks every destination's wave would add up all of them:
-    // first each block is summed once, in wave order, by the 8 / RB waves that
+    // first each block is summed once, in wave order, by the 8 / NB waves that
     // share it (a part of the lanes each), and left in the first wave's place.
-    constexpr int WPB = SKINNY_WAVES / RB, LPW = 64 / WPB;  // waves per block, lanes of a block per wave
+    constexpr int WPB = SKINNY_WAVES / NB, LPW = 64 / WPB;  // waves per block, lanes of a block per wave
     const int blk = wave / WPB, l0 = (wave % WPB) * LPW;
     f32x4 s = {0.f, 0.f, 0.f, 0.f};
     const bool mine = lane >= l0 && lane < l0 + LPW;
     if (mine) {
       s = red[blk * 64 + lane];
 #pragma unroll
-      for (int w = 1; w < SKINNY_WAVES; ++w) s += red[(w * RB + blk) * 64 + lane];  // wave order
+      for (int w = 1; w < SKINNY_WAVES; ++w) s += red[(w * NB + blk) * 64 + lane];  // wave order
     }
     __syncthreads();  // all partial sums have been read
     if (mine) red[blk * 64 + lane] = s;
@@ -219,15 +262,14 @@ gemm_skinny_kernel(const GemmKArgs p) {
     // K shared out over gridDim.z groups: each leaves its sum in `partials` (register order, 1 KiB a block), and
     // the last to arrive at the blocks' counter adds all of them up, in the order of K, and goes on to the
     // stores.  Nobody waits: any number of the groups can be resident.
-    const int cell = blockIdx.y * gridDim.x + blockIdx.x;
-    const uint32_t span = (uint32_t)(gridDim.x * gridDim.y) * (RB * 1024);  // bytes of one share's sums
-    IRIS_LDS int* is_last = (IRIS_LDS int*)(lds + RB * 1024);  // (behind the blocks' sums)
+    const uint32_t span = (uint32_t)(CB == 2 ? p.cells : (int)(gridDim.x * gridDim.y)) * (NB * 1024);  // bytes of one share's sums
+    IRIS_LDS int* is_last = (IRIS_LDS int*)(lds + NB * 1024);  // (behind the blocks' sums)
     if (wave == 0) {
-      f32x4 s[RB];
+      f32x4 s[NB];
 #pragma unroll
-      for (int b = 0; b < RB; ++b) {
+      for (int b = 0; b < NB; ++b) {
         s[b] = red[b * 64 + lane];
-        if constexpr (RB == 1) {
+        if constexpr (NB == 1) {
 #pragma unroll
           for (int w = 1; w < SKINNY_WAVES; ++w) s[b] += red[w * 64 + lane];
         }
@@ -235,9 +277,9 @@ gemm_skinny_kernel(const GemmKArgs p) {
       const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
           (void*)p.partials, 0, (int)(span * gridDim.z), 0x00020000);
 #pragma unroll
-      for (int b = 0; b < RB; ++b)
+      for (int b = 0; b < NB; ++b)
         __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, s[b]), rs,
-                                               (int)(blockIdx.z * span + (cell * RB + b) * 1024 + lane * 16), 0, AUX_SC1);
+                                               (int)(blockIdx.z * span + (cell * NB + b) * 1024 + lane * 16), 0, AUX_SC1);
       IRIS_WAIT_VMCNT(0);
       asm volatile("" ::: "memory");
       IRIS_GLOBAL int32_t* cnt = (IRIS_GLOBAL int32_t*)(p.locks + p.total_tiles + cell);
@@ -249,24 +291,24 @@ gemm_skinny_kernel(const GemmKArgs p) {
       last = __builtin_amdgcn_readfirstlane(last);
       asm volatile("" ::: "memory");
       if (last) {
-        constexpr int G = 8 / RB;  // shares in flight
+        constexpr int G = 8 / NB;  // shares in flight
 #pragma unroll
-        for (int b = 0; b < RB; ++b) s[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int b = 0; b < NB; ++b) s[b] = f32x4{0.f, 0.f, 0.f, 0.f};
         for (int z0 = 0; z0 < (int)gridDim.z; z0 += G) {
-          u32x4 v[G][RB];
+          u32x4 v[G][NB];
 #pragma unroll
           for (int g = 0; g < G; ++g)
 #pragma unroll
-            for (int b = 0; b < RB; ++b)  // (shares past the last lie past the descriptor: zero)
+            for (int b = 0; b < NB; ++b)  // (shares past the last lie past the descriptor: zero)
               v[g][b] = __builtin_amdgcn_raw_buffer_load_b128(
-                  rs, (int)((z0 + g) * span + (cell * RB + b) * 1024 + lane * 16), 0, AUX_SC1);
+                  rs, (int)((z0 + g) * span + (cell * NB + b) * 1024 + lane * 16), 0, AUX_SC1);
 #pragma unroll
           for (int g = 0; g < G; ++g)
 #pragma unroll
-            for (int b = 0; b < RB; ++b) s[b] += __builtin_bit_cast(f32x4, v[g][b]);
+            for (int b = 0; b < NB; ++b) s[b] += __builtin_bit_cast(f32x4, v[g][b]);
         }
 #pragma unroll
-        for (int b = 0; b < RB; ++b) red[b * 64 + lane] = s[b];
+        for (int b = 0; b < NB; ++b) red[b * 64 + lane] = s[b];
       }
       if (lane == 0) *is_last = last;
     }
@@ -276,68 +318,85 @@ gemm_skinny_kernel(const GemmKArgs p) {
 
   const int r_begin = p.dest_all ? 0 : p.cur_rank;
   const int r_end = p.dest_all ? p.ws : p.cur_rank + 1;
-  if (r_begin + wave < r_end) {
-#pragma unroll
-    for (int i = 0; i < RB; ++i) {
-      const int m = m0 + i * 16 + lr, n = n0 + lq * 4;
-      if (m >= p.M || n >= p.N) continue;
-      f32x4 s = red[i * 64 + lane];
-      if (RB == 1 && !split) {
-#pragma unroll
-        for (int w = 1; w < SKINNY_WAVES; ++w) s += red[w * 64 + lane];  // wave order: the sum does not depend on timing
-      }
-      constexpr int ES = F32 ? 4 : 2;
-      for (int r = r_begin + wave; r < r_end; r += SKINNY_WAVES) {
-        IRIS_GLOBAL char* dst = rank_ptr(p, p.out, r);
-        if constexpr (ATOMIC) {
-          // 08: add into the destination (gemm_atomics_all_reduce.py:236-248)
-          if constexpr (OP == OP_ATOMIC16) {
-            if (p.row_out) {
-              const int valid = min(4, p.N - n);
-              atomic_add16_strip<ODT>(dst + ((int64_t)m * p.som + n) * ES, s, valid, n > 0, n + valid < p.N);
-              continue;
-            }
-          }
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            if (n + e >= p.N) continue;
-            IRIS_GLOBAL char* d = dst + ((int64_t)m * p.som + (int64_t)(n + e) * p.son) * ES;
-            const float f = s[e];
-            if constexpr (OP == OP_ATOMIC32)
-              __hip_atomic_fetch_add((IRIS_GLOBAL float*)d, f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            else
-              atomic_add16_cas<ODT>((IRIS_GLOBAL unsigned short*)d, from16<ODT>(to16<ODT>(f)));
-          }
-        } else if (p.row_out && n + 4 <= p.N) {
-          // four columns in one store (at any address: rows of an odd length are no exception)
-          IRIS_GLOBAL char* d = dst + ((int64_t)m * p.som + n) * ES;
-          if constexpr (F32) {
-            const u32x4 v = __builtin_bit_cast(u32x4, s);
-            if (p.sys)
-              store16_any<AUX_SC0 | AUX_SC1>(d, v);
-            else
-              store16_any<AUX_SC1>(d, v);
-          } else {
-            const u32x2 v = {pack2<ODT>(s[0], s[1]), pack2<ODT>(s[2], s[3])};
-            if (p.sys)
-              store8_any<AUX_SC0 | AUX_SC1>(d, v);
-            else
-              store8_any<AUX_SC1>(d, v);
-          }
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            if (n + e >= p.N) continue;
-            IRIS_GLOBAL char* d = dst + ((int64_t)m * p.som + (int64_t)(n + e) * p.son) * ES;
-            const float f = s[e];
-            if constexpr (F32)
-              store_through((IRIS_GLOBAL unsigned int*)d, __builtin_bit_cast(unsigned int, f), p.sys != 0);
-            else
-              store_through((IRIS_GLOBAL unsigned short*)d, to16<ODT>(s[e]), p.sys != 0);
-          }
+  constexpr int ES = F32 ? 4 : 2;
+  // four columns of a row, from column n on
+  auto store4 = [&](IRIS_GLOBAL char* dst, int m, int n, f32x4 s) __attribute__((always_inline)) {
+    if constexpr (ATOMIC) {
+      // 08: add into the destination (gemm_atomics_all_reduce.py:236-248)
+      if constexpr (OP == OP_ATOMIC16) {
+        if (p.row_out) {
+          const int valid = min(4, p.N - n);
+          atomic_add16_strip<ODT>(dst + ((int64_t)m * p.som + n) * ES, s, valid, n > 0, n + valid < p.N);
+          return;
         }
       }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (n + e >= p.N) continue;
+        IRIS_GLOBAL char* d = dst + ((int64_t)m * p.som + (int64_t)(n + e) * p.son) * ES;
+        const float f = s[e];
+        if constexpr (OP == OP_ATOMIC32)
+          __hip_atomic_fetch_add((IRIS_GLOBAL float*)d, f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        else
+          atomic_add16_cas<ODT>((IRIS_GLOBAL unsigned short*)d, from16<ODT>(to16<ODT>(f)));
+      }
+    } else if (p.row_out && n + 4 <= p.N) {
+      // four columns in one store (at any address: rows of an odd length are no exception)
+      IRIS_GLOBAL char* d = dst + ((int64_t)m * p.som + n) * ES;
+      if constexpr (F32) {
+        const u32x4 v = __builtin_bit_cast(u32x4, s);
+        if (p.sys)
+          store16_any<AUX_SC0 | AUX_SC1>(d, v);
+        else
+          store16_any<AUX_SC1>(d, v);
+      } else {
+        const u32x2 v = {pack2<ODT>(s[0], s[1]), pack2<ODT>(s[2], s[3])};
+        if (p.sys)
+          store8_any<AUX_SC0 | AUX_SC1>(d, v);
+        else
+          store8_any<AUX_SC1>(d, v);
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (n + e >= p.N) continue;
+        IRIS_GLOBAL char* d = dst + ((int64_t)m * p.som + (int64_t)(n + e) * p.son) * ES;
+        const float f = s[e];
+        if constexpr (F32)
+          store_through((IRIS_GLOBAL unsigned int*)d, __builtin_bit_cast(unsigned int, f), p.sys != 0);
+        else
+          store_through((IRIS_GLOBAL unsigned short*)d, to16<ODT>(s[e]), p.sys != 0);
+      }
     }
+  };
+  // (rank, row block) pairs over the waves
+  for (int it = wave; it < (r_end - r_begin) * RB; it += SKINNY_WAVES) {
+    const int r = r_begin + it / RB, i = it % RB;
+    const int m = m0 + i * 16 + lr, n = n0 + lq * (4 * CB);
+    if (m >= p.M || n >= p.N) continue;
+    IRIS_GLOBAL char* dst = rank_ptr(p, p.out, r);
+    f32x4 s[CB];
+#pragma unroll
+    for (int j = 0; j < CB; ++j) s[j] = red[(i * CB + j) * 64 + lane];
+    if (NB == 1 && !split) {
+#pragma unroll
+      for (int w = 1; w < SKINNY_WAVES; ++w) s[0] += red[w * 64 + lane];  // wave order: the sum does not depend on timing
+    }
+    if constexpr (CB == 2 && !ATOMIC && !F32) {
+      if (p.row_out && n + 8 <= p.N) {
+        IRIS_GLOBAL char* d = dst + ((int64_t)m * p.som + n) * ES;
+        const u32x4 v = {pack2<ODT>(s[0][0], s[0][1]), pack2<ODT>(s[0][2], s[0][3]), pack2<ODT>(s[1][0], s[1][1]),
+                         pack2<ODT>(s[1][2], s[1][3])};
+        if (p.sys)
+          store16_any<AUX_SC0 | AUX_SC1>(d, v);
+        else
+          store16_any<AUX_SC1>(d, v);
+        continue;
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < CB; ++j)
+      if (n + 4 * j < p.N) store4(dst, m, n + 4 * j, s[j]);
   }
   if (p.flag_mode == 0) return;
 
@@ -349,7 +408,8 @@ gemm_skinny_kernel(const GemmKArgs p) {
     const int pid_m = m0 / p.BM, pid_n = n0 / p.BN;
     const int tile_id = tile_id_of(pid_m, pid_n, p.num_pid_m, p.num_pid_n, p.G);
     const int cols = min(p.N, (pid_n + 1) * p.BN) - pid_n * p.BN, rows = min(p.M, (pid_m + 1) * p.BM) - pid_m * p.BM;
-    const int parts = ((cols + SKINNY_COLS - 1) / SKINNY_COLS) * ((rows + SKINNY_ROWS * RB - 1) / (SKINNY_ROWS * RB));
+    constexpr int COLS = SKINNY_COLS * CB;
+    const int parts = ((cols + COLS - 1) / COLS) * ((rows + SKINNY_ROWS * RB - 1) / (SKINNY_ROWS * RB));
     int last = 1;
     if (parts > 1) {
       IRIS_GLOBAL int32_t* cnt = (IRIS_GLOBAL int32_t*)(p.locks + tile_id);
@@ -363,7 +423,7 @@ gemm_skinny_kernel(const GemmKArgs p) {
   }
 }
 
-// The kernel for (operand type, store op, rows of A in a block, blocks of rows a workgroup), or null.
-GemmKernelFn gemm_skinny_kernel_for(int dt, int op, int arows, int rb);
+// The kernel for (operand type, store op, rows of A in a block, blocks of rows and of columns a workgroup), or null.
+GemmKernelFn gemm_skinny_kernel_for(int dt, int op, int arows, int rb, int cb = 1);
 
 }  // namespace iris_amd
