@@ -73,6 +73,12 @@ const GemmKernelEntry* plain_twin(const GemmKernelEntry* list, int count, const 
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
+// Whether every row of both operands (K-contiguous) starts on a cache line; strides in 16-bit units.
+bool whole_lines(const iris_gemm_args& a) {
+  return a.stride_am % 64 == 0 && a.stride_bn % 64 == 0 &&
+         ((reinterpret_cast<uintptr_t>(a.a) | reinterpret_cast<uintptr_t>(a.b)) & 127) == 0;
+}
+
 // 16-byte vector access on a row-major [rows, cols] view of `es`-byte elements
 bool vec_ok(const void* base, int64_t stride_m, int64_t stride_n, int es) {
   return stride_n == 1 && aligned16(base) && ((stride_m * es) % 16) == 0;
@@ -190,6 +196,7 @@ bool plan_few_rows(const iris_gemm_args& a, int op, bool dma_ok, Plan* plan) {
 // 9.0; fp32 [475,2560] x [2560,480] 21.7 / 17.6.  In two rounds the second starts from nothing and the tiles are as good
 // or better: [728,3072] x [3072,448] 13.8 / 13.8, [1113,832] x [832,393] 8.9 / 10.3.  Only for a launch that owns the
 // device and says how many XCDs it has: the cells are dealt to them so that each fetches its own part of an operand.
+// Whether it is better than tiles at the launch's K is for plan_small to say.
 bool plan_cells(const iris_gemm_args& a, int op, bool dma_ok, Plan* plan) {
   GemmKArgs& k = plan->k;
   const int64_t lim = (int64_t)1 << 31, cus = current_cu_count();
@@ -222,6 +229,18 @@ bool plan_cells(const iris_gemm_args& a, int op, bool dma_ok, Plan* plan) {
   k.locks = a.locks;
   k.partials = a.partials;
   return true;
+}
+
+// Parts of K for `tiles` tiles of `steps` K-steps of 64 (1: unsplit).  The hand-over of partials costs about as much as ten
+// K-steps of a small tile: as many parts as there are idle programs, at least four K-steps each, and a K loop shorter
+// than 32 steps is only split in four or more parts (measured on [M, 1376] x [1376, 4096], 22 steps of 128 x 128 tiles:
+// 4 parts 16.4 against 19.5 us unsplit at 128 rows, 2 parts 25.9 against 20.2 at 512).
+int auto_split(int64_t tiles, int steps, int programs) {
+  if (tiles * 2 > programs || steps < 16) return 1;
+  int sk = (int)(programs / tiles);
+  if (sk > steps / 4) sk = steps / 4;
+  if (sk > 16) sk = 16;
+  return sk >= 4 || steps >= 32 ? sk : 1;
 }
 
 // Split-K and stream-K.  The owner of a tile waits for the programs that hold
@@ -272,21 +291,9 @@ hipError_t plan_split(const iris_gemm_args& a, const GemmKernelEntry& pick, bool
         return hipErrorInvalidValue;
       k.split_k = a.split_k;
     } else if (possible || pair_ok) {
-      if (k.total_tiles * 2 <= a.num_sms && nk * d >= 16) {
-        // The hand-over of partials costs about as much as ten K-steps of a
-        // small tile: as many parts as there are idle programs, at least four
-        // K-steps each, and a K loop shorter than 32 steps is only split in
-        // four or more parts (measured on [M, 1376] x [1376, 4096], 22 steps of
-        // 128 x 128 tiles: 4 parts 16.4 against 19.5 us unsplit at 128 rows,
-        // 2 parts 25.9 against 20.2 at 512).
-        int sk = a.num_sms / k.total_tiles;
-        if (sk > nk * d / 4) sk = nk * d / 4;
-        if (sk > 16) sk = 16;
-        if (!possible && sk > 2) sk = 2;  // (slots of half a tile: two parts)
-        if (sk >= 4 || (sk > 1 && nk * d >= 32)) {
-          k.split_k = sk;
-        }
-      }
+      int sk = auto_split(k.total_tiles, nk * d, a.num_sms);
+      if (!possible && sk > 2) sk = 2;  // (slots of half a tile: two parts)
+      if (sk >= 4 || (sk > 1 && nk * d >= 32)) k.split_k = sk;
       // Stream-K is only taken on request.  With the plain four-wave tiles it beat both the
       // unsplit and the split launch where the tiles left programs idle and the walk was long
       // (132 tiles of 64 steps on 256 programs: -17 %).  The tiles with fetching waves made
@@ -430,7 +437,8 @@ void launch_constants(const iris_gemm_args& a, const GemmKernelEntry& pick, Gemm
 // Validate `a` and build the launch plan.  Returns hipSuccess,
 // hipErrorInvalidValue, or a pseudo-success with entry == nullptr when there
 // is no GEMM work to do.
-hipError_t make_plan_body(const iris_gemm_args& a, Plan* plan);
+// `cells`: as cells of 32 x 32, if the launch can be (the caller asks with `skinny_cb`).
+hipError_t make_plan_body(const iris_gemm_args& a, Plan* plan, bool cells = false);
 
 // A long GEMM whose tiles are a few more than a multiple of the programs spends a whole round on those few:
 // 288 tiles on 256 programs take two rounds for 1.125 rounds of work.  Where a tile's walk over K is long
@@ -570,67 +578,188 @@ hipError_t make_plan(const iris_gemm_args& a, Plan* plan) {
   return make_plan_units(b, plan);
 }
 
-// A caller's tile is the unit of a flag, not of work: where its tiles are too few for the programs, the launch is
-// planned in parts of them, 64 x 64 or the next larger tile that still gives every part a program of its own in one
-// round.  The parts of a tile count their arrivals in the caller's locks; the last one raises its flag.
-// [1000,1504] x [1504,999] in 256 x 64 tiles: 64 tiles, K in four parts, 21.6 us; 256 parts of 64 x 64, 10.7.
-// [1418,384] x [384,224] in 256 x 256 tiles: 13.9 as 6 tiles, 6.7 as 92 parts.  [627,14528] x [14528,3208] in
-// 128 x 128 tiles: 130 tiles for 256 programs 82.7 us, 255 parts of 128 x 64 69.7.  Only what the few-rows kernel does
-// not take, for a launch that owns the device and leaves tile and split to the launcher.
-bool plan_parts(const iris_gemm_args& a, Plan* plan) {
-  if (a.variant != 0 || a.split_k != 0 || a.mm_begin_timestamp || a.mm_end_timestamp || a.M <= 0 || a.N <= 0 || a.K <= 0) return false;
-  if (a.block_m <= 0 || a.block_n <= 0 || a.num_sms != current_cu_count()) return false;
+// A plan whose tiles are the caller's.
+void own_flags(Plan* plan) {
+  GemmKArgs& k = plan->k;
+  k.merge_m = k.merge_n = 1;
+  k.flag_num_pid_m = k.num_pid_m;
+  k.flag_num_pid_n = k.num_pid_n;
+  k.flag_pn_base = 0;
+}
+
+// Estimated times of a small product's launch, in us: what plan_small compares its plans by.  A CU fetches 108 KB a us
+// (its L1), an eighth less when all of them do (L2); rows that start anywhere on a cache line touch half as many lines
+// again, and a gathering tile's fetching waves need three times as long.  A K-step takes as long as its operands, or as
+// the matrix cores where those are slower.  Around the K loop: the launch, the arrival counters of parts, the epilogue
+// (each rank's copy), and for a shared K the hand-over, which grows with the partials that cross memory.  The constants
+// are a fit to 8200 timings of 33 shapes ([24,8192] .. [96,2560] .. [4477,136] .. [1500,1500]) at K from 152 to 36864:
+// every tile, cells, up to 16 parts of K, 16-bit and fp32, weights in rows of either direction and at any alignment,
+// stores and atomics.  The plan with the least of these times is on average 0.4 % over the fastest one timed, in one case
+// of 100 more than 8 %.
+struct TileLaunch {
+  int cm, cn;
+  int64_t tiles;  // (the caller's, `subs` of these to one, or parts of the caller's)
+  int subs, split_k;
+  bool sliced, parts;
+};
+struct Operands {
+  bool f32, lines, gather, atomic, vec_out;
+  int copies;     // of the output
+  int64_t tile;   // elements of a caller's tile that lie in the output
+};
+double tiles_us(const iris_gemm_args& a, const TileLaunch& t, const Operands& o, int64_t cus) {
+  const int64_t items = t.tiles * t.split_k, programs = items < cus ? items : cus;
+  const bool split = t.split_k > 1;
+  const double cover = programs * 5 > cus * 4 ? 1.0 : 0.0;  // (nearly) every CU fetches
+  const double area = (double)t.cm * t.cn / 4096, partials = programs * area / 64;  // tiles of 64 x 64; MB
+  const bool deep = t.cm == 64 && t.cn == 64;  // (K-steps of 128: whole lines, mostly)
+  const double fetch = (t.cm + t.cn) / (8 * 108.0) * (1 + 0.13 * cover + (split ? 0.17 : 0.0)) *
+                       (o.gather ? 2.9 : o.lines ? 1.0 : deep ? 1.37 : 1.69);
+  const double multiply = o.f32 ? area * 0.452 * (1 + 0.04 * cover) + 0.1 : area * 0.0535;
+  const int64_t unit = deep ? 2 : 1, nk = ((int64_t)a.K + 64 * unit - 1) / (64 * unit);
+  const int64_t part_steps = (nk + t.split_k - 1) / t.split_k * unit, steps = (items + cus - 1) / cus * t.subs * part_steps;
+  const double loop = steps * (fetch > multiply ? fetch : multiply);
+  // (from the last-level cache, or from HBM, which a few programs do not keep busy)
+  const double mb = ((double)a.M + a.N) * a.K * 2e-6, rate = mb > 200 ? 2 + 3.5 * programs / cus : 5.5;
+  const double stream = mb / rate - 6.9;
+  double us = 7.4 + 0.005 * programs + 0.1 * area * (o.copies - 1) + (loop > stream ? loop : stream);
+  if (o.gather) us += 2.3 + 0.24 * area;
+  if (o.atomic) us += 1.5 * area;
+  if (t.parts && !o.atomic) {
+    const double per_tile = (double)o.tile / (t.cm * t.cn) / 16;  // (the more parts count on one word, the longer it takes)
+    us += 0.1 + 0.008 * programs * (per_tile < 1 ? per_tile : 1.0);
+  }
+  if (!split) {
+    us += area > 4 ? 2.4 : 0.1 * area;
+    if (!o.vec_out) us += area < 4 ? 1.5 * area : 6.0;  // (rows that 16-byte stores don't fit)
+  } else {
+    us += 3.1 + 0.53 * area + 0.2 * (partials < 16 ? partials : 16) + (partials > 16 ? 0.4 * (partials - 16) : 0.0);
+    // (an owner adds the parts of a tile one after another)
+    if (!t.sliced && area > 1) us += 0.31 * area * (t.split_k - 1);
+    // (a short part pays for the 256 x 64 tile's prefetch hints)
+    if (!o.f32 && t.cm == 256 && t.cn == 64 && nk >= 128 && part_steps < 64) us += 5;
+  }
+  return us;
+}
+double cells_us(const iris_gemm_args& a, int64_t cells, int parts, const Operands& o, int64_t cus) {
+  const int64_t groups = cells * parts, nk = ((int64_t)a.K + 63) / 64;
+  const double lines = o.lines ? 1.0 : 1.0 + 1.35 * (groups < 256 ? groups : 256) / 256;  // (both operands come in by lines of K = 64)
+  const double step = 0.083 * (groups * 5 > cus * 4 ? 1.09 : 1.0) * (o.f32 && lines < 1.65 ? 1.65 : lines);
+  // (a workgroup's first sixteen blocks of K are in flight together)
+  const double loop = ((groups + cus - 1) / cus * ((nk + parts - 1) / parts) - 16) * step;
+  const double mb = ((double)a.M + a.N) * a.K * 2e-6;
+  const double stream = mb / (mb > 200 ? 4.4 : 8.4) - 3, k_time = loop > stream ? loop : stream;
+  const double per_tile = o.atomic ? 0.0 : (double)o.tile / (CELL * CELL) / 64;
+  return 5.85 + (0.0075 + 0.004 * (per_tile < 1 ? per_tile : 1.0)) * groups + 0.025 * (o.copies - 1) + (parts > 1 ? 0.7 : 0.0) +
+         (o.atomic ? 0.4 : 0.0) + (k_time > 0 ? k_time : 0.0);
+}
+
+// The launch in parts of the caller's tiles, `cm` x `cn` each, every part with a program of its own in one round, K
+// shared out in split_k.  A caller's tile is the unit of a flag, not of work: the parts of a tile count their arrivals in
+// the caller's locks (`words` of them), and the last one raises its flag.
+bool plan_parts(const iris_gemm_args& a, int cm, int cn, int split_k, int64_t words, Plan* plan) {
+  iris_gemm_args b = a;
+  b.block_m = cm;
+  b.block_n = cn;
+  b.variant = IRIS_GEMM_VARIANT_PERSISTENT;
+  b.split_k = split_k;
+  if (make_plan_body(b, plan) != hipSuccess) return false;
+  GemmKArgs& k = plan->k;
+  if (!plan->entry || plan->entry->cm != cm || plan->entry->cn != cn || k.sub_m != 1 || k.sub_n != 1 ||
+      plan->entry->fetch_waves == 0 || k.num_sms != a.num_sms)
+    return false;
+  own_flags(plan);
+  k.flag_num_pid_m = (a.M + a.block_m - 1) / a.block_m;
+  k.flag_num_pid_n = (a.N + a.block_n - 1) / a.block_n;
+  if (words > 0) {
+    k.part_m = a.block_m / cm;
+    k.part_n = a.block_n / cn;
+    k.tile_arrivals = a.locks + (a.num_sms - words);
+  }
+  plan->parts = 1;
+  return true;
+}
+
+// A small product: the caller's tiles, cells of 32 x 32, or parts of the caller's tiles, whichever is expected to finish
+// first, each with K shared out as its own rule has it, parts also without.  Returns false for the caller's
+// tiles.  us a pass, the caller's tiles / the best parts / cells:
+//   [1000,1504] x [1504,999] in 256 x 64 tiles  21.6 (K in four) / 10.7 / -
+//   [512,512] in 256 x 128 tiles                K 1024 12.3 / 10.2 / 9.0   16384 26.6 / 25.8 / 28.8   36864 33.5 / 33.3 / 61
+//   [256,2048] in 128 x 128 tiles               K 2048 17.8 / 13.3 / -     8192 25.7 / 24.8 / -       36864 48 / 65 / -
+// Small tiles fill the chip and fetch more for the work they do: their K-steps are many times as many as those of a
+// large tile whose K is shared out, so they lose to it from some K on.  Only what the few-rows kernel does not take;
+// parts for a launch that owns the device and leaves tile and split to the launcher.
+bool plan_small(const iris_gemm_args& a, Plan* plan) {
+  const int64_t cus = current_cu_count();
+  if (a.variant != 0 || (a.split_k != 0 && a.split_k != 1) || a.mm_begin_timestamp || a.mm_end_timestamp) return false;
+  if (a.M <= 0 || a.N <= 0 || a.K <= 0 || a.block_m <= 0 || a.block_n <= 0 || a.num_sms < cus) return false;
   if (a.epilogue == IRIS_EPI_ONE_SHOT && (a.phase == IRIS_PHASE_FUSED || a.phase == IRIS_PHASE_CONSUME)) return false;
+  auto tiles_of = [&](int cm, int cn) { return ((int64_t)a.M + cm - 1) / cm * (((int64_t)a.N + cn - 1) / cn); };
+  if (tiles_of(128, 128) > a.num_sms) return false;
+  Plan whole;
+  if (make_plan_body(a, &whole) != hipSuccess || whole.skinny || !whole.entry) return false;
+  const GemmKArgs& w = whole.k;
+  const Operands o{a.ab_dtype == IRIS_DTYPE_F32, whole_lines(a), !whole.entry->dma,
+                   a.epilogue == IRIS_EPI_ATOMIC_ADD, w.vec_out != 0, w.dest_all ? a.world_size : 1,
+                   (int64_t)(a.block_m < a.M ? a.block_m : a.M) * (a.block_n < a.N ? a.block_n : a.N)};
+  double least = tiles_us(a, TileLaunch{whole.entry->cm, whole.entry->cn, w.total_tiles, w.sub_m * w.sub_n, w.split_k,
+                                        w.sliced != 0, false}, o, cus);
+  bool found = false;
+  if (tiles_of(CELL, CELL) <= cus) {
+    Plan cells;
+    if (make_plan_body(a, &cells, true) == hipSuccess && cells.skinny_cb == 2) {
+      const double us = cells_us(a, cells.k.cells, cells.skinny_grid_z, o, cus);
+      if (us < least) {
+        least = us;
+        own_flags(&cells);
+        *plan = cells;
+        found = true;
+      }
+    }
+  }
   // (fp32 operands, K in 16-bit units here: the tiles for longer K)
-  if (a.ab_dtype == IRIS_DTYPE_F32 && a.K < 1024) return false;
+  if (a.split_k != 0 || a.num_sms != cus || (a.ab_dtype == IRIS_DTYPE_F32 && a.K < 1024)) return found;
   const bool flags = a.epilogue == IRIS_EPI_ALL_SCATTER ? a.notify != 0 : a.epilogue == IRIS_EPI_ONE_SHOT && a.world_size > 1;
-  const int64_t flag_m = (a.M + (int64_t)a.block_m - 1) / a.block_m, flag_n = (a.N + (int64_t)a.block_n - 1) / a.block_n;
-  const int64_t words = flags ? flag_m * flag_n : 0;
-  if (words > 0 && (!a.locks || words > a.num_sms)) return false;
+  const int64_t words = flags ? tiles_of(a.block_m, a.block_n) : 0;
+  if (words > 0 && (!a.locks || words > a.num_sms)) return found;
   static const int shapes[4][2] = {{64, 64}, {128, 64}, {64, 128}, {128, 128}};
+  TileLaunch list[8];
+  double times[8];
+  int count = 0;
   for (const auto& s : shapes) {
-    const int cm = s[0], cn = s[1];
-    if (a.block_m % cm != 0 || a.block_n % cn != 0) continue;
-    const int64_t tiles = ((a.M + (int64_t)cm - 1) / cm) * ((a.N + (int64_t)cn - 1) / cn);
+    if (a.block_m % s[0] != 0 || a.block_n % s[1] != 0) continue;
+    const int64_t tiles = tiles_of(s[0], s[1]);
     if (tiles > a.num_sms) continue;
-    if (cm == a.block_m && cn == a.block_n) return false;  // (the caller's tile is the smallest that fits)
-    Plan whole;
-    if (make_plan_body(a, &whole) != hipSuccess || whole.skinny) return false;
+    if (s[0] == a.block_m && s[1] == a.block_n) break;  // (the caller's tile is the smallest that fits)
     // (a larger part than 64 x 64 only halves or quarters the tile; where K is shared out over as many programs that
     // has been done)
-    if (cm * cn > 64 * 64 && whole.k.split_k > 1) return false;
-    iris_gemm_args b = a;
-    b.block_m = cm;
-    b.block_n = cn;
-    b.variant = IRIS_GEMM_VARIANT_PERSISTENT;
-    Plan parts;
-    if (make_plan_body(b, &parts) != hipSuccess || !parts.entry) return false;
-    auto fits = [&](const Plan& q) {
-      return q.entry && q.entry->cm == cm && q.entry->cn == cn && q.k.sub_m == 1 && q.k.sub_n == 1 && !q.k.stream_k &&
-             q.entry->fetch_waves > 0 && q.k.num_sms == a.num_sms;
-    };
-    if (!fits(parts)) continue;
-    if (parts.k.split_k > 1 && parts.k.total_tiles * (int64_t)parts.k.split_k + words > a.num_sms) {
-      // (the parts of a part's K use the locks, too)
-      const int64_t sk = (a.num_sms - words) / parts.k.total_tiles;
-      b.split_k = sk >= 2 ? (int)sk : 1;
-      parts = Plan();
-      if (make_plan_body(b, &parts) != hipSuccess || !fits(parts)) continue;
+    if (s[0] * s[1] > 64 * 64 && w.split_k > 1) break;
+    const int bk = s[0] == 64 && s[1] == 64 ? 128 : 64;  // (the 64 x 64 tile's K-step)
+    int sk = a.partials && a.locks ? auto_split(tiles, (int)(((int64_t)a.K + bk - 1) / bk) * (bk / 64), a.num_sms) : 1;
+    // (the parts of a part's K use the locks, too)
+    if (tiles * sk + words > a.num_sms) sk = (int)((a.num_sms - words) / tiles);
+    for (int split_k = 1;; split_k = sk) {
+      const TileLaunch t{s[0], s[1], tiles, 1, split_k, split_k >= 8, true};
+      list[count] = t;
+      times[count++] = tiles_us(a, t, o, cus);
+      if (split_k >= sk) break;
     }
-    parts.k.merge_m = parts.k.merge_n = 1;
-    parts.k.flag_num_pid_m = (int)flag_m;
-    parts.k.flag_num_pid_n = (int)flag_n;
-    parts.k.flag_pn_base = 0;
-    if (words > 0) {
-      parts.k.part_m = a.block_m / cm;
-      parts.k.part_n = a.block_n / cn;
-      parts.k.tile_arrivals = a.locks + (a.num_sms - words);
-    }
-    parts.parts = 1;
-    *plan = parts;
-    return true;
+    // (the gathering tiles' times scatter more: the first shape that fits, unless another is clearly ahead of it)
+    if (o.gather && s[0] * s[1] == 64 * 64) times[count - 1] *= 0.9;
   }
-  return false;
+  // the best of them that there is a kernel for
+  for (;;) {
+    int best = -1;
+    for (int i = 0; i < count; ++i)
+      if (times[i] < least && (best < 0 || times[i] < times[best])) best = i;
+    if (best < 0) return found;
+    Plan parts;
+    if (plan_parts(a, list[best].cm, list[best].cn, list[best].split_k, words, &parts)) {
+      *plan = parts;
+      return true;
+    }
+    times[best] = 1e30;
+  }
 }
 
 // Whether a launch of IRIS_PHASE_FUSED is better off reducing inside the program than behind it, `producer` being the
@@ -666,7 +795,7 @@ hipError_t make_plan_units(const iris_gemm_args& a, Plan* plan) {
       return hipSuccess;
     }
   }
-  if (plan_parts(a, plan)) return hipSuccess;
+  if (plan_small(a, plan)) return hipSuccess;
   const bool plain = a.variant == 0 && a.split_k == 0 && !a.mm_begin_timestamp && !a.mm_end_timestamp &&
                      !(a.epilogue == IRIS_EPI_ONE_SHOT && a.phase != IRIS_PHASE_PRODUCE) &&
                      a.epilogue != IRIS_EPI_ATOMIC_ADD && a.num_sms > 0 && (a.block_m == 128 || a.block_m == 256) &&
@@ -706,15 +835,12 @@ hipError_t make_plan_units(const iris_gemm_args& a, Plan* plan) {
     }
   }
   const hipError_t err = make_plan_body(a, plan);
-  plan->k.merge_m = plan->k.merge_n = 1;
-  plan->k.flag_num_pid_m = plan->k.num_pid_m;
-  plan->k.flag_num_pid_n = plan->k.num_pid_n;
-  plan->k.flag_pn_base = 0;
+  own_flags(plan);
   if (err == hipSuccess) split_last_round(a, plan);
   return err;
 }
 
-hipError_t make_plan_body(const iris_gemm_args& a, Plan* plan) {
+hipError_t make_plan_body(const iris_gemm_args& a, Plan* plan, bool cells) {
   if (a.M < 0 || a.N < 0 || a.K < 0) return hipErrorInvalidValue;
   if (a.block_m <= 0 || a.block_n <= 0 || a.group_size_m <= 0) return hipErrorInvalidValue;
   if (a.num_sms <= 0 || a.num_xcds <= 0 || (a.num_sms % a.num_xcds) != 0) return hipErrorInvalidValue;
@@ -859,7 +985,7 @@ hipError_t make_plan_body(const iris_gemm_args& a, Plan* plan) {
 
   if (a.variant == 0 || a.variant == IRIS_GEMM_VARIANT_FEW_ROWS) {
     if (plan_few_rows(a, op, dma_ok, plan)) return hipSuccess;
-    if (a.variant == 0 && plan_cells(a, op, dma_ok, plan)) return hipSuccess;
+    if (cells && plan_cells(a, op, dma_ok, plan)) return hipSuccess;
     if (a.variant == IRIS_GEMM_VARIANT_FEW_ROWS) return hipErrorInvalidValue;
   }
 

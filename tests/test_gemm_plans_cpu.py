@@ -1,0 +1,75 @@
+"""Which kernel the launcher plans for small products, on both sides of every line where the faster one changes
+(``iris_gemm_plan_name`` reads the arguments only: no GPU, and the pointers below are never followed)."""
+
+import ctypes
+
+import pytest
+
+from iris_amd import _native, ops
+
+BF16, F32 = 2, 0
+
+
+def plan(M, N, K, BM, BN, dtype=BF16, ws=1, base=1 << 32, row=None, **kw):
+    args = _native.GemmArgs()
+    args.a, args.b, args.c_global = base, 2 << 32, 4 << 32
+    args.tile_completed, args.heap_bases = 5 << 32, 6 << 32
+    args.partials, args.locks, args.partials_slot_elems = 7 << 32, 8 << 32, BM * BN
+    args.M, args.N, args.K = M, N, K
+    args.stride_am, args.stride_ak, args.stride_bk, args.stride_bn = row or K, 1, 1, row or K
+    args.stride_cm_global, args.stride_cn_global = N * ws, 1
+    args.block_m, args.block_n, args.block_k, args.group_size_m = BM, BN, 64, 4
+    args.num_sms, args.num_xcds, args.world_size = 256, 8, ws
+    args.ab_dtype = args.c_dtype = args.c_global_dtype = dtype
+    args.epilogue, args.notify = ops.EPI_ALL_SCATTER, 1
+    for name, value in kw.items():
+        setattr(args, name, value)
+    lib = _native.lib()
+    name, parts = ctypes.create_string_buffer(256), ctypes.c_int(0)
+    assert lib.iris_gemm_plan_name(ctypes.byref(args), name, 256) == 0
+    assert lib.iris_gemm_split_k(ctypes.byref(args), ctypes.byref(parts)) == 0
+    return name.value.decode(), parts.value
+
+
+PARTS = "64x64x128_w2x2_s4_f4+parts_of_tiles"
+
+
+@pytest.mark.parametrize("M,N,BM,BN,K,want", [
+    # 32 tiles of 128 x 128 and the like: parts fill the chip, a long K is shared out instead
+    (256, 2048, 128, 128, 512, (PARTS, 1)),
+    (256, 2048, 128, 128, 2048, (PARTS, 1)),
+    (256, 2048, 128, 128, 16384, ("128x128x64_w2x2_s4_f4", 8)),
+    (256, 2048, 128, 128, 36864, ("128x128x64_w2x2_s4_f4", 8)),
+    (256, 2048, 256, 64, 2048, (PARTS, 1)),
+    (256, 2048, 256, 64, 36864, ("256x64x64_w4x1_s3_f4", 8)),
+    (256, 2048, 256, 128, 2048, (PARTS, 1)),
+    (256, 2048, 256, 128, 36864, ("256x128x64_w2x2_s3_f4", 16)),
+    (256, 2048, 256, 256, 2048, (PARTS, 1)),
+    (256, 2048, 256, 256, 36864, ("256x256x64_w2x4_s2", 16)),
+    (256, 2048, 64, 64, 36864, ("64x64x128_w2x2_s4_f4", 2)),
+    # 256 cells of 32 x 32
+    (512, 512, 64, 64, 2048, ("cells_32x32", 1)),
+    (512, 512, 64, 64, 36864, ("64x64x128_w2x2_s4_f4", 4)),
+    (512, 512, 128, 128, 8192, ("cells_32x32", 1)),
+    (512, 512, 128, 128, 36864, ("128x128x64_w2x2_s4_f4", 16)),
+    (512, 512, 256, 64, 36864, ("256x64x64_w4x1_s3_f4", 16)),
+    (512, 512, 256, 128, 36864, ("256x128x64_w2x2_s3_f4", 16)),
+    (512, 512, 256, 256, 36864, (PARTS, 3)),
+    # a batch too tall for the few-rows kernel
+    (128, 1376, 64, 64, 4096, ("cells_32x32", 1)),
+    (128, 1376, 128, 128, 36864, ("128x128x64_w2x2_s4_f4", 16)),
+])
+def test_small_products(M, N, BM, BN, K, want):
+    assert plan(M, N, K, BM, BN) == want
+
+
+def test_no_split_asked_for_stays_unsplit():
+    for K in (512, 36864):
+        assert plan(512, 512, K, 128, 128, split_k=1)[1] == 1
+        assert plan(256, 2048, K, 128, 128, split_k=1) == ("128x128x64_w2x2_s4_f4", 1)
+
+
+def test_fp32():
+    assert plan(512, 512, 512, 128, 128, dtype=F32)[0] == "cells_32x32"
+    name, parts = plan(512, 512, 36864, 128, 128, dtype=F32)
+    assert name == "128x128x32_w2x2_s4_f4_fp32" and parts == 16
