@@ -159,9 +159,16 @@ bool plan_few_rows(const iris_gemm_args& a, int op, bool dma_ok, Plan* plan) {
   const bool f32_room = a.M <= SKINNY_MID_MAX_ROWS ||
                         (a.M <= SKINNY_F32_MAX_ROWS && (cells <= cus || cells * 4 >= (cells + cus - 1) / cus * cus * 3));
   const bool room = !mid || (f32 && f32_room) || (cells <= (int64_t)current_cu_count() && a.M <= SKINNY_MID_MAX_ROWS && a.K >= SKINNY_MID_MIN_K);
+  // 17 to 32 rows of a long K are left to the persistent kernel where the workgroups need a second round, or where
+  // rows that start anywhere on a cache line cost more than B's stream ([17..32,16384] x [16384,4776] 40-42 us here and
+  // 31.5 there, [27,21136] x [21136,4776] 63 and 39, [32,21136] x [21136,4096] 41 and 36; but at K = 4096 14 and 16.6,
+  // [32,16384] x [16384,4096] 28.2 and 30.5, [17,21136] x [21136,4096] 34.2 and 35.6, [32,21136] x [21136,1376] 21 and 23).
+  const bool lines = whole_lines(a);
+  const bool long_k = a.variant == 0 && !mid && rb == 2 && !f32 &&
+                      (cells > cus ? a.K >= 8192 : !lines && a.M > 24 && a.K >= 20480 && b_bytes > (96 << 20));
   // (the workgroups' rows belong to one tile)
   const bool rows_ok = a.block_m >= a.M || (f32 && a.block_m % (SKINNY_ROWS * rb) == 0);
-  const bool ok = room && a.K > 0 && dma_ok && !plan->in_program && rows_ok && (a.block_n % SKINNY_COLS) == 0 &&
+  const bool ok = room && !long_k && a.K > 0 && dma_ok && !plan->in_program && rows_ok && (a.block_n % SKINNY_COLS) == 0 &&
                   !a.mm_begin_timestamp && !a.mm_end_timestamp && (a.split_k == 0 || a.split_k == 1) && counters &&
                   ((int64_t)SKINNY_ROWS * rb * a.stride_am + a.K) * 2 < lim &&
                   ((int64_t)SKINNY_COLS * a.stride_bn + a.K) * 2 < lim;
@@ -171,7 +178,6 @@ bool plan_few_rows(const iris_gemm_args& a, int op, bool dma_ok, Plan* plan) {
   if (a.split_k == 0 && a.partials && aligned16(a.partials) && a.locks && k.total_tiles + cells <= a.num_sms) {
     // a block of K of a workgroup alone on its CU, by what it fetches; rows that do not start on a cache line
     // touch half as many lines again ([31,11800] x [11800,1360] 0.85 us, [40,16384] x [16384,512] 0.48)
-    const bool lines = a.stride_am % 64 == 0 && a.stride_bn % 64 == 0;
     const double block_us = (rb == 2 ? 0.5 : 0.3) * (lines ? 1 : 1.6);
     parts = few_rows_parts(cells, (a.K + 63) / 64, block_us, b_bytes);
     const int64_t elems = cells * rb * (SKINNY_ROWS * SKINNY_COLS);  // of one part's sums

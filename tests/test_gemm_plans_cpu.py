@@ -63,6 +63,24 @@ def test_small_products(M, N, BM, BN, K, want):
     assert plan(M, N, K, BM, BN) == want
 
 
+@pytest.mark.parametrize("M,N,K,few", [
+    (17, 4096, 21136, True), (32, 4096, 16384, True), (24, 4096, 21136, True), (32, 4096, 21136, False),
+    (32, 1376, 21136, True), (17, 4776, 4096, True), (17, 4776, 8192, False), (32, 8192, 36864, False),
+    (16, 8192, 36864, True),
+])
+def test_rows_of_a_long_k(M, N, K, few):
+    assert plan(M, N, K, 64, 64)[0].startswith("few_rows") == few
+    # ... asked for by name, the kernel still takes them
+    assert plan(M, N, K, 64, 64, variant=ops.VARIANT_FEW_ROWS)[0].startswith("few_rows")
+
+
+def test_rows_off_the_cache_lines():
+    # a shard of a wider operand whose rows do not start on cache lines, by their stride or by the first of them
+    assert plan(32, 8192, 1024 * 16, 64, 64, row=1 << 17) == plan(32, 8192, 1024 * 16, 64, 64)
+    on, off = plan(32, 4096, 20480, 64, 64, row=1 << 16)[0], plan(32, 4096, 20480, 64, 64, row=1 << 16, base=(1 << 32) + 32)[0]
+    assert on.startswith("few_rows") and not off.startswith("few_rows")
+
+
 def test_no_split_asked_for_stays_unsplit():
     for K in (512, 36864):
         assert plan(512, 512, K, 128, 128, split_k=1)[1] == 1
