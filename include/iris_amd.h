@@ -114,7 +114,8 @@ int iris_hip_arch_name(int device, char* buf, size_t len);
 
 /* status word values (max-reduced by the kernels into *status) */
 #define IRIS_STATUS_OK 0
-#define IRIS_STATUS_SPIN_TIMEOUT 1 /* a flag wait gave up; that tile was not reduced */
+#define IRIS_STATUS_SPIN_TIMEOUT 1 /* a flag wait gave up; that tile was not reduced, or (one-shot reduce, tiles that
+                                    * several groups share) not all of it, and its flag keeps the count it has */
 
 /* Special values of iris_gemm_args.variant.  A launch with at most 32 rows of
  * A (64 when K >= 2048) whose operands are K-contiguous normally takes a kernel

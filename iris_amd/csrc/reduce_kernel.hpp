@@ -45,7 +45,32 @@ struct ReduceKArgs {
 // The row-band and flat kernels count their finished groups in the upper half
 // of the first tile's flag (a producer's +1 only ever touches the lower half),
 // so a flag's value is its lower half.
-constexpr int FLAG_COUNT_SHIFT = 16, FLAG_VALUE_MASK = 0xFFFF;
+constexpr int FLAG_COUNT_SHIFT = 16, FLAG_VALUE_MASK = 0xFFFF, FLAG_COUNT_MASK = 0x7FFF;
+// A tile that an item has given up waiting for carries this bit until the end of the launch (a negative flag): what the
+// item leaves out is missing from the tile, so no other item waits for it or starts on it, and the count that comes
+// in meanwhile is not consumed.  A flag is taken back to 0 only where the whole tile was reduced.
+constexpr int FLAG_GIVEN_UP = (int)0x80000000;
+
+// Bounded wait, without consuming it, for the flag of a tile that several items share.  False: one of them has given up.
+__device__ inline bool wait_shared_tile(const ReduceKArgs& p, int tile_id) {
+  IRIS_GLOBAL int32_t* flag = (IRIS_GLOBAL int32_t*)(p.flags + tile_id);
+  const uint64_t t0 = wall_clock64();
+  for (;;) {
+    const int v = p.sys ? __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM)
+                        : __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (v & FLAG_GIVEN_UP) return false;
+    if ((v & FLAG_VALUE_MASK) >= p.ws - 1) return true;
+    if (wall_clock64() - t0 > p.timeout) {
+      if (p.status) atomicMax(p.status, (uint32_t)IRIS_STATUS_SPIN_TIMEOUT);
+      const int before = p.sys ? __hip_atomic_fetch_or(flag, FLAG_GIVEN_UP, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM)
+                               : __hip_atomic_fetch_or(flag, FLAG_GIVEN_UP, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      // (the old value in hand: the mark is set before the caller's barrier)
+      asm volatile("" ::"v"(before) : "memory");
+      return false;
+    }
+    __builtin_amdgcn_s_sleep(8);
+  }
+}
 
 // Block-wide wait for one tile's flag.  One lane polls; the outcome is
 // broadcast through LDS and every wave then acquires.
@@ -159,10 +184,10 @@ __global__ __launch_bounds__(256) void reduce_tiles_vec_kernel(const ReduceKArgs
   }
 }
 
-// This group is past all its waits.  Groups count themselves on the upper half of flags[0]; the one that counts last
+// This group (all of its waves) is past its last look at a flag.  Groups count themselves on the upper half of flags[0]; the one that counts last
 // knows that nobody polls any more and takes every flag that reached ws-1 back to 0, which is what the consumer's
 // CAS(ws-1 -> 0) leaves (gemm_one_shot_all_reduce.py:228-234).  The count comes off with one atomic per flag, so a
-// +1 of the next round that lands meanwhile is kept.  (Spread over sixteen flags, the count takes as long.)
+// +1 of the next round that lands meanwhile is kept.  A flag that was given up on keeps its count and loses the mark.  (Spread over sixteen flags, the count takes as long.)
 __device__ inline void reset_by_last_group(const ReduceKArgs& p, IRIS_LDS int* last) {
   const int tid = threadIdx.x;
   if (tid == 0) {
@@ -171,7 +196,7 @@ __device__ inline void reset_by_last_group(const ReduceKArgs& p, IRIS_LDS int* l
                                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM)
                              : __hip_atomic_fetch_add((IRIS_GLOBAL int32_t*)p.flags, 1 << FLAG_COUNT_SHIFT,
                                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    *last = (before >> FLAG_COUNT_SHIFT) == (int)gridDim.x - 1 ? 1 : 0;
+    *last = ((before >> FLAG_COUNT_SHIFT) & FLAG_COUNT_MASK) == (int)gridDim.x - 1 ? 1 : 0;
   }
   __syncthreads();
   if (!*last) return;
@@ -180,7 +205,13 @@ __device__ inline void reset_by_last_group(const ReduceKArgs& p, IRIS_LDS int* l
     IRIS_GLOBAL int32_t* f = (IRIS_GLOBAL int32_t*)(p.flags + t);
     const int v = p.sys ? __hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM)
                         : __hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    int take = (v & FLAG_VALUE_MASK) >= consumed ? consumed : 0;
+    int take = v >= 0 && (v & FLAG_VALUE_MASK) >= consumed ? consumed : 0;
+    if (v < 0) {
+      if (p.sys)
+        __hip_atomic_fetch_and(f, ~FLAG_GIVEN_UP, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      else
+        __hip_atomic_fetch_and(f, ~FLAG_GIVEN_UP, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
     if (t == 0) take += (int)gridDim.x << FLAG_COUNT_SHIFT;  // the groups' count, too
     if (take) flag_add_relaxed(f, -take, p.sys != 0);
   }
@@ -196,7 +227,7 @@ __device__ inline void reset_by_last_group(const ReduceKArgs& p, IRIS_LDS int* l
 //
 // Flags: an item waits for every tile its rows cross (its columns only, when it lies inside one row) without
 // consuming them; the flags go back to 0 as in the row-band kernel.  When one does not arrive within the timeout the
-// item goes element by element and leaves that tile's elements alone.
+// item goes element by element, leaves that tile's elements alone and marks the tile (FLAG_GIVEN_UP).
 //
 // STREAM, for launches of many items: a lane keeps two loads in flight where it could keep dozens.  HBM likes that
 // better: 8 x fp32 [8192,8192] with 1 / 2 / 3 / 4 / 8 / 12 loads ahead 382 / 359 / 366 / 375 / 386 / 388 us, two groups a
@@ -258,9 +289,7 @@ __global__ __launch_bounds__(256) void reduce_flat_kernel(const ReduceKArgs p) {
       for (int i = tid; i < count; i += 256) {
         const int dm = i / width;
         const int t = tile_id_of(m0 + dm, t0 + i - dm * width, p.num_pid_m, p.num_pid_n, p.G);
-        ok &= wait_tile_ready((IRIS_GLOBAL int32_t*)(p.flags + t), p.ws - 1, p.sys != 0, p.timeout, p.status, FLAG_VALUE_MASK)
-                  ? 1
-                  : 0;
+        ok &= wait_shared_tile(p, t) ? 1 : 0;
       }
       all = __syncthreads_and(ok) != 0;
       if (p.acquire) {
@@ -277,8 +306,10 @@ __global__ __launch_bounds__(256) void reduce_flat_kernel(const ReduceKArgs p) {
         const IRIS_GLOBAL int32_t* f = (const IRIS_GLOBAL int32_t*)(p.flags + t);
         const int v = p.sys ? __hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM)
                             : __hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if ((v & FLAG_VALUE_MASK) >= p.ws - 1) sum_element(e);
+        // (what this item waited for in vain is marked by now, whatever has arrived since; the rest is ready)
+        if (v >= 0 && (v & FLAG_VALUE_MASK) >= p.ws - 1) sum_element(e);
       }
+      __syncthreads();  // every wave has read its flags before the group counts itself and they may be reset
       continue;
     }
     // whole strips through descriptors that end with the last one; what is left of the array by elements
@@ -385,8 +416,8 @@ __global__ __launch_bounds__(256) void reduce_flat_kernel(const ReduceKArgs p) {
 //
 // Flags: the band crosses every tile of its tile row, so the group waits for
 // all of them (one lane per tile) without consuming them; a tile that does
-// not arrive within the timeout only masks its own columns.  The flags that
-// reached ws-1 are reset to 0 by the group that finishes last (the groups
+// not arrive within the timeout only masks its own columns and is marked
+// (FLAG_GIVEN_UP).  The other flags that reached ws-1 are reset to 0 by the group that finishes last (the groups
 // count themselves on the upper half of the first flag), or, for grids too
 // large for that count, by reset_consumed_flags_kernel, which the launcher
 // then enqueues behind this kernel.  The sum is in rank order 0..ws-1.
@@ -435,10 +466,7 @@ __global__ __launch_bounds__(256) void reduce_rows_kernel(const ReduceKArgs p) {
       int ok = 1;
       if (tid < ntn) {
         const int t = tile_id_of(row0 / p.BM, tn0 + tid, p.num_pid_m, p.num_pid_n, p.G);
-        ok = wait_tile_ready((IRIS_GLOBAL int32_t*)(p.flags + t), p.ws - 1, p.sys != 0, p.timeout, p.status,
-                             FLAG_VALUE_MASK)
-                 ? 1
-                 : 0;
+        ok = wait_shared_tile(p, t) ? 1 : 0;
         ready[tid] = ok;
       }
       all = __syncthreads_and(ok) != 0;
@@ -534,7 +562,10 @@ __global__ __launch_bounds__(256) void reset_consumed_flags_kernel(int32_t* flag
   const int t = blockIdx.x * 256 + threadIdx.x;
   if (t >= total) return;
   IRIS_GLOBAL int32_t* f = (IRIS_GLOBAL int32_t*)(flags + t);
-  if (__hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= consumed)
+  const int v = __hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (v < 0)
+    __hip_atomic_fetch_and(f, ~FLAG_GIVEN_UP, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  else if (v >= consumed)
     __hip_atomic_fetch_add(f, -consumed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 

@@ -192,3 +192,43 @@ def test_matrices_without_gaps_are_reduced_as_arrays(shmem, in_dt, out_dt, ws, M
     want = want.clone()
     want[pm * BM:(pm + 1) * BM, pn * BN:(pn + 1) * BN] = 3
     assert torch.equal(cg.cpu(), want) and not flags.any() and int(status.item()) == 1
+
+
+@pytest.mark.parametrize("M,N,BM,BN,variant", [
+    (1030, 1021, 128, 128, 0),   # as an array, odd rows
+    (512, 384, 128, 64, 7),      # in bands of rows
+    (37, 131, 32, 64, 0),        # as an array, one strip a lane
+])
+@pytest.mark.parametrize("scope", [ops.SCOPE_AGENT, ops.SCOPE_SYSTEM])
+def test_a_tile_given_up_by_one_group_is_left_by_all(shmem, M, N, BM, BN, variant, scope):
+    """Two tiles, the first among them, that another group of the launch has
+    given up on (bit 31) while their last increment comes in: they are left
+    alone, keep their count and lose the mark; the rest is reduced."""
+    ws = 3
+    c = shmem.zeros((M, N), dtype=torch.float32)
+    cg = shmem.full((M, N), 3, dtype=torch.float32)
+    total = ops.cdiv(M, BM) * ops.cdiv(N, BN)
+    flags = shmem.zeros((total,), dtype=torch.int32)
+    status = torch.zeros(1, dtype=torch.int32, device="cuda")
+    host = fill_partials(shmem, c, ws)
+    want = O.one_shot_reduce(host, torch.float32)
+    left = [0, total // 2]
+    f = torch.full((total,), ws - 1, dtype=torch.int32)
+    f[left] -= 1 << 31
+    args = (c, cg, flags, shmem.get_heap_bases(), 0, ws, BM, BN, 4)
+    for again in range(2):
+        cg.fill_(3)
+        flags.copy_(f)
+        ops.one_shot_reduce(*args, scope=scope, status=status, variant=variant)
+        torch.cuda.synchronize()
+        out, some = cg.cpu(), want.clone()
+        for t in left:
+            pm, pn = O.tile_map(t, M, N, BM, BN, 4)
+            some[pm * BM:(pm + 1) * BM, pn * BN:(pn + 1) * BN] = 3
+        assert torch.equal(out, some)
+        assert flags.cpu().tolist() == [ws - 1 if t in left else 0 for t in range(total)]
+    # what is left is reduced by the next launch
+    flags.fill_(ws - 1)
+    ops.one_shot_reduce(*args, scope=scope, status=status, variant=variant)
+    torch.cuda.synchronize()
+    assert torch.equal(cg.cpu(), want) and not flags.any() and int(status.item()) == 0
