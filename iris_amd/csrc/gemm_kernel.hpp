@@ -997,9 +997,12 @@ __device__ __attribute__((always_inline)) inline bool store_acc(const GemmKArgs&
             // (element by element throughout, 32 round trips to LDS instead of 4 a block and rank, the epilogue of
             // [1000,1500] x [1500,999] in 256 x 64 tiles on two ranks took half of the launch's 47 us)
             if constexpr (OP == OP_STORE16 || OP == OP_STORE32) {
+              int at = lane;
+              // (128 accumulators: the offsets are computed here, not kept in registers across the K loop)
+              if constexpr (Cfg::IM * Cfg::IN * 4 > 64) asm volatile("" : "+v"(at));
 #pragma nounroll
               for (int t = 0; t < 32 * Cfg::U16 / 64; ++t) {
-                const int row = t * (64 / Cfg::U16) + lane / Cfg::U16, u = lane % Cfg::U16;
+                const int row = t * (64 / Cfg::U16) + at / Cfg::U16, u = at % Cfg::U16;
                 const int m = row0 + row, n = col0 + u * EPV;
                 if (m >= m_end || n >= n_end) continue;
                 const IRIS_LDS char* src = ws + row * Cfg::WS_PITCH + (u ^ ((row / Cfg::ERPB) % Cfg::U16)) * 16;
@@ -1782,6 +1785,13 @@ __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKAr
       }
       }
     }
+    // (The 128-accumulator tiles with fetching waves have no register to spare: what the stores read of the arguments is
+    // read here, as in the split hand-over above, not held in spilled scalar registers across the K loop.)
+    constexpr bool LATE = !SPLIT && !FUSED && Cfg::DMA && Cfg::LW != 0 && Cfg::IM * Cfg::IN * 4 > 64;
+    typedef const __attribute__((address_space(4))) GemmKArgs* KernArgPtr;
+    KernArgPtr late_args = (KernArgPtr)__builtin_amdgcn_kernarg_segment_ptr();
+    if constexpr (LATE) asm volatile("" : "+s"(late_args));
+    const GemmKArgs& p = LATE ? *(const GemmKArgs*)late_args : p_outer;
     bool fast = true;  // (a fetching wave has no stores to count)
     if (worker)
       fast = store_acc<Cfg, OP, ODT>(p, acc, ws, c_it.m0 + wm * Cfg::TM, c_it.n0 + wn * Cfg::TN, c_it.m_end, c_it.n_end,
