@@ -772,20 +772,32 @@ bool plan_small(const iris_gemm_args& a, Plan* plan) {
 // plan of the same launch without the reduce.  Inside, a tile is one program's from its first K-step to its last
 // strip: K is not shared out, the caller's tiles are not blocked, the fetching waves' registers are not there, and
 // CUs whose tiles are done do not help with the others' reduces.  Behind, a kernel boundary is paid, 4 us.  So inside
-// for one round of small tiles with a short K, whose producer would run the same way (K-shard [785,216] x [216,2752],
-// 8 fp32 partials, 256 x 64 tiles: 27.8 against 30.7 us; 64^3 10 against 13); behind otherwise ([1999,1376] x
-// [1376,4096] in 256 x 128 tiles 68 against 55 us, in two rounds of 256 x 256 tiles 200 against 175, 25 tiles of
-// K = 29408 838 against 106).  A launch that shares the device with its peers' (fewer programs than CUs) stays inside:
-// every program's CU is counted there.
+// for one round of small tiles with a short K, whose producer would run the same way (us a pass, inside / behind:
+// K-shard [785,216] x [216,2752], 8 fp32 partials, 256 x 64 tiles 25.3 / 28; 64^3 8.9 / 12); behind otherwise
+// ([1999,1376] x [1376,4096] in 256 x 128 tiles 67 / 54, in 256 x 256 tiles 78 / 62, 25 tiles of K = 29408 741 / 103).
+// Where the producer would run in smaller units than the caller's tiles, those win from a shorter K on: [64,K] x [K,640],
+// 8 bf16 partials, 256 x 64 tiles 11.6 / 13.5 at K = 128, 12.4 / 13.5 at 320, 13.9 / 14.0 at 640, 16.7 / 14.6 at 1376;
+// [128,K] x [K,4096] 13.1 / 17.2 at 128, 17.2 / 18.9 at 640; [128,K] x [K,320] 13.2 / 12.7 at 128 (5 tiles: 5 CUs);
+// [2000,320] x [320,640], 2 fp32 partials 18.0 / 21.4; [16,K] x [K,4096] 10.8 / 12.2 at 128, 11.9 / 12.0 at 320.
+// A launch that shares the device with its peers' (fewer programs than CUs) stays inside: every program's CU is counted
+// there.
 bool reduce_in_program(const iris_gemm_args& a, const Plan& producer) {
   if (a.num_sms < current_cu_count() || a.variant != 0 || a.split_k != 0 || a.mm_begin_timestamp || a.mm_end_timestamp) return true;
   if (!producer.entry && !producer.skinny) return true;  // (nothing to compute)
-  if ((producer.skinny && producer.skinny_cb == 1) || producer.last_round || producer.rest || producer.parts) return false;
   const GemmKArgs& k = producer.k;
+  const int steps = (a.K + 63) / 64;
+  const int64_t tiles = ((int64_t)a.M + a.block_m - 1) / a.block_m * (((int64_t)a.N + a.block_n - 1) / a.block_n);
+  const int64_t inside = (int64_t)(a.block_m < a.M ? a.block_m : a.M) * (a.block_n < a.N ? a.block_n : a.N);
+  const int64_t strips = inside * a.world_size * dtype_size(a.c_dtype);  // bytes that a program's tile is reduced from
+  if (tiles <= a.num_sms && k.vec_out && (producer.skinny || producer.entry->dma)) {
+    const bool few = producer.skinny && producer.skinny_cb == 1;
+    if (inside <= 64 * 64 && (few ? steps <= 2 && a.block_n <= 64 : steps <= 10)) return true;
+    if (!few && tiles >= 16 && a.block_n <= 64 && steps <= 5 && (inside <= 128 * 64 || strips <= (128 << 10))) return true;
+  }
+  if ((producer.skinny && producer.skinny_cb == 1) || producer.last_round || producer.rest || producer.parts) return false;
   // (cells: the caller's tiles inside, when they are as small as the parts they would be run in)
   if (producer.skinny && a.block_m * a.block_n > 64 * 64) return false;
   if (k.split_k > 1 || k.merge_m * k.merge_n > 1 || k.total_tiles > a.num_sms || !k.vec_out) return false;
-  const int steps = (a.K + 63) / 64;
   return steps <= 8 || (steps <= 24 && a.block_m * a.block_n <= 128 * 128);
 }
 

@@ -91,3 +91,17 @@ def test_fp32():
     assert plan(512, 512, 512, 128, 128, dtype=F32)[0] == "cells_32x32"
     name, parts = plan(512, 512, 36864, 128, 128, dtype=F32)
     assert name == "128x128x32_w2x2_s4_f4_fp32" and parts == 16
+
+
+@pytest.mark.parametrize("M,N,K,BM,BN,ws,partial,inside", [
+    (64, 640, 320, 256, 64, 2, F32, True), (64, 640, 1376, 256, 64, 2, F32, False),
+    (64, 4096, 640, 256, 64, 8, BF16, True),
+    (128, 4096, 128, 256, 64, 8, F32, True), (128, 320, 128, 256, 64, 8, F32, False),  # 64 tiles, and 5
+    (2000, 640, 320, 256, 64, 2, F32, True), (2000, 640, 320, 256, 64, 8, F32, False),
+    (16, 4096, 128, 64, 64, 2, F32, True), (16, 4096, 320, 64, 64, 2, F32, False), (1, 320, 128, 256, 128, 2, F32, False),
+    (1999, 4096, 1376, 256, 128, 8, BF16, False), (785, 2752, 216, 256, 64, 8, F32, True),
+])
+def test_the_reduce_inside_the_program_or_behind_it(M, N, K, BM, BN, ws, partial, inside):
+    name, _ = plan(M, N, K, BM, BN, ws=ws, epilogue=ops.EPI_ONE_SHOT, phase=ops.PHASE_FUSED, c=3 << 32, c_dtype=partial,
+                   stride_cm=N, stride_cn=1, stride_cm_global=N)
+    assert name.endswith("+reduce") and name.endswith("+kernel+reduce") != inside
