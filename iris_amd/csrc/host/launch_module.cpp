@@ -13,9 +13,11 @@
 
 #include <ATen/core/Tensor.h>
 #include <ATen/core/grad_mode.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 
 #include "../../../include/iris_amd.h"
 
@@ -36,6 +38,28 @@ bool plain(const at::Tensor& t) {
                                             DispatchKey::Negative, DispatchKey::ZeroTensor, DispatchKey::FuncTorchBatched,
                                             DispatchKey::FuncTorchGradWrapper});
   return t.defined() && t.layout() == c10::kStrided && t.has_storage() && !t.key_set().has_any(wrapped);
+}
+
+// Whether this thread is being traced, or inside a transform or a dispatch mode (torch.func, functionalization,
+// make_fx, ...): autograd's apply records a function there, or refuses it, and a launch of our own would pass it by.
+bool watched() {
+  using c10::DispatchKey;
+  static const c10::DispatchKeySet modes({DispatchKey::FuncTorchDynamicLayerFrontMode, DispatchKey::FuncTorchDynamicLayerBackMode,
+                                          DispatchKey::FuncTorchVmapMode, DispatchKey::FuncTorchBatched,
+                                          DispatchKey::FuncTorchGradWrapper, DispatchKey::Functionalize, DispatchKey::Python,
+                                          DispatchKey::PythonTLSSnapshot, DispatchKey::PythonDispatcher, DispatchKey::PreDispatch,
+                                          DispatchKey::Tracer});
+  return torch::jit::tracer::isTracing() || c10::impl::tls_local_dispatch_key_set().included_.has_any(modes);
+}
+
+// Whether autograd has business with a tensor among the arguments: a gradient, or a tangent (forward mode).
+bool differentiated(PyObject* const* x, Py_ssize_t n) {
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    if (!THPVariable_Check(x[i])) continue;
+    const at::Tensor& t = THPVariable_Unpack(x[i]);
+    if (!plain(t) || (at::GradMode::is_enabled() && t.requires_grad()) || t._fw_grad(/*level=*/0).defined()) return true;
+  }
+  return false;
 }
 
 bool operand(PyObject* o, int device, Operand* out) {
@@ -243,8 +267,8 @@ struct Attr {
 };
 
 // matmul_apply(cls, epilogue, args): the positional `matmul.apply(*args)` of a wrapper class, when it is not in debug
-// mode and no operand wants a gradient.  -> what autograd's apply returns (a view of `c`, or None), or NotImplemented:
-// declined or failed, the caller takes the long way.
+// mode, no operand wants a gradient or carries a tangent, and nothing traces or transforms the call.  -> what autograd's
+// apply returns (a view of `c`, or None), or NotImplemented: declined or failed, the caller takes the long way.
 PyObject* matmul_apply(PyObject*, PyObject* const* v, Py_ssize_t n) {
   if (n != 3 || !PyTuple_Check(v[2])) {
     PyErr_SetString(PyExc_TypeError, "matmul_apply(cls, epilogue, args)");
@@ -281,9 +305,7 @@ PyObject* matmul_apply(PyObject*, PyObject* const* v, Py_ssize_t n) {
   if (nx > 23 && (collect = PyObject_IsTrue(x[23])) < 0) return decline();
   if (collect && ((nx > 24 && !operand(x[24], device, &t.ts_begin)) || (nx > 25 && !operand(x[25], device, &t.ts_end))))
     return decline();
-  if (at::GradMode::is_enabled())
-    for (Py_ssize_t i = 0; i < nx; ++i)
-      if (THPVariable_Check(x[i]) && THPVariable_Unpack(x[i]).requires_grad()) return decline();
+  if (watched() || differentiated(x, nx)) return decline();
   // (ops.default_num_xcds)
   g.num_xcds = (cu_count == 304 || cu_count == 256) && g.num_sms % 8 == 0 ? 8 : 1;
   if (g.num_sms > 0 && g.block_m > 0 && g.block_n > 0) workspace(x[5], x[6], device, &g, &t);

@@ -112,8 +112,8 @@ def make_matmul(epilogue: int, name: str):
 
         @classmethod
         def apply(cls, *args, **kwargs):
-            # The ordinary call (no debug report, no operand that wants a gradient) goes to the launch in native
-            # code; what that declines takes autograd's way to `forward` below.  (One token's gate / up projection
+            # The ordinary call (no debug report, no operand that wants a gradient, nobody tracing) goes to the launch
+            # in native code; what that declines takes autograd's way to `forward` below.  (One token's gate / up projection
             # behind a fill of its flags, launched back to back: 30 us a pass through autograd and ctypes, 8 us now.)
             out = NotImplemented
             if cls is matmul and not kwargs:
