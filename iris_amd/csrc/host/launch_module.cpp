@@ -268,7 +268,8 @@ struct Attr {
 
 // matmul_apply(cls, epilogue, args): the positional `matmul.apply(*args)` of a wrapper class, when it is not in debug
 // mode, no operand wants a gradient or carries a tangent, and nothing traces or transforms the call.  -> what autograd's
-// apply returns (a view of `c`, or None), or NotImplemented: declined or failed, the caller takes the long way.
+// apply returns (a view of `c`, or None); NotImplemented: declined, nothing launched, the caller takes the long way; or the
+// hipError_t of a launch that failed (its first kernel may have run, so it is not tried again).
 PyObject* matmul_apply(PyObject*, PyObject* const* v, Py_ssize_t n) {
   if (n != 3 || !PyTuple_Check(v[2])) {
     PyErr_SetString(PyExc_TypeError, "matmul_apply(cls, epilogue, args)");
@@ -311,7 +312,8 @@ PyObject* matmul_apply(PyObject*, PyObject* const* v, Py_ssize_t n) {
   if (g.num_sms > 0 && g.block_m > 0 && g.block_n > 0) workspace(x[5], x[6], device, &g, &t);
   if (!fill_gemm(t, &g)) return decline();
   void* stream = current_stream(device);
-  if (unlocked([&] { return iris_gemm_launch(&g, stream); }) != hipSuccess) return decline();
+  const int err = unlocked([&] { return iris_gemm_launch(&g, stream); });
+  if (err != hipSuccess) return PyLong_FromLong(err);
   if (!t.c) Py_RETURN_NONE;
   try {
     at::NoGradGuard guard;
@@ -383,7 +385,7 @@ PyObject* memset_i32(PyObject*, PyObject* const* v, Py_ssize_t n) {
 
 PyMethodDef methods[] = {
     {"gemm", (PyCFunction)(void (*)(void))gemm, METH_FASTCALL, "launch a shard GEMM; -1: declined"},
-    {"matmul_apply", (PyCFunction)(void (*)(void))matmul_apply, METH_FASTCALL, "matmul.apply; NotImplemented: declined"},
+    {"matmul_apply", (PyCFunction)(void (*)(void))matmul_apply, METH_FASTCALL, "matmul.apply; NotImplemented: declined, int: failed"},
     {"one_shot_reduce", (PyCFunction)(void (*)(void))one_shot_reduce, METH_FASTCALL, "launch the reduce; -1: declined"},
     {"memset_i32", (PyCFunction)(void (*)(void))memset_i32, METH_FASTCALL, "int32 fill; -1: declined"},
     {nullptr, nullptr, 0, nullptr}};

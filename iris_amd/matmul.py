@@ -118,7 +118,11 @@ def make_matmul(epilogue: int, name: str):
             out = NotImplemented
             if cls is matmul and not kwargs:
                 out = _native.host().matmul_apply(matmul, epilogue, args)
-            return super().apply(*args, **kwargs) if out is NotImplemented else out
+            if out is NotImplemented:
+                return super().apply(*args, **kwargs)
+            if isinstance(out, int):
+                ops._gemm_launch_failed(out)
+            return out
 
         @staticmethod
         def forward(ctx, a, b, c, c_global, bias, P, locks, tile_completed, rank, world_size, grid, BLK_M=128,
