@@ -198,6 +198,12 @@ def host():
     global _host
     if _host is None:
         lib()  # what the module is linked against; raises its own message when missing
+        from . import build
+
+        built_for = build.host_built_for()
+        if built_for is not None and built_for != build.host_abi():
+            raise RuntimeError(f"iris_amd native launch module was built for {built_for}, this is {build.host_abi()}. "
+                               "Build it again with `python -m iris_amd.build`.")
         try:
             from . import _launch
         except ImportError as e:

@@ -20,6 +20,7 @@ from __future__ import annotations
 import argparse
 import concurrent.futures
 import os
+import re
 import shutil
 import subprocess
 import sys
@@ -91,6 +92,23 @@ def _run(cmd):
     return proc
 
 
+def host_abi() -> str:
+    """What ``_launch.so`` is bound to besides its sources: this Python's and this torch's binary interface."""
+    import torch
+
+    return f"{sysconfig.get_config_var('SOABI')}, torch {torch.__version__}, cxx11abi {int(torch._C._GLIBCXX_USE_CXX11_ABI)}"
+
+
+def host_built_for() -> str | None:
+    """``host_abi()`` as it was when ``_launch.so`` was built (the text is in the file), None without one."""
+    found = re.search(rb"iris_amd\._launch built for ([^\0]*)\0", HOST_EXT.read_bytes()) if HOST_EXT.exists() else None
+    return found.group(1).decode() if found else None
+
+
+def host_stale() -> bool:
+    return _stale(HOST_EXT, [HOST_SRC, PKG.parent / "include" / "iris_amd.h"]) or host_built_for() != host_abi()
+
+
 def _build_host_module() -> None:
     import torch
 
@@ -100,7 +118,7 @@ def _build_host_module() -> None:
                 sysconfig.get_paths()["include"]]
     _run([cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-D__HIP_PLATFORM_AMD__=1",
           "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
-          *(f"-isystem{d}" for d in includes), f"-isystem{Path(hipcc()).resolve().parent.parent / 'include'}",
+          f'-DIRIS_BUILT_FOR="{host_abi()}"', *(f"-isystem{d}" for d in includes), f"-isystem{Path(hipcc()).resolve().parent.parent / 'include'}",
           str(HOST_SRC), "-o", str(HOST_EXT), f"-L{PKG}", f"-l:{LIB.name}", f"-L{torch_dir / 'lib'}",
           "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN"])
 
@@ -138,7 +156,7 @@ def build(force: bool = False, jobs: int | None = None, verbose: bool = True) ->
         if verbose:
             print(f"[iris_amd.build] linked {TESTING_LIB.name}", flush=True)
 
-    if force or _stale(HOST_EXT, [HOST_SRC, PKG.parent / "include" / "iris_amd.h"]):
+    if force or host_stale():
         _build_host_module()
         if verbose:
             print(f"[iris_amd.build] linked {HOST_EXT.name}", flush=True)

@@ -25,6 +25,9 @@ namespace {
 
 constexpr int DECLINED = -1;
 
+// Read off the file by iris_amd/build.py and iris_amd/_native.py before it is loaded.
+__attribute__((used)) const char built_for[] = "iris_amd._launch built for " IRIS_BUILT_FOR;
+
 // A plain strided tensor of the device, or (for None) nothing.  False: not for this module.
 struct Operand {
   const at::Tensor* t = nullptr;
