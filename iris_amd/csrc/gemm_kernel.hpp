@@ -1114,7 +1114,7 @@ __device__ __attribute__((always_inline)) inline void publish_tile(const GemmKAr
       IRIS_GLOBAL int32_t* cnt = (IRIS_GLOBAL int32_t*)(p.tile_arrivals + first);
       int last = 0;
       if (lane == 0) {
-        last = __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == parts - 1;
+        last = arrive(cnt, (p.flag_mode & FLAG_RELEASE) != 0, p.sys != 0) == parts - 1;
         if (last) __hip_atomic_store(cnt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
       }
       if (!__builtin_amdgcn_readfirstlane(last)) return;
@@ -1739,7 +1739,7 @@ __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKAr
         if (wave == 0 && ok) {
           IRIS_GLOBAL int32_t* done = (IRIS_GLOBAL int32_t*)(p.locks + slot0 + 1);
           int before = 0;
-          if (lane == 0) before = __hip_atomic_fetch_add(done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          if (lane == 0) before = arrive(done, (p.flag_mode & FLAG_RELEASE) != 0, p.sys != 0);
           before = __builtin_amdgcn_readfirstlane(before);
           if (before == parts - 1) {
             // every slice is in memory: publish, and leave both counters at 0

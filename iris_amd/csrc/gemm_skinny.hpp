@@ -414,7 +414,7 @@ gemm_skinny_kernel(const GemmKArgs p) {
     if (parts > 1) {
       IRIS_GLOBAL int32_t* cnt = (IRIS_GLOBAL int32_t*)(p.locks + tile_id);
       if (lane == 0) {
-        last = __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == parts - 1;
+        last = arrive(cnt, (p.flag_mode & FLAG_RELEASE) != 0, p.sys != 0) == parts - 1;
         if (last) __hip_atomic_store(cnt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
       }
       last = __builtin_amdgcn_readfirstlane(last);
