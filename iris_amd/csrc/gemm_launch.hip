@@ -693,7 +693,7 @@ bool plan_parts(const iris_gemm_args& a, int cm, int cn, int split_k, int64_t wo
 //   [512,512] in 256 x 128 tiles                K 1024 12.3 / 10.2 / 9.0   16384 26.6 / 25.8 / 28.8   36864 33.5 / 33.3 / 61
 //   [256,2048] in 128 x 128 tiles               K 2048 17.8 / 13.3 / -     8192 25.7 / 24.8 / -       36864 48 / 65 / -
 // Small tiles fill the chip and fetch more for the work they do: their K-steps are many times as many as those of a
-// large tile whose K is shared out, so they lose to it from some K on.  Only what the few-rows kernel does not take;
+// large tile whose K is shared out, so they lose to it from some K on.  What the few-rows kernel takes is its;
 // parts for a launch that owns the device and leaves tile and split to the launcher.
 bool plan_small(const iris_gemm_args& a, Plan* plan) {
   const int64_t cus = current_cu_count();
@@ -703,7 +703,13 @@ bool plan_small(const iris_gemm_args& a, Plan* plan) {
   auto tiles_of = [&](int cm, int cn) { return ((int64_t)a.M + cm - 1) / cm * (((int64_t)a.N + cn - 1) / cn); };
   if (tiles_of(128, 128) > a.num_sms) return false;
   Plan whole;
-  if (make_plan_body(a, &whole) != hipSuccess || whole.skinny || !whole.entry) return false;
+  if (make_plan_body(a, &whole) != hipSuccess) return false;
+  if (whole.skinny) {  // few rows
+    own_flags(&whole);
+    *plan = whole;
+    return true;
+  }
+  if (!whole.entry) return false;
   const GemmKArgs& w = whole.k;
   const Operands o{a.ab_dtype == IRIS_DTYPE_F32, whole_lines(a), !whole.entry->dma,
                    a.epilogue == IRIS_EPI_ATOMIC_ADD, w.vec_out != 0, w.dest_all ? a.world_size : 1,

@@ -58,7 +58,8 @@ bool watched() {
 // Whether autograd has business with a tensor among the arguments: a gradient, or a tangent (forward mode).
 bool differentiated(PyObject* const* x, Py_ssize_t n) {
   for (Py_ssize_t i = 0; i < n; ++i) {
-    if (!THPVariable_Check(x[i])) continue;
+    // (what most arguments are: the check for a tensor asks its metaclass about each of these)
+    if (x[i] == Py_None || PyLong_Check(x[i]) || PyUnicode_Check(x[i]) || !THPVariable_Check(x[i])) continue;
     const at::Tensor& t = THPVariable_Unpack(x[i]);
     if (!plain(t) || (at::GradMode::is_enabled() && t.requires_grad()) || t._fw_grad(/*level=*/0).defined()) return true;
   }
