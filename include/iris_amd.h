@@ -118,11 +118,13 @@ int iris_hip_arch_name(int device, char* buf, size_t len);
                                     * several groups share) not all of it, and its flag keeps the count it has */
 
 /* Special values of iris_gemm_args.variant.  A launch with at most 32 rows of
- * A (64 when K >= 2048) whose operands are K-contiguous normally takes a kernel
- * of its own that streams B (one workgroup per 16 or 32 rows x 16 columns of C,
- * all fetches in flight);
+ * A (64 when K >= 2048, 128 of fp32) whose operands are K-contiguous and 16-byte
+ * aligned normally takes a kernel of its own that streams B (workgroups of 16 or
+ * 32 rows x 16 columns of C, a long K shared out over several); 17 to 32 rows of a
+ * long K over many columns are left to the persistent kernel.
  * FEW_ROWS insists on it (hipErrorInvalidValue when the launch does not
- * qualify), PERSISTENT keeps the default choice among the persistent kernels.
+ * qualify), PERSISTENT keeps the default choice among the persistent kernels
+ * (and the caller's tiles: no cells of 32 x 32, no parts of tiles).
  * The reference has one Triton kernel for every M (gemm_all_scatter.py:95). */
 #define IRIS_GEMM_VARIANT_FEW_ROWS 1000
 #define IRIS_GEMM_VARIANT_PERSISTENT 1001
@@ -187,13 +189,20 @@ typedef struct iris_gemm_args {
   int32_t scope;        /* IRIS_SCOPE_*                                           */
   int32_t variant;      /* 0 = default kernel choice; >0 selects a tuning variant, or IRIS_GEMM_VARIANT_* */
   uint64_t spin_timeout_ticks; /* bound on a flag wait in 100 MHz ticks; 0 = default (2 s) */
-  /* Split-K workspace: the `P` and `locks` buffers that matmul.apply receives
-   * (matmul_wrapper.py:29-31,73-92; allocated at benchmark.py:136-142).  With both
-   * given, a launch whose tiles would leave most programs idle shares each
-   * tile's K range over several programs: partial tiles go through `partials`
-   * in fp32, `locks` (all zero before the first launch, left all zero) orders
-   * the hand-over.  Results differ from the unsplit ones only in fp32
-   * summation order. */
+  /* Workspace: the `P` and `locks` buffers that matmul.apply receives
+   * (matmul_wrapper.py:29-31,73-92; allocated at benchmark.py:136-142).
+   * `partials`, with `locks`: a launch whose tiles would leave most programs idle
+   * shares each tile's K range over several programs, whose partial sums go
+   * through it in fp32.  Results differ from the unsplit ones only in fp32
+   * summation order.
+   * `locks` (all zero before the first launch, left all zero): the words on which
+   * the programs of a launch meet.  Parts of a shared K hand over there; where a
+   * tile is computed by several workgroups (the few-rows kernel, cells of 32 x 32,
+   * parts of the caller's tiles), they count their arrivals there, and the last one
+   * raises the tile's flag, whether K is shared or not.  So a launch of any shape
+   * may write them, and both buffers belong to ONE launch at a time: launches that
+   * can run at the same time (other streams, other ranks of the device) need
+   * buffers of their own, or NULL, without which no such plan is taken. */
   float* partials;      /* [num_sms][partials_slot_elems] fp32, or NULL           */
   int32_t* locks;       /* int32[num_sms], or NULL (a tile in n parts uses the n words of its programs) */
   int64_t partials_slot_elems; /* >= block_m * block_n                            */
@@ -254,8 +263,9 @@ int iris_gemm_kernel_info(const iris_gemm_args* args, int* n_regs, int* n_spills
 int iris_gemm_split_k(const iris_gemm_args* args, int* split_k);
 
 /* Name of the kernel `iris_gemm_launch` would run for `args` ("" when there is
- * no GEMM work): a tuning variant's name, or "few_rows_16xN" / "few_rows_32xN",
- * followed by "+stream_k", "+reduce" (the in-program reduce) or "+two_per_cu"
+ * no GEMM work): a tuning variant's name, that of a tile behind the table
+ * ("..._gather": operands that lie across K or at any alignment; fp32 tiles for a
+ * longer K), or "few_rows_16xN" / "few_rows_32xN" / "cells_32x32", followed by "+stream_k", "+reduce" (the in-program reduce) or "+two_per_cu"
  * (two programs a CU), and by "+two_tiles_each" / "+four_tiles_each" /
  * "+eight_tiles_each" where the launch computes a block of that many of the
  * caller's tiles as one (each tile keeps its own id and flag), and by
@@ -288,7 +298,7 @@ typedef struct iris_reduce_args {
   int64_t stride_cm, stride_cn;
   int64_t stride_cm_global, stride_cn_global;
   int32_t block_m, block_n, group_size_m;
-  int32_t num_sms;   /* grid size; 0 = one program per tile */
+  int32_t num_sms;   /* grid size; 0 = the launcher's choice, two groups a CU at most */
   int32_t num_xcds;
   int32_t cur_rank, world_size;
   int32_t c_dtype, c_global_dtype;

@@ -12,8 +12,10 @@ Arguments that only steer the Triton compiler (``num_stages``, ``num_warps``,
 ``waves_per_eu``, ``mfmaInstrSize``, ``kpack``) and ``two_tiles`` are accepted
 and ignored; ``BLK_K`` does not change any result.  ``P`` and ``locks``, which
 the reference allocates and never reads, serve as workspace when they have
-the reference's shapes (split-K partials; arrival counters of the few-rows
-kernel) and are ignored otherwise.  ``bias`` is never applied (the reference
+the reference's shapes (partial sums of a shared K; the counters on which the
+programs of one launch meet) and are ignored otherwise.  They belong to one
+launch at a time: launches that can run at the same time need their own.
+``bias`` is never applied (the reference
 forces ``BIAS=False``, matmul_wrapper.py:104).
 """
 
