@@ -867,22 +867,15 @@ def run_decoder(args, emit=True):
             got = shmem.on_rank(gate_all, 5)[:, rank * ffn:(rank + 1) * ffn].float()
             assert torch.allclose(got, ref_up, rtol=1e-2, atol=1e-2), "gate/up scatter differs from the fp32 product"
             assert torch.allclose(shmem.on_rank(part, rank), ref_dn, rtol=1e-2, atol=1e-2), "down partial differs"
-            sk = {"gate_up": ops.gemm_split_k(x, wg.T, None, shmem.on_rank(gate_all, rank),
-                                              shmem.on_rank(flags_up, rank), hb, rank, ws, grid_up, bm, bn, 64, 4,
-                                              ops.EPI_ALL_SCATTER, partials=P, locks=locks, split_k=args.decoder_split_k),
-                  "down": ops.gemm_split_k(h, wd.T, shmem.on_rank(part, rank), shmem.on_rank(out, rank),
-                                           shmem.on_rank(flags_dn, rank), hb, rank, ws, grid_dn, bm, bn, 64, 6,
-                                           ops.EPI_ONE_SHOT, phase=ops.PHASE_PRODUCE, partials=P, locks=locks,
-                                           split_k=args.decoder_split_k),
-                  "reduce": 1}
-            kern = {"gate_up": ops.gemm_plan_name(x, wg.T, None, shmem.on_rank(gate_all, rank),
-                                                  shmem.on_rank(flags_up, rank), hb, rank, ws, grid_up, bm, bn, 64, 4,
-                                                  ops.EPI_ALL_SCATTER, partials=P, locks=locks, split_k=args.decoder_split_k),
-                    "down": ops.gemm_plan_name(h, wd.T, shmem.on_rank(part, rank), shmem.on_rank(out, rank),
-                                               shmem.on_rank(flags_dn, rank), hb, rank, ws, grid_dn, bm, bn, 64, 6,
-                                               ops.EPI_ONE_SHOT, phase=ops.PHASE_PRODUCE, partials=P, locks=locks,
-                                           split_k=args.decoder_split_k),
-                    "reduce": "reduce"}
+            up_args = (x, wg.T, None, shmem.on_rank(gate_all, rank), shmem.on_rank(flags_up, rank), hb, rank, ws,
+                       grid_up, bm, bn, 64, 4, ops.EPI_ALL_SCATTER)
+            dn_args = (h, wd.T, shmem.on_rank(part, rank), shmem.on_rank(out, rank), shmem.on_rank(flags_dn, rank),
+                       hb, rank, ws, grid_dn, bm, bn, 64, 6, ops.EPI_ONE_SHOT)
+            plan_kw = dict(partials=P, locks=locks, num_xcds=xcds, split_k=args.decoder_split_k)
+            sk = {"gate_up": ops.gemm_split_k(*up_args, **plan_kw),
+                  "down": ops.gemm_split_k(*dn_args, phase=ops.PHASE_PRODUCE, **plan_kw), "reduce": 1}
+            kern = {"gate_up": ops.gemm_plan_name(*up_args, **plan_kw),
+                    "down": ops.gemm_plan_name(*dn_args, phase=ops.PHASE_PRODUCE, **plan_kw), "reduce": "reduce"}
             plain_variant = plain_build_of(kern["gate_up"])
             runs = [("gate_up", up), ("down", down), ("reduce", reduce), ("gate_up_one", up_one)]
             if plain_variant is not None:

@@ -214,7 +214,7 @@ constexpr GemmKernelEntry make_entry_f32(const char* name) {
   X(IRIS_DTYPE_F32, OP, 64, 64, 32, 2, 2, 1, LOAD_GENERIC, 0, "64x64x16_w2x2_generic_fp32")
 // Tiles behind the fp32 table: the launcher takes them for a K of eight K-steps or more.
 // The scripts' 256 x 64 tile as one compute tile ([2048,1024] x [1024,2048]: as four of 64 x 64, fetch-bound, 131 us;
-// 66 so), split-K builds, and the gathering loader.
+// 70 so), split-K builds, and the gathering loader.
 #define IRIS_GEMM_F32_LONG_VARIANTS(X, OP)                                                        \
   X(IRIS_DTYPE_F32, OP, 128, 128, 64, 2, 2, 4, LOAD_DMA, 4, "128x128x32_w2x2_s4_f4_fp32")        \
   X(IRIS_DTYPE_F32, OP, 256, 64, 64, 4, 1, 3, LOAD_DMA, 4, "256x64x32_w4x1_s3_f4_fp32")          \

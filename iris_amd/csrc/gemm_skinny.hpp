@@ -19,16 +19,16 @@
 // A block that has been multiplied gives its place to the fetches of the one
 // after next.  Two blocks a wave are enough, as three workgroups then share a
 // CU: with eight (one workgroup a CU, all fetches of a K of 4096 issued before
-// the first MFMA) [16,3584] x [3584,8192] took 17.6 us a pass and takes 14.3,
-// [6,2560] x [2560,6208] 13.9 -> 10.6, and nothing measured is slower.  What a
+// the first MFMA) [16,3584] x [3584,8192] took 17.6 us a pass and takes 14.1,
+// [6,2560] x [2560,6208] 13.9 -> 8.9, and nothing measured is slower.  What a
 // workgroup alone on its CU is bound by is the addresses: 16 clocks an
 // instruction, whichever of its lanes are in range.  So up to eight rows of A
 // are one instruction a block, not two ([1,1376] .. [8,4096] x [4096,1376]
-// 8.6 -> 7.3 us at eight rows).
+// 8.6 -> 7.9 us at eight rows).
 // A K too long for that is shared out over workgroups (gridDim.z of them a
 // block of C), which leave their sums in the caller's workspace; the last one
-// to arrive adds them up.  [2,23680] x [23680,736] 18.6 -> 10.4 us,
-// [4,36864] x [36864,512] 28.8 -> 13.0.
+// to arrive adds them up.  [2,23680] x [23680,736] 18.6 -> 11.0 us,
+// [4,36864] x [36864,512] 28.8 -> 12.3.
 // The waves' partial 16x16 accumulators meet in LDS; wave w then stores the
 // sum on destination rank w, w+8, ...
 //
@@ -38,7 +38,7 @@
 //
 // fp32 operands: the launcher counts K and the strides in 16-bit units, so a
 // block of K is 32 elements of the same 128 bytes, a chunk four of them
-// (gemm_kernel.hpp, Mfma<IRIS_DTYPE_F32>).  [16,4096] x [4096,4096] takes 19.5 us a
+// (gemm_kernel.hpp, Mfma<IRIS_DTYPE_F32>).  [16,4096] x [4096,4096] takes 19.1 us a
 // pass, 14.1 of them B's 67 MB at the rate of a large copy.
 #pragma once
 
@@ -66,7 +66,8 @@ constexpr int skinny_lds_bytes(int rb) { return skinny_a_bytes(rb) + SKINNY_WAVE
 // persistent kernel's tiles are too few to fill the chip or too short to pay for its fixed costs (its prologue, hand-over
 // and flag take 3 us more than this kernel's; sharing K out over programs 4 to 6 us).  Here the eight waves share K
 // inside the workgroup.  A comes in like B, by LDS-DMA, two blocks a wave in flight: 8 KiB a block of K, 128 KiB a
-// workgroup, one workgroup a CU.  It is bound by the CU's L1, 64 bytes a clock: 0.06 us for every 64 of K.
+// workgroup, one workgroup a CU.  It is bound by the CU's L1: 0.08 us for every 64 of K, 0.09 on
+// all CUs at once ([512,512], 256 workgroups: 9.0 us at K = 1024, 61 at 36864), where 64 bytes a clock would be 0.053.
 // A lane's columns are eight in a row: the block j of a row of 32 columns takes columns 8q + 4j .. + 3, so that a row
 // leaves in 16-byte stores.  The cells are dealt to the XCDs in consecutive runs (the shorter direction first), so that
 // each XCD's L2 fetches its share of the longer operand once.
