@@ -38,7 +38,7 @@ PEAK_HBM_GBPS = 8000.0     # MI355X HBM3E, published
 # kernel (profiles/gemm_all_scatter_bf16_8192x8192x1024.txt, profiles/one_shot_reduce_fp32x8_8192x8192.txt).
 # Counters cannot be read from inside a run, so these are carried here and dropped for non-default variants.
 GEMM_TRAFFIC_BYTES = 335108222
-REDUCE_TRAFFIC_BYTES = 2280882394
+REDUCE_TRAFFIC_BYTES = 2281096192
 
 M, N, K_SHARD, K_TOTAL = 8192, 8192, 1024, 8192
 BLK_M, BLK_N, BLK_K, GSIZE_M, GRID = 256, 256, 64, 4, 256
@@ -786,9 +786,10 @@ def run_decoder(args, emit=True):
 
     def plain_build_of(kernel):
         """Variant number of the build of `kernel`'s tile shape and wave layout in which every wave fetches its
-        share of the operands, or None if `kernel` is such a build already."""
+        share of the operands, or None if `kernel` is such a build already (or is run in parts of the caller's tiles,
+        which a launch that names a variant is not)."""
         base = kernel.split("+")[0]
-        if not base.endswith("_f4"):
+        if not base.endswith("_f4") or "+parts_of_tiles" in kernel:
             return None
         shape, waves = base.split("x")[:2], base.split("_")[1]
         for cand, num in variants.items():
