@@ -118,7 +118,8 @@ def _build_host_module() -> None:
                 sysconfig.get_paths()["include"]]
     _run([cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-D__HIP_PLATFORM_AMD__=1",
           "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
-          f'-DIRIS_BUILT_FOR="{host_abi()}"', *(f"-isystem{d}" for d in includes), f"-isystem{Path(hipcc()).resolve().parent.parent / 'include'}",
+          f'-DIRIS_BUILT_FOR="{host_abi()}"', *(f"-isystem{d}" for d in includes),
+          f"-isystem{Path(hipcc()).resolve().parent.parent / 'include'}",
           str(HOST_SRC), "-o", str(HOST_EXT), f"-L{PKG}", f"-l:{LIB.name}", f"-L{torch_dir / 'lib'}",
           "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN"])
 

@@ -315,8 +315,6 @@ __device__ inline void flag_add_relaxed(IRIS_GLOBAL int32_t* p, int v, bool sys)
     __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Store that is written through to the coherence point of the agent (or of
-// the system): nothing stays dirty in this XCD's L2.
 // Counts one of the groups that share a tile and returns how many had come before; the last one raises the tile's flag.
 // `release`: the flag is a release (IRIS_FLAG_SEM_RELEASE_ACQUIRE) and has to release what every group stored, not its
 // own group's stores alone, so each arrival releases and acquires at the flag's scope.
@@ -326,6 +324,8 @@ __device__ inline int arrive(IRIS_GLOBAL int32_t* count, bool release, bool sys)
              : __hip_atomic_fetch_add(count, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// Store that is written through to the coherence point of the agent (or of
+// the system): nothing stays dirty in this XCD's L2.
 template <typename T>
 __device__ inline void store_through(IRIS_GLOBAL T* p, T v, bool sys) {
   if (sys)

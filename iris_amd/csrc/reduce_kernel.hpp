@@ -184,10 +184,11 @@ __global__ __launch_bounds__(256) void reduce_tiles_vec_kernel(const ReduceKArgs
   }
 }
 
-// This group (all of its waves) is past its last look at a flag.  Groups count themselves on the upper half of flags[0]; the one that counts last
-// knows that nobody polls any more and takes every flag that reached ws-1 back to 0, which is what the consumer's
-// CAS(ws-1 -> 0) leaves (gemm_one_shot_all_reduce.py:228-234).  The count comes off with one atomic per flag, so a
-// +1 of the next round that lands meanwhile is kept.  A flag that was given up on keeps its count and loses the mark.  (Spread over sixteen flags, the count takes as long.)
+// This group (all of its waves) is past its last look at a flag.  Groups count themselves on the upper half of flags[0];
+// the one that counts last knows that nobody polls any more and takes every flag that reached ws-1 back to 0, which is
+// what the consumer's CAS(ws-1 -> 0) leaves (gemm_one_shot_all_reduce.py:228-234).  The count comes off with one atomic
+// per flag, so a +1 of the next round that lands meanwhile is kept.  A flag that was given up on keeps its count and
+// loses the mark.  (Spread over sixteen flags, the count takes as long.)
 __device__ inline void reset_by_last_group(const ReduceKArgs& p, IRIS_LDS int* last) {
   const int tid = threadIdx.x;
   if (tid == 0) {
@@ -417,9 +418,10 @@ __global__ __launch_bounds__(256) void reduce_flat_kernel(const ReduceKArgs p) {
 // Flags: the band crosses every tile of its tile row, so the group waits for
 // all of them (one lane per tile) without consuming them; a tile that does
 // not arrive within the timeout only masks its own columns and is marked
-// (FLAG_GIVEN_UP).  The other flags that reached ws-1 are reset to 0 by the group that finishes last (the groups
-// count themselves on the upper half of the first flag), or, for grids too
-// large for that count, by reset_consumed_flags_kernel, which the launcher
+// (FLAG_GIVEN_UP).  The other flags that reached ws-1 are reset to 0 by the
+// group that finishes last (the groups count themselves on the upper half of
+// the first flag), or, for grids too large for that count, by
+// reset_consumed_flags_kernel, which the launcher
 // then enqueues behind this kernel.  The sum is in rank order 0..ws-1.
 template <int IN_DT, int OUT_DT, int LAUX, int WS>
 __global__ __launch_bounds__(256) void reduce_rows_kernel(const ReduceKArgs p) {
