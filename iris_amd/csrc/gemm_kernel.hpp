@@ -1786,8 +1786,10 @@ __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKAr
       }
     }
     // (The 128-accumulator tiles with fetching waves have no register to spare: what the stores read of the arguments is
-    // read here, as in the split hand-over above, not held in spilled scalar registers across the K loop.)
-    constexpr bool LATE = !SPLIT && !FUSED && Cfg::DMA && Cfg::LW != 0 && Cfg::IM * Cfg::IN * 4 > 64;
+    // read here, as in the split hand-over above, not held in spilled scalar registers across the K loop.  Atomics read
+    // less and fit as they are: 8 x [4096,512] x [512,4096] 527 us, 530 with the arguments read late.)
+    constexpr bool LATE = !SPLIT && !FUSED && (OP == OP_STORE16 || OP == OP_STORE32) && Cfg::DMA && Cfg::LW != 0 &&
+                          Cfg::IM * Cfg::IN * 4 > 64;
     typedef const __attribute__((address_space(4))) GemmKArgs* KernArgPtr;
     KernArgPtr late_args = (KernArgPtr)__builtin_amdgcn_kernarg_segment_ptr();
     if constexpr (LATE) asm volatile("" : "+s"(late_args));
