@@ -1110,11 +1110,14 @@ __device__ __attribute__((always_inline)) inline void publish_tile(const GemmKAr
       const int pm = t.pid_m / p.part_m, pn = t.pid_n / p.part_n;
       first = tile_id_of(pm, pn, p.flag_num_pid_m, p.flag_num_pid_n, p.G);
       const int parts = min(p.part_m, p.num_pid_m - pm * p.part_m) * min(p.part_n, p.num_pid_n - pn * p.part_n);
-      // (the group's stores of the part have completed, written through: the part that counts last finds all of them)
+      // (the group's stores of the part have completed, written through: the part that counts last finds all of them.
+      // Flags that are releases need more than that, and launches with such flags are not run in parts: an arrival
+      // that can also release and acquire, here, cost the default launches 0.3 to 1 us, [823,1024] x [1024,1096] with 16-bit
+      // atomics 11.0 -> 12.0 a launch, by where it moved the compiler's scalar spills.)
       IRIS_GLOBAL int32_t* cnt = (IRIS_GLOBAL int32_t*)(p.tile_arrivals + first);
       int last = 0;
       if (lane == 0) {
-        last = arrive(cnt, (p.flag_mode & FLAG_RELEASE) != 0, p.sys != 0) == parts - 1;
+        last = __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == parts - 1;
         if (last) __hip_atomic_store(cnt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
       }
       if (!__builtin_amdgcn_readfirstlane(last)) return;

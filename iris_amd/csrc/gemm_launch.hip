@@ -734,6 +734,8 @@ bool plan_small(const iris_gemm_args& a, Plan* plan) {
   const bool flags = a.epilogue == IRIS_EPI_ALL_SCATTER ? a.notify != 0 : a.epilogue == IRIS_EPI_ONE_SHOT && a.world_size > 1;
   const int64_t words = flags ? tiles_of(a.block_m, a.block_n) : 0;
   if (words > 0 && (!a.locks || words > a.num_sms)) return found;
+  // (the last part raises the flag for all: where it is a release, only its own stores would be covered, see publish_tile)
+  if (words > 0 && a.flag_sem == IRIS_FLAG_SEM_RELEASE_ACQUIRE) return found;
   static const int shapes[4][2] = {{64, 64}, {128, 64}, {64, 128}, {128, 128}};
   TileLaunch list[8];
   double times[8];
