@@ -594,8 +594,8 @@ void own_flags(Plan* plan) {
 }
 
 // Estimated times of a small product's launch, in us: what plan_small compares its plans by.  A CU fetches 108 KB a us
-// (its L1), an eighth less when all of them do (L2); rows that start anywhere on a cache line touch half as many lines
-// again, and a gathering tile's fetching waves need three times as long.  A K-step takes as long as its operands, or as
+// (its L1), an eighth less when all of them do (L2); rows that start anywhere on a cache line touch a third to a half as
+// many lines again, and a gathering tile's fetching waves need three times as long.  A K-step takes as long as its operands, or as
 // the matrix cores where those are slower.  Around the K loop: the launch, the arrival counters of parts, the epilogue
 // (each rank's copy), and for a shared K the hand-over, which grows with the partials that cross memory.  The constants
 // are a fit to 8200 timings of 33 shapes ([24,8192] .. [96,2560] .. [4477,136] .. [1500,1500]) at K from 152 to 36864:
@@ -620,7 +620,7 @@ double tiles_us(const iris_gemm_args& a, const TileLaunch& t, const Operands& o,
   const double area = (double)t.cm * t.cn / 4096, partials = programs * area / 64;  // tiles of 64 x 64; MB
   const bool deep = t.cm == 64 && t.cn == 64;  // (K-steps of 128: whole lines, mostly)
   const double fetch = (t.cm + t.cn) / (8 * 108.0) * (1 + 0.13 * cover + (split ? 0.17 : 0.0)) *
-                       (o.gather ? 2.9 : o.lines ? 1.0 : deep ? 1.37 : 1.69);
+                       (o.gather ? 2.9 : o.lines ? 1.0 : deep ? 1.3 : 1.5);
   const double multiply = o.f32 ? area * 0.452 * (1 + 0.04 * cover) + 0.1 : area * 0.0535;
   const int64_t unit = deep ? 2 : 1, nk = ((int64_t)a.K + 64 * unit - 1) / (64 * unit);
   const int64_t part_steps = (nk + t.split_k - 1) / t.split_k * unit, steps = (items + cus - 1) / cus * t.subs * part_steps;
@@ -649,7 +649,7 @@ double tiles_us(const iris_gemm_args& a, const TileLaunch& t, const Operands& o,
 }
 double cells_us(const iris_gemm_args& a, int64_t cells, int parts, const Operands& o, int64_t cus) {
   const int64_t groups = cells * parts, nk = ((int64_t)a.K + 63) / 64;
-  const double lines = o.lines ? 1.0 : 1.0 + 1.35 * (groups < 256 ? groups : 256) / 256;  // (both operands come in by lines of K = 64)
+  const double lines = o.lines ? 1.0 : 1.6;  // (both operands come in by lines of K = 64: [128,8200] x [8200,1376] 19.2 us)
   const double step = 0.083 * (groups * 5 > cus * 4 ? 1.09 : 1.0) * (o.f32 && lines < 1.65 ? 1.65 : lines);
   // (a workgroup's first sixteen blocks of K are in flight together)
   const double loop = ((groups + cus - 1) / cus * ((nk + parts - 1) / parts) - 16) * step;
