@@ -611,6 +611,7 @@ struct TileLaunch {
 struct Operands {
   bool f32, lines, gather, atomic, vec_out;
   int copies;     // of the output
+  bool peers;     // other ranks wait for it
   int64_t tile;   // elements of a caller's tile that lie in the output
 };
 double tiles_us(const iris_gemm_args& a, const TileLaunch& t, const Operands& o, int64_t cus) {
@@ -637,6 +638,9 @@ double tiles_us(const iris_gemm_args& a, const TileLaunch& t, const Operands& o,
   }
   if (!split) {
     us += area > 4 ? 2.4 : 0.1 * area;
+    // (more where peers wait for it: us a pass in 64 x 64 / 128 x 64 parts, [4318,576] x [576,192] to four ranks 11.8 / 12.4,
+    // [518,256] x [256,928] and its reduce over eight 17.2 / 17.9; [389,512] x [512,2240] alone 10.24 / 10.28)
+    if (o.peers && !o.atomic) us += 0.45 * (area - 1);
     if (!o.vec_out) us += area < 4 ? 1.5 * area : 6.0;  // (rows that 16-byte stores don't fit)
   } else {
     us += 3.1 + 0.53 * area + 0.2 * (partials < 16 ? partials : 16) + (partials > 16 ? 0.4 * (partials - 16) : 0.0);
@@ -649,11 +653,13 @@ double tiles_us(const iris_gemm_args& a, const TileLaunch& t, const Operands& o,
 }
 double cells_us(const iris_gemm_args& a, int64_t cells, int parts, const Operands& o, int64_t cus) {
   const int64_t groups = cells * parts, nk = ((int64_t)a.K + 63) / 64;
-  const double lines = o.lines ? 1.0 : 1.6;  // (both operands come in by lines of K = 64: [128,8200] x [8200,1376] 19.2 us)
-  const double step = 0.083 * (groups * 5 > cus * 4 ? 1.09 : 1.0) * (o.f32 && lines < 1.65 ? 1.65 : lines);
+  const double mb = ((double)a.M + a.N) * a.K * 2e-6;
+  // us for 64 of K, operands in whole lines / not: [512,512] 256 cells 0.090 / 0.13; [128,1376] 172 cells 0.083 / 0.11;
+  // [200,512] 112 cells 0.048 / 0.066 as long as the L2s hold the operands, 0.07 / 0.08 beyond
+  const double lines = o.lines ? 1.0 : 1.45;
+  const double step = 0.083 * (groups * 5 > cus * 4 ? 1.09 : groups * 2 <= cus && mb <= 30 ? 0.7 : 1.0) * (o.f32 && lines < 1.65 ? 1.65 : lines);
   // (a workgroup's first sixteen blocks of K are in flight together)
   const double loop = ((groups + cus - 1) / cus * ((nk + parts - 1) / parts) - 16) * step;
-  const double mb = ((double)a.M + a.N) * a.K * 2e-6;
   const double stream = mb / (mb > 200 ? 4.4 : 8.4) - 3, k_time = loop > stream ? loop : stream;
   const double per_tile = o.atomic ? 0.0 : (double)o.tile / (CELL * CELL) / 64;
   return 5.85 + (0.0075 + 0.004 * (per_tile < 1 ? per_tile : 1.0)) * groups + 0.025 * (o.copies - 1) + (parts > 1 ? 0.7 : 0.0) +
@@ -712,7 +718,7 @@ bool plan_small(const iris_gemm_args& a, Plan* plan) {
   if (!whole.entry) return false;
   const GemmKArgs& w = whole.k;
   const Operands o{a.ab_dtype == IRIS_DTYPE_F32, whole_lines(a), !whole.entry->dma,
-                   a.epilogue == IRIS_EPI_ATOMIC_ADD, w.vec_out != 0, w.dest_all ? a.world_size : 1,
+                   a.epilogue == IRIS_EPI_ATOMIC_ADD, w.vec_out != 0, w.dest_all ? a.world_size : 1, a.world_size > 1,
                    (int64_t)(a.block_m < a.M ? a.block_m : a.M) * (a.block_n < a.N ? a.block_n : a.N)};
   double least = tiles_us(a, TileLaunch{whole.entry->cm, whole.entry->cn, w.total_tiles, w.sub_m * w.sub_n, w.split_k,
                                         w.sliced != 0, false}, o, cus);
