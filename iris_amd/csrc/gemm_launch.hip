@@ -600,8 +600,8 @@ void own_flags(Plan* plan) {
 // (each rank's copy), and for a shared K the hand-over, which grows with the partials that cross memory.  The constants
 // are a fit to 8200 timings of 33 shapes ([24,8192] .. [96,2560] .. [4477,136] .. [1500,1500]) at K from 152 to 36864:
 // every tile, cells, up to 16 parts of K, 16-bit and fp32, weights in rows of either direction and at any alignment,
-// stores and atomics.  The plan with the least of these times is on average 0.4 % over the fastest one timed, in one case
-// of 100 more than 8 %.
+// stores and atomics.  The plan with the least of these times is on average 0.5 % over the fastest one timed, in three
+// cases of 200 more than 8 %.
 struct TileLaunch {
   int cm, cn;
   int64_t tiles;  // (the caller's, `subs` of these to one, or parts of the caller's)
@@ -657,7 +657,8 @@ double cells_us(const iris_gemm_args& a, int64_t cells, int parts, const Operand
   // us for 64 of K, operands in whole lines / not: [512,512] 256 cells 0.090 / 0.13; [128,1376] 172 cells 0.083 / 0.11;
   // [200,512] 112 cells 0.048 / 0.066 as long as the L2s hold the operands, 0.07 / 0.08 beyond
   const double lines = o.lines ? 1.0 : 1.45;
-  const double step = 0.083 * (groups * 5 > cus * 4 ? 1.09 : groups * 2 <= cus && mb <= 30 ? 0.7 : 1.0) * (o.f32 && lines < 1.65 ? 1.65 : lines);
+  const double step = 0.083 * (groups * 5 > cus * 4 ? 1.09 : groups * 2 <= cus && mb <= 30 ? 0.7 : 1.0) *
+                      (o.f32 && lines < 1.65 ? 1.65 : lines);
   // (a workgroup's first sixteen blocks of K are in flight together)
   const double loop = ((groups + cus - 1) / cus * ((nk + parts - 1) / parts) - 16) * step;
   const double stream = mb / (mb > 200 ? 4.4 : 8.4) - 3, k_time = loop > stream ? loop : stream;
