@@ -209,12 +209,15 @@ struct Mfma<IRIS_DTYPE_F32> {
 // issue no memory instruction in the K loop.
 // LOAD_: how the slabs get into LDS.  LOAD_DMA: see the top of the file.  LOAD_GATHER: through the fetching waves'
 // registers, for operands with any alignment that are contiguous along k or across it (see Gather).  LOAD_GENERIC:
-// element by element, for what is contiguous along neither.
-enum SlabLoad { LOAD_GENERIC = 0, LOAD_DMA = 1, LOAD_GATHER = 2 };
+// element by element, for what is contiguous along neither.  LOAD_DMA_ROWS: LOAD_DMA for a B whose rows are its k (a row-major
+// [K, N]): the slab of B lies in LDS as it does in memory, BK rows of CN columns, and is transposed on its way to the
+// MFMAs, by ds_read_b64_tr_b16 (see load_b).
+enum SlabLoad { LOAD_GENERIC = 0, LOAD_DMA = 1, LOAD_GATHER = 2, LOAD_DMA_ROWS = 3 };
 template <int DT_, int CM_, int CN_, int BK_, int WM_, int WN_, int S_, int LOAD_, int LW_ = 0, bool TOUCH_ = false>
 struct GemmCfg {
   static constexpr int DT = DT_, CM = CM_, CN = CN_, BK = BK_, WM = WM_, WN = WN_, S = S_;
-  static constexpr bool DMA = LOAD_ == LOAD_DMA, GATHER = LOAD_ == LOAD_GATHER;
+  static constexpr bool B_ROWS = LOAD_ == LOAD_DMA_ROWS;
+  static constexpr bool DMA = LOAD_ == LOAD_DMA || B_ROWS, GATHER = LOAD_ == LOAD_GATHER;
   static constexpr bool PIPE = LOAD_ != LOAD_GENERIC;  // the K loop runs as a pipeline across tiles
   static constexpr int NW = WM * WN, NT = NW * 64;  // the waves (threads) that multiply and store
   static constexpr int LW = LW_;
@@ -228,6 +231,7 @@ struct GemmCfg {
   static constexpr int CPR = BK / 8;    // 16-byte chunks per slab row
   static constexpr int RP = 16 / CPR;   // slab rows per 256 bytes
   static constexpr int RPB = 64 / CPR;  // slab rows per 1 KiB block (one wave-wide DMA)
+  static constexpr int B_CPR = CN / 8, B_RPB = 64 / B_CPR;  // (B_ROWS) chunks per k of the slab of B, k per 1 KiB block
   static constexpr int A_BYTES = CM * BK * 2, B_BYTES = CN * BK * 2;
   static constexpr int STAGE = A_BYTES + B_BYTES;
   static constexpr int A_LOADS = CM * CPR / (NL * 64), B_LOADS = CN * CPR / (NL * 64);
@@ -264,6 +268,7 @@ struct GemmCfg {
   static_assert(IM * IN * 4 <= 128, "accumulators of a wave tile: at most 128 registers (two waves a SIMD)");
   static_assert(TN == 32 || TN == 64 || TN == 128, "wave tile width");
   static_assert(LDS_BYTES <= 160 * 1024, "LDS budget of one CU");
+  static_assert(!B_ROWS || (DT != IRIS_DTYPE_F32 && IN <= 4 && CN % 64 == 0), "B by rows of k: 16-bit elements, wave tiles of at most 64 columns");
 };
 
 // One compute tile of work.
@@ -403,6 +408,21 @@ struct Loader {
   int k_limit;  // K
   // (Cfg::TOUCH) byte offset of the row whose line this lane touches ahead of the loads, out of range for none
   uint32_t ta, tb;
+  int step_kb;  // (Cfg::B_ROWS) bytes from a K-step of B to the next
+
+  // (Cfg::B_ROWS) The slab of B holds, for each k, CN columns as 32-byte pieces (what the transposing read of one 16-column
+  // block takes from one k) XOR-ed by this number: 32 lanes of that read take eight k, 8 q .. 8 q + 3 and 8 q + 8 .. 8 q + 11,
+  // and find them in eight different 32-byte pieces of the 256 bytes that LDS delivers at a time.
+  __device__ static inline int rows_swizzle(int k) {
+    return Cfg::CN >= 128 ? (k & 3) | ((k >> 1) & 4) : ((k >> 1) & 1) | ((k >> 2) & 2);
+  }
+  // ... the k of the slab of B that this lane fetches with its first load (load j: j * NL * B_RPB further down; the
+  // swizzle repeats every sixteen k, so a lane's chunk is the same for all its loads), and the chunk's first column
+  static_assert(!Cfg::B_ROWS || (Cfg::NL * Cfg::B_RPB) % 16 == 0, "the lane's chunk must not depend on the load");
+  __device__ static inline int rows_k(int wave, int lane) { return wave * Cfg::B_RPB + lane / Cfg::B_CPR; }
+  __device__ static inline int rows_col(int wave, int lane) {
+    return ((lane % Cfg::B_CPR) ^ (rows_swizzle(rows_k(wave, lane)) * 2)) * 8;
+  }
 
   // The chunk of the row that a lane fetches is the same for every load:
   // the swizzle period divides the rows between two loads of a wave.
@@ -421,15 +441,25 @@ struct Loader {
     const char* abase = p.a + (int64_t)m0c * p.sam * 2;
     const char* bbase = p.b + (int64_t)n0c * p.sbn * 2;
     const uint32_t arec = rows_a > 0 ? (uint32_t)(((int64_t)(rows_a - 1) * p.sam + p.K) * 2) : 0;
-    const uint32_t brec = rows_b > 0 ? (uint32_t)(((int64_t)(rows_b - 1) * p.sbn + p.K) * 2) : 0;
+    const uint32_t brec = rows_b <= 0   ? 0
+                          : Cfg::B_ROWS ? (uint32_t)(((int64_t)(p.K - 1) * p.sbk + rows_b) * 2)
+                                        : (uint32_t)(((int64_t)(rows_b - 1) * p.sbn + p.K) * 2);
     ra = __builtin_amdgcn_make_buffer_rsrc((void*)abase, 0, arec, 0x00020000);
     rb = __builtin_amdgcn_make_buffer_rsrc((void*)bbase, 0, brec, 0x00020000);
     k_limit = p.K;
     const int row = wave * Cfg::RPB + lane / Cfg::CPR, ck = chunk_k(wave, lane);
     va = (uint32_t)(((int64_t)row * p.sam + ck) * 2);
-    vb = (uint32_t)(((int64_t)row * p.sbn + ck) * 2);
     step_a = (int)((int64_t)Cfg::NL * Cfg::RPB * p.sam * 2);
-    step_b = (int)((int64_t)Cfg::NL * Cfg::RPB * p.sbn * 2);
+    if constexpr (Cfg::B_ROWS) {
+      const int col = rows_col(wave, lane);
+      // (N is a multiple of eight: a chunk lies inside the matrix or past its edge)
+      vb = col < rows_b ? (uint32_t)(((int64_t)rows_k(wave, lane) * p.sbk + col) * 2) : 0x80000000u;
+      step_b = (int)((int64_t)Cfg::NL * Cfg::B_RPB * p.sbk * 2);
+      step_kb = (int)((int64_t)Cfg::BK * p.sbk * 2);
+    } else {
+      vb = (uint32_t)(((int64_t)row * p.sbn + ck) * 2);
+      step_b = (int)((int64_t)Cfg::NL * Cfg::RPB * p.sbn * 2);
+    }
     if constexpr (Cfg::TOUCH) {
       // this program's share of the panels' rows: `first`, `first + share`, ... (the shares are powers of two)
       const int q = wave * 64 + lane;
@@ -453,7 +483,10 @@ struct Loader {
   // The load cursor is about to load step `k`: park the chunks past K.
   __device__ inline void before_step(int k, int wave, int lane) {
     if (k_limit - k * Cfg::BK >= Cfg::BK) return;  // a full step: nothing to mask
-    if (k * Cfg::BK + chunk_k(wave, lane) >= k_limit) va = vb = 0x80000000u;
+    if (k * Cfg::BK + chunk_k(wave, lane) >= k_limit) {
+      va = 0x80000000u;
+      if constexpr (!Cfg::B_ROWS) vb = 0x80000000u;  // (else the loads of the step are masked one by one, see issue_at)
+    }
   }
   // The program has no more steps to load: the loads are still issued, so
   // that every K-step keeps the same number of loads in flight, but fetch
@@ -464,21 +497,29 @@ struct Loader {
   }
 
   // Issue load `i` of K-step `k` into the stage at LDS address `stage`.  The
-  // K offset rides in the scalar offset.
-  __device__ inline void issue_at(const GemmKArgs& p, IRIS_LDS char* stage, int k, int wave, int i) const {
+  // K offset rides in the scalar offset.  FULL: the step is known to lie inside K.
+  template <bool FULL>
+  __device__ inline void issue_at(const GemmKArgs& p, IRIS_LDS char* stage, int k, int wave, int lane, int i) const {
     const bool isA = i < Cfg::A_LOADS;
     const int j = isA ? i : i - Cfg::A_LOADS;
     const int k0 = k * Cfg::BK;
     IRIS_LDS char* dst = stage + (isA ? 0 : Cfg::A_BYTES) + (j * Cfg::NL + wave) * 1024;
     // (a parked offset stays out of range: j * step is far below 2 GiB)
-    const uint32_t off = isA ? va + (uint32_t)(j * step_a) : vb + (uint32_t)(j * step_b);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(isA ? ra : rb, (IRIS_LDS void*)dst, 16, off, k0 * 2, 0, 0);
+    uint32_t off = isA ? va + (uint32_t)(j * step_a) : vb + (uint32_t)(j * step_b);
+    int at_k = k0 * 2;
+    if constexpr (Cfg::B_ROWS) {
+      if (!isA) {
+        at_k = k * step_kb;
+        if (!FULL && k0 + j * Cfg::NL * Cfg::B_RPB + rows_k(wave, lane) >= k_limit) off = 0x80000000u;
+      }
+    }
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(isA ? ra : rb, (IRIS_LDS void*)dst, 16, off, at_k, 0, 0);
   }
-  template <int I = 0>
-  __device__ inline void issue(const GemmKArgs& p, IRIS_LDS char* stage, int k, int wave) const {
+  template <bool FULL, int I = 0>
+  __device__ inline void issue(const GemmKArgs& p, IRIS_LDS char* stage, int k, int wave, int lane) const {
     if constexpr (I < Cfg::L) {
-      issue_at(p, stage, k, wave, I);
-      issue<I + 1>(p, stage, k, wave);
+      issue_at<FULL>(p, stage, k, wave, lane, I);
+      issue<FULL, I + 1>(p, stage, k, wave, lane);
     }
   }
 };
@@ -747,26 +788,38 @@ template <class Cfg>
 __device__ inline typename Mfma<Cfg::DT>::vec8 load_a(const IRIS_LDS char* sA, int i) {
   return *reinterpret_cast<const IRIS_LDS typename Mfma<Cfg::DT>::vec8*>(sA + i * 16 * Cfg::BK * 2);
 }
+// (B_ROWS) `sB` is the substep's 32 k of the slab, `lane_off` where this lane reads of its wave's first block of 16 columns.
+// ds_read_b64_tr_b16 takes from each 16 lanes four k of 16 columns, 8 bytes a lane, and hands lane i the four k of
+// column i; the fragment's eight k are two of them, four k apart.  The swizzle (Loader::rows_swizzle) leaves a block's
+// 32 bytes together, so that block j's are at the first one's address with j XOR-ed into its 32-byte piece.
 template <class Cfg>
-__device__ inline typename Mfma<Cfg::DT>::vec8 load_b(const IRIS_LDS char* sB, int j) {
-  return *reinterpret_cast<const IRIS_LDS typename Mfma<Cfg::DT>::vec8*>(sB + j * 16 * Cfg::BK * 2);
+__device__ inline typename Mfma<Cfg::DT>::vec8 load_b(const IRIS_LDS char* sB, int lane_off, int j) {
+  if constexpr (Cfg::B_ROWS) {
+    typedef short s16x4 __attribute__((ext_vector_type(4)));
+    const IRIS_LDS char* at = sB + (lane_off ^ (j * 32));
+    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((IRIS_LDS s16x4*)at);
+    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((IRIS_LDS s16x4*)(at + 4 * Cfg::CN * 2));
+    return __builtin_bit_cast(typename Mfma<Cfg::DT>::vec8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+  } else {
+    return *reinterpret_cast<const IRIS_LDS typename Mfma<Cfg::DT>::vec8*>(sB + j * 16 * Cfg::BK * 2);
+  }
 }
 
 // B fragments fetched next to A block i, so that all IN of them are spread
 // over the IM blocks of a substep.
 template <class Cfg>
-__device__ inline void load_b_share(const IRIS_LDS char* sB, int i, typename Mfma<Cfg::DT>::vec8 (&b)[Cfg::IN]) {
+__device__ inline void load_b_share(const IRIS_LDS char* sB, int lane_off, int i, typename Mfma<Cfg::DT>::vec8 (&b)[Cfg::IN]) {
   constexpr int PER = (Cfg::IN + Cfg::IM - 1) / Cfg::IM;
 #pragma unroll
   for (int j = i * PER; j < (i + 1) * PER; ++j)
-    if (j < Cfg::IN) b[j] = load_b<Cfg>(sB, j);
+    if (j < Cfg::IN) b[j] = load_b<Cfg>(sB, lane_off, j);
 }
 
 // Whole substep's fragments at once (pipeline prologue, generic loader).
 template <class Cfg>
-__device__ inline void load_all(const IRIS_LDS char* sA, const IRIS_LDS char* sB, Frags<Cfg>& f, int cb) {
+__device__ inline void load_all(const IRIS_LDS char* sA, const IRIS_LDS char* sB, int lane_off, Frags<Cfg>& f, int cb) {
 #pragma unroll
-  for (int j = 0; j < Cfg::IN; ++j) f.b[cb][j] = load_b<Cfg>(sB, j);
+  for (int j = 0; j < Cfg::IN; ++j) f.b[cb][j] = load_b<Cfg>(sB, lane_off, j);
 #pragma unroll
   for (int i = 0; i < Cfg::IM; ++i) f.a[i] = load_a<Cfg>(sA, i);
 }
@@ -1582,10 +1635,17 @@ __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKAr
   // row only depends on l%16)
   const int lrow = lane & 15, lq = lane >> 4;
   const int a_row_off = (wm * Cfg::TM + lrow) * Cfg::BK * 2;
-  const int b_row_off = (wn * Cfg::TN + lrow) * Cfg::BK * 2;
+  // (B_ROWS: added by load_b, with the block's place XOR-ed in)
+  const int b_row_off = Cfg::B_ROWS ? (8 * lq + (lrow >> 2)) * Cfg::CN * 2 +
+                                          ((wn * Cfg::IN) ^ Loader<Cfg>::rows_swizzle(8 * lq + (lrow >> 2))) * 32 + (lrow & 3) * 8
+                                    : (wn * Cfg::TN + lrow) * Cfg::BK * 2;
   int xoff[Cfg::KSUB];
 #pragma unroll
   for (int kk = 0; kk < Cfg::KSUB; ++kk) xoff[kk] = ((kk * 4 + lq) ^ ((lrow / Cfg::RP) % Cfg::CPR)) * 16;
+  // where substep kk of a stage's slab of B is read from
+  auto b_at = [&](const IRIS_LDS char* stage, int kk) __attribute__((always_inline)) {
+    return stage + Cfg::A_BYTES + (Cfg::B_ROWS ? kk * 32 * Cfg::CN * 2 : b_row_off + xoff[kk]);
+  };
 
   f32x4 acc[Cfg::IM][Cfg::IN];
 #pragma unroll
@@ -1616,7 +1676,7 @@ __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKAr
   // descriptor of the current tile's panel and each lane the offset of the row whose line it touches.
   // (compiled into the 256 x 64 tile only: a test and a branch per K-step are felt by the small tiles, whose
   // steps take 0.2 us: [512,4096] x [4096,1376] in 64 x 64 x 128 tiles 19.9 -> 24.3 us)
-  constexpr bool PF = Cfg::LW != 0 && Cfg::DMA && !FUSED && Cfg::CM == 256 && Cfg::CN == 64;
+  constexpr bool PF = Cfg::LW != 0 && Cfg::DMA && !Cfg::B_ROWS && !FUSED && Cfg::CM == 256 && Cfg::CN == 64;
   // a third build of the K-step, without the hand-over's tests (see `step`; not with the reduce inside the program,
   // where the K loop is the smaller part and a third copy of the step adds to what the 128-accumulator tiles spill)
   constexpr bool LEAN_STEPS = Cfg::PIPE && !FUSED;
@@ -1945,7 +2005,7 @@ __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKAr
         } else {
 #pragma unroll
           for (int s = 0; s < Cfg::S; ++s) {
-            ld.issue(p, lds + s * Cfg::STAGE, l_k, fwave);
+            ld.template issue<false>(p, lds + s * Cfg::STAGE, l_k, fwave, lane);
             advance_load_cursor();
           }
           // stage 0 has landed once at most S-1 younger slabs are outstanding
@@ -1955,7 +2015,7 @@ __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKAr
       if (worker) touch_line(p.heap_bases);  // (read in the epilogue; the multiplying waves have nothing else to do here)
       block_barrier_raw();
       if (worker) {
-        load_all<Cfg>(lds + a_row_off + xoff[0], lds + Cfg::A_BYTES + b_row_off + xoff[0], fr, 0);
+        load_all<Cfg>(lds + a_row_off + xoff[0], b_at(lds, 0), b_row_off, fr, 0);
         IRIS_WAIT_LGKMCNT0();
       }
     }
@@ -1998,7 +2058,7 @@ __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKAr
         for (int kk = 0; kk < Cfg::KSUB - 1; ++kk) {
           const int cb = (PAR + kk) & 1;
           const IRIS_LDS char* sA = stage + a_row_off + xoff[kk + 1];
-          const IRIS_LDS char* sB = stage + Cfg::A_BYTES + b_row_off + xoff[kk + 1];
+          const IRIS_LDS char* sB = b_at(stage, kk + 1);
 #pragma unroll
           for (int i = 0; i < Cfg::IM; ++i) {
             if (FIRST && kk == 0)
@@ -2006,7 +2066,7 @@ __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKAr
             else
               mma_row<Cfg, false>(acc, fr, cb, i);
             fr.a[i] = load_a<Cfg>(sA, i);
-            load_b_share<Cfg>(sB, i, fr.b[cb ^ 1]);
+            load_b_share<Cfg>(sB, b_row_off, i, fr.b[cb ^ 1]);
             __builtin_amdgcn_sched_barrier(0);
           }
         }
@@ -2062,23 +2122,23 @@ __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKAr
         }
         const IRIS_LDS char* nstage = lds + slot_n * Cfg::STAGE;
         const IRIS_LDS char* sA = nstage + a_row_off + xoff[0];
-        const IRIS_LDS char* sB = nstage + Cfg::A_BYTES + b_row_off + xoff[0];
+        const IRIS_LDS char* sB = b_at(nstage, 0);
         IRIS_LDS char* rstage = lds + slot_g * Cfg::STAGE;
         if (worker) {
           fr.a[0] = load_a<Cfg>(sA, 0);
-          load_b_share<Cfg>(sB, 0, fr.b[cb ^ 1]);
+          load_b_share<Cfg>(sB, b_row_off, 0, fr.b[cb ^ 1]);
           __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
           for (int i = 1; i < Cfg::IM; ++i) {
             mma_row<Cfg, F>(acc, fr, cb, i);
             fr.a[i] = load_a<Cfg>(sA, i);
-            load_b_share<Cfg>(sB, i, fr.b[cb ^ 1]);
+            load_b_share<Cfg>(sB, b_row_off, i, fr.b[cb ^ 1]);
             // every wave is past its reads of stage g: refill it with step g+S,
             // the L loads shared out over the blocks
             if constexpr (Cfg::LW == 0) {
 #pragma unroll
               for (int q = (i - 1) * Cfg::L / (Cfg::IM - 1); q < i * Cfg::L / (Cfg::IM - 1); ++q)
-                ld.issue_at(p, rstage, l_k, wave, q);
+                ld.template issue_at<LEAN>(p, rstage, l_k, wave, lane, q);
             }
             __builtin_amdgcn_sched_barrier(0);
           }
@@ -2091,7 +2151,7 @@ __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKAr
               // (the other set's stores, which wait for their own loads, stay behind these)
               __builtin_amdgcn_sched_barrier(0);
             } else
-              ld.issue(p, rstage, l_k, fwave);
+              ld.template issue<LEAN>(p, rstage, l_k, fwave, lane);
             if constexpr (LEAN)
               ++l_k;
             else
@@ -2230,7 +2290,7 @@ __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKAr
         __syncthreads();
 #pragma unroll
         for (int kk = 0; kk < Cfg::KSUB; ++kk) {
-          load_all<Cfg>(lds + a_row_off + xoff[kk], lds + Cfg::A_BYTES + b_row_off + xoff[kk], fr, 0);
+          load_all<Cfg>(lds + a_row_off + xoff[kk], b_at(lds, kk), b_row_off, fr, 0);
 #pragma unroll
           for (int i = 0; i < Cfg::IM; ++i) {
             if (k == kr.k_begin && kk == 0)

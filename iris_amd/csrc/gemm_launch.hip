@@ -63,7 +63,7 @@ const GemmKernelEntry* more_entries_for(int dt, int op, int* count) {
 // The plain build (every wave fetches its share) of the tile shape of `e`, an
 // entry with fetching waves; null if `e` has none or the list holds no such build.
 const GemmKernelEntry* plain_twin(const GemmKernelEntry* list, int count, const GemmKernelEntry& e) {
-  if (e.fetch_waves == 0 || !e.dma) return nullptr;
+  if (e.fetch_waves == 0 || !e.dma || e.b_rows) return nullptr;
   for (int i = 0; i < count; ++i)
     if (list[i].dma && list[i].fetch_waves == 0 && list[i].cm == e.cm && list[i].cn == e.cn && list[i].wm == e.wm &&
         list[i].wn == e.wn)
@@ -73,9 +73,10 @@ const GemmKernelEntry* plain_twin(const GemmKernelEntry* list, int count, const 
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
-// Whether every row of both operands (K-contiguous) starts on a cache line; strides in 16-bit units.
+// Whether every row of both operands (A's K-contiguous, B's along K or across it) starts on a cache line; strides in 16-bit
+// units.
 bool whole_lines(const iris_gemm_args& a) {
-  return a.stride_am % 64 == 0 && a.stride_bn % 64 == 0 &&
+  return a.stride_am % 64 == 0 && (a.stride_bn == 1 ? a.stride_bk : a.stride_bn) % 64 == 0 &&
          ((reinterpret_cast<uintptr_t>(a.a) | reinterpret_cast<uintptr_t>(a.b)) & 127) == 0;
 }
 
@@ -389,7 +390,7 @@ void launch_constants(const iris_gemm_args& a, const GemmKernelEntry& pick, Gemm
   }
   k.pf_dist = k.pf_sa = k.pf_sb = 0;
   const int pf_dist = 8;
-  if (pick.fetch_waves > 0 && pick.cm == 256 && pick.cn == 64 && !k.stream_k && k.sub_m == 1 && k.sub_n == 1 && nk >= 16 * pf_dist &&
+  if (pick.fetch_waves > 0 && pick.cm == 256 && pick.cn == 64 && !pick.b_rows && !k.stream_k && k.sub_m == 1 && k.sub_n == 1 && nk >= 16 * pf_dist &&
       a.num_xcds > 1) {
     const int64_t per_xcd = k.xcd_per > 0 ? k.xcd_per : (k.num_sms / a.num_xcds);
     int64_t tiles_per_xcd = k.split_k > 1 ? (per_xcd + k.split_k - 1) / k.split_k : per_xcd;
@@ -804,7 +805,7 @@ bool reduce_in_program(const iris_gemm_args& a, const Plan& producer) {
   const int64_t tiles = ((int64_t)a.M + a.block_m - 1) / a.block_m * (((int64_t)a.N + a.block_n - 1) / a.block_n);
   const int64_t inside = (int64_t)(a.block_m < a.M ? a.block_m : a.M) * (a.block_n < a.N ? a.block_n : a.N);
   const int64_t strips = inside * a.world_size * dtype_size(a.c_dtype);  // bytes that a program's tile is reduced from
-  if (tiles <= a.num_sms && k.vec_out && (producer.skinny || producer.entry->dma)) {
+  if (tiles <= a.num_sms && k.vec_out && (producer.skinny || (producer.entry->dma && !producer.entry->b_rows))) {
     const bool few = producer.skinny && producer.skinny_cb == 1;
     if (inside <= 64 * 64 && (few ? steps <= 2 && a.block_n <= 64 : steps <= 10)) return true;
     if (!few && tiles >= 16 && a.block_n <= 64 && steps <= 5 && (inside <= 128 * 64 || strips <= (128 << 10))) return true;
@@ -1001,6 +1002,14 @@ hipError_t make_plan_body(const iris_gemm_args& a, Plan* plan, bool cells) {
   const bool a_across = !a_along && a.stride_am == unit && a.M >= 8, b_across = !b_along && a.stride_bn == unit && a.N >= 8;
   k.a_across = a_across;
   k.b_across = b_across;
+  // A row-major B goes through the LDS-DMA too where its rows are whole aligned 16-byte chunks and all of it, K rows, lies
+  // within the 2 GiB window of a descriptor.  (us a pass gathered / so, row-major, operands from HBM: [2048,4096] x
+  // [4096,1376] 43.8 / 32.7, [2697,1936] x [1936,1600] 66.8 / 40.1, [50,2752] x [2752,7040] 27.1 / 16.2, [1232,29704] x
+  // [29704,512] 87.8 / 75.9, [42,320] x [320,3968] 11.8 / 9.4; the same weights along K take within 5 % of the latter.)
+  const bool rows_ok = !dma_ok && unit == 1 && a.stride_ak == 1 && a.stride_am > 0 && (a.stride_am % 8) == 0 && (a.K % 8) == 0 &&
+                       a.stride_bn == 1 && a.stride_bk > 0 && (a.stride_bk % 8) == 0 && (a.N % 8) == 0 && aligned16(a.a) &&
+                       aligned16(a.b) && ((int64_t)256 * a.stride_am + a.K) * 2 < ((int64_t)1 << 31) &&
+                       ((int64_t)(a.K > 128 ? a.K : 128) * a.stride_bk + 256) * 2 < ((int64_t)1 << 31);
   auto gatherable = [&](bool along, bool across, int rows, int bk, int64_t ld_row, int64_t ld_k, int64_t extent) {
     const int64_t lim = (int64_t)1 << 30;  // 16-bit units
     return (along && ld_row >= 0 && rows * ld_row + a.K < lim) ||
@@ -1011,6 +1020,7 @@ hipError_t make_plan_body(const iris_gemm_args& a, Plan* plan, bool cells) {
       return gatherable(a_along, a_across, e.cm, e.bk, a.stride_am, a.stride_ak, a.M) &&
              gatherable(b_along, b_across, e.cn, e.bk, a.stride_bn, a.stride_bk, a.N);
     if (!e.dma) return true;
+    if (e.b_rows) return rows_ok;
     if (!dma_ok) return false;
     const int64_t lim = (int64_t)1 << 31;
     return ((int64_t)e.cm * a.stride_am + a.K) * 2 < lim && ((int64_t)e.cn * a.stride_bn + a.K) * 2 < lim;
@@ -1039,8 +1049,9 @@ hipError_t make_plan_body(const iris_gemm_args& a, Plan* plan, bool cells) {
     for (int i = 0; i < more + count && !pick; ++i) {
       const GemmKernelEntry& e = i < more ? more_list[i] : list[i - more];
       if (i < more && a.ab_dtype == IRIS_DTYPE_F32 && a.K < LONG_STEPS * e.bk) continue;
-      // (the gathering tiles are for what the DMA does not take)
-      if (!fits(e) || (e.gather && dma_ok)) continue;
+      // (the gathering tiles are for what the DMA does not take, and for the reduce inside the program, of which there is
+      // no build for a row-major B)
+      if (!fits(e) || (e.gather && (dma_ok || (rows_ok && !plan->in_program)))) continue;
       if (plan->in_program && !e.fn_fused) continue;
       // (a caller's split needs a K-step per part: a tile with a deeper step may not have them)
       if (a.split_k > 1 && a.split_k > (a.K + e.bk - 1) / e.bk && e.bk > 64) continue;
