@@ -38,9 +38,21 @@ const GemmKernelEntry* entries_for(int dt, int op, int* count) {
   return nullptr;
 }
 
-// Tiles behind the table (`variant` does not number them): the fp32 ones for a K of at least LONG_STEPS of their
-// K-steps, the gathering ones.
+// Tiles behind the table (`variant` does not number them), in two lists: those for a row-major B, and the fp32 ones for a K of
+// at least LONG_STEPS of their K-steps and the gathering ones.
 constexpr int LONG_STEPS = 8;
+const GemmKernelEntry* rows_entries_for(int dt, int op, int* count) {
+  *count = 0;
+  if (dt != IRIS_DTYPE_BF16 && dt != IRIS_DTYPE_F16) return nullptr;
+  const bool bf16 = dt == IRIS_DTYPE_BF16;
+  switch (op) {
+    case OP_STORE16: return bf16 ? gemm_entries_bf16_store16_rows(count) : gemm_entries_f16_store16_rows(count);
+    case OP_STORE32: return bf16 ? gemm_entries_bf16_store32_rows(count) : gemm_entries_f16_store32_rows(count);
+    case OP_ATOMIC32: return bf16 ? gemm_entries_bf16_atomic32_rows(count) : gemm_entries_f16_atomic32_rows(count);
+    case OP_ATOMIC16: return bf16 ? gemm_entries_bf16_atomic16_rows(count) : gemm_entries_f16_atomic16_rows(count);
+  }
+  return nullptr;
+}
 const GemmKernelEntry* more_entries_for(int dt, int op, int* count) {
   *count = 0;
   switch (op) {
@@ -1044,10 +1056,11 @@ hipError_t make_plan_body(const iris_gemm_args& a, Plan* plan, bool cells) {
   if (!pick) {
     // first entry whose compute tile divides the logical tile; the rows and
     // columns a small matrix cannot fill are not worth a tall compute tile
-    int more = 0;
+    int more = 0, rows = 0;
     const GemmKernelEntry* more_list = more_entries_for(a.ab_dtype, op, &more);
-    for (int i = 0; i < more + count && !pick; ++i) {
-      const GemmKernelEntry& e = i < more ? more_list[i] : list[i - more];
+    const GemmKernelEntry* rows_list = rows_entries_for(a.ab_dtype, op, &rows);
+    for (int i = -rows; i < more + count && !pick; ++i) {
+      const GemmKernelEntry& e = i < 0 ? rows_list[i + rows] : i < more ? more_list[i] : list[i - more];
       if (i < more && a.ab_dtype == IRIS_DTYPE_F32 && a.K < LONG_STEPS * e.bk) continue;
       // (the gathering tiles are for what the DMA does not take, and for the reduce inside the program, of which there is
       // no build for a row-major B)

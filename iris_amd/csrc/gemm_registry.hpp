@@ -140,7 +140,7 @@ constexpr GemmKernelEntry make_entry(const char* name) {
   X(DT, OP, 64, 128, 64, 2, 2, 2, LOAD_GATHER, 4, 1, "64x128x64_w2x2_gather")   \
   X(DT, OP, 64, 64, 128, 2, 2, 2, LOAD_GATHER, 4, 1, "64x64x128_w2x2_gather")
 
-// ... and in front of those, the LDS-DMA tiles for a row-major B, the first for the store epilogues only (atomics take half
+// ... and, in a list of their own in front of those, the LDS-DMA tiles for a row-major B, the first for the store epilogues only (atomics take half
 // tiles).  The gathering tiles transpose such a B in the fetching waves' registers, and a K-step waits for them: a step of
 // 128 x 128 x 64 in 1.2 us.  Here the DMA brings the rows as they lie and the transposing LDS read costs what a plain one
 // does: 0.45 us, as for a B along K ([2697,1936] x [1936,1600], 275 tiles in two rounds, 66.8 -> 40.1 us a pass).
@@ -268,6 +268,14 @@ IRIS_GEMM_DECLARE(f32_store32)
 IRIS_GEMM_DECLARE(f32_atomic32)
 IRIS_GEMM_DECLARE(f32_store32_long)
 IRIS_GEMM_DECLARE(f32_atomic32_long)
+IRIS_GEMM_DECLARE(bf16_store16_rows)
+IRIS_GEMM_DECLARE(bf16_store32_rows)
+IRIS_GEMM_DECLARE(bf16_atomic32_rows)
+IRIS_GEMM_DECLARE(bf16_atomic16_rows)
+IRIS_GEMM_DECLARE(f16_store16_rows)
+IRIS_GEMM_DECLARE(f16_store32_rows)
+IRIS_GEMM_DECLARE(f16_atomic32_rows)
+IRIS_GEMM_DECLARE(f16_atomic16_rows)
 IRIS_GEMM_DECLARE(bf16_store16_gather)
 IRIS_GEMM_DECLARE(bf16_store32_gather)
 IRIS_GEMM_DECLARE(bf16_atomic32_gather)
