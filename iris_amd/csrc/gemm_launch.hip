@@ -756,6 +756,12 @@ bool plan_small(const iris_gemm_args& a, Plan* plan) {
   if (words > 0 && (!a.locks || words > a.num_sms)) return found;
   // (the last part raises the flag for all: where it is a release, only its own stores would be covered, see publish_tile)
   if (words > 0 && a.flag_sem == IRIS_FLAG_SEM_RELEASE_ACQUIRE) return found;
+  // Where K of the caller's tiles is shared out, parts larger than 64 x 64 are taken up to this K only: they fetch no less
+  // than the shared tiles do, and the longer the K the less their hand-over weighs.  (us a pass, the caller's tiles / parts:
+  // 256 x 256 tiles [2534,1664] x [1664,896] 35.5 / 19.1, [667,5888] x [5888,4160] 72 / 58, [1669,30872] x [30872,320] 91 /
+  // 95; 256 x 128 [3319,1792] x [1792,312] 24.3 / 17.0, [7069,13376] x [13376,512] 117 / 138; 256 x 64 [797,2048] x
+  // [2048,1856] 32.1 / 27.6, [786,25064] x [25064,1368] 154 / 232; 128 x 128 tiles [1024,2048] x [2048,1376] keep theirs.)
+  const int whole_k = a.ab_dtype == IRIS_DTYPE_F32 || a.block_m < 256 ? 0 : a.block_n >= 256 ? 6144 : 2560;
   static const int shapes[4][2] = {{64, 64}, {128, 64}, {64, 128}, {128, 128}};
   TileLaunch list[8];
   double times[8];
@@ -765,9 +771,7 @@ bool plan_small(const iris_gemm_args& a, Plan* plan) {
     const int64_t tiles = tiles_of(s[0], s[1]);
     if (tiles > a.num_sms) continue;
     if (s[0] == a.block_m && s[1] == a.block_n) break;  // (the caller's tile is the smallest that fits)
-    // (a larger part than 64 x 64 only halves or quarters the tile; where K is shared out over as many programs that
-    // has been done)
-    if (s[0] * s[1] > 64 * 64 && w.split_k > 1) break;
+    if (s[0] * s[1] > 64 * 64 && w.split_k > 1 && a.K > whole_k) break;
     const int bk = s[0] == 64 && s[1] == 64 ? 128 : 64;  // (the 64 x 64 tile's K-step)
     int sk = a.partials && a.locks ? auto_split(tiles, (int)(((int64_t)a.K + bk - 1) / bk) * (bk / 64), a.num_sms) : 1;
     // (the parts of a part's K use the locks, too)
