@@ -496,43 +496,6 @@ void split_last_round(const iris_gemm_args& a, Plan* plan) {
   plan->last_round = 1;
 }
 
-// How a plain launch's tiles are blocked: merge_m x merge_n of the caller's tiles as one 256 x 256 or 256 x 128
-// tile, when the `tiles_n` columns of tiles suffice for it.  Returns false for "the caller's tiles as they are".
-bool choose_merge(const iris_gemm_args& a, int64_t tiles_n, int* merge_m, int* merge_n) {
-  *merge_m = *merge_n = 1;
-  const int64_t tiles_m = (a.M + a.block_m - 1) / a.block_m;
-  const int mm = 256 / a.block_m;  // 1 or 2
-  const int64_t rows = (tiles_m + mm - 1) / mm;
-  // 256 x 256 or 256 x 128, whichever finishes first among those that give (almost) every program a tile: rounds
-  // of tiles times the tile's time (a 256 x 256 tile does twice the work at 1.25 times the rate, as measured)
-  double best = 0;
-  for (int width = 256; width >= 128; width /= 2) {
-    const int mn = width / a.block_n;
-    const int64_t merged_tiles = rows * ((tiles_n + mn - 1) / mn);
-    // (seven programs in eight busy is enough: [8192,14336] x [14336,1792] as 224 tiles of 256 x 256 in one
-    // round against 448 of 256 x 128 in two)
-    if (mm * mn == 1 || merged_tiles * 8 < (int64_t)a.num_sms * 7) continue;
-    const double cost = (double)((merged_tiles + a.num_sms - 1) / a.num_sms) * (width == 256 ? 1.6 : 1.0);
-    if (best == 0 || cost < best) best = cost, *merge_m = mm, *merge_n = mn;
-  }
-  if (*merge_m * *merge_n > 1) return true;
-  if (!a.partials || !a.locks || a.K < 4096) return false;
-  // No block of the caller's tiles gives every program one.  Blocks that give every OTHER program one do, with
-  // each block's K range shared by two programs; their hand-over takes slots of half a (merged) tile, which is
-  // what the caller's workspace holds when the blocks are pairs of its tiles ([8192,14336] x [14336,448] in
-  // 256 x 64 tiles: 175 -> 114 us).
-  for (int width = 256; width >= 128; width /= 2) {
-    const int mn = width / a.block_n;
-    const int64_t merged_tiles = rows * ((tiles_n + mn - 1) / mn);
-    if (mm * mn == 1 || mn < 1) continue;
-    if (merged_tiles * 2 > a.num_sms || merged_tiles * 16 < (int64_t)a.num_sms * 7) continue;
-    if (a.partials_slot_elems * 2 < (int64_t)256 * width) continue;
-    *merge_m = mm, *merge_n = mn;
-    return true;
-  }
-  return false;
-}
-
 // The plan for the caller's tiles blocked merge_m x merge_n; false when the launcher has no kernel for it.
 bool plan_merged(const iris_gemm_args& a, int merge_m, int merge_n, Plan* plan) {
   iris_gemm_args b = a;
@@ -833,6 +796,111 @@ bool reduce_in_program(const iris_gemm_args& a, const Plan& producer) {
   return steps <= 8 || (steps <= 24 && a.block_m * a.block_n <= 128 * 128);
 }
 
+// Times of a launch in large tiles, by which plan_blocks compares its plans: us = fixed + rounds of tiles * (tile + K-steps
+// of a part * step), a step being dearer by `cover` when every CU takes one (the board's power, the L2s), by `off_lines`
+// where rows do not start on cache lines, by `streamed` where the operands come from HBM (none of it up to 50 MB, all from
+// 150 MB on: a program has other data in the 256 MB of the last-level cache between two launches).  Fitted to 22000 timings
+// of 3750 random shapes ([500 .. 8192, 256 .. 36864] x [.., 400 .. 8192], operands changed from launch to launch): rms 6 %.
+struct BlockTime {
+  int cm, cn, split;
+  double fixed, tile, step, cover, off_lines, streamed;
+};
+constexpr BlockTime BLOCK_TIMES[] = {
+    {128, 64, 1, 4.4, 2.0, 0.249, 0.03, 0.45, 0.45},  {128, 128, 1, 4.4, 2.3, 0.384, 0.00, 0.35, 0.35},
+    {256, 64, 1, 4.6, 2.2, 0.443, 0.00, 0.44, 0.32},  {256, 128, 1, 3.7, 3.5, 0.511, 0.25, 0.34, 0.34},
+    {256, 128, 2, 9.2, 4.5, 0.693, 0.00, 0.40, 0.31}, {256, 256, 1, 2.6, 5.2, 0.899, 0.32, 0.22, 0.31},
+    {256, 256, 2, 10.6, 6.4, 0.719, 0.78, 0.23, 0.26},
+};
+// The plan's time in us, or a negative number for a launch that the table does not know.
+double block_us(const iris_gemm_args& a, const Plan& plan) {
+  const GemmKArgs& k = plan.k;
+  if (!plan.entry || plan.skinny || k.stream_k || k.sub_m != 1 || k.sub_n != 1 || plan.entry->bk != 64) return -1;
+  const bool lines = whole_lines(a);
+  double streamed = (((double)a.M + a.N) * a.K * 2e-6 - 50) / 100;
+  streamed = streamed < 0 ? 0 : streamed > 1 ? 1 : streamed;
+  const int nk = (a.K + 63) / 64, cus = current_cu_count();
+  for (const BlockTime& t : BLOCK_TIMES) {
+    if (t.cm != plan.entry->cm || t.cn != plan.entry->cn || t.split != k.split_k) continue;
+    const int64_t items = (int64_t)k.total_tiles * t.split, rounds = (items + k.num_sms - 1) / k.num_sms;
+    const double busy = (double)(rounds > 1 ? k.num_sms : items) / cus;
+    const double step = t.step * (1 + t.cover * busy) * (lines ? 1.0 : 1 + t.off_lines) * (1 + t.streamed * streamed);
+    // (the other copies of the output, or its wider elements: 6.5 TB/s of stores on all CUs)
+    const double copies = (k.dest_all ? a.world_size : 1) * (plan.entry->op == OP_STORE32 ? 2 : 1);
+    const double tile = t.tile + (copies - 1) * t.cm * t.cn * 2 / 25400.0 / t.split;
+    const double us = t.fixed + rounds * (tile + (nk + t.split - 1) / t.split * step);
+    if (!plan.last_round) return us;
+    // The tiles of a last round that are shared out over all programs, as a launch of their own, whose programs share less of
+    // what they fetch.  ([8192,36864] x [36864,576] in 256 x 64 tiles, 256 and then 32 in eight parts, 565 us, 717 in two
+    // rounds; [2624,26328] x [26328,1520], 256 and 8 in twelve parts, 352)
+    const double apart = 1 + plan.k_last.total_tiles / (t.cm * t.cn >= 256 * 128 ? 256.0 : 32.0);
+    return us + 8 + tile + (nk + plan.k_last.split_k - 1) / plan.k_last.split_k * step * apart;
+  }
+  return -1;
+}
+
+// A large launch in the caller's tiles or in blocks of them, as 256 x 128 or 256 x 256 tiles, whichever is expected to
+// finish first; K shared by two programs a block where half of them suffice for the blocks and the caller's workspace has
+// the slots; or the columns of tiles that block well first and the rest as a launch of their own.  (us, [8192,K] x [K,N] in
+// 256 x 64 tiles, the caller's / 256 x 128 / 256 x 256: N 576, K 1024 23 / 16 / 24; N 704, K 4128 98 / 53 / -; N 1152, K 12288
+// 337 / 299 / 263; N 1344, K 4096 100 / 100 / 82.  By number of tiles alone, blocks only where they gave seven programs in
+// eight a tile, the plan of a random shape took 1.16, 1.07 and 1.12 times the best one's time for 256 x 64, 256 x 128 and
+// 128 x 128 tiles; by these times 1.001 to 1.003.)
+bool plan_blocks(const iris_gemm_args& a, Plan* plan) {
+  Plan best;
+  if (make_plan_body(a, &best) != hipSuccess) return false;
+  own_flags(&best);
+  split_last_round(a, &best);
+  double least = block_us(a, best);
+  if (least < 0) return false;  // (K of the caller's tiles shared out, or no such tile)
+  auto blocked = [&](const iris_gemm_args& b, Plan* into, double limit) {
+    double us = -1;
+    for (int width = 256; width >= 128; width /= 2) {
+      const int mm = 256 / b.block_m, mn = width / b.block_n;
+      Plan merged;
+      if (mn < 1 || mm * mn == 1 || !plan_merged(b, mm, mn, &merged)) continue;
+      // (a launch on fewer programs than CUs leaves room for others: none of its own stays idle for a larger block)
+      if (b.num_sms < current_cu_count() && (int64_t)merged.k.total_tiles * merged.k.split_k * 8 < (int64_t)b.num_sms * 7) continue;
+      const double t = block_us(b, merged);
+      if (t > 0 && t < (us < 0 ? limit : us)) us = t, *into = merged;
+    }
+    return us;
+  };
+  // (what is as good by the estimate is better off in larger blocks: [8192,4096] x [4096,384] in 256 x 64 tiles 33.2 us, in
+  // 256 x 128 with K in two 32.1)
+  const double us = blocked(a, &best, best.last_round ? least : least * 1.04);
+  if (us > 0) least = us;
+  // The columns of tiles may be one or a few too many for blocks that fill the programs: [8192,36864] x [36864,576] is nine
+  // columns of 256 x 64 tiles, eight of which make 128 blocks with K in two parts.  (For a K that can be shared out.)
+  const int64_t tiles_n = a.N / a.block_n;
+  const bool two_kernels = a.epilogue == IRIS_EPI_ONE_SHOT && a.phase != IRIS_PHASE_PRODUCE;
+  if (a.N % a.block_n == 0 && a.K >= 4096 && a.partials && a.locks && !two_kernels) {
+    for (int width = 256; width >= 128; width /= 2) {
+      const int mn = width / a.block_n;
+      if (mn < 2) continue;
+      const int64_t main_n = tiles_n / mn * mn, rest_n = tiles_n - main_n;
+      if (main_n == 0 || rest_n == 0 || rest_n * 4 > main_n) continue;
+      const iris_gemm_args am = column_range(a, 0, main_n * a.block_n);
+      const iris_gemm_args ar = column_range(a, main_n * a.block_n, rest_n * a.block_n);
+      Plan first;
+      auto rest = std::make_shared<Plan>();
+      const double main_us = blocked(am, &first, least);
+      // (the remaining columns as the caller's tiles; their flags sit at their place in the caller's grid)
+      if (main_us < 0 || !plan_merged(ar, 1, 1, rest.get())) continue;
+      // K of the rest shared out so far that A streams through again: at 5.2 MB a us
+      const double rest_us = 12 + ((double)ar.M + ar.N) * ar.K * 2e-6 / 5.2;
+      if (main_us + rest_us >= least) continue;
+      least = main_us + rest_us;
+      best = first;
+      best.k.flag_num_pid_n = (int)tiles_n;
+      rest->k.flag_num_pid_n = (int)tiles_n;
+      rest->k.flag_pn_base = (int)main_n;
+      best.rest = rest;
+    }
+  }
+  *plan = best;
+  return true;
+}
+
 hipError_t make_plan_units(const iris_gemm_args& a, Plan* plan) {
   if (a.epilogue == IRIS_EPI_ONE_SHOT && a.phase == IRIS_PHASE_FUSED) {
     iris_gemm_args b = a;
@@ -847,43 +915,10 @@ hipError_t make_plan_units(const iris_gemm_args& a, Plan* plan) {
   }
   if (plan_small(a, plan)) return hipSuccess;
   const bool plain = a.variant == 0 && a.split_k == 0 && !a.mm_begin_timestamp && !a.mm_end_timestamp &&
-                     !(a.epilogue == IRIS_EPI_ONE_SHOT && a.phase != IRIS_PHASE_PRODUCE) &&
+                     !(a.epilogue == IRIS_EPI_ONE_SHOT && a.phase != IRIS_PHASE_PRODUCE && a.phase != IRIS_PHASE_TWO_KERNELS) &&
                      a.epilogue != IRIS_EPI_ATOMIC_ADD && a.num_sms > 0 && (a.block_m == 128 || a.block_m == 256) &&
                      (a.block_n == 64 || a.block_n == 128) && a.M >= 256;
-  const bool plain_two_kernels = a.variant == 0 && a.split_k == 0 && !a.mm_begin_timestamp && !a.mm_end_timestamp &&
-                                 a.epilogue == IRIS_EPI_ONE_SHOT && a.phase == IRIS_PHASE_TWO_KERNELS && a.num_sms > 0 &&
-                                 (a.block_m == 128 || a.block_m == 256) && (a.block_n == 64 || a.block_n == 128) &&
-                                 a.M >= 256;
-  if (plain || plain_two_kernels) {
-    const int64_t tiles_n = (a.N + a.block_n - 1) / a.block_n;
-    int merge_m = 1, merge_n = 1;
-    if (choose_merge(a, tiles_n, &merge_m, &merge_n)) {
-      if (plan_merged(a, merge_m, merge_n, plan)) return hipSuccess;
-    } else if (plain && a.N % a.block_n == 0) {
-      // The columns of tiles are one or a few too many for a blocking that pays: [8192,36864] x [36864,576] is nine
-      // columns of 256 x 64 tiles, eight of which block into 128 pairs with K in two parts.  The launch then
-      // takes the columns that block first and the remaining ones as a launch of their own behind it.
-      for (int width = 256; width >= 128; width /= 2) {
-        const int mn = width / a.block_n;
-        const int64_t main_n = tiles_n / mn * mn, rest_n = tiles_n - main_n;
-        if (mn < 2 || main_n == 0 || rest_n == 0 || rest_n * 4 > main_n) continue;
-        const iris_gemm_args am = column_range(a, 0, main_n * a.block_n);
-        if (!choose_merge(am, main_n, &merge_m, &merge_n)) continue;
-        Plan first;
-        if (!plan_merged(am, merge_m, merge_n, &first)) continue;
-        const iris_gemm_args ar = column_range(a, main_n * a.block_n, rest_n * a.block_n);
-        auto rest = std::make_shared<Plan>();
-        // (the remaining columns as the caller's tiles; their flags sit at their place in the caller's grid)
-        if (!plan_merged(ar, 1, 1, rest.get())) continue;
-        first.k.flag_num_pid_n = (int)tiles_n;
-        rest->k.flag_num_pid_n = (int)tiles_n;
-        rest->k.flag_pn_base = (int)main_n;
-        *plan = first;
-        plan->rest = rest;
-        return hipSuccess;
-      }
-    }
-  }
+  if (plain && plan_blocks(a, plan)) return hipSuccess;
   const hipError_t err = make_plan_body(a, plan);
   own_flags(plan);
   if (err == hipSuccess) split_last_round(a, plan);
