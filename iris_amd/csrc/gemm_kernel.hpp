@@ -211,13 +211,15 @@ struct Mfma<IRIS_DTYPE_F32> {
 // registers, for operands with any alignment that are contiguous along k or across it (see Gather).  LOAD_GENERIC:
 // element by element, for what is contiguous along neither.  LOAD_DMA_ROWS: LOAD_DMA for a B whose rows are its k (a row-major
 // [K, N]): the slab of B lies in LDS as it does in memory, BK rows of CN columns, and is transposed on its way to the
-// MFMAs, by ds_read_b64_tr_b16 (see load_b).
-enum SlabLoad { LOAD_GENERIC = 0, LOAD_DMA = 1, LOAD_GATHER = 2, LOAD_DMA_ROWS = 3 };
+// MFMAs, by ds_read_b64_tr_b16 (see load_b).  LOAD_DMA_LOOSE: LOAD_DMA for operands along k at any alignment and of any K from
+// eight on (see Loader::before_step and mask_tail).
+enum SlabLoad { LOAD_GENERIC = 0, LOAD_DMA = 1, LOAD_GATHER = 2, LOAD_DMA_ROWS = 3, LOAD_DMA_LOOSE = 4 };
 template <int DT_, int CM_, int CN_, int BK_, int WM_, int WN_, int S_, int LOAD_, int LW_ = 0, bool TOUCH_ = false>
 struct GemmCfg {
   static constexpr int DT = DT_, CM = CM_, CN = CN_, BK = BK_, WM = WM_, WN = WN_, S = S_;
   static constexpr bool B_ROWS = LOAD_ == LOAD_DMA_ROWS;
-  static constexpr bool DMA = LOAD_ == LOAD_DMA || B_ROWS, GATHER = LOAD_ == LOAD_GATHER;
+  static constexpr bool LOOSE = LOAD_ == LOAD_DMA_LOOSE;
+  static constexpr bool DMA = LOAD_ == LOAD_DMA || B_ROWS || LOOSE, GATHER = LOAD_ == LOAD_GATHER;
   static constexpr bool PIPE = LOAD_ != LOAD_GENERIC;  // the K loop runs as a pipeline across tiles
   static constexpr int NW = WM * WN, NT = NW * 64;  // the waves (threads) that multiply and store
   static constexpr int LW = LW_;
@@ -409,6 +411,9 @@ struct Loader {
   // (Cfg::TOUCH) byte offset of the row whose line this lane touches ahead of the loads, out of range for none
   uint32_t ta, tb;
   int step_kb;  // (Cfg::B_ROWS) bytes from a K-step of B to the next
+  // (Cfg::LOOSE) A row's last chunk may reach past K.  It is fetched moved back to end at K, so that nothing outside the
+  // row is read: the descriptors begin a chunk in front of the operands, and no offset is ever below zero.
+  static constexpr int LEAD = Cfg::LOOSE ? 16 : 0;
 
   // (Cfg::B_ROWS) The slab of B holds, for each k, CN columns as 32-byte pieces (what the transposing read of one 16-column
   // block takes from one k) XOR-ed by this number: 32 lanes of that read take eight k, 8 q .. 8 q + 3 and 8 q + 8 .. 8 q + 11,
@@ -444,11 +449,11 @@ struct Loader {
     const uint32_t brec = rows_b <= 0   ? 0
                           : Cfg::B_ROWS ? (uint32_t)(((int64_t)(p.K - 1) * p.sbk + rows_b) * 2)
                                         : (uint32_t)(((int64_t)(rows_b - 1) * p.sbn + p.K) * 2);
-    ra = __builtin_amdgcn_make_buffer_rsrc((void*)abase, 0, arec, 0x00020000);
-    rb = __builtin_amdgcn_make_buffer_rsrc((void*)bbase, 0, brec, 0x00020000);
+    ra = __builtin_amdgcn_make_buffer_rsrc((void*)(abase - LEAD), 0, arec > 0 ? arec + LEAD : 0, 0x00020000);
+    rb = __builtin_amdgcn_make_buffer_rsrc((void*)(bbase - LEAD), 0, brec > 0 ? brec + LEAD : 0, 0x00020000);
     k_limit = p.K;
     const int row = wave * Cfg::RPB + lane / Cfg::CPR, ck = chunk_k(wave, lane);
-    va = (uint32_t)(((int64_t)row * p.sam + ck) * 2);
+    va = (uint32_t)(((int64_t)row * p.sam + ck) * 2) + LEAD;
     step_a = (int)((int64_t)Cfg::NL * Cfg::RPB * p.sam * 2);
     if constexpr (Cfg::B_ROWS) {
       const int col = rows_col(wave, lane);
@@ -457,7 +462,7 @@ struct Loader {
       step_b = (int)((int64_t)Cfg::NL * Cfg::B_RPB * p.sbk * 2);
       step_kb = (int)((int64_t)Cfg::BK * p.sbk * 2);
     } else {
-      vb = (uint32_t)(((int64_t)row * p.sbn + ck) * 2);
+      vb = (uint32_t)(((int64_t)row * p.sbn + ck) * 2) + LEAD;
       step_b = (int)((int64_t)Cfg::NL * Cfg::RPB * p.sbn * 2);
     }
     if constexpr (Cfg::TOUCH) {
@@ -480,12 +485,17 @@ struct Loader {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (IRIS_LDS void*)scratch, 4, ta, k * Cfg::BK * 2, 0, 0);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (IRIS_LDS void*)scratch, 4, tb, k * Cfg::BK * 2, 0, 0);
   }
-  // The load cursor is about to load step `k`: park the chunks past K.
+  // The load cursor is about to load step `k`: park the chunks past K.  (LOOSE: and move a chunk that K cuts back to end
+  // there.  What it then holds in front of its own k, mask_tail clears in the fragments.)
   __device__ inline void before_step(int k, int wave, int lane) {
     if (k_limit - k * Cfg::BK >= Cfg::BK) return;  // a full step: nothing to mask
     if (k * Cfg::BK + chunk_k(wave, lane) >= k_limit) {
       va = 0x80000000u;
       if constexpr (!Cfg::B_ROWS) vb = 0x80000000u;  // (else the loads of the step are masked one by one, see issue_at)
+    } else if (Cfg::LOOSE) {
+      const uint32_t back = (uint32_t)max(0, k * Cfg::BK + chunk_k(wave, lane) + 8 - k_limit) * 2;
+      va -= back;
+      vb -= back;
     }
   }
   // The program has no more steps to load: the loads are still issued, so
@@ -803,6 +813,17 @@ __device__ inline typename Mfma<Cfg::DT>::vec8 load_b(const IRIS_LDS char* sB, i
   } else {
     return *reinterpret_cast<const IRIS_LDS typename Mfma<Cfg::DT>::vec8*>(sB + j * 16 * Cfg::BK * 2);
   }
+}
+
+// (Operands at any alignment) Clear what stands in front of its own k in a chunk that was moved back to end at K: the first `n` of this
+// lane's eight elements (none in lanes that hold another chunk).  Both operands' fragments, so that an infinity which the
+// moved chunk repeats is not multiplied by the other's zero.
+template <int DT>
+__device__ inline void mask_tail(typename Mfma<DT>::vec8& v, int n) {
+  u32x4 x = __builtin_bit_cast(u32x4, v);
+#pragma unroll
+  for (int w = 0; w < 4; ++w) x[w] &= n >= 2 * w + 2 ? 0u : n == 2 * w + 1 ? 0xFFFF0000u : 0xFFFFFFFFu;
+  v = __builtin_bit_cast(typename Mfma<DT>::vec8, x);
 }
 
 // B fragments fetched next to A block i, so that all IN of them are spread
@@ -1676,7 +1697,7 @@ __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKAr
   // descriptor of the current tile's panel and each lane the offset of the row whose line it touches.
   // (compiled into the 256 x 64 tile only: a test and a branch per K-step are felt by the small tiles, whose
   // steps take 0.2 us: [512,4096] x [4096,1376] in 64 x 64 x 128 tiles 19.9 -> 24.3 us)
-  constexpr bool PF = Cfg::LW != 0 && Cfg::DMA && !Cfg::B_ROWS && !FUSED && Cfg::CM == 256 && Cfg::CN == 64;
+  constexpr bool PF = Cfg::LW != 0 && Cfg::DMA && !Cfg::B_ROWS && !Cfg::LOOSE && !FUSED && Cfg::CM == 256 && Cfg::CN == 64;
   // a third build of the K-step, without the hand-over's tests (see `step`; not with the reduce inside the program,
   // where the K loop is the smaller part and a third copy of the step adds to what the 128-accumulator tiles spill)
   constexpr bool LEAN_STEPS = Cfg::PIPE && !FUSED;
@@ -2034,6 +2055,20 @@ __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKAr
     // too; what it fetches is never used (loads past the last step fetch
     // nothing).
     int ring_slot = 0;  // slot of the step about to run (rings whose depth is no power of two)
+    // (LOOSE) the step about to run, of those the tile's K has, where it is not a lean one; the step, the substep and the
+    // chunk of it that K cuts
+    int cur_k = 0;
+    const int cut_step = Cfg::LOOSE && (p.K & 7) ? nk - 1 : -1, cut_chunk = (p.K % Cfg::BK) / 8;
+    auto mask_cut = [&](Frags<Cfg>& f, int cb, int kk) __attribute__((always_inline)) {
+      if constexpr (Cfg::LOOSE) {
+        if (cur_k != cut_step || kk != cut_chunk / 4) return;
+        const int n = lq == (cut_chunk & 3) ? 8 - (p.K & 7) : 0;
+#pragma unroll
+        for (int j = 0; j < Cfg::IN; ++j) mask_tail<Cfg::DT>(f.b[cb][j], n);
+#pragma unroll
+        for (int i = 0; i < Cfg::IM; ++i) mask_tail<Cfg::DT>(f.a[i], n);
+      }
+    };
     // LEAN: a step in the middle of a tile's K loop.  No tile waits to be published at its hand-over (the
     // previous tile's flag went up at this tile's second hand-over) and the load cursor's next step lies inside
     // the tile and is a full one, so the hand-over is a wait, the barrier and the refill, with no test between
@@ -2059,6 +2094,7 @@ __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKAr
           const int cb = (PAR + kk) & 1;
           const IRIS_LDS char* sA = stage + a_row_off + xoff[kk + 1];
           const IRIS_LDS char* sB = b_at(stage, kk + 1);
+          if constexpr (!LEAN) mask_cut(fr, cb, kk);
 #pragma unroll
           for (int i = 0; i < Cfg::IM; ++i) {
             if (FIRST && kk == 0)
@@ -2076,6 +2112,7 @@ __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKAr
         constexpr int cb = (PAR + kk) & 1;
         constexpr bool F = FIRST && kk == 0;
         if (worker) {
+          if constexpr (!LEAN) mask_cut(fr, cb, kk);
           mma_row<Cfg, F>(acc, fr, cb, 0);
           __builtin_amdgcn_sched_barrier(0);
           // this wave's reads of stage g have returned (they were issued a
@@ -2207,6 +2244,7 @@ __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKAr
       const KRange kr = k_range<Cfg, SPLIT>(p, sr, pid, it, nk);
       prefetch_setup(c_it);
       prefetch_step(kr.k_begin + p.pf_dist, kr.k_end);
+      cur_k = kr.k_begin;
       run_step(g, std::true_type{}, std::false_type{});
       ++g;
       const int steps = kr.k_end - kr.k_begin;
@@ -2216,6 +2254,7 @@ __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKAr
       int k = 1;
       for (; k < steps && k < 2; ++k, ++g) {
         prefetch_step(kr.k_begin + k + p.pf_dist, kr.k_end);
+        cur_k = kr.k_begin + k;
         run_step(g, std::false_type{}, std::false_type{});
       }
       if constexpr (PF8) {
@@ -2261,6 +2300,7 @@ __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKAr
       }
       for (; k < steps; ++k, ++g) {
         prefetch_step(kr.k_begin + k + p.pf_dist, kr.k_end);
+        cur_k = kr.k_begin + k;
         run_step(g, std::false_type{}, std::false_type{});
       }
       if constexpr (ONE_ITEM) IRIS_WAIT_VMCNT(0);  // (the loads past the last step fetch nothing, and nothing follows)

@@ -38,8 +38,8 @@ const GemmKernelEntry* entries_for(int dt, int op, int* count) {
   return nullptr;
 }
 
-// Tiles behind the table (`variant` does not number them), in two lists: those for a row-major B, and the fp32 ones for a K of
-// at least LONG_STEPS of their K-steps and the gathering ones.
+// Tiles behind the table (`variant` does not number them), in three lists: those for a row-major B, those for operands at any
+// alignment, and the fp32 ones for a K of at least LONG_STEPS of their K-steps with the gathering ones.
 constexpr int LONG_STEPS = 8;
 const GemmKernelEntry* rows_entries_for(int dt, int op, int* count) {
   *count = 0;
@@ -50,6 +50,18 @@ const GemmKernelEntry* rows_entries_for(int dt, int op, int* count) {
     case OP_STORE32: return bf16 ? gemm_entries_bf16_store32_rows(count) : gemm_entries_f16_store32_rows(count);
     case OP_ATOMIC32: return bf16 ? gemm_entries_bf16_atomic32_rows(count) : gemm_entries_f16_atomic32_rows(count);
     case OP_ATOMIC16: return bf16 ? gemm_entries_bf16_atomic16_rows(count) : gemm_entries_f16_atomic16_rows(count);
+  }
+  return nullptr;
+}
+const GemmKernelEntry* loose_entries_for(int dt, int op, int* count) {
+  *count = 0;
+  if (dt != IRIS_DTYPE_BF16 && dt != IRIS_DTYPE_F16) return nullptr;
+  const bool bf16 = dt == IRIS_DTYPE_BF16;
+  switch (op) {
+    case OP_STORE16: return bf16 ? gemm_entries_bf16_store16_loose(count) : gemm_entries_f16_store16_loose(count);
+    case OP_STORE32: return bf16 ? gemm_entries_bf16_store32_loose(count) : gemm_entries_f16_store32_loose(count);
+    case OP_ATOMIC32: return bf16 ? gemm_entries_bf16_atomic32_loose(count) : gemm_entries_f16_atomic32_loose(count);
+    case OP_ATOMIC16: return bf16 ? gemm_entries_bf16_atomic16_loose(count) : gemm_entries_f16_atomic16_loose(count);
   }
   return nullptr;
 }
@@ -75,7 +87,7 @@ const GemmKernelEntry* more_entries_for(int dt, int op, int* count) {
 // The plain build (every wave fetches its share) of the tile shape of `e`, an
 // entry with fetching waves; null if `e` has none or the list holds no such build.
 const GemmKernelEntry* plain_twin(const GemmKernelEntry* list, int count, const GemmKernelEntry& e) {
-  if (e.fetch_waves == 0 || !e.dma || e.b_rows) return nullptr;
+  if (e.fetch_waves == 0 || !e.dma || e.b_rows || e.loose) return nullptr;
   for (int i = 0; i < count; ++i)
     if (list[i].dma && list[i].fetch_waves == 0 && list[i].cm == e.cm && list[i].cn == e.cn && list[i].wm == e.wm &&
         list[i].wn == e.wn)
@@ -402,7 +414,7 @@ void launch_constants(const iris_gemm_args& a, const GemmKernelEntry& pick, Gemm
   }
   k.pf_dist = k.pf_sa = k.pf_sb = 0;
   const int pf_dist = 8;
-  if (pick.fetch_waves > 0 && pick.cm == 256 && pick.cn == 64 && !pick.b_rows && !k.stream_k && k.sub_m == 1 && k.sub_n == 1 && nk >= 16 * pf_dist &&
+  if (pick.fetch_waves > 0 && pick.cm == 256 && pick.cn == 64 && !pick.b_rows && !pick.loose && !k.stream_k && k.sub_m == 1 && k.sub_n == 1 && nk >= 16 * pf_dist &&
       a.num_xcds > 1) {
     const int64_t per_xcd = k.xcd_per > 0 ? k.xcd_per : (k.num_sms / a.num_xcds);
     int64_t tiles_per_xcd = k.split_k > 1 ? (per_xcd + k.split_k - 1) / k.split_k : per_xcd;
@@ -784,7 +796,7 @@ bool reduce_in_program(const iris_gemm_args& a, const Plan& producer) {
   const int64_t tiles = ((int64_t)a.M + a.block_m - 1) / a.block_m * (((int64_t)a.N + a.block_n - 1) / a.block_n);
   const int64_t inside = (int64_t)(a.block_m < a.M ? a.block_m : a.M) * (a.block_n < a.N ? a.block_n : a.N);
   const int64_t strips = inside * a.world_size * dtype_size(a.c_dtype);  // bytes that a program's tile is reduced from
-  if (tiles <= a.num_sms && k.vec_out && (producer.skinny || (producer.entry->dma && !producer.entry->b_rows))) {
+  if (tiles <= a.num_sms && k.vec_out && (producer.skinny || (producer.entry->dma && !producer.entry->b_rows && !producer.entry->loose))) {
     const bool few = producer.skinny && producer.skinny_cb == 1;
     if (inside <= 64 * 64 && (few ? steps <= 2 && a.block_n <= 64 : steps <= 10)) return true;
     if (!few && tiles >= 16 && a.block_n <= 64 && steps <= 5 && (inside <= 128 * 64 || strips <= (128 << 10))) return true;
@@ -1061,6 +1073,13 @@ hipError_t make_plan_body(const iris_gemm_args& a, Plan* plan, bool cells) {
                        a.stride_bn == 1 && a.stride_bk > 0 && (a.stride_bk % 8) == 0 && (a.N % 8) == 0 && aligned16(a.a) &&
                        aligned16(a.b) && ((int64_t)256 * a.stride_am + a.K) * 2 < ((int64_t)1 << 31) &&
                        ((int64_t)(a.K > 128 ? a.K : 128) * a.stride_bk + 256) * 2 < ((int64_t)1 << 31);
+  // Operands along K at any alignment and of any K from eight on: the same tiles, built to take them (LOAD_DMA_LOOSE; us a
+  // pass gathered / so: [1000,1500] x [1500,999] 18.3 / 17.0, [346,1849] x [1849,4544] 49 / 34, [2518,2911] x [2911,4744] 207 /
+  // 155; 50 random calls of a K that is no multiple of eight 1.11x, none slower).  Rows
+  // that overlap stay with the gathering tiles: past the edge, a chunk could straddle the end of the descriptor.
+  const bool loose_ok = !dma_ok && unit == 1 && a.stride_ak == 1 && a.stride_bk == 1 && a.K >= 8 && a.stride_am >= a.K &&
+                        a.stride_bn >= a.K && ((int64_t)256 * a.stride_am + a.K + 8) * 2 < ((int64_t)1 << 31) &&
+                        ((int64_t)256 * a.stride_bn + a.K + 8) * 2 < ((int64_t)1 << 31);
   auto gatherable = [&](bool along, bool across, int rows, int bk, int64_t ld_row, int64_t ld_k, int64_t extent) {
     const int64_t lim = (int64_t)1 << 30;  // 16-bit units
     return (along && ld_row >= 0 && rows * ld_row + a.K < lim) ||
@@ -1072,6 +1091,7 @@ hipError_t make_plan_body(const iris_gemm_args& a, Plan* plan, bool cells) {
              gatherable(b_along, b_across, e.cn, e.bk, a.stride_bn, a.stride_bk, a.N);
     if (!e.dma) return true;
     if (e.b_rows) return rows_ok;
+    if (e.loose) return loose_ok;
     if (!dma_ok) return false;
     const int64_t lim = (int64_t)1 << 31;
     return ((int64_t)e.cm * a.stride_am + a.K) * 2 < lim && ((int64_t)e.cn * a.stride_bn + a.K) * 2 < lim;
@@ -1095,15 +1115,17 @@ hipError_t make_plan_body(const iris_gemm_args& a, Plan* plan, bool cells) {
   if (!pick) {
     // first entry whose compute tile divides the logical tile; the rows and
     // columns a small matrix cannot fill are not worth a tall compute tile
-    int more = 0, rows = 0;
+    int more = 0, dma = 0;
     const GemmKernelEntry* more_list = more_entries_for(a.ab_dtype, op, &more);
-    const GemmKernelEntry* rows_list = rows_entries_for(a.ab_dtype, op, &rows);
-    for (int i = -rows; i < more + count && !pick; ++i) {
-      const GemmKernelEntry& e = i < 0 ? rows_list[i + rows] : i < more ? more_list[i] : list[i - more];
+    const GemmKernelEntry* dma_list = rows_ok    ? rows_entries_for(a.ab_dtype, op, &dma)
+                                      : loose_ok ? loose_entries_for(a.ab_dtype, op, &dma)
+                                                 : nullptr;
+    for (int i = -dma; i < more + count && !pick; ++i) {
+      const GemmKernelEntry& e = i < 0 ? dma_list[i + dma] : i < more ? more_list[i] : list[i - more];
       if (i < more && a.ab_dtype == IRIS_DTYPE_F32 && a.K < LONG_STEPS * e.bk) continue;
-      // (the gathering tiles are for what the DMA does not take, and for the reduce inside the program, of which there is
-      // no build for a row-major B)
-      if (!fits(e) || (e.gather && (dma_ok || (rows_ok && !plan->in_program)))) continue;
+      // (the gathering tiles are for what the DMA does not take, and for the reduce inside the program, of which there are
+      // builds for aligned operands along K only)
+      if (!fits(e) || (e.gather && (dma_ok || ((rows_ok || loose_ok) && !plan->in_program)))) continue;
       if (plan->in_program && !e.fn_fused) continue;
       // (a caller's split needs a K-step per part: a tile with a deeper step may not have them)
       if (a.split_k > 1 && a.split_k > (a.K + e.bk - 1) / e.bk && e.bk > 64) continue;

@@ -16,6 +16,7 @@ struct GemmKernelEntry {
   int bk, wm, wn, stages;  // (bk in 16-bit units: half as many elements of fp32 operands)
   bool dma;    // LDS-DMA loader (needs K-contiguous, 16-byte aligned operands)
   bool b_rows;  // ... of a B whose rows are its k (row-major [K, N], 16-byte aligned rows)
+  bool loose;   // ... of operands along K at any alignment and of any K from eight on
   bool gather;  // gathering loader (operands contiguous along K or across it, at any alignment); neither: generic
   bool splitk;  // the kernel can share a tile's K range with other programs
   bool split_owner;  // ... and its first part can add the others' partials itself (needed for stream-K runs)
@@ -45,7 +46,7 @@ constexpr GemmKernelFn fused_fn() {
   // (the DMA tiles with fetching waves have no such build: the reduce wants the registers their
   // fetch state takes, and the launcher takes the plain tile of the same shape instead; the gathering tiles, which
   // have no plain twin, have one where the accumulators leave room)
-  if constexpr ((OP == OP_STORE16 || OP == OP_STORE32) && !Cfg::B_ROWS && (Cfg::LW == 0 || (Cfg::GATHER && Cfg::IM * Cfg::IN * 4 <= 64)))
+  if constexpr ((OP == OP_STORE16 || OP == OP_STORE32) && !Cfg::B_ROWS && !Cfg::LOOSE && (Cfg::LW == 0 || (Cfg::GATHER && Cfg::IM * Cfg::IN * 4 <= 64)))
     return &gemm_persistent_kernel<Cfg, OP, ODT, false, true>;
   else
     return nullptr;
@@ -76,7 +77,7 @@ constexpr GemmKernelFn split_merged_fn() {
 
 // The eight-wave 256 x 256 tile's builds with the touches of Loader::touch (store epilogues).
 template <class Cfg>
-constexpr bool touch_build = Cfg::CM == 256 && Cfg::CN == 256 && Cfg::DMA && !Cfg::B_ROWS && Cfg::BK == 64 && Cfg::LW == 0 && Cfg::NW == 8 &&
+constexpr bool touch_build = Cfg::CM == 256 && Cfg::CN == 256 && Cfg::DMA && !Cfg::B_ROWS && !Cfg::LOOSE && Cfg::BK == 64 && Cfg::LW == 0 && Cfg::NW == 8 &&
                              Cfg::S == 2 && Cfg::WM == 2;
 template <int DT>
 using TouchCfg = GemmCfg<DT, 256, 256, 64, 2, 4, 2, true, 0, true>;
@@ -92,7 +93,7 @@ template <class Cfg, int OP>
 constexpr GemmKernelEntry make_entry(const char* name) {
   constexpr int ODT = (OP == OP_STORE32 || OP == OP_ATOMIC32) ? IRIS_DTYPE_F32 : Cfg::DT;
   return GemmKernelEntry{Cfg::DT, OP,      Cfg::CM, Cfg::CN, Cfg::BK,        Cfg::WM,
-                         Cfg::WN, Cfg::S,  Cfg::DMA, Cfg::B_ROWS, Cfg::GATHER, Cfg::SPLITK, Cfg::SPLIT_OWNER, Cfg::THREADS, Cfg::LW, Cfg::LDS_BYTES,
+                         Cfg::WN, Cfg::S,  Cfg::DMA, Cfg::B_ROWS, Cfg::LOOSE, Cfg::GATHER, Cfg::SPLITK, Cfg::SPLIT_OWNER, Cfg::THREADS, Cfg::LW, Cfg::LDS_BYTES,
                          &gemm_persistent_kernel<Cfg, OP, ODT, false>, split_fn<Cfg, OP, ODT>(), fused_fn<Cfg, OP, ODT>(),
                          merged_fn<Cfg, OP, ODT>(), split_merged_fn<Cfg, OP, ODT>(), touch_fn<Cfg, OP, ODT, false>(),
                          touch_fn<Cfg, OP, ODT, true>(), name};
@@ -140,20 +141,28 @@ constexpr GemmKernelEntry make_entry(const char* name) {
   X(DT, OP, 64, 128, 64, 2, 2, 2, LOAD_GATHER, 4, 1, "64x128x64_w2x2_gather")   \
   X(DT, OP, 64, 64, 128, 2, 2, 2, LOAD_GATHER, 4, 1, "64x64x128_w2x2_gather")
 
-// ... and, in a list of their own in front of those, the LDS-DMA tiles for a row-major B, the first for the store epilogues only (atomics take half
+// ... and, in a list of their own in front of those, the LDS-DMA tiles for a row-major B (LOAD_DMA_ROWS), the first for the store epilogues only (atomics take half
 // tiles).  The gathering tiles transpose such a B in the fetching waves' registers, and a K-step waits for them: a step of
 // 128 x 128 x 64 in 1.2 us.  Here the DMA brings the rows as they lie and the transposing LDS read costs what a plain one
 // does: 0.45 us, as for a B along K ([2697,1936] x [1936,1600], 275 tiles in two rounds, 66.8 -> 40.1 us a pass).
-#define IRIS_GEMM_ROWS_VARIANTS(X, DT, OP)                                         \
-  X(DT, OP, 256, 128, 64, 2, 2, 3, LOAD_DMA_ROWS, 4, 1, "256x128x64_w2x2_s3_f4_rows") \
-  X(DT, OP, 128, 128, 64, 2, 2, 4, LOAD_DMA_ROWS, 4, 1, "128x128x64_w2x2_s4_f4_rows") \
-  X(DT, OP, 256, 64, 64, 4, 1, 3, LOAD_DMA_ROWS, 4, 1, "256x64x64_w4x1_s3_f4_rows")   \
-  X(DT, OP, 128, 64, 64, 2, 2, 4, LOAD_DMA_ROWS, 4, 1, "128x64x64_w2x2_s4_f4_rows")   \
-  X(DT, OP, 64, 128, 64, 2, 2, 4, LOAD_DMA_ROWS, 4, 1, "64x128x64_w2x2_s4_f4_rows")   \
-  X(DT, OP, 64, 64, 128, 2, 2, 4, LOAD_DMA_ROWS, 4, 1, "64x64x128_w2x2_s4_f4_rows")
-#define IRIS_GEMM_ROWS_STORE_VARIANTS(X, DT, OP)                            \
-  X(DT, OP, 256, 256, 64, 2, 4, 2, LOAD_DMA_ROWS, 0, 1, "256x256x64_w2x4_s2_rows") \
-  IRIS_GEMM_ROWS_VARIANTS(X, DT, OP)
+// The same tiles (LOOSE) for operands along K that the plain ones do not take: rows at any alignment, a K that is no multiple
+// of eight.  The DMA brings 16 bytes from any address at little more than the aligned ones' cost; the gathering tiles, which
+// shift such rows in registers, are left for what lies across K ([4096,4096] x [4096,4096] on rows 8 bytes off, 256 x 256 tiles:
+// 144 us gathered, 116 so, 100 aligned).
+#define IRIS_GEMM_DMA_VARIANTS(X, DT, OP, LOAD, SUFFIX)                           \
+  X(DT, OP, 256, 128, 64, 2, 2, 3, LOAD, 4, 1, "256x128x64_w2x2_s3_f4" SUFFIX)    \
+  X(DT, OP, 128, 128, 64, 2, 2, 4, LOAD, 4, 1, "128x128x64_w2x2_s4_f4" SUFFIX)    \
+  X(DT, OP, 256, 64, 64, 4, 1, 3, LOAD, 4, 1, "256x64x64_w4x1_s3_f4" SUFFIX)      \
+  X(DT, OP, 128, 64, 64, 2, 2, 4, LOAD, 4, 1, "128x64x64_w2x2_s4_f4" SUFFIX)      \
+  X(DT, OP, 64, 128, 64, 2, 2, 4, LOAD, 4, 1, "64x128x64_w2x2_s4_f4" SUFFIX)      \
+  X(DT, OP, 64, 64, 128, 2, 2, 4, LOAD, 4, 1, "64x64x128_w2x2_s4_f4" SUFFIX)
+#define IRIS_GEMM_DMA_STORE_VARIANTS(X, DT, OP, LOAD, SUFFIX)                     \
+  X(DT, OP, 256, 256, 64, 2, 4, 2, LOAD, 0, 1, "256x256x64_w2x4_s2" SUFFIX)       \
+  IRIS_GEMM_DMA_VARIANTS(X, DT, OP, LOAD, SUFFIX)
+#define IRIS_GEMM_ROWS_VARIANTS(X, DT, OP) IRIS_GEMM_DMA_VARIANTS(X, DT, OP, LOAD_DMA_ROWS, "_rows")
+#define IRIS_GEMM_ROWS_STORE_VARIANTS(X, DT, OP) IRIS_GEMM_DMA_STORE_VARIANTS(X, DT, OP, LOAD_DMA_ROWS, "_rows")
+#define IRIS_GEMM_LOOSE_VARIANTS(X, DT, OP) IRIS_GEMM_DMA_VARIANTS(X, DT, OP, LOAD_DMA_LOOSE, "_gather_dma")
+#define IRIS_GEMM_LOOSE_STORE_VARIANTS(X, DT, OP) IRIS_GEMM_DMA_STORE_VARIANTS(X, DT, OP, LOAD_DMA_LOOSE, "_gather_dma")
 
 // extra variants, compiled for the bf16 store op only (tuning runs, and the
 // one-substep stage whose fragment buffers alternate from step to step)
@@ -210,19 +219,16 @@ constexpr GemmKernelEntry make_entry(const char* name) {
   template __global__ void gemm_persistent_kernel<TouchCfg<DT>, OP, IRIS_GEMM_ODT(DT, OP), false, false, true>(   \
       const GemmKArgs);
 
-#define IRIS_GEMM_INSTANTIATE_MERGED_ROWS(DT, OP)                                                                       \
-  template __global__ void gemm_persistent_kernel<GemmCfg<DT, 256, 256, 64, 2, 4, 2, LOAD_DMA_ROWS, 0>, OP,           \
-                                                  IRIS_GEMM_ODT(DT, OP), false, false, true>(const GemmKArgs);     \
-  template __global__ void gemm_persistent_kernel<GemmCfg<DT, 256, 128, 64, 2, 2, 3, LOAD_DMA_ROWS, 4>, OP,           \
-                                                  IRIS_GEMM_ODT(DT, OP), false, false, true>(const GemmKArgs);     \
-  template __global__ void gemm_persistent_kernel<GemmCfg<DT, 256, 256, 64, 2, 4, 2, LOAD_DMA_ROWS, 0>, OP,           \
-                                                  IRIS_GEMM_ODT(DT, OP), true, false, true>(const GemmKArgs);      \
-  template __global__ void gemm_persistent_kernel<GemmCfg<DT, 256, 128, 64, 2, 2, 3, LOAD_DMA_ROWS, 4>, OP,           \
-                                                  IRIS_GEMM_ODT(DT, OP), true, false, true>(const GemmKArgs);      \
-  template __global__ void gemm_persistent_kernel<GemmCfg<DT, 256, 64, 64, 4, 1, 3, LOAD_DMA_ROWS, 4>, OP,            \
-                                                  IRIS_GEMM_ODT(DT, OP), false, false, true>(const GemmKArgs);     \
-  template __global__ void gemm_persistent_kernel<GemmCfg<DT, 256, 64, 64, 4, 1, 3, LOAD_DMA_ROWS, 4>, OP,            \
-                                                  IRIS_GEMM_ODT(DT, OP), true, false, true>(const GemmKArgs);
+#define IRIS_GEMM_MERGED_KERNEL(DT, OP, CN, WM, WN, S, LOAD, LW, SPLIT)                                      \
+  template __global__ void gemm_persistent_kernel<GemmCfg<DT, 256, CN, 64, WM, WN, S, LOAD, LW>, OP,         \
+                                                  IRIS_GEMM_ODT(DT, OP), SPLIT, false, true>(const GemmKArgs);
+#define IRIS_GEMM_INSTANTIATE_MERGED_DMA(DT, OP, LOAD)           \
+  IRIS_GEMM_MERGED_KERNEL(DT, OP, 256, 2, 4, 2, LOAD, 0, false)  \
+  IRIS_GEMM_MERGED_KERNEL(DT, OP, 256, 2, 4, 2, LOAD, 0, true)   \
+  IRIS_GEMM_MERGED_KERNEL(DT, OP, 128, 2, 2, 3, LOAD, 4, false)  \
+  IRIS_GEMM_MERGED_KERNEL(DT, OP, 128, 2, 2, 3, LOAD, 4, true)   \
+  IRIS_GEMM_MERGED_KERNEL(DT, OP, 64, 4, 1, 3, LOAD, 4, false)   \
+  IRIS_GEMM_MERGED_KERNEL(DT, OP, 64, 4, 1, 3, LOAD, 4, true)
 
 // fp32 operands (fp32 output only): a short table.  The tiles are the 16-bit ones' (a stage of BK 16-bit units holds
 // BK / 2 elements of K; the names count elements); the matrix cores run fp32 at a sixteenth of the 16-bit rate, so any
@@ -233,7 +239,7 @@ constexpr GemmKernelEntry make_entry_f32(const char* name) {
   static_assert(Cfg::DT == IRIS_DTYPE_F32 && (OP == OP_STORE32 || OP == OP_ATOMIC32), "fp32 operands, fp32 output");
   GemmKernelFn split = nullptr;
   if constexpr (SPLIT) split = split_fn<Cfg, OP, IRIS_DTYPE_F32>();
-  return GemmKernelEntry{Cfg::DT, OP, Cfg::CM, Cfg::CN, Cfg::BK, Cfg::WM, Cfg::WN, Cfg::S, Cfg::DMA, Cfg::B_ROWS, Cfg::GATHER, SPLIT, SPLIT && Cfg::SPLIT_OWNER,
+  return GemmKernelEntry{Cfg::DT, OP, Cfg::CM, Cfg::CN, Cfg::BK, Cfg::WM, Cfg::WN, Cfg::S, Cfg::DMA, Cfg::B_ROWS, Cfg::LOOSE, Cfg::GATHER, SPLIT, SPLIT && Cfg::SPLIT_OWNER,
                          Cfg::THREADS, Cfg::LW, Cfg::LDS_BYTES, &gemm_persistent_kernel<Cfg, OP, IRIS_DTYPE_F32, false>,
                          split, fused_fn<Cfg, OP, IRIS_DTYPE_F32>(), nullptr, nullptr, nullptr, nullptr, name};
 }
@@ -276,6 +282,14 @@ IRIS_GEMM_DECLARE(f16_store16_rows)
 IRIS_GEMM_DECLARE(f16_store32_rows)
 IRIS_GEMM_DECLARE(f16_atomic32_rows)
 IRIS_GEMM_DECLARE(f16_atomic16_rows)
+IRIS_GEMM_DECLARE(bf16_store16_loose)
+IRIS_GEMM_DECLARE(bf16_store32_loose)
+IRIS_GEMM_DECLARE(bf16_atomic32_loose)
+IRIS_GEMM_DECLARE(bf16_atomic16_loose)
+IRIS_GEMM_DECLARE(f16_store16_loose)
+IRIS_GEMM_DECLARE(f16_store32_loose)
+IRIS_GEMM_DECLARE(f16_atomic32_loose)
+IRIS_GEMM_DECLARE(f16_atomic16_loose)
 IRIS_GEMM_DECLARE(bf16_store16_gather)
 IRIS_GEMM_DECLARE(bf16_store32_gather)
 IRIS_GEMM_DECLARE(bf16_atomic32_gather)
