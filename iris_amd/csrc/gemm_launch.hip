@@ -115,6 +115,7 @@ struct Plan {
   int fused_reduce = 0;  // ONE_SHOT, CONSUME on its own or IRIS_PHASE_TWO_KERNELS: follow with the reduce kernel
   int in_program = 0;    // ONE_SHOT, IRIS_PHASE_FUSED: the build of the kernel that reduces each tile itself
   int parts = 0;         // the launch's tiles are parts of the caller's (plan_parts)
+  int loose = 0;         // the few-rows kernel's build for operands at any alignment
   int two_kernels = 0;   // ... or, for such a launch too, producer and reduce as two kernels (reduce_in_program)
   // the few-rows kernel instead of a table entry: workgroups along the columns, the rows and K
   GemmKernelFn skinny = nullptr;
@@ -159,7 +160,8 @@ int few_rows_parts(int64_t cells, int64_t nb, double block_us, int64_t b_bytes) 
 // takes it when the operands allow the 16-byte fetches, the logical tile
 // covers every row (or whole workgroups of them) and the tiles' arrival counters have a home.  Fills the
 // plan and returns true when the launch qualifies.
-bool plan_few_rows(const iris_gemm_args& a, int op, bool dma_ok, Plan* plan) {
+// `loose`: the operands are not aligned, or K is no multiple of eight (dma_ok says that the kernel's build for those takes them).
+bool plan_few_rows(const iris_gemm_args& a, int op, bool dma_ok, bool loose, Plan* plan) {
   GemmKArgs& k = plan->k;
   const int64_t lim = (int64_t)1 << 31;
   // Up to 32 rows: a workgroup per 16 rows x 16 columns, unless B is more than the 16 MB that are as well read
@@ -208,8 +210,9 @@ bool plan_few_rows(const iris_gemm_args& a, int op, bool dma_ok, Plan* plan) {
     const int64_t elems = cells * rb * (SKINNY_ROWS * SKINNY_COLS);  // of one part's sums
     if (parts * elems > (int64_t)a.num_sms * a.partials_slot_elems) parts = 1;
   }
-  plan->skinny = gemm_skinny_kernel_for(a.ab_dtype, op, a.M <= 8 ? 8 : 16, rb);
+  plan->skinny = gemm_skinny_kernel_for(a.ab_dtype, op, a.M <= 8 ? 8 : 16, rb, 1, loose);
   if (!plan->skinny) return false;
+  plan->loose = loose;
   plan->skinny_lds = skinny_lds_bytes(rb);
   plan->skinny_grid = n_blocks;
   plan->skinny_grid_y = m_blocks;
@@ -228,7 +231,7 @@ bool plan_few_rows(const iris_gemm_args& a, int op, bool dma_ok, Plan* plan) {
 // or better: [728,3072] x [3072,448] 13.8 / 13.8, [1113,832] x [832,393] 8.9 / 10.3.  Only for a launch that owns the
 // device and says how many XCDs it has: the cells are dealt to them so that each fetches its own part of an operand.
 // Whether it is better than tiles at the launch's K is for plan_small to say.
-bool plan_cells(const iris_gemm_args& a, int op, bool dma_ok, Plan* plan) {
+bool plan_cells(const iris_gemm_args& a, int op, bool dma_ok, bool loose, Plan* plan) {
   GemmKArgs& k = plan->k;
   const int64_t lim = (int64_t)1 << 31, cus = current_cu_count();
   const int64_t m_cells = (a.M + CELL - 1) / CELL, n_cells = (a.N + CELL - 1) / CELL, cells = m_cells * n_cells;
@@ -242,7 +245,7 @@ bool plan_cells(const iris_gemm_args& a, int op, bool dma_ok, Plan* plan) {
     parts = few_rows_parts(cells, (a.K + 63) / 64, 0.6, (int64_t)a.N * a.K * 2);
     if (parts * cells * (CELL * CELL) > (int64_t)a.num_sms * a.partials_slot_elems) parts = 1;
   }
-  plan->skinny = gemm_skinny_kernel_for(a.ab_dtype, op, 16, 2, 2);
+  plan->skinny = gemm_skinny_kernel_for(a.ab_dtype, op, 16, 2, 2, loose);
   if (!plan->skinny) return false;
   k.cells = (int)cells;
   k.cells_by_row = a.M > a.N;
@@ -250,6 +253,7 @@ bool plan_cells(const iris_gemm_args& a, int op, bool dma_ok, Plan* plan) {
   k.xcd_per = (int)((cells + a.num_xcds - 1) / a.num_xcds);
   k.div_inner = make_fast_div((uint32_t)k.cells_inner, (uint64_t)cells + 1);
   k.div_xcd = make_fast_div((uint32_t)a.num_xcds, (uint64_t)k.xcd_per * a.num_xcds + 1);
+  plan->loose = loose;
   plan->skinny_lds = cells_lds_bytes();
   plan->skinny_grid = k.xcd_per * a.num_xcds;
   plan->skinny_grid_y = 1;
@@ -796,7 +800,8 @@ bool reduce_in_program(const iris_gemm_args& a, const Plan& producer) {
   const int64_t tiles = ((int64_t)a.M + a.block_m - 1) / a.block_m * (((int64_t)a.N + a.block_n - 1) / a.block_n);
   const int64_t inside = (int64_t)(a.block_m < a.M ? a.block_m : a.M) * (a.block_n < a.N ? a.block_n : a.N);
   const int64_t strips = inside * a.world_size * dtype_size(a.c_dtype);  // bytes that a program's tile is reduced from
-  if (tiles <= a.num_sms && k.vec_out && (producer.skinny || (producer.entry->dma && !producer.entry->b_rows && !producer.entry->loose))) {
+  // (inside, operands at any alignment are gathered)
+  if (tiles <= a.num_sms && k.vec_out && !producer.loose && (producer.skinny || (producer.entry->dma && !producer.entry->b_rows && !producer.entry->loose))) {
     const bool few = producer.skinny && producer.skinny_cb == 1;
     if (inside <= 64 * 64 && (few ? steps <= 2 && a.block_n <= 64 : steps <= 10)) return true;
     if (!few && tiles >= 16 && a.block_n <= 64 && steps <= 5 && (inside <= 128 * 64 || strips <= (128 << 10))) return true;
@@ -1077,7 +1082,7 @@ hipError_t make_plan_body(const iris_gemm_args& a, Plan* plan, bool cells) {
   // pass gathered / so: [1000,1500] x [1500,999] 18.3 / 17.0, [346,1849] x [1849,4544] 49 / 34, [2518,2911] x [2911,4744] 207 /
   // 155; 50 random calls of a K that is no multiple of eight 1.11x, none slower).  Rows
   // that overlap stay with the gathering tiles: past the edge, a chunk could straddle the end of the descriptor.
-  const bool loose_ok = !dma_ok && unit == 1 && a.stride_ak == 1 && a.stride_bk == 1 && a.K >= 8 && a.stride_am >= a.K &&
+  const bool loose_ok = !dma_ok && a.stride_ak == unit && a.stride_bk == unit && a.K >= 8 && a.stride_am >= a.K &&
                         a.stride_bn >= a.K && ((int64_t)256 * a.stride_am + a.K + 8) * 2 < ((int64_t)1 << 31) &&
                         ((int64_t)256 * a.stride_bn + a.K + 8) * 2 < ((int64_t)1 << 31);
   auto gatherable = [&](bool along, bool across, int rows, int bk, int64_t ld_row, int64_t ld_k, int64_t extent) {
@@ -1098,8 +1103,10 @@ hipError_t make_plan_body(const iris_gemm_args& a, Plan* plan, bool cells) {
   };
 
   if (a.variant == 0 || a.variant == IRIS_GEMM_VARIANT_FEW_ROWS) {
-    if (plan_few_rows(a, op, dma_ok, plan)) return hipSuccess;
-    if (cells && plan_cells(a, op, dma_ok, plan)) return hipSuccess;
+    // (insisted on, it is for aligned operands)
+    const bool any_ok = dma_ok || (loose_ok && a.variant == 0);
+    if (plan_few_rows(a, op, any_ok, !dma_ok, plan)) return hipSuccess;
+    if (cells && plan_cells(a, op, any_ok, !dma_ok, plan)) return hipSuccess;
     if (a.variant == IRIS_GEMM_VARIANT_FEW_ROWS) return hipErrorInvalidValue;
   }
 
@@ -1125,7 +1132,7 @@ hipError_t make_plan_body(const iris_gemm_args& a, Plan* plan, bool cells) {
       if (i < more && a.ab_dtype == IRIS_DTYPE_F32 && a.K < LONG_STEPS * e.bk) continue;
       // (the gathering tiles are for what the DMA does not take, and for the reduce inside the program, of which there are
       // builds for aligned operands along K only)
-      if (!fits(e) || (e.gather && (dma_ok || ((rows_ok || loose_ok) && !plan->in_program)))) continue;
+      if (!fits(e) || (e.gather && (dma_ok || (dma > 0 && !plan->in_program)))) continue;
       if (plan->in_program && !e.fn_fused) continue;
       // (a caller's split needs a K-step per part: a tile with a deeper step may not have them)
       if (a.split_k > 1 && a.split_k > (a.K + e.bk - 1) / e.bk && e.bk > 64) continue;
@@ -1458,7 +1465,7 @@ extern "C" int iris_gemm_plan_name(const iris_gemm_args* args, char* buf, size_t
   hipError_t err = make_plan(*args, &plan);
   if (err != hipSuccess) return err;
   const char* few = plan.skinny_cb == 2 ? "cells_32x32" : plan.skinny_rb == 2 ? "few_rows_32xN" : "few_rows_16xN";
-  std::snprintf(buf, len, "%s%s%s", plan.skinny ? few : plan.entry ? plan.entry->name : "",
+  std::snprintf(buf, len, "%s%s%s%s", plan.skinny ? few : plan.entry ? plan.entry->name : "", plan.loose ? "_gather_dma" : "",
                 plan.entry && plan.k.stream_k                   ? "+stream_k"
                 : plan.entry && plan.in_program                 ? "+reduce"
                 : plan.entry && plan.k.num_sms > args->num_sms ? "+two_per_cu"

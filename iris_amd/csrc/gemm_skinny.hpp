@@ -79,7 +79,11 @@ constexpr int cells_lds_bytes() { return SKINNY_WAVES * SKINNY_UN * 4 * SKINNY_B
 // RB: blocks of 16 rows a workgroup computes (1 for up to 32 rows; 2 up to 64
 // rows of a long K, and from 17 rows on where B is large).
 // CB: blocks of 16 columns, 1 or (with RB 2) 2.
-template <int DT, int OP, int ODT, int AROWS, int RB = 1, int CB = 1>
+// LOOSE: operands along K at any alignment and of any K from eight on (see Loader in gemm_kernel.hpp): a chunk that K cuts is
+// fetched moved back to end there, and what it repeats is cleared in the fragments.  (us a pass, by the gathering tiles / so:
+// [1,8229] x [8229,3816] 29.0 / 15.5, [15,2293] x [2293,1344] 17.0 / 9.8, [2,29690] x [29690,336] 22.3 / 11.8, [25,137] x
+// [137,4864] and its reduce 17.2 / 16.8; 40 random calls of up to 32 rows 1.48x.)
+template <int DT, int OP, int ODT, int AROWS, int RB = 1, int CB = 1, bool LOOSE = false>
 __global__ __launch_bounds__(SKINNY_THREADS) __attribute__((amdgpu_waves_per_eu(2, 8))) void
 gemm_skinny_kernel(const GemmKArgs p) {
   constexpr bool ATOMIC = OP == OP_ATOMIC32 || OP == OP_ATOMIC16;
@@ -118,12 +122,13 @@ gemm_skinny_kernel(const GemmKArgs p) {
 
   // Rows past the edge of either operand lie past the end of its buffer
   // descriptor and read as zero; chunks past K are parked out of range.
+  constexpr int LEAD = LOOSE ? 16 : 0;  // (no offset of a chunk moved back is below zero)
   const int rows_b = min(SKINNY_COLS * CB, p.N - n0);
   const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)(p.b + (int64_t)n0 * p.sbn * 2), 0, (int)((((int64_t)rows_b - 1) * p.sbn + p.K) * 2), 0x00020000);
+      (void*)(p.b + (int64_t)n0 * p.sbn * 2 - LEAD), 0, (int)((((int64_t)rows_b - 1) * p.sbn + p.K) * 2) + LEAD, 0x00020000);
   const int rows_a = min(SKINNY_ROWS * RB, p.M - m0);
   const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)(p.a + (int64_t)m0 * p.sam * 2), 0, (int)((((int64_t)rows_a - 1) * p.sam + p.K) * 2), 0x00020000);
+      (void*)(p.a + (int64_t)m0 * p.sam * 2 - LEAD), 0, (int)((((int64_t)rows_a - 1) * p.sam + p.K) * 2) + LEAD, 0x00020000);
   // B: lane l of fetch j of a block brings row 8j + l/8 and lands at byte
   // l*16 of the fetch's 1 KiB, i.e. at physical chunk l%8 of that row; the
   // chunk of the row it must bring there is (l%8) ^ (row/2 % 8).
@@ -153,13 +158,17 @@ gemm_skinny_kernel(const GemmKArgs p) {
   for (int i = 0; i < NB; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   u32x4 va[A_DMA ? 1 : UN][RB][AH];
+  // bytes by which chunk ch of K block kb is moved back
+  auto back = [&](int kb, int ch) __attribute__((always_inline)) -> uint32_t {
+    return LOOSE ? (uint32_t)max(0, kb * 64 + ch * 8 + 8 - p.K) * 2 : 0u;
+  };
   // fetches of K block kb into set u (blocks past the end are parked: the number of loads never changes)
   auto fetch = [&](int u, int kb) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < 2 * CB; ++j) {
       const int ch = bchunk ^ ((j & 1) << 2);
       const bool ok = kb < nb && kb * 64 + ch * 8 < p.K;
-      const uint32_t off = (uint32_t)(((int64_t)b_column(j) * p.sbn) * 2 + kb * 128 + ch * 16);
+      const uint32_t off = (uint32_t)(((int64_t)b_column(j) * p.sbn) * 2 + kb * 128 + ch * 16) + LEAD - back(kb, ch);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (IRIS_LDS void*)(wb + u * (CB * SKINNY_BLOCK_BYTES) + j * 1024), 16,
                                                ok ? (int)off : (int)0x80000000, 0, 0, 0);
     }
@@ -169,7 +178,7 @@ gemm_skinny_kernel(const GemmKArgs p) {
       for (int j = 0; j < AH; ++j) {
         const int ch = bchunk ^ (j << 2);
         const bool ok = kb < nb && kb * 64 + ch * 8 < p.K;
-        const uint32_t off = (uint32_t)(((int64_t)(i * 16 + brow + 8 * j) * p.sam) * 2 + kb * 128 + ch * 16);
+        const uint32_t off = (uint32_t)(((int64_t)(i * 16 + brow + 8 * j) * p.sam) * 2 + kb * 128 + ch * 16) + LEAD - back(kb, ch);
         if constexpr (A_DMA)
           __builtin_amdgcn_raw_ptr_buffer_load_lds(
               ra, (IRIS_LDS void*)(wa + (u * RB + i) * SKINNY_BLOCK_BYTES + j * 1024), 16, ok ? (int)off : (int)0x80000000, 0, 0, 0);
@@ -177,7 +186,7 @@ gemm_skinny_kernel(const GemmKArgs p) {
           va[u][i][j] = __builtin_amdgcn_raw_buffer_load_b128(ra, ok ? (int)off : (int)0x80000000, 0, 0);
       }
   };
-  auto multiply = [&](int u) __attribute__((always_inline)) {
+  auto multiply = [&](int u, int kb) __attribute__((always_inline)) {
     // (the wave's LDS operations execute in order: these writes land after
     // the previous block's reads and before this block's)
     if constexpr (!A_DMA) {
@@ -195,9 +204,15 @@ gemm_skinny_kernel(const GemmKArgs p) {
 #pragma unroll
       for (int j = 0; j < CB; ++j)
         fb[j] = *reinterpret_cast<const IRIS_LDS vec8*>(wb + (u * CB + j) * SKINNY_BLOCK_BYTES + lr * 128 + pc * 16);
+      const bool cut = LOOSE && (p.K & 7) != 0 && kb == nb_all - 1;
+      const int front = lq * 2 + h == (p.K & 63) / 8 ? 8 - (p.K & 7) : 0;
+      if (cut)
+#pragma unroll
+        for (int j = 0; j < CB; ++j) mask_tail<DT>(fb[j], front);
 #pragma unroll
       for (int i = 0; i < RB; ++i) {
-        const vec8 fa = *reinterpret_cast<const IRIS_LDS vec8*>(sa + i * SKINNY_BLOCK_BYTES + lr * 128 + pc * 16);
+        vec8 fa = *reinterpret_cast<const IRIS_LDS vec8*>(sa + i * SKINNY_BLOCK_BYTES + lr * 128 + pc * 16);
+        if (cut) mask_tail<DT>(fa, front);
 #pragma unroll
         for (int j = 0; j < CB; ++j) acc[i * CB + j] = Mfma<DT>::run(fb[j], fa, acc[i * CB + j]);
       }
@@ -220,7 +235,7 @@ gemm_skinny_kernel(const GemmKArgs p) {
     for (int u = 0; u < UN; ++u) {
       IRIS_WAIT_VMCNT(LOADS * (UN - 1));
       asm volatile("" ::: "memory");
-      multiply(u);
+      multiply(u, b0 + SKINNY_WAVES * u);
       IRIS_WAIT_LGKMCNT0();  // the reads have returned before the next fetch overwrites the region
       asm volatile("" ::: "memory");
       fetch(u, b0 + SKINNY_WAVES * (UN + u));
@@ -230,7 +245,7 @@ gemm_skinny_kernel(const GemmKArgs p) {
   IRIS_WAIT_VMCNT(0);
   asm volatile("" ::: "memory");
 #pragma unroll
-  for (int u = 0; u < UN; ++u) multiply(u);
+  for (int u = 0; u < UN; ++u) multiply(u, b0 + SKINNY_WAVES * u);
   IRIS_WAIT_LGKMCNT0();
   asm volatile("" ::: "memory");
 
@@ -425,6 +440,7 @@ gemm_skinny_kernel(const GemmKArgs p) {
 }
 
 // The kernel for (operand type, store op, rows of A in a block, blocks of rows and of columns a workgroup), or null.
-GemmKernelFn gemm_skinny_kernel_for(int dt, int op, int arows, int rb, int cb = 1);
+// `loose`: for operands at any alignment.
+GemmKernelFn gemm_skinny_kernel_for(int dt, int op, int arows, int rb, int cb, bool loose);
 
 }  // namespace iris_amd

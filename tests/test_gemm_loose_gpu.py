@@ -163,3 +163,55 @@ def test_what_stays_as_it_was(shmem, M, N, K, lda, dtype):
     ops.gemm_launch(*args)
     torch.cuda.synchronize()
     check_close(cg, O.shard_gemm(A, B, dtype), "as it was")
+
+
+@pytest.mark.parametrize("M,N,K,BM,BN,pad,shift,kernel", [
+    (1, 300, 4099, 64, 64, 0, 0, "few_rows_16xN"),     # one k in the last chunk
+    (3, 50, 9, 64, 64, 0, 1, "few_rows_16xN"),         # two chunks, N no multiple of a workgroup's columns
+    (8, 72, 8, 64, 64, 1, 0, "few_rows_16xN"),         # one whole chunk off the 16 bytes
+    (9, 200, 1407, 64, 64, 3, 5, "few_rows_16xN"),
+    (17, 130, 2111, 64, 64, 0, 0, "few_rows_16xN"),
+    (30, 201, 63, 64, 128, 0, 0, "few_rows_16xN"),     # one block of K, cut in its last chunk
+    (20, 4200, 2050, 64, 64, 0, 0, "few_rows_32xN"),   # blocks of 32 rows
+    (50, 272, 3001, 64, 64, 1, 0, "few_rows_32xN"),
+    (4, 192, 8197, 64, 64, 0, 0, "few_rows_16xN"),     # K shared out over workgroups
+    (130, 330, 1021, 64, 64, 0, 3, "cells_32x32"),
+    (200, 500, 515, 128, 64, 0, 0, "cells_32x32"),
+])
+@pytest.mark.parametrize("dtype,out", [(BF16, BF16), (F16, F32)])
+def test_few_rows_and_cells(shmem, M, N, K, BM, BN, pad, shift, kernel, dtype, out):
+    A, B, a, b = operands(shmem, M, N, K, dtype, pad, shift)
+    cg = shmem.full((M, N), 7, dtype=out)
+    total = ops.cdiv(M, BM) * ops.cdiv(N, BN)
+    flags = shmem.zeros((total + 1,), dtype=torch.int32)
+    P = shmem.zeros((256, BM * BN), dtype=F32)
+    locks = shmem.zeros((256,), dtype=torch.int32)
+    args = (a, b, None, cg, flags, None, 0, 1, 256, BM, BN, 64, 2, ops.EPI_ALL_SCATTER)
+    kw = dict(partials=P, locks=locks, num_xcds=8)
+    assert ops.gemm_plan_name(*args, **kw) == kernel + "_gather_dma"
+    for launch in (1, 2):
+        ops.gemm_launch(*args, **kw)
+        torch.cuda.synchronize()
+        check_close(cg, O.shard_gemm(A, B, out), f"launch {launch}")
+        assert flags.cpu().tolist() == [launch] * total + [0] and not locks.any()
+
+
+@pytest.mark.parametrize("M,N,K", [(5, 70, 1031), (70, 130, 517)])
+def test_fp32_few_rows(shmem, M, N, K):
+    A, B, a, b = operands(shmem, M, N, K, F32, 1, 1)
+    cg = shmem.zeros((M, N), dtype=F32)
+    flags = shmem.zeros((16,), dtype=torch.int32)
+    locks = shmem.zeros((256,), dtype=torch.int32)
+    args = (a, b, None, cg, flags, None, 0, 1, 256, 64, 64, 64, 2, ops.EPI_ALL_SCATTER)
+    ops.gemm_launch(*args, locks=locks, num_xcds=8)
+    torch.cuda.synchronize()
+    check_close(cg, O.shard_gemm(A, B, F32), "fp32", block_rtol=1e-5)
+
+
+def test_the_few_rows_kernel_is_not_to_be_had_for_them_by_name(shmem):
+    A, B, a, b = operands(shmem, 4, 64, 131, BF16, 0, 0)
+    cg = shmem.zeros((4, 64), dtype=BF16)
+    flags = shmem.zeros((1,), dtype=torch.int32)
+    with pytest.raises(ValueError):
+        ops.gemm_plan_name(a, b, None, cg, flags, None, 0, 1, 256, 64, 64, 64, 2, ops.EPI_ALL_SCATTER,
+                           variant=ops.VARIANT_FEW_ROWS)
