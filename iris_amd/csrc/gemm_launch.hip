@@ -116,6 +116,7 @@ struct Plan {
   int in_program = 0;    // ONE_SHOT, IRIS_PHASE_FUSED: the build of the kernel that reduces each tile itself
   int parts = 0;         // the launch's tiles are parts of the caller's (plan_parts)
   int loose = 0;         // the few-rows kernel's build for operands at any alignment
+  int b_rows = 0;        // ... for a row-major B (cells)
   int two_kernels = 0;   // ... or, for such a launch too, producer and reduce as two kernels (reduce_in_program)
   // the few-rows kernel instead of a table entry: workgroups along the columns, the rows and K
   GemmKernelFn skinny = nullptr;
@@ -231,7 +232,10 @@ bool plan_few_rows(const iris_gemm_args& a, int op, bool dma_ok, bool loose, Pla
 // or better: [728,3072] x [3072,448] 13.8 / 13.8, [1113,832] x [832,393] 8.9 / 10.3.  Only for a launch that owns the
 // device and says how many XCDs it has: the cells are dealt to them so that each fetches its own part of an operand.
 // Whether it is better than tiles at the launch's K is for plan_small to say.
-bool plan_cells(const iris_gemm_args& a, int op, bool dma_ok, bool loose, Plan* plan) {
+// `b_rows`: a row-major B, up to 32 rows of A too, which the few-rows kernel does not take with it (us a pass, operands changed
+// from call to call, tiles / cells: [1,4096] x [4096,1376] 14.4 / 9.4, [4,1376] x [1376,4096] 12.3 / 8.2, [95,4224] x [4224,1280]
+// 14.2 / 11.0, [251,1344] x [1344,384] 10.6 / 7.9; 90 random calls 1.27x).
+bool plan_cells(const iris_gemm_args& a, int op, bool dma_ok, bool loose, bool b_rows, Plan* plan) {
   GemmKArgs& k = plan->k;
   const int64_t lim = (int64_t)1 << 31, cus = current_cu_count();
   const int64_t m_cells = (a.M + CELL - 1) / CELL, n_cells = (a.N + CELL - 1) / CELL, cells = m_cells * n_cells;
@@ -241,11 +245,12 @@ bool plan_cells(const iris_gemm_args& a, int op, bool dma_ok, bool loose, Plan* 
                   counters && (CELL * a.stride_am + a.K) * 2 < lim && (CELL * a.stride_bn + a.K) * 2 < lim;
   if (!ok) return false;
   int parts = 1;
-  if (a.split_k == 0 && a.partials && aligned16(a.partials) && a.locks && k.total_tiles + cells <= a.num_sms) {
-    parts = few_rows_parts(cells, (a.K + 63) / 64, 0.6, (int64_t)a.N * a.K * 2);
+  // (K of a row-major B is shared out for one row of cells only: [138,32000] x [32000,128] in twelve parts 24.4 us, 18.0 in tiles)
+  if (a.split_k == 0 && a.partials && aligned16(a.partials) && a.locks && k.total_tiles + cells <= a.num_sms && (!b_rows || m_cells == 1)) {
+    parts = few_rows_parts(cells, (a.K + 63) / 64, b_rows ? 0.9 : 0.6, (int64_t)a.N * a.K * 2);
     if (parts * cells * (CELL * CELL) > (int64_t)a.num_sms * a.partials_slot_elems) parts = 1;
   }
-  plan->skinny = gemm_skinny_kernel_for(a.ab_dtype, op, 16, 2, 2, loose);
+  plan->skinny = gemm_skinny_kernel_for(a.ab_dtype, op, 16, 2, 2, loose, b_rows);
   if (!plan->skinny) return false;
   k.cells = (int)cells;
   k.cells_by_row = a.M > a.N;
@@ -254,6 +259,7 @@ bool plan_cells(const iris_gemm_args& a, int op, bool dma_ok, bool loose, Plan* 
   k.div_inner = make_fast_div((uint32_t)k.cells_inner, (uint64_t)cells + 1);
   k.div_xcd = make_fast_div((uint32_t)a.num_xcds, (uint64_t)k.xcd_per * a.num_xcds + 1);
   plan->loose = loose;
+  plan->b_rows = b_rows;
   plan->skinny_lds = cells_lds_bytes();
   plan->skinny_grid = k.xcd_per * a.num_xcds;
   plan->skinny_grid_y = 1;
@@ -601,7 +607,7 @@ struct TileLaunch {
   bool sliced, parts;
 };
 struct Operands {
-  bool f32, lines, gather, atomic, vec_out;
+  bool f32, lines, gather, b_rows, atomic, vec_out;
   int copies;     // of the output
   bool peers;     // other ranks wait for it
   int64_t tile;   // elements of a caller's tile that lie in the output
@@ -648,12 +654,13 @@ double cells_us(const iris_gemm_args& a, int64_t cells, int parts, const Operand
   const double mb = ((double)a.M + a.N) * a.K * 2e-6;
   // us for 64 of K, operands in whole lines / not: [512,512] 256 cells 0.090 / 0.13; [128,1376] 172 cells 0.083 / 0.11;
   // [200,512] 112 cells 0.048 / 0.066 as long as the L2s hold the operands, 0.07 / 0.08 beyond
-  const double lines = o.lines ? 1.0 : 1.45;
+  // (a row-major B comes in half lines, from HBM at half the rate: [28,7936] x [7936,4864] 33.8, in tiles 23.5)
+  const double lines = o.b_rows ? 1.8 : o.lines ? 1.0 : 1.45;
   const double step = 0.083 * (groups * 5 > cus * 4 ? 1.09 : groups * 2 <= cus && mb <= 30 ? 0.7 : 1.0) *
                       (o.f32 && lines < 1.65 ? 1.65 : lines);
   // (a workgroup's first sixteen blocks of K are in flight together)
   const double loop = ((groups + cus - 1) / cus * ((nk + parts - 1) / parts) - 16) * step;
-  const double stream = mb / (mb > 200 ? 4.4 : 8.4) - 3, k_time = loop > stream ? loop : stream;
+  const double stream = mb / (o.b_rows ? 3.2 : mb > 200 ? 4.4 : 8.4) - 3, k_time = loop > stream ? loop : stream;
   const double per_tile = o.atomic ? 0.0 : (double)o.tile / (CELL * CELL) / 64;
   return 5.85 + (0.0075 + 0.004 * (per_tile < 1 ? per_tile : 1.0)) * groups + 0.025 * (o.copies - 1) + (parts > 1 ? 0.7 : 0.0) +
          (o.atomic ? 0.4 : 0.0) + (k_time > 0 ? k_time : 0.0);
@@ -710,7 +717,7 @@ bool plan_small(const iris_gemm_args& a, Plan* plan) {
   }
   if (!whole.entry) return false;
   const GemmKArgs& w = whole.k;
-  const Operands o{a.ab_dtype == IRIS_DTYPE_F32, whole_lines(a), !whole.entry->dma,
+  const Operands o{a.ab_dtype == IRIS_DTYPE_F32, whole_lines(a), !whole.entry->dma, whole.entry->b_rows,
                    a.epilogue == IRIS_EPI_ATOMIC_ADD, w.vec_out != 0, w.dest_all ? a.world_size : 1, a.world_size > 1,
                    (int64_t)(a.block_m < a.M ? a.block_m : a.M) * (a.block_n < a.N ? a.block_n : a.N)};
   double least = tiles_us(a, TileLaunch{whole.entry->cm, whole.entry->cn, w.total_tiles, w.sub_m * w.sub_n, w.split_k,
@@ -800,8 +807,8 @@ bool reduce_in_program(const iris_gemm_args& a, const Plan& producer) {
   const int64_t tiles = ((int64_t)a.M + a.block_m - 1) / a.block_m * (((int64_t)a.N + a.block_n - 1) / a.block_n);
   const int64_t inside = (int64_t)(a.block_m < a.M ? a.block_m : a.M) * (a.block_n < a.N ? a.block_n : a.N);
   const int64_t strips = inside * a.world_size * dtype_size(a.c_dtype);  // bytes that a program's tile is reduced from
-  // (inside, operands at any alignment are gathered)
-  if (tiles <= a.num_sms && k.vec_out && !producer.loose && (producer.skinny || (producer.entry->dma && !producer.entry->b_rows && !producer.entry->loose))) {
+  // (inside, operands at any alignment and a row-major B are gathered)
+  if (tiles <= a.num_sms && k.vec_out && !producer.loose && !producer.b_rows && (producer.skinny || (producer.entry->dma && !producer.entry->b_rows && !producer.entry->loose))) {
     const bool few = producer.skinny && producer.skinny_cb == 1;
     if (inside <= 64 * 64 && (few ? steps <= 2 && a.block_n <= 64 : steps <= 10)) return true;
     if (!few && tiles >= 16 && a.block_n <= 64 && steps <= 5 && (inside <= 128 * 64 || strips <= (128 << 10))) return true;
@@ -1106,7 +1113,7 @@ hipError_t make_plan_body(const iris_gemm_args& a, Plan* plan, bool cells) {
     // (insisted on, it is for aligned operands)
     const bool any_ok = dma_ok || (loose_ok && a.variant == 0);
     if (plan_few_rows(a, op, any_ok, !dma_ok, plan)) return hipSuccess;
-    if (cells && plan_cells(a, op, any_ok, !dma_ok, plan)) return hipSuccess;
+    if (cells && plan_cells(a, op, any_ok || (rows_ok && a.variant == 0), !dma_ok && !rows_ok, rows_ok, plan)) return hipSuccess;
     if (a.variant == IRIS_GEMM_VARIANT_FEW_ROWS) return hipErrorInvalidValue;
   }
 
@@ -1465,7 +1472,7 @@ extern "C" int iris_gemm_plan_name(const iris_gemm_args* args, char* buf, size_t
   hipError_t err = make_plan(*args, &plan);
   if (err != hipSuccess) return err;
   const char* few = plan.skinny_cb == 2 ? "cells_32x32" : plan.skinny_rb == 2 ? "few_rows_32xN" : "few_rows_16xN";
-  std::snprintf(buf, len, "%s%s%s%s", plan.skinny ? few : plan.entry ? plan.entry->name : "", plan.loose ? "_gather_dma" : "",
+  std::snprintf(buf, len, "%s%s%s%s", plan.skinny ? few : plan.entry ? plan.entry->name : "", plan.loose ? "_gather_dma" : plan.b_rows ? "_rows" : "",
                 plan.entry && plan.k.stream_k                   ? "+stream_k"
                 : plan.entry && plan.in_program                 ? "+reduce"
                 : plan.entry && plan.k.num_sms > args->num_sms ? "+two_per_cu"

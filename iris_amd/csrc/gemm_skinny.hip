@@ -14,26 +14,32 @@ GemmKernelFn pick(int arows, int rb, int cb) {
 }
 
 template <int DT, int OP>
-GemmKernelFn pick(int arows, int rb, int cb, bool loose) {
+GemmKernelFn pick(int arows, int rb, int cb, bool loose, bool b_rows) {
+  if (b_rows) {
+    if constexpr (DT == IRIS_DTYPE_F32)
+      return nullptr;
+    else
+      return cb == 2 ? &gemm_skinny_kernel<DT, OP, (OP == OP_STORE32 || OP == OP_ATOMIC32) ? IRIS_DTYPE_F32 : DT, 16, 2, 2, false, true> : nullptr;
+  }
   return loose ? pick<DT, OP, true>(arows, rb, cb) : pick<DT, OP, false>(arows, rb, cb);
 }
 
 }  // namespace
 
-GemmKernelFn gemm_skinny_kernel_for(int dt, int op, int arows, int rb, int cb, bool loose) {
+GemmKernelFn gemm_skinny_kernel_for(int dt, int op, int arows, int rb, int cb, bool loose, bool b_rows) {
   if (dt == IRIS_DTYPE_BF16) {
-    if (op == OP_STORE16) return pick<IRIS_DTYPE_BF16, OP_STORE16>(arows, rb, cb, loose);
-    if (op == OP_STORE32) return pick<IRIS_DTYPE_BF16, OP_STORE32>(arows, rb, cb, loose);
-    if (op == OP_ATOMIC32) return pick<IRIS_DTYPE_BF16, OP_ATOMIC32>(arows, rb, cb, loose);
-    if (op == OP_ATOMIC16) return pick<IRIS_DTYPE_BF16, OP_ATOMIC16>(arows, rb, cb, loose);
+    if (op == OP_STORE16) return pick<IRIS_DTYPE_BF16, OP_STORE16>(arows, rb, cb, loose, b_rows);
+    if (op == OP_STORE32) return pick<IRIS_DTYPE_BF16, OP_STORE32>(arows, rb, cb, loose, b_rows);
+    if (op == OP_ATOMIC32) return pick<IRIS_DTYPE_BF16, OP_ATOMIC32>(arows, rb, cb, loose, b_rows);
+    if (op == OP_ATOMIC16) return pick<IRIS_DTYPE_BF16, OP_ATOMIC16>(arows, rb, cb, loose, b_rows);
   } else if (dt == IRIS_DTYPE_F16) {
-    if (op == OP_STORE16) return pick<IRIS_DTYPE_F16, OP_STORE16>(arows, rb, cb, loose);
-    if (op == OP_STORE32) return pick<IRIS_DTYPE_F16, OP_STORE32>(arows, rb, cb, loose);
-    if (op == OP_ATOMIC32) return pick<IRIS_DTYPE_F16, OP_ATOMIC32>(arows, rb, cb, loose);
-    if (op == OP_ATOMIC16) return pick<IRIS_DTYPE_F16, OP_ATOMIC16>(arows, rb, cb, loose);
+    if (op == OP_STORE16) return pick<IRIS_DTYPE_F16, OP_STORE16>(arows, rb, cb, loose, b_rows);
+    if (op == OP_STORE32) return pick<IRIS_DTYPE_F16, OP_STORE32>(arows, rb, cb, loose, b_rows);
+    if (op == OP_ATOMIC32) return pick<IRIS_DTYPE_F16, OP_ATOMIC32>(arows, rb, cb, loose, b_rows);
+    if (op == OP_ATOMIC16) return pick<IRIS_DTYPE_F16, OP_ATOMIC16>(arows, rb, cb, loose, b_rows);
   } else if (dt == IRIS_DTYPE_F32) {
-    if (op == OP_STORE32) return pick<IRIS_DTYPE_F32, OP_STORE32>(arows, rb, cb, loose);
-    if (op == OP_ATOMIC32) return pick<IRIS_DTYPE_F32, OP_ATOMIC32>(arows, rb, cb, loose);
+    if (op == OP_STORE32) return pick<IRIS_DTYPE_F32, OP_STORE32>(arows, rb, cb, loose, b_rows);
+    if (op == OP_ATOMIC32) return pick<IRIS_DTYPE_F32, OP_ATOMIC32>(arows, rb, cb, loose, b_rows);
   }
   return nullptr;
 }

@@ -83,7 +83,10 @@ constexpr int cells_lds_bytes() { return SKINNY_WAVES * SKINNY_UN * 4 * SKINNY_B
 // fetched moved back to end there, and what it repeats is cleared in the fragments.  (us a pass, by the gathering tiles / so:
 // [1,8229] x [8229,3816] 29.0 / 15.5, [15,2293] x [2293,1344] 17.0 / 9.8, [2,29690] x [29690,336] 22.3 / 11.8, [25,137] x
 // [137,4864] and its reduce 17.2 / 16.8; 40 random calls of up to 32 rows 1.48x.)
-template <int DT, int OP, int ODT, int AROWS, int RB = 1, int CB = 1, bool LOOSE = false>
+// BROWS (cells, 16-bit operands): a B whose rows are its k (row-major [K, N]), in whole aligned 16-byte chunks.  A block of B lies
+// in LDS as in memory, 64 k of 32 columns, and is transposed on its way to the MFMAs by ds_read_b64_tr_b16.  A row of 64
+// bytes is half a cache line, so that such a block costs the L1 twice what one along K does.
+template <int DT, int OP, int ODT, int AROWS, int RB = 1, int CB = 1, bool LOOSE = false, bool BROWS = false>
 __global__ __launch_bounds__(SKINNY_THREADS) __attribute__((amdgpu_waves_per_eu(2, 8))) void
 gemm_skinny_kernel(const GemmKArgs p) {
   constexpr bool ATOMIC = OP == OP_ATOMIC32 || OP == OP_ATOMIC16;
@@ -92,6 +95,7 @@ gemm_skinny_kernel(const GemmKArgs p) {
   static_assert(AROWS == 16 || (AROWS == 8 && RB == 1), "rows of a block of A");
   static_assert(RB == 1 || RB == 2, "blocks of rows per workgroup");
   static_assert(CB == 1 || (CB == 2 && RB == 2 && AROWS == 16), "blocks of columns per workgroup");
+  static_assert(!BROWS || (CB == 2 && !LOOSE && DT != IRIS_DTYPE_F32), "B by rows of k: cells of 16-bit operands");
   constexpr bool A_DMA = CB == 2;  // A in LDS, UN blocks a wave, like B
   constexpr int NB = RB * CB;
   using vec8 = typename Mfma<DT>::vec8;
@@ -125,7 +129,8 @@ gemm_skinny_kernel(const GemmKArgs p) {
   constexpr int LEAD = LOOSE ? 16 : 0;  // (no offset of a chunk moved back is below zero)
   const int rows_b = min(SKINNY_COLS * CB, p.N - n0);
   const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)(p.b + (int64_t)n0 * p.sbn * 2 - LEAD), 0, (int)((((int64_t)rows_b - 1) * p.sbn + p.K) * 2) + LEAD, 0x00020000);
+      (void*)(p.b + (int64_t)n0 * p.sbn * 2 - LEAD), 0,
+      (int)((BROWS ? ((int64_t)p.K - 1) * p.sbk + rows_b : ((int64_t)rows_b - 1) * p.sbn + p.K) * 2) + LEAD, 0x00020000);
   const int rows_a = min(SKINNY_ROWS * RB, p.M - m0);
   const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
       (void*)(p.a + (int64_t)m0 * p.sam * 2 - LEAD), 0, (int)((((int64_t)rows_a - 1) * p.sam + p.K) * 2) + LEAD, 0x00020000);
@@ -166,6 +171,14 @@ gemm_skinny_kernel(const GemmKArgs p) {
   auto fetch = [&](int u, int kb) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < 2 * CB; ++j) {
+      if constexpr (BROWS) {
+        // lane l of fetch j: columns 8 (l % 4) .. + 7 of k 16j + l / 4 (N is a multiple of eight: inside the matrix or past it)
+        const int k = kb * 64 + 16 * j + (lane >> 2), col = (lane & 3) * 8;
+        const bool ok = kb < nb && k < p.K && col < rows_b;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (IRIS_LDS void*)(wb + u * (CB * SKINNY_BLOCK_BYTES) + j * 1024), 16,
+                                                 ok ? (int)(((int64_t)k * p.sbk + col) * 2) : (int)0x80000000, 0, 0, 0);
+        continue;
+      }
       const int ch = bchunk ^ ((j & 1) << 2);
       const bool ok = kb < nb && kb * 64 + ch * 8 < p.K;
       const uint32_t off = (uint32_t)(((int64_t)b_column(j) * p.sbn) * 2 + kb * 128 + ch * 16) + LEAD - back(kb, ch);
@@ -202,8 +215,21 @@ gemm_skinny_kernel(const GemmKArgs p) {
       const int pc = (lq * 2 + h) ^ ((lr >> 1) & 7);
       vec8 fb[CB];
 #pragma unroll
-      for (int j = 0; j < CB; ++j)
-        fb[j] = *reinterpret_cast<const IRIS_LDS vec8*>(wb + (u * CB + j) * SKINNY_BLOCK_BYTES + lr * 128 + pc * 16);
+      for (int j = 0; j < CB; ++j) {
+        if constexpr (BROWS) {
+          // Each 16 lanes read four k of the 16 columns of block j, lane l four of them of k l / 4: those of its own
+          // chunk (l % 4) that are block j's.  They are handed out so that lane l holds the four k of the block's column l.
+          // Twice, four k apart.  (Two of the wave's quarters meet on the same banks: 8 reads of 16 clocks a block, beside 270
+          // that its fetches take.)
+          typedef short s16x4 __attribute__((ext_vector_type(4)));
+          const IRIS_LDS char* at = wb + u * (CB * SKINNY_BLOCK_BYTES) + (lq * 16 + h * 8 + (lr >> 2)) * 64 + (lr & 3) * 16 + j * 8;
+          const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((IRIS_LDS s16x4*)at);
+          const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((IRIS_LDS s16x4*)(at + 4 * 64));
+          fb[j] = __builtin_bit_cast(vec8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+        } else {
+          fb[j] = *reinterpret_cast<const IRIS_LDS vec8*>(wb + (u * CB + j) * SKINNY_BLOCK_BYTES + lr * 128 + pc * 16);
+        }
+      }
       const bool cut = LOOSE && (p.K & 7) != 0 && kb == nb_all - 1;
       const int front = lq * 2 + h == (p.K & 63) / 8 ? 8 - (p.K & 7) : 0;
       if (cut)
@@ -440,7 +466,7 @@ gemm_skinny_kernel(const GemmKArgs p) {
 }
 
 // The kernel for (operand type, store op, rows of A in a block, blocks of rows and of columns a workgroup), or null.
-// `loose`: for operands at any alignment.
-GemmKernelFn gemm_skinny_kernel_for(int dt, int op, int arows, int rb, int cb, bool loose);
+// `loose`: for operands at any alignment.  `b_rows` (cells): for a row-major B.
+GemmKernelFn gemm_skinny_kernel_for(int dt, int op, int arows, int rb, int cb, bool loose, bool b_rows = false);
 
 }  // namespace iris_amd

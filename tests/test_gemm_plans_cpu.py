@@ -34,6 +34,20 @@ def plan(M, N, K, BM, BN, dtype=BF16, ws=1, base=1 << 32, row=None, **kw):
 PARTS = "64x64x128_w2x2_s4_f4+parts_of_tiles"
 
 
+@pytest.mark.parametrize("M,N,K,BM,BN,want", [
+    # a row-major weight: cells up to a K whose half lines no longer come in time, and for what 32 rows of them share
+    (1, 1376, 4096, 64, 64, ("cells_32x32_rows", 1)),
+    (27, 256, 28032, 256, 64, ("cells_32x32_rows", 1)),
+    (128, 1376, 4096, 64, 64, ("cells_32x32_rows", 1)),
+    (28, 4864, 7936, 64, 64, ("64x64x128_w2x2_s4_f4_rows", 3)),
+    (138, 128, 32000, 64, 64, ("64x64x128_w2x2_s4_f4_rows", 16)),
+    # rows off the 16 bytes
+    (16, 1380, 1024, 64, 64, ("64x64x128_w2x2_gather", 4)),
+])
+def test_row_major_weights(M, N, K, BM, BN, want):
+    assert plan(M, N, K, BM, BN, stride_bk=N, stride_bn=1) == want
+
+
 @pytest.mark.parametrize("M,N,BM,BN,K,want", [
     # 32 tiles of 128 x 128 and the like: parts fill the chip, a long K is shared out instead
     (256, 2048, 128, 128, 512, (PARTS, 1)),

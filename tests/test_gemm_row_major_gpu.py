@@ -138,3 +138,60 @@ def test_what_stays_gathered(shmem, M, N, K, pad, shift, dtype):
     ops.gemm_launch(*args)
     torch.cuda.synchronize()
     check_close(cg, O.shard_gemm(A, B, dtype), "gathered")
+
+
+@pytest.mark.parametrize("M,N,K,BM,BN,pad,shift", [
+    (1, 64, 8, 64, 64, 0, 0),         # one chunk of K, one row
+    (3, 40, 72, 64, 64, 8, 0),        # N inside a cell, a block of K that holds a single chunk
+    (16, 1376, 200, 64, 64, 0, 8),
+    (32, 520, 1032, 64, 128, 0, 0),   # two blocks a wave in flight and one more
+    (33, 328, 1024, 64, 64, 16, 0),
+    (200, 504, 2056, 128, 64, 0, 0),
+    (250, 120, 576, 256, 128, 24, 8),
+])
+@pytest.mark.parametrize("dtype,out", [(BF16, BF16), (F16, F32)])
+def test_cells(shmem, M, N, K, BM, BN, pad, shift, dtype, out):
+    A, B, a, b = operands(shmem, M, N, K, dtype, pad, shift)
+    cg = shmem.full((M, N), 7, dtype=out)
+    total = ops.cdiv(M, BM) * ops.cdiv(N, BN)
+    flags = shmem.zeros((total + 1,), dtype=torch.int32)
+    locks = shmem.zeros((256,), dtype=torch.int32)
+    args = (a, b, None, cg, flags, None, 0, 1, 256, BM, BN, 64, 2, ops.EPI_ALL_SCATTER)
+    kw = dict(locks=locks, num_xcds=8)
+    assert ops.gemm_plan_name(*args, **kw) == "cells_32x32_rows"
+    for launch in (1, 2):
+        ops.gemm_launch(*args, **kw)
+        torch.cuda.synchronize()
+        check_close(cg, O.shard_gemm(A, B, out), f"launch {launch}")
+        assert flags.cpu().tolist() == [launch] * total + [0] and not locks.any()
+
+
+@pytest.mark.parametrize("M,N,K", [(16, 256, 8200), (5, 1376, 4096)])
+def test_cells_that_share_k(shmem, M, N, K):
+    A, B, a, b = operands(shmem, M, N, K, BF16)
+    cg = shmem.zeros((M, N), dtype=BF16)
+    total = ops.cdiv(N, 64)
+    flags = shmem.zeros((total,), dtype=torch.int32)
+    P = shmem.zeros((256, 64 * 64), dtype=F32)
+    locks = shmem.zeros((256,), dtype=torch.int32)
+    args = (a, b, None, cg, flags, None, 0, 1, 256, 64, 64, 64, 2, ops.EPI_ALL_SCATTER)
+    kw = dict(partials=P, locks=locks, num_xcds=8)
+    assert ops.gemm_plan_name(*args, **kw) == "cells_32x32_rows"
+    for launch in (1, 2):
+        ops.gemm_launch(*args, **kw)
+        torch.cuda.synchronize()
+        check_close(cg, O.shard_gemm(A, B, BF16), f"launch {launch}")
+        assert flags.cpu().tolist() == [launch] * total and not locks.any()
+
+
+@pytest.mark.parametrize("out_dtype", [F32, F16])
+def test_cells_add_with_atomics(shmem, out_dtype):
+    M, N, ks, ws = 40, 136, 72, 4
+    A, B, a, b = operands(shmem, M, N, ks * ws, F16)
+    cg = shmem.zeros((M, N), dtype=out_dtype)
+    for r in range(ws):
+        args = (a[:, r * ks:(r + 1) * ks], b[r * ks:(r + 1) * ks, :], None, cg, None, None, 0, 1, 256, 64, 64, 64, 6, ops.EPI_ATOMIC_ADD)
+        assert ops.gemm_plan_name(*args, num_xcds=8) == "cells_32x32_rows"
+        ops.gemm_launch(*args, num_xcds=8)
+    torch.cuda.synchronize()
+    check_close(cg, O.atomics_all_reduce(O.k_shards(A, B, ws)), "sum", block_rtol=2 ** -7 if out_dtype == F32 else None)
