@@ -808,15 +808,30 @@ bool reduce_in_program(const iris_gemm_args& a, const Plan& producer) {
   const int64_t inside = (int64_t)(a.block_m < a.M ? a.block_m : a.M) * (a.block_n < a.N ? a.block_n : a.N);
   const int64_t strips = inside * a.world_size * dtype_size(a.c_dtype);  // bytes that a program's tile is reduced from
   // (inside, operands at any alignment and a row-major B are gathered)
-  if (tiles <= a.num_sms && k.vec_out && !producer.loose && !producer.b_rows && (producer.skinny || (producer.entry->dma && !producer.entry->b_rows && !producer.entry->loose))) {
+  const bool rows = producer.skinny ? producer.b_rows != 0 : producer.entry->b_rows;
+  const bool loose = producer.skinny ? producer.loose != 0 : producer.entry->loose;
+  if (tiles <= a.num_sms && k.vec_out && !rows && !loose && (producer.skinny || producer.entry->dma)) {
     const bool few = producer.skinny && producer.skinny_cb == 1;
     if (inside <= 64 * 64 && (few ? steps <= 2 && a.block_n <= 64 : steps <= 10)) return true;
     if (!few && tiles >= 16 && a.block_n <= 64 && steps <= 5 && (inside <= 128 * 64 || strips <= (128 << 10))) return true;
   }
+  // (few rows off the 16 bytes: [16,133] x [133,4096] of 8 bf16 partials 12.0 / 13.2, K 389 12.9 / 13.2, 637 14.7 / 13.2)
+  if (loose && producer.skinny && producer.skinny_cb == 1 && tiles <= a.num_sms && k.vec_out && inside <= 64 * 64 && a.block_n <= 64 && steps <= 7)
+    return true;
   if ((producer.skinny && producer.skinny_cb == 1) || producer.last_round || producer.rest || producer.parts) return false;
   // (cells: the caller's tiles inside, when they are as small as the parts they would be run in)
   if (producer.skinny && a.block_m * a.block_n > 64 * 64) return false;
   if (k.split_k > 1 || k.merge_m * k.merge_n > 1 || k.total_tiles > a.num_sms || !k.vec_out) return false;
+  // Behind, those operands go through the DMA, so they stay inside for less: up to fewer K-steps the larger the tile, and not
+  // where a program has 256 KB to reduce.  (us a pass, inside / behind, bf16 partials; row-major B, 64 x 64 tiles [1000,1024] of 8,
+  // K 1024 17.9 / 19.7, 1504 21.7 / 20.9; cells [16,4096] of 8, K 256 11.6 / 13.8, 520 14.7 / 13.2; 128 x 128 tiles [2048,2048] of 2,
+  // K 392 21.4 / 24.1, 1288 37.8 / 27.6, of 8, K 1024 37.3 / 31.0; 256 x 128 [4096,2048] of 2, K 136 28.2 / 30.0, 392 35.7 / 31.5;
+  // along K off the 16 bytes, 128 x 128 tiles of 2, K 709 24.2 / 27.7, 1285 34.8 / 31.7; 256 x 64 [4096,1024] of 8, K 1501 48.7 / 43.6.)
+  if (rows || loose) {
+    const int area = a.block_m * a.block_n;
+    const int most = area > 128 * 128 ? 4 : area > 64 * 64 ? (rows ? 8 : 12) : rows ? (producer.skinny ? 7 : 16) : 24;
+    return steps <= most && (area <= 64 * 64 || strips < (256 << 10));
+  }
   return steps <= 8 || (steps <= 24 && a.block_m * a.block_n <= 128 * 128);
 }
 

@@ -119,3 +119,22 @@ def test_the_reduce_inside_the_program_or_behind_it(M, N, K, BM, BN, ws, partial
     name, _ = plan(M, N, K, BM, BN, ws=ws, epilogue=ops.EPI_ONE_SHOT, phase=ops.PHASE_FUSED, c=3 << 32, c_dtype=partial,
                    stride_cm=N, stride_cn=1, stride_cm_global=N)
     assert name.endswith("+reduce") and name.endswith("+kernel+reduce") != inside
+
+
+@pytest.mark.parametrize("M,N,K,BM,BN,ws,rows,inside", [
+    # a row-major weight, whose producer is faster than the program that also reduces
+    (1000, 1024, 1024, 64, 64, 8, True, True), (1000, 1024, 1504, 64, 64, 8, True, False),
+    (16, 4096, 256, 64, 64, 8, True, True), (16, 4096, 1376, 64, 64, 8, True, False),
+    (2048, 2048, 392, 128, 128, 2, True, True), (2048, 2048, 1288, 128, 128, 2, True, False),
+    (2048, 2048, 392, 128, 128, 8, True, False),
+    (4096, 2048, 136, 256, 128, 2, True, True), (4096, 2048, 392, 256, 128, 2, True, False),
+    # rows along K off the 16 bytes
+    (16, 4096, 133, 64, 64, 8, False, True), (16, 4096, 637, 64, 64, 8, False, False),
+    (2048, 2048, 573, 128, 128, 2, False, True), (2048, 2048, 1285, 128, 128, 2, False, False),
+    (4096, 1024, 389, 256, 64, 8, False, False), (1000, 1024, 1501, 64, 64, 8, False, True),
+])
+def test_where_operands_that_are_gathered_inside_are_reduced(M, N, K, BM, BN, ws, rows, inside):
+    kw = dict(stride_bk=N, stride_bn=1) if rows else {}
+    name, _ = plan(M, N, K, BM, BN, ws=ws, epilogue=ops.EPI_ONE_SHOT, phase=ops.PHASE_FUSED, c=9 << 32, stride_cm=N, stride_cn=1,
+                   stride_cm_global=N, **kw)
+    assert name.endswith("+kernel+reduce") != inside, name
