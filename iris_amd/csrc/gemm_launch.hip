@@ -250,7 +250,9 @@ bool plan_cells(const iris_gemm_args& a, int op, bool dma_ok, bool loose, bool b
     parts = few_rows_parts(cells, (a.K + 63) / 64, b_rows ? 0.9 : 0.6, (int64_t)a.N * a.K * 2);
     if (parts * cells * (CELL * CELL) > (int64_t)a.num_sms * a.partials_slot_elems) parts = 1;
   }
-  plan->skinny = gemm_skinny_kernel_for(a.ab_dtype, op, 16, 2, 2, loose, b_rows);
+  // (a row-major B with up to 16 rows of A: cells of 16 x 32, which fetch the half or the quarter of A that there is)
+  const int rb = b_rows && a.M <= SKINNY_ROWS ? 1 : 2;
+  plan->skinny = gemm_skinny_kernel_for(a.ab_dtype, op, rb == 1 && a.M <= 8 ? 8 : 16, rb, 2, loose, b_rows);
   if (!plan->skinny) return false;
   k.cells = (int)cells;
   k.cells_by_row = a.M > a.N;

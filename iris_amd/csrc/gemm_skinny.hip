@@ -16,10 +16,14 @@ GemmKernelFn pick(int arows, int rb, int cb) {
 template <int DT, int OP>
 GemmKernelFn pick(int arows, int rb, int cb, bool loose, bool b_rows) {
   if (b_rows) {
-    if constexpr (DT == IRIS_DTYPE_F32)
+    if constexpr (DT == IRIS_DTYPE_F32) {
       return nullptr;
-    else
-      return cb == 2 ? &gemm_skinny_kernel<DT, OP, (OP == OP_STORE32 || OP == OP_ATOMIC32) ? IRIS_DTYPE_F32 : DT, 16, 2, 2, false, true> : nullptr;
+    } else {
+      constexpr int ODT = (OP == OP_STORE32 || OP == OP_ATOMIC32) ? IRIS_DTYPE_F32 : DT;
+      if (cb != 2) return nullptr;
+      if (rb == 2) return &gemm_skinny_kernel<DT, OP, ODT, 16, 2, 2, false, true>;
+      return arows == 8 ? &gemm_skinny_kernel<DT, OP, ODT, 8, 1, 2, false, true> : &gemm_skinny_kernel<DT, OP, ODT, 16, 1, 2, false, true>;
+    }
   }
   return loose ? pick<DT, OP, true>(arows, rb, cb) : pick<DT, OP, false>(arows, rb, cb);
 }

@@ -85,7 +85,9 @@ constexpr int cells_lds_bytes() { return SKINNY_WAVES * SKINNY_UN * 4 * SKINNY_B
 // [137,4864] and its reduce 17.2 / 16.8; 40 random calls of up to 32 rows 1.48x.)
 // BROWS (cells, 16-bit operands): a B whose rows are its k (row-major [K, N]), in whole aligned 16-byte chunks.  A block of B lies
 // in LDS as in memory, 64 k of 32 columns, and is transposed on its way to the MFMAs by ds_read_b64_tr_b16.  A row of 64
-// bytes is half a cache line, so that such a block costs the L1 twice what one along K does.
+// bytes is half a cache line, so that such a block costs the L1 twice what one along K does.  With up to 16 rows of A, RB is 1
+// ([4,1376] x [1376,4096] 8.0 -> 7.4 us, 27 random calls of 1 to 16 rows 1.08x, same bits; RB 2 fetched as many rows of A again,
+// and for up to eight three times as many, all out of range).
 template <int DT, int OP, int ODT, int AROWS, int RB = 1, int CB = 1, bool LOOSE = false, bool BROWS = false>
 __global__ __launch_bounds__(SKINNY_THREADS) __attribute__((amdgpu_waves_per_eu(2, 8))) void
 gemm_skinny_kernel(const GemmKArgs p) {
@@ -94,7 +96,7 @@ gemm_skinny_kernel(const GemmKArgs p) {
   constexpr int UN = SKINNY_UN, AH = AROWS / 8;  // fetches of a block of A
   static_assert(AROWS == 16 || (AROWS == 8 && RB == 1), "rows of a block of A");
   static_assert(RB == 1 || RB == 2, "blocks of rows per workgroup");
-  static_assert(CB == 1 || (CB == 2 && RB == 2 && AROWS == 16), "blocks of columns per workgroup");
+  static_assert(CB == 1 || (CB == 2 && ((RB == 2 && AROWS == 16) || BROWS)), "blocks of columns per workgroup");
   static_assert(!BROWS || (CB == 2 && !LOOSE && DT != IRIS_DTYPE_F32), "B by rows of k: cells of 16-bit operands");
   constexpr bool A_DMA = CB == 2;  // A in LDS, UN blocks a wave, like B
   constexpr int NB = RB * CB;

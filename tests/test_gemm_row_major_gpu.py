@@ -184,9 +184,10 @@ def test_cells_that_share_k(shmem, M, N, K):
         assert flags.cpu().tolist() == [launch] * total and not locks.any()
 
 
+@pytest.mark.parametrize("M", [7, 13, 40])  # (8, 16 and 32 rows of A a cell)
 @pytest.mark.parametrize("out_dtype", [F32, F16])
-def test_cells_add_with_atomics(shmem, out_dtype):
-    M, N, ks, ws = 40, 136, 72, 4
+def test_cells_add_with_atomics(shmem, M, out_dtype):
+    N, ks, ws = 136, 72, 4
     A, B, a, b = operands(shmem, M, N, ks * ws, F16)
     cg = shmem.zeros((M, N), dtype=out_dtype)
     for r in range(ws):
