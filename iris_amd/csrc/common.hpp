@@ -236,6 +236,23 @@ __device__ inline __amdgpu_buffer_rsrc_t tile_rsrc(const IRIS_GLOBAL char* base,
   return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, (int)bytes, 0x00020000);
 }
 
+// 16 bytes a lane by LDS-DMA, for waves that read LDS with ds_read_b64_tr_b16: the caller waits for them by count.  The
+// compiler takes that read (not a plain one) for one that may meet any LDS-DMA it knows to be in flight and puts
+// s_waitcnt vmcnt(0) in front of it; of these loads it does not know.  (m0 holds the LDS address, which may be read one
+// instruction after its write; nothing else in the kernels that load this way uses it.  dst, rs and at are the wave's.)
+// us a pass, the compiler's loads / these: a K-step of the 256 x 256 tile, whose waves fetch what they multiply, stood still
+// three times, [1816,34048] x [34048,6016] 1196 / 709, [8020,4224] x [4224,1472] 171 / 111, 46 random calls 1.24x; cells had one
+// set in flight for two, [14,4032] x [4032,192] 6.3 / 5.8; tiles with fetching waves waited for the tile before's stores, 1.01x.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+__device__ __attribute__((always_inline)) inline void lds_dma16(__amdgpu_buffer_rsrc_t rs, IRIS_LDS void* dst, uint32_t off, int at) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+               :
+               : "s"(__builtin_amdgcn_readfirstlane((int)(uintptr_t)dst)), "v"(off), "s"(rs), "s"(__builtin_amdgcn_readfirstlane(at))
+               : "m0", "memory");
+}
+#pragma clang diagnostic pop
+
 template <int DT>
 __device__ inline void unpack_vec(u32x4 x, float (&v)[Vec<DT>::N]) {
   if constexpr (DT == IRIS_DTYPE_F32) {

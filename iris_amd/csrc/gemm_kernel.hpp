@@ -522,6 +522,8 @@ struct Loader {
         at_k = k * step_kb;
         if (!FULL && k0 + j * Cfg::NL * Cfg::B_RPB + rows_k(wave, lane) >= k_limit) off = 0x80000000u;
       }
+      lds_dma16(isA ? ra : rb, dst, off, at_k);
+      return;
     }
     __builtin_amdgcn_raw_ptr_buffer_load_lds(isA ? ra : rb, (IRIS_LDS void*)dst, 16, off, at_k, 0, 0);
   }

@@ -177,8 +177,7 @@ gemm_skinny_kernel(const GemmKArgs p) {
         // lane l of fetch j: columns 8 (l % 4) .. + 7 of k 16j + l / 4 (N is a multiple of eight: inside the matrix or past it)
         const int k = kb * 64 + 16 * j + (lane >> 2), col = (lane & 3) * 8;
         const bool ok = kb < nb && k < p.K && col < rows_b;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (IRIS_LDS void*)(wb + u * (CB * SKINNY_BLOCK_BYTES) + j * 1024), 16,
-                                                 ok ? (int)(((int64_t)k * p.sbk + col) * 2) : (int)0x80000000, 0, 0, 0);
+        lds_dma16(rb, wb + u * (CB * SKINNY_BLOCK_BYTES) + j * 1024, ok ? (uint32_t)(((int64_t)k * p.sbk + col) * 2) : 0x80000000u, 0);
         continue;
       }
       const int ch = bchunk ^ ((j & 1) << 2);
@@ -194,7 +193,9 @@ gemm_skinny_kernel(const GemmKArgs p) {
         const int ch = bchunk ^ (j << 2);
         const bool ok = kb < nb && kb * 64 + ch * 8 < p.K;
         const uint32_t off = (uint32_t)(((int64_t)(i * 16 + brow + 8 * j) * p.sam) * 2 + kb * 128 + ch * 16) + LEAD - back(kb, ch);
-        if constexpr (A_DMA)
+        if constexpr (BROWS)
+          lds_dma16(ra, wa + (u * RB + i) * SKINNY_BLOCK_BYTES + j * 1024, ok ? off : 0x80000000u, 0);
+        else if constexpr (A_DMA)
           __builtin_amdgcn_raw_ptr_buffer_load_lds(
               ra, (IRIS_LDS void*)(wa + (u * RB + i) * SKINNY_BLOCK_BYTES + j * 1024), 16, ok ? (int)off : (int)0x80000000, 0, 0, 0);
         else
