@@ -194,9 +194,21 @@ bool plan_few_rows(const iris_gemm_args& a, int op, bool dma_ok, bool loose, Pla
   const bool lines = whole_lines(a);
   const bool long_k = a.variant == 0 && !mid && rb == 2 && !f32 &&
                       (cells > cus ? a.K >= 8192 : !lines && a.M > 24 && a.K >= 20480 && b_bytes > (96 << 20));
+  // Off the 16 bytes the L1 is the bound earlier, and the tiles no longer gather.  (us a pass, here / there: [9,12977] x
+  // [12977,4352] 52 / 46, [15,19393] x [19393,3392] 45 / 42, [24,449] x [449,5824] 11.6 / 10.5, [23,29889] x [29889,2368] 54 / 45,
+  // [36,26745] x [26745,1376] 42 / 31, fp32 [43,10433] x [10433,3136] 101 / 69, [109,2913] x [2913,7152] 95 / 79; but [1,23937] x
+  // [23937,3584] 37 / 46, [24,15489] x [15489,1600] 16.7 / 18.3, [63,27009] x [27009,528] 23 / 29, fp32 [58,17025] x [17025,192] 18 / 20.)
+  const bool off = loose && a.variant == 0;
+  const bool off_f32 = off && f32 && (mid ? (cells >= 128 && a.K >= 32768) || (cells > cus && a.K >= 8192) || (cells > 4 * cus && a.K >= 1024)
+                                          : a.M > 16 && cells > cus && a.K >= 8192);
+  const bool off_16 =
+      off && !f32 && (mid        ? (cells >= 72 && a.K >= 16384) || (cells >= 192 && a.K >= 12288)
+                      : rb == 2  ? (cells >= 128 && a.K >= 18432) || (cells > cus && a.K >= 6144)
+                      : a.M > 16 ? cells > 2 * cus
+                                 : (cells > cus && a.K >= (a.M > 8 ? 8192 : 16384)) || (a.M > 8 && b_bytes > (128 << 20)));
   // (the workgroups' rows belong to one tile)
   const bool rows_ok = a.block_m >= a.M || (f32 && a.block_m % (SKINNY_ROWS * rb) == 0);
-  const bool ok = room && !long_k && a.K > 0 && dma_ok && !plan->in_program && rows_ok && (a.block_n % SKINNY_COLS) == 0 &&
+  const bool ok = room && !long_k && !off_f32 && !off_16 && a.K > 0 && dma_ok && !plan->in_program && rows_ok && (a.block_n % SKINNY_COLS) == 0 &&
                   !a.mm_begin_timestamp && !a.mm_end_timestamp && (a.split_k == 0 || a.split_k == 1) && counters &&
                   ((int64_t)SKINNY_ROWS * rb * a.stride_am + a.K) * 2 < lim &&
                   ((int64_t)SKINNY_COLS * a.stride_bn + a.K) * 2 < lim;

@@ -1,0 +1,25 @@
+"""Which kernel is planned for operands off the 16 bytes and for a row-major B, on both sides of lines where the faster one changes
+(plan names only: no GPU)."""
+
+import pytest
+
+from iris_amd import ops
+from test_gemm_plans_cpu import F32, plan
+
+ROWS = lambda N: dict(stride_bk=N, stride_bn=1)
+
+
+@pytest.mark.parametrize("M,N,K,BM,BN,dtype,few", [
+    # an odd K: rows off the 16 bytes
+    (9, 4352, 12977, 256, 64, 2, False), (9, 4352, 4097, 256, 64, 2, True), (1, 4288, 32705, 128, 128, 2, False),
+    (1, 3584, 23937, 256, 64, 2, True), (15, 3392, 20993, 128, 128, 2, False), (15, 1360, 19393, 128, 128, 2, True),
+    (24, 5824, 449, 128, 128, 2, False), (23, 2368, 29889, 128, 128, 2, False), (24, 1600, 15489, 256, 64, 2, True),
+    (36, 1376, 26745, 64, 64, 2, False), (63, 528, 27009, 64, 64, 2, True),
+    # fp32, where a row of workgroups more is a round more
+    (115, 6400, 10753, 128, 128, F32, False), (118, 7424, 641, 64, 64, F32, False), (118, 2368, 833, 256, 64, F32, True),
+    (58, 192, 17025, 128, 128, F32, True), (40, 7552, 257, 64, 64, F32, True),
+])
+def test_few_rows(M, N, K, BM, BN, dtype, few):
+    assert plan(M, N, K, BM, BN, dtype=dtype)[0].startswith("few_rows") == few
+    # (on aligned rows the line is another)
+    assert dtype == F32 or M > 16 or plan(M, N, K // 64 * 64, BM, BN)[0].startswith("few_rows")
