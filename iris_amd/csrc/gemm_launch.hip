@@ -257,8 +257,11 @@ bool plan_cells(const iris_gemm_args& a, int op, bool dma_ok, bool loose, bool b
                   counters && (CELL * a.stride_am + a.K) * 2 < lim && (CELL * a.stride_bn + a.K) * 2 < lim;
   if (!ok) return false;
   int parts = 1;
-  // (K of a row-major B is shared out for one row of cells only: [138,32000] x [32000,128] in twelve parts 24.4 us, 18.0 in tiles)
-  if (a.split_k == 0 && a.partials && aligned16(a.partials) && a.locks && k.total_tiles + cells <= a.num_sms && (!b_rows || m_cells == 1)) {
+  // (K of a row-major B is shared out for one row of cells only: [138,32000] x [32000,128] in twelve parts 24.4 us, 18.0 in tiles;
+  // not off the 16 bytes for more than four rows of cells of a long K: [152,29953] x [29953,320] in five 39, in tiles 27,
+  // [209,20041] x [20041,168] 26.6 / 21.9; but [119,17089] x [17089,384] 17.8 / 20.9, [273,16001] x [16001,192] 19.6 / 22.9)
+  const bool far = loose && a.ab_dtype != IRIS_DTYPE_F32 && m_cells > 4 && a.K >= 19000;
+  if (a.split_k == 0 && a.partials && aligned16(a.partials) && a.locks && k.total_tiles + cells <= a.num_sms && (m_cells == 1 || !b_rows) && !far) {
     parts = few_rows_parts(cells, (a.K + 63) / 64, b_rows ? 0.9 : 0.6, (int64_t)a.N * a.K * 2);
     if (parts * cells * (CELL * CELL) > (int64_t)a.num_sms * a.partials_slot_elems) parts = 1;
   }
