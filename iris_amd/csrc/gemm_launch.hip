@@ -624,11 +624,17 @@ struct TileLaunch {
   bool sliced, parts;
 };
 struct Operands {
-  bool f32, lines, gather, b_rows, atomic, vec_out;
+  bool f32, lines, gather, b_rows, loose, atomic, vec_out;
   int copies;     // of the output
   bool peers;     // other ranks wait for it
   int64_t tile;   // elements of a caller's tile that lie in the output
 };
+// How much of the operands comes from HBM: none of it up to 60 MB, all from 110 MB on (a program has other data in the 256 MB
+// of the last-level cache between two launches).
+double streamed(const iris_gemm_args& a) {
+  const double of = (((double)a.M + a.N) * a.K * 2e-6 - 60) / 50;
+  return of < 0 ? 0 : of > 1 ? 1 : of;
+}
 double tiles_us(const iris_gemm_args& a, const TileLaunch& t, const Operands& o, int64_t cus) {
   const int64_t items = t.tiles * t.split_k, programs = items < cus ? items : cus;
   const bool split = t.split_k > 1;
@@ -636,7 +642,8 @@ double tiles_us(const iris_gemm_args& a, const TileLaunch& t, const Operands& o,
   const double area = (double)t.cm * t.cn / 4096, partials = programs * area / 64;  // tiles of 64 x 64; MB
   const bool deep = t.cm == 64 && t.cn == 64;  // (K-steps of 128: whole lines, mostly)
   const double fetch = (t.cm + t.cn) / (8 * 108.0) * (1 + 0.13 * cover + (split ? 0.17 : 0.0)) *
-                       (o.gather ? 2.9 : o.lines ? 1.0 : deep ? 1.3 : 1.5);
+                       (o.gather ? 2.9 : o.lines ? 1.0 : o.loose ? (deep ? 1.9 : 2.1) : deep ? 1.3 : 1.5) *
+                       ((o.b_rows || o.loose) && !split ? 1 + 0.5 * streamed(a) : 1.0);
   const double multiply = o.f32 ? area * 0.452 * (1 + 0.04 * cover) + 0.1 : area * 0.0535;
   const int64_t unit = deep ? 2 : 1, nk = ((int64_t)a.K + 64 * unit - 1) / (64 * unit);
   const int64_t part_steps = (nk + t.split_k - 1) / t.split_k * unit, steps = (items + cus - 1) / cus * t.subs * part_steps;
@@ -671,13 +678,14 @@ double cells_us(const iris_gemm_args& a, int64_t cells, int parts, const Operand
   const double mb = ((double)a.M + a.N) * a.K * 2e-6;
   // us for 64 of K, operands in whole lines / not: [512,512] 256 cells 0.090 / 0.13; [128,1376] 172 cells 0.083 / 0.11;
   // [200,512] 112 cells 0.048 / 0.066 as long as the L2s hold the operands, 0.07 / 0.08 beyond
-  // (a row-major B comes in half lines, from HBM at half the rate: [28,7936] x [7936,4864] 33.8, in tiles 23.5)
-  const double lines = o.b_rows ? 1.8 : o.lines ? 1.0 : 1.45;
+  // (a row-major B comes in half lines, from HBM at half the rate: [28,7936] x [7936,4864] 33.8, in tiles 23.5; with up to 16
+  // rows of A a cell fetches half of A)
+  const double lines = o.b_rows ? (a.M <= SKINNY_ROWS ? 1.08 : 1.8) : o.lines ? 1.0 : o.loose ? 2.1 : 1.45;
   const double step = 0.083 * (groups * 5 > cus * 4 ? 1.09 : groups * 2 <= cus && mb <= 30 ? 0.7 : 1.0) *
                       (o.f32 && lines < 1.65 ? 1.65 : lines);
   // (a workgroup's first sixteen blocks of K are in flight together)
   const double loop = ((groups + cus - 1) / cus * ((nk + parts - 1) / parts) - 16) * step;
-  const double stream = mb / (o.b_rows ? 3.2 : mb > 200 ? 4.4 : 8.4) - 3, k_time = loop > stream ? loop : stream;
+  const double stream = mb / (o.b_rows ? (mb > 80 ? 3.2 : 4.8) : o.loose ? (mb > 100 ? 3.2 : 6.0) : mb > 200 ? 4.4 : 8.4) - 3, k_time = loop > stream ? loop : stream;
   const double per_tile = o.atomic ? 0.0 : (double)o.tile / (CELL * CELL) / 64;
   return 5.85 + (0.0075 + 0.004 * (per_tile < 1 ? per_tile : 1.0)) * groups + 0.025 * (o.copies - 1) + (parts > 1 ? 0.7 : 0.0) +
          (o.atomic ? 0.4 : 0.0) + (k_time > 0 ? k_time : 0.0);
@@ -734,7 +742,7 @@ bool plan_small(const iris_gemm_args& a, Plan* plan) {
   }
   if (!whole.entry) return false;
   const GemmKArgs& w = whole.k;
-  const Operands o{a.ab_dtype == IRIS_DTYPE_F32, whole_lines(a), !whole.entry->dma, whole.entry->b_rows,
+  const Operands o{a.ab_dtype == IRIS_DTYPE_F32, whole_lines(a), !whole.entry->dma, whole.entry->b_rows, whole.entry->loose,
                    a.epilogue == IRIS_EPI_ATOMIC_ADD, w.vec_out != 0, w.dest_all ? a.world_size : 1, a.world_size > 1,
                    (int64_t)(a.block_m < a.M ? a.block_m : a.M) * (a.block_n < a.N ? a.block_n : a.N)};
   double least = tiles_us(a, TileLaunch{whole.entry->cm, whole.entry->cn, w.total_tiles, w.sub_m * w.sub_n, w.split_k,
@@ -1180,6 +1188,8 @@ hipError_t make_plan_body(const iris_gemm_args& a, Plan* plan, bool cells) {
       // the tall tiles are the ones whose K range can be shared out over idle programs)
       if (e.cm > 64 && e.cm >= 4 * a.M) continue;
       if (e.cn > 64 && e.cn >= 4 * a.N) continue;
+      // (a row-major B, and rows off the 16 bytes, come at no more than half the rate into the half of a tile that is padding)
+      if (e.cn > 128 && (e.b_rows || e.loose) && e.cn >= 2 * a.N) continue;
       // An atomic epilogue is bound by the chip's atomic rate (329 G fp32
       // adds a second, 51 us for 4096 x 4096), and while a program walks its
       // K loop it sends none: with two half tiles per logical tile the

@@ -32,3 +32,23 @@ def test_few_rows(M, N, K, BM, BN, dtype, few):
 ])
 def test_cells_that_share_k(M, N, K, BM, BN, cells):
     assert plan(M, N, K, BM, BN)[0].startswith("cells_32x32") == cells
+
+
+@pytest.mark.parametrize("M,N,K,BM,BN,rows,want", [
+    # operands that come from HBM: not a program per 64 x 64 part with all of K
+    (83, 7936, 32384, 128, 128, True, ("128x128x64_w2x2_s4_f4_rows", 4)),
+    (6745, 128, 22528, 256, 128, True, ("256x128x64_w2x2_s3_f4_rows", 9)),
+    (401, 1320, 9745, 128, 128, False, ("128x128x64_w2x2_s4_f4_gather_dma", 5)),
+    (73, 5824, 9281, 128, 128, False, ("128x128x64_w2x2_s4_f4_gather_dma", 5)),
+    (569, 960, 3873, 256, 256, False, ("64x64x128_w2x2_s4_f4_gather_dma+parts_of_tiles", 1)),
+    # cells with up to 16 rows of A
+    (5, 2432, 9536, 256, 256, True, ("cells_32x32_rows", 1)),
+    (2, 5696, 3840, 256, 128, True, ("cells_32x32_rows", 1)),
+    (28, 4864, 7936, 64, 64, True, ("64x64x128_w2x2_s4_f4_rows", 3)),
+    # a tile that is no more than half padding
+    (4705, 128, 14912, 256, 256, True, ("256x128x64_w2x2_s3_f4_rows", 13)),
+    (7388, 128, 22209, 256, 256, False, ("256x128x64_w2x2_s3_f4_gather_dma", 8)),
+    (7388, 129, 22209, 256, 256, False, ("256x256x64_w2x4_s2_gather_dma", 8)),
+])
+def test_small_products(M, N, K, BM, BN, rows, want):
+    assert plan(M, N, K, BM, BN, **(ROWS(N) if rows else {})) == want
