@@ -841,7 +841,7 @@ bool reduce_in_program(const iris_gemm_args& a, const Plan& producer) {
     if (!few && tiles >= 16 && a.block_n <= 64 && steps <= 5 && (inside <= 128 * 64 || strips <= (128 << 10))) return true;
   }
   // (few rows off the 16 bytes: [16,133] x [133,4096] of 8 bf16 partials 12.0 / 13.2, K 389 12.9 / 13.2, 637 14.7 / 13.2)
-  if (loose && producer.skinny && producer.skinny_cb == 1 && tiles <= a.num_sms && k.vec_out && inside <= 64 * 64 && a.block_n <= 64 && steps <= 7)
+  if (loose && producer.skinny && tiles <= a.num_sms && k.vec_out && inside <= 64 * 64 && a.block_n <= 64 && steps <= 7)
     return true;
   if ((producer.skinny && producer.skinny_cb == 1) || producer.last_round || producer.rest || producer.parts) return false;
   // (cells: the caller's tiles inside, when they are as small as the parts they would be run in)
@@ -854,6 +854,12 @@ bool reduce_in_program(const iris_gemm_args& a, const Plan& producer) {
   // along K off the 16 bytes, 128 x 128 tiles of 2, K 709 24.2 / 27.7, 1285 34.8 / 31.7; 256 x 64 [4096,1024] of 8, K 1501 48.7 / 43.6.)
   if (rows || loose) {
     const int area = a.block_m * a.block_n;
+    // (along K off the 16 bytes, a short shard: 128 x 128 tiles [2048,2048] of 8, bf16, K 129 27.0 / 28.5, 385 30.5 / 30.9, of 8,
+    // fp32, 37.2 / 40.2, 41.0 / 42.7, of 4, fp32, 26.2 / 32.2, 29.7 / 34.5, 641 33.3 / 37.1; 256 x 128 tiles, fp32, [1534,3008] of 4, 144 tiles, 34 / 42,
+    // 41 / 46.5, [4096,2048], 256 tiles, 46.5 / 46.0, 54 / 50.4; bf16 there as the line below)
+    const bool wide = a.c_dtype == IRIS_DTYPE_F32;
+    if (loose && steps <= (!wide ? 6 : strips > (256 << 10) ? 7 : 12) && strips <= (512 << 10) && area <= 128 * 128) return true;
+    if (loose && steps <= 7 && wide && area <= 256 * 128 && tiles * 4 <= (int64_t)a.num_sms * 3) return true;
     const int most = area > 128 * 128 ? 4 : area > 64 * 64 ? (rows ? 8 : 12) : rows ? (producer.skinny ? 7 : 16) : 24;
     return steps <= most && (area <= 64 * 64 || strips < (256 << 10));
   }
