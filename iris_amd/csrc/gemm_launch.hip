@@ -881,29 +881,65 @@ constexpr BlockTime BLOCK_TIMES[] = {
     {256, 128, 2, 9.2, 4.5, 0.693, 0.00, 0.40, 0.31}, {256, 256, 1, 2.6, 5.2, 0.899, 0.32, 0.22, 0.31},
     {256, 256, 2, 10.6, 6.4, 0.719, 0.78, 0.23, 0.26},
 };
-// The plan's time in us, or a negative number for a launch that the table does not know.
-double block_us(const iris_gemm_args& a, const Plan& plan) {
+// A launch in tiles of cm x cn as plan_split and split_last_round make it, before there is a plan of it: K in `split` parts, or
+// the last `last_tiles` tiles in `last_parts`.  (The plan is asked whether that is what it is: as_expected.)
+struct BlockLaunch {
+  int cm, cn, split;
+  int64_t tiles;
+  int last_tiles, last_parts;
+};
+BlockLaunch block_launch(const iris_gemm_args& a, int cm, int cn, bool callers, int cus) {
+  BlockLaunch l{cm, cn, 1, ((int64_t)a.M + cm - 1) / cm * (((int64_t)a.N + cn - 1) / cn), 0, 0};
+  const int nk = (a.K + 63) / 64;
+  if (!a.partials || !a.locks || a.num_sms > cus) return l;
+  const bool slots = a.partials_slot_elems >= (int64_t)cm * cn;
+  if (slots || (cm * cn >= 256 * 128 && a.partials_slot_elems * 2 >= (int64_t)cm * cn)) {
+    int sk = auto_split(l.tiles, nk, a.num_sms);
+    if (!slots && sk > 2) sk = 2;
+    if (sk >= 4 || (sk > 1 && nk >= 32)) l.split = sk;
+  }
+  if (callers && slots && l.split == 1) {
+    const int64_t last = l.tiles % a.num_sms;
+    int parts = last > 0 && l.tiles > a.num_sms && last * 2 <= a.num_sms ? (int)(a.num_sms / last) : 1;
+    if (parts > 16) parts = 16;
+    if (parts > nk / 32) parts = nk / 32;
+    if (parts >= 2) {
+      l.last_tiles = (int)last;
+      l.last_parts = parts;
+      l.tiles -= last;
+    }
+  }
+  return l;
+}
+bool as_expected(const BlockLaunch& l, const Plan& plan) {
   const GemmKArgs& k = plan.k;
-  if (!plan.entry || plan.skinny || k.stream_k || k.sub_m != 1 || k.sub_n != 1 || plan.entry->bk != 64) return -1;
+  return plan.entry && !plan.skinny && !k.stream_k && k.sub_m == 1 && k.sub_n == 1 && plan.entry->bk == 64 && plan.entry->cm == l.cm &&
+         plan.entry->cn == l.cn && k.split_k == l.split && k.total_tiles == l.tiles && plan.last_round == (l.last_parts > 0) &&
+         (!plan.last_round || (plan.k_last.split_k == l.last_parts && plan.k_last.total_tiles == l.last_tiles));
+}
+
+// The launch's time in us, or a negative number for one that the table does not know.
+double block_us(const iris_gemm_args& a, const BlockLaunch& l, int cus) {
   const bool lines = whole_lines(a);
   double streamed = (((double)a.M + a.N) * a.K * 2e-6 - 50) / 100;
   streamed = streamed < 0 ? 0 : streamed > 1 ? 1 : streamed;
-  const int nk = (a.K + 63) / 64, cus = current_cu_count();
+  const int nk = (a.K + 63) / 64;
+  const bool scatter = a.epilogue == IRIS_EPI_ALL_SCATTER, wide = (scatter ? a.c_global_dtype : a.c_dtype) == IRIS_DTYPE_F32;
   for (const BlockTime& t : BLOCK_TIMES) {
-    if (t.cm != plan.entry->cm || t.cn != plan.entry->cn || t.split != k.split_k) continue;
-    const int64_t items = (int64_t)k.total_tiles * t.split, rounds = (items + k.num_sms - 1) / k.num_sms;
-    const double busy = (double)(rounds > 1 ? k.num_sms : items) / cus;
+    if (t.cm != l.cm || t.cn != l.cn || t.split != l.split) continue;
+    const int64_t items = l.tiles * t.split, rounds = (items + a.num_sms - 1) / a.num_sms;
+    const double busy = (double)(rounds > 1 ? a.num_sms : items) / cus;
     const double step = t.step * (1 + t.cover * busy) * (lines ? 1.0 : 1 + t.off_lines) * (1 + t.streamed * streamed);
     // (the other copies of the output, or its wider elements: 6.5 TB/s of stores on all CUs)
-    const double copies = (k.dest_all ? a.world_size : 1) * (plan.entry->op == OP_STORE32 ? 2 : 1);
+    const double copies = (scatter ? a.world_size : 1) * (wide ? 2 : 1);
     const double tile = t.tile + (copies - 1) * t.cm * t.cn * 2 / 25400.0 / t.split;
     const double us = t.fixed + rounds * (tile + (nk + t.split - 1) / t.split * step);
-    if (!plan.last_round) return us;
+    if (l.last_parts == 0) return us;
     // The tiles of a last round that are shared out over all programs, as a launch of their own, whose programs share less of
     // what they fetch.  ([8192,36864] x [36864,576] in 256 x 64 tiles, 256 and then 32 in eight parts, 565 us, 717 in two
     // rounds; [2624,26328] x [26328,1520], 256 and 8 in twelve parts, 352)
-    const double apart = 1 + plan.k_last.total_tiles / (t.cm * t.cn >= 256 * 128 ? 256.0 : 32.0);
-    return us + 8 + tile + (nk + plan.k_last.split_k - 1) / plan.k_last.split_k * step * apart;
+    const double apart = 1 + l.last_tiles / (t.cm * t.cn >= 256 * 128 ? 256.0 : 32.0);
+    return us + 8 + tile + (nk + l.last_parts - 1) / l.last_parts * step * apart;
   }
   return -1;
 }
@@ -914,34 +950,38 @@ double block_us(const iris_gemm_args& a, const Plan& plan) {
 // 256 x 64 tiles, the caller's / 256 x 128 / 256 x 256: N 576, K 1024 23 / 16 / 24; N 704, K 4128 98 / 53 / -; N 1152, K 12288
 // 337 / 299 / 263; N 1344, K 4096 100 / 100 / 82.  By number of tiles alone, blocks only where they gave seven programs in
 // eight a tile, the plan of a random shape took 1.16, 1.07 and 1.12 times the best one's time for 256 x 64, 256 x 128 and
-// 128 x 128 tiles; by these times 1.001 to 1.003.)
+// 128 x 128 tiles; by these times 1.001 to 1.003.)  The times are weighed first and only what is taken is planned.
 bool plan_blocks(const iris_gemm_args& a, Plan* plan) {
-  Plan best;
-  if (make_plan_body(a, &best) != hipSuccess) return false;
-  own_flags(&best);
-  split_last_round(a, &best);
-  double least = block_us(a, best);
-  if (least < 0) return false;  // (K of the caller's tiles shared out, or no such tile)
-  auto blocked = [&](const iris_gemm_args& b, Plan* into, double limit) {
-    double us = -1;
-    for (int width = 256; width >= 128; width /= 2) {
-      const int mm = 256 / b.block_m, mn = width / b.block_n;
-      Plan merged;
-      if (mn < 1 || mm * mn == 1 || !plan_merged(b, mm, mn, &merged)) continue;
-      // (a launch on fewer programs than CUs leaves room for others: none of its own stays idle for a larger block)
-      if (b.num_sms < current_cu_count() && (int64_t)merged.k.total_tiles * merged.k.split_k * 8 < (int64_t)b.num_sms * 7) continue;
-      const double t = block_us(b, merged);
-      if (t > 0 && t < (us < 0 ? limit : us)) us = t, *into = merged;
-    }
-    return us;
+  if (a.ab_dtype == IRIS_DTYPE_F32) return false;
+  const int cus = current_cu_count();
+  const BlockLaunch own = block_launch(a, a.block_m, a.block_n, true, cus);
+  const double own_us = block_us(a, own, cus);
+  if (own_us < 0) return false;  // (K of the caller's tiles shared out, or no such tile)
+  auto blocks = [&](const iris_gemm_args& b, int width) { return block_launch(b, 256, width, false, cus); };
+  auto blocks_us = [&](const iris_gemm_args& b, int width) {
+    const int mm = 256 / b.block_m, mn = width / b.block_n;
+    if (mn < 1 || mm * mn == 1) return -1.0;
+    const BlockLaunch l = blocks(b, width);
+    // (a launch on fewer programs than CUs leaves room for others: none of its own stays idle for a larger block)
+    if (b.num_sms < cus && l.tiles * l.split * 8 < (int64_t)b.num_sms * 7) return -1.0;
+    return block_us(b, l, cus);
   };
+  struct Candidate {
+    double us;
+    int width;       // of the blocks; 0: the caller's tiles
+    int64_t main_n;  // columns of tiles in blocks, the others apart
+  };
+  const int64_t tiles_n = ((int64_t)a.N + a.block_n - 1) / a.block_n;
   // (what is as good by the estimate is better off in larger blocks: [8192,4096] x [4096,384] in 256 x 64 tiles 33.2 us, in
   // 256 x 128 with K in two 32.1)
-  const double us = blocked(a, &best, best.last_round ? least : least * 1.04);
-  if (us > 0) least = us;
+  Candidate list[5] = {{own.last_parts > 0 ? own_us : own_us * 1.04, 0, tiles_n}};
+  int count = 1;
+  for (int width = 256; width >= 128; width /= 2) {
+    const double us = blocks_us(a, width);
+    if (us > 0) list[count++] = {us, width, tiles_n};
+  }
   // The columns of tiles may be one or a few too many for blocks that fill the programs: [8192,36864] x [36864,576] is nine
   // columns of 256 x 64 tiles, eight of which make 128 blocks with K in two parts.  (For a K that can be shared out.)
-  const int64_t tiles_n = a.N / a.block_n;
   const bool two_kernels = a.epilogue == IRIS_EPI_ONE_SHOT && a.phase != IRIS_PHASE_PRODUCE;
   if (a.N % a.block_n == 0 && a.K >= 4096 && a.partials && a.locks && !two_kernels) {
     for (int width = 256; width >= 128; width /= 2) {
@@ -950,25 +990,40 @@ bool plan_blocks(const iris_gemm_args& a, Plan* plan) {
       const int64_t main_n = tiles_n / mn * mn, rest_n = tiles_n - main_n;
       if (main_n == 0 || rest_n == 0 || rest_n * 4 > main_n) continue;
       const iris_gemm_args am = column_range(a, 0, main_n * a.block_n);
-      const iris_gemm_args ar = column_range(a, main_n * a.block_n, rest_n * a.block_n);
-      Plan first;
-      auto rest = std::make_shared<Plan>();
-      const double main_us = blocked(am, &first, least);
-      // (the remaining columns as the caller's tiles; their flags sit at their place in the caller's grid)
-      if (main_us < 0 || !plan_merged(ar, 1, 1, rest.get())) continue;
+      const double wide_us = blocks_us(am, 256), half_us = blocks_us(am, 128);
+      if (wide_us < 0 && half_us < 0) continue;
+      const bool half = wide_us < 0 || (half_us > 0 && half_us < wide_us);
       // K of the rest shared out so far that A streams through again: at 5.2 MB a us
-      const double rest_us = 12 + ((double)ar.M + ar.N) * ar.K * 2e-6 / 5.2;
-      if (main_us + rest_us >= least) continue;
-      least = main_us + rest_us;
-      best = first;
-      best.k.flag_num_pid_n = (int)tiles_n;
-      rest->k.flag_num_pid_n = (int)tiles_n;
-      rest->k.flag_pn_base = (int)main_n;
-      best.rest = rest;
+      const double rest_us = 12 + ((double)a.M + (double)rest_n * a.block_n) * a.K * 2e-6 / 5.2;
+      list[count++] = {(half ? half_us : wide_us) + rest_us, half ? 128 : 256, main_n};
     }
   }
-  *plan = best;
-  return true;
+  // the least of them that there is a kernel for
+  for (;;) {
+    Candidate* c = &list[0];
+    for (int i = 1; i < count; ++i)
+      if (list[i].us < c->us) c = &list[i];
+    if (c->width == 0) break;
+    const iris_gemm_args am = c->main_n < tiles_n ? column_range(a, 0, c->main_n * a.block_n) : a;
+    Plan blocked;
+    if (plan_merged(am, 256 / a.block_m, c->width / a.block_n, &blocked) && as_expected(blocks(am, c->width), blocked)) {
+      // (the remaining columns as the caller's tiles; their flags sit at their place in the caller's grid)
+      bool found = true;
+      if (c->main_n < tiles_n) {
+        const iris_gemm_args ar = column_range(a, c->main_n * a.block_n, (tiles_n - c->main_n) * a.block_n);
+        blocked.rest = std::make_shared<Plan>();
+        found = plan_merged(ar, 1, 1, blocked.rest.get());
+        blocked.k.flag_num_pid_n = blocked.rest->k.flag_num_pid_n = (int)tiles_n;
+        blocked.rest->k.flag_pn_base = (int)c->main_n;
+      }
+      if (found) {
+        *plan = std::move(blocked);
+        return true;
+      }
+    }
+    c->us = 1e30;
+  }
+  return false;
 }
 
 hipError_t make_plan_units(const iris_gemm_args& a, Plan* plan) {

@@ -10,7 +10,7 @@ from iris_amd import _native, ops
 BF16, F32 = 2, 0
 
 
-def plan(M, N, K, BM, BN, dtype=BF16, ws=1, base=1 << 32, row=None, **kw):
+def plan_args(M, N, K, BM, BN, dtype=BF16, ws=1, base=1 << 32, row=None, **kw):
     args = _native.GemmArgs()
     args.a, args.b, args.c_global = base, 2 << 32, 4 << 32
     args.tile_completed, args.heap_bases = 5 << 32, 6 << 32
@@ -24,7 +24,11 @@ def plan(M, N, K, BM, BN, dtype=BF16, ws=1, base=1 << 32, row=None, **kw):
     args.epilogue, args.notify = ops.EPI_ALL_SCATTER, 1
     for name, value in kw.items():
         setattr(args, name, value)
-    lib = _native.lib()
+    return args
+
+
+def plan(*args, **kw):
+    args, lib = plan_args(*args, **kw), _native.lib()
     name, parts = ctypes.create_string_buffer(256), ctypes.c_int(0)
     assert lib.iris_gemm_plan_name(ctypes.byref(args), name, 256) == 0
     assert lib.iris_gemm_split_k(ctypes.byref(args), ctypes.byref(parts)) == 0
