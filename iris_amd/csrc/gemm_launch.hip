@@ -869,17 +869,19 @@ bool reduce_in_program(const iris_gemm_args& a, const Plan& producer) {
 // Times of a launch in large tiles, by which plan_blocks compares its plans: us = fixed + rounds of tiles * (tile + K-steps
 // of a part * step), a step being dearer by `cover` when every CU takes one (the board's power, the L2s), by `off_lines`
 // where rows do not start on cache lines, by `streamed` where the operands come from HBM (none of it up to 50 MB, all from
-// 150 MB on: a program has other data in the 256 MB of the last-level cache between two launches).  Fitted to 22000 timings
-// of 3750 random shapes ([500 .. 8192, 256 .. 36864] x [.., 400 .. 8192], operands changed from launch to launch): rms 6 %.
+// 150 MB on: a program has other data in the 256 MB of the last-level cache between two launches).  Fitted to two thirds of
+// 7000 random calls ([256 .. 8192, 128 .. 36864] x [.., 128 .. 8192], weights in rows of either direction and at any alignment,
+// up to eight copies of the output, operands changed from launch to launch); on the other third the error is 7.4 % rms.
+// (128 x 64 from an earlier fit.)
 struct BlockTime {
   int cm, cn, split;
   double fixed, tile, step, cover, off_lines, streamed;
 };
 constexpr BlockTime BLOCK_TIMES[] = {
-    {128, 64, 1, 4.4, 2.0, 0.249, 0.03, 0.45, 0.45},  {128, 128, 1, 4.4, 2.3, 0.384, 0.00, 0.35, 0.35},
-    {256, 64, 1, 4.6, 2.2, 0.443, 0.00, 0.44, 0.32},  {256, 128, 1, 3.7, 3.5, 0.511, 0.25, 0.34, 0.34},
-    {256, 128, 2, 9.2, 4.5, 0.693, 0.00, 0.40, 0.31}, {256, 256, 1, 2.6, 5.2, 0.899, 0.32, 0.22, 0.31},
-    {256, 256, 2, 10.6, 6.4, 0.719, 0.78, 0.23, 0.26},
+    {128, 64, 1, 4.4, 2.0, 0.249, 0.03, 0.45, 0.45},  {128, 128, 1, 4.1, 2.3, 0.375, 0.12, 0.26, 0.33},
+    {256, 64, 1, 4.0, 2.2, 0.464, 0.00, 0.39, 0.41},  {256, 128, 1, 3.7, 4.1, 0.634, 0.07, 0.29, 0.22},
+    {256, 128, 2, 8.9, 4.6, 0.505, 0.31, 0.36, 0.34}, {256, 256, 1, 2.9, 5.5, 0.999, 0.23, 0.20, 0.20},
+    {256, 256, 2, 9.4, 4.9, 0.977, 0.37, 0.17, 0.21},
 };
 // A launch in tiles of cm x cn as plan_split and split_last_round make it, before there is a plan of it: K in `split` parts, or
 // the last `last_tiles` tiles in `last_parts`.  (The plan is asked whether that is what it is: as_expected.)
@@ -924,33 +926,59 @@ double block_us(const iris_gemm_args& a, const BlockLaunch& l, int cus) {
   double streamed = (((double)a.M + a.N) * a.K * 2e-6 - 50) / 100;
   streamed = streamed < 0 ? 0 : streamed > 1 ? 1 : streamed;
   const int nk = (a.K + 63) / 64;
+  const bool along = a.stride_ak == 1 && a.stride_bk == 1;
+  const bool loose = along && ((a.K | a.stride_am | a.stride_bn) % 8 != 0 || !aligned16(a.a) || !aligned16(a.b));
   const bool scatter = a.epilogue == IRIS_EPI_ALL_SCATTER, wide = (scatter ? a.c_global_dtype : a.c_dtype) == IRIS_DTYPE_F32;
   for (const BlockTime& t : BLOCK_TIMES) {
     if (t.cm != l.cm || t.cn != l.cn || t.split != l.split) continue;
     const int64_t items = l.tiles * t.split, rounds = (items + a.num_sms - 1) / a.num_sms;
     const double busy = (double)(rounds > 1 ? a.num_sms : items) / cus;
-    const double step = t.step * (1 + t.cover * busy) * (lines ? 1.0 : 1 + t.off_lines) * (1 + t.streamed * streamed);
-    // (the other copies of the output, or its wider elements: 6.5 TB/s of stores on all CUs)
-    const double copies = (scatter ? a.world_size : 1) * (wide ? 2 : 1);
-    const double tile = t.tile + (copies - 1) * t.cm * t.cn * 2 / 25400.0 / t.split;
-    const double us = t.fixed + rounds * (tile + (nk + t.split - 1) / t.split * step);
+    const double step = t.step * (1 + t.cover * busy) * (lines ? 1.0 : 1 + t.off_lines) * (1 + t.streamed * streamed) * (loose ? 1.23 : 1.0);
+    // (the other copies of the output, or its wider elements: 6.5 TB/s of stores on all CUs, a third of them hidden behind the
+    // next round's products)
+    const double copies = (scatter ? a.world_size : 1) * (wide ? 2 : 1), store = (copies - 1) * t.cm * t.cn * 2 / 25400.0 / t.split;
+    const double us = t.fixed + rounds * (t.tile + (nk + t.split - 1) / t.split * step) +
+                      store * (busy > 0.37 ? busy : 0.37) * (1 + (rounds - 1) * 0.67);
     if (l.last_parts == 0) return us;
-    // The tiles of a last round that are shared out over all programs, as a launch of their own, whose programs share less of
-    // what they fetch.  ([8192,36864] x [36864,576] in 256 x 64 tiles, 256 and then 32 in eight parts, 565 us, 717 in two
-    // rounds; [2624,26328] x [26328,1520], 256 and 8 in twelve parts, 352)
-    const double apart = 1 + l.last_tiles / (t.cm * t.cn >= 256 * 128 ? 256.0 : 32.0);
-    return us + 8 + tile + (nk + l.last_parts - 1) / l.last_parts * step * apart;
+    // the tiles of a last round that are shared out over all programs, as a launch of their own
+    return us + 17.7 + t.tile + store * 0.37 + (nk + l.last_parts - 1) / l.last_parts * step;
   }
   return -1;
 }
 
-// A large launch in the caller's tiles or in blocks of them, as 256 x 128 or 256 x 256 tiles, whichever is expected to
-// finish first; K shared by two programs a block where half of them suffice for the blocks and the caller's workspace has
-// the slots; or the columns of tiles that block well first and the rest as a launch of their own.  (us, [8192,K] x [K,N] in
-// 256 x 64 tiles, the caller's / 256 x 128 / 256 x 256: N 576, K 1024 23 / 16 / 24; N 704, K 4128 98 / 53 / -; N 1152, K 12288
-// 337 / 299 / 263; N 1344, K 4096 100 / 100 / 82.  By number of tiles alone, blocks only where they gave seven programs in
-// eight a tile, the plan of a random shape took 1.16, 1.07 and 1.12 times the best one's time for 256 x 64, 256 x 128 and
-// 128 x 128 tiles; by these times 1.001 to 1.003.)  The times are weighed first and only what is taken is planned.
+// Columns of the blocks (256 rows high) that a large launch is run in by number of tiles alone, 0 for the caller's tiles: blocks
+// that give seven programs in eight one, by rounds of them and a tile's time (a 256 x 256 tile does twice the work at 1.25
+// times the rate), or every other one with K in two.
+int blocks_by_count(const iris_gemm_args& a, int64_t tiles_n) {
+  const int64_t rows = ((int64_t)a.M + 255) / 256;
+  const int mm = 256 / a.block_m;
+  double best = 0;
+  int found = 0;
+  for (int width = 256; width >= 128; width /= 2) {
+    const int mn = width / a.block_n;
+    const int64_t tiles = rows * ((tiles_n + mn - 1) / mn);
+    if (mm * mn == 1 || tiles * 8 < (int64_t)a.num_sms * 7) continue;
+    const double cost = (double)((tiles + a.num_sms - 1) / a.num_sms) * (width == 256 ? 1.6 : 1.0);
+    if (!found || cost < best) best = cost, found = width;
+  }
+  if (found || !a.partials || !a.locks || a.K < 4096) return found;
+  for (int width = 256; width >= 128; width /= 2) {
+    const int mn = width / a.block_n;
+    const int64_t tiles = rows * ((tiles_n + mn - 1) / mn);
+    if (mm * mn > 1 && tiles * 2 <= a.num_sms && tiles * 16 >= (int64_t)a.num_sms * 7 && a.partials_slot_elems * 2 >= (int64_t)256 * width)
+      return width;
+  }
+  return 0;
+}
+
+// A large launch in the caller's tiles or in blocks of them, as 256 x 128 or 256 x 256 tiles; K shared by two programs a block
+// where half of them suffice for the blocks and the caller's workspace has the slots; or the columns of tiles that block well
+// first and the rest as a launch of their own.  What blocks_by_count says, unless another is expected to be faster by more than
+// 5 % (2 % where it says the caller's tiles): the times above are not good for less.  (us, [8192,K] x [K,N] in 256 x 64 tiles, the caller's / 256 x 128 / 256 x
+// 256: N 576, K 1024 23 / 16 / 24; N 704, K 4128 98 / 53 / -; N 1152, K 12288 337 / 299 / 263; N 1344, K 4096 100 / 100 / 82.
+// 6000 random calls, on average over the fastest plan timed: by count alone 9 % for a weight along K and 14 to 17 % for others, so
+// 0.3 %; slower than by count by more than 3 %: 79 by the times alone, 45 so.)  The plans are weighed first, and only the one that
+// is taken is made.
 bool plan_blocks(const iris_gemm_args& a, Plan* plan) {
   if (a.ab_dtype == IRIS_DTYPE_F32) return false;
   const int cus = current_cu_count();
@@ -972,13 +1000,13 @@ bool plan_blocks(const iris_gemm_args& a, Plan* plan) {
     int64_t main_n;  // columns of tiles in blocks, the others apart
   };
   const int64_t tiles_n = ((int64_t)a.N + a.block_n - 1) / a.block_n;
-  // (what is as good by the estimate is better off in larger blocks: [8192,4096] x [4096,384] in 256 x 64 tiles 33.2 us, in
-  // 256 x 128 with K in two 32.1)
-  Candidate list[5] = {{own.last_parts > 0 ? own_us : own_us * 1.04, 0, tiles_n}};
-  int count = 1;
+  Candidate list[5] = {{own_us, 0, tiles_n}};
+  int count = 1, by_count = blocks_by_count(a, tiles_n), first = 0;
   for (int width = 256; width >= 128; width /= 2) {
     const double us = blocks_us(a, width);
-    if (us > 0) list[count++] = {us, width, tiles_n};
+    if (us <= 0) continue;
+    if (width == by_count) first = count;
+    list[count++] = {us, width, tiles_n};
   }
   // The columns of tiles may be one or a few too many for blocks that fill the programs: [8192,36864] x [36864,576] is nine
   // columns of 256 x 64 tiles, eight of which make 128 blocks with K in two parts.  (For a K that can be shared out.)
@@ -993,11 +1021,17 @@ bool plan_blocks(const iris_gemm_args& a, Plan* plan) {
       const double wide_us = blocks_us(am, 256), half_us = blocks_us(am, 128);
       if (wide_us < 0 && half_us < 0) continue;
       const bool half = wide_us < 0 || (half_us > 0 && half_us < wide_us);
-      // K of the rest shared out so far that A streams through again: at 5.2 MB a us
-      const double rest_us = 12 + ((double)a.M + (double)rest_n * a.block_n) * a.K * 2e-6 / 5.2;
+      // K of the rest shared out so far that A streams through again
+      const double rest_us = 12.8 + ((double)a.M + (double)rest_n * a.block_n) * a.K * 2e-6 / 3.3;
+      if (by_count == 0 && first == 0 && blocks_by_count(am, main_n) > 0) first = count;
       list[count++] = {(half ? half_us : wide_us) + rest_us, half ? 128 : 256, main_n};
     }
   }
+  // (blocks that share K are a plan like the others)
+  if (first == 0)
+    list[0].us *= 0.98;
+  else if (list[first].main_n < tiles_n || blocks(a, by_count).split == 1)
+    list[first].us *= 0.95;
   // the least of them that there is a kernel for
   for (;;) {
     Candidate* c = &list[0];
