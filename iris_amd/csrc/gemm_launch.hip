@@ -843,6 +843,12 @@ bool reduce_in_program(const iris_gemm_args& a, const Plan& producer) {
   // (few rows off the 16 bytes: [16,133] x [133,4096] of 8 bf16 partials 12.0 / 13.2, K 389 12.9 / 13.2, 637 14.7 / 13.2)
   if (loose && producer.skinny && tiles <= a.num_sms && k.vec_out && inside <= 64 * 64 && a.block_n <= 64 && steps <= 7)
     return true;
+  // (parts of those, for what is behind them: row-major [3587,K] x [K,448] in 256 x 64 tiles of 4, K 128 15.2 / 17.1, fp32 19.2 / 21.5, 256
+  // 18.1 / 18.0, fp32 21.3 / 22.4, 384 20.8 / 19.0; of 8, bf16, K 128 19.7 / 18.6)
+  const bool wide = a.c_dtype == IRIS_DTYPE_F32;
+  if ((rows || loose) && producer.parts && tiles <= a.num_sms && k.vec_out && a.block_m * a.block_n <= 128 * 128 && steps <= 4 &&
+      strips < (wide ? (256 << 10) + 1 : 256 << 10))
+    return true;
   if ((producer.skinny && producer.skinny_cb == 1) || producer.last_round || producer.rest || producer.parts) return false;
   // (cells: the caller's tiles inside, when they are as small as the parts they would be run in)
   if (producer.skinny && a.block_m * a.block_n > 64 * 64) return false;
@@ -854,12 +860,13 @@ bool reduce_in_program(const iris_gemm_args& a, const Plan& producer) {
   // along K off the 16 bytes, 128 x 128 tiles of 2, K 709 24.2 / 27.7, 1285 34.8 / 31.7; 256 x 64 [4096,1024] of 8, K 1501 48.7 / 43.6.)
   if (rows || loose) {
     const int area = a.block_m * a.block_n;
-    // (along K off the 16 bytes, a short shard: 128 x 128 tiles [2048,2048] of 8, bf16, K 129 27.0 / 28.5, 385 30.5 / 30.9, of 8,
-    // fp32, 37.2 / 40.2, 41.0 / 42.7, of 4, fp32, 26.2 / 32.2, 29.7 / 34.5, 641 33.3 / 37.1; 256 x 128 tiles, fp32, [1534,3008] of 4, 144 tiles, 34 / 42,
-    // 41 / 46.5, [4096,2048], 256 tiles, 46.5 / 46.0, 54 / 50.4; bf16 there as the line below)
-    const bool wide = a.c_dtype == IRIS_DTYPE_F32;
-    if (loose && steps <= (!wide ? 6 : strips > (256 << 10) ? 7 : 12) && strips <= (512 << 10) && area <= 128 * 128) return true;
-    if (loose && steps <= 7 && wide && area <= 256 * 128 && tiles * 4 <= (int64_t)a.num_sms * 3) return true;
+    // (a short shard, inside / behind: along K off the 16 bytes, 128 x 128 tiles [2048,2048] of 8, bf16, K 129 27.0 / 28.5, 385 30.5 /
+    // 30.9, of 8, fp32, 37.2 / 40.2, 41.0 / 42.7, of 4, fp32, 26.2 / 32.2, 29.7 / 34.5, 641 33.3 / 37.1; row-major, of 8, bf16, K 128 25.5 /
+    // 27.3, 384 29.5 / 28.9, of 4, fp32, 24.4 / 31.0, 512 30.3 / 33.7; 256 x 128 tiles, fp32, 144 tiles of 4, 34 / 42, 41 / 46.5, 256 tiles
+    // 46.5 / 46.0, 54 / 50.4; bf16 there, and 256 x 64 tiles [2580,185] x [185,1000] of 8 29.1 / 24.3, as the line below)
+    const int few = loose ? (!wide ? 6 : strips > (256 << 10) ? 7 : 12) : strips > (256 << 10) ? (wide ? 4 : 0) : wide ? 8 : 4;
+    if (steps <= few && strips <= (512 << 10) && area <= 128 * 128 && a.block_m <= 128) return true;
+    if (steps <= (loose ? 7 : 8) && wide && area > 128 * 128 && area <= 256 * 128 && tiles * 4 <= (int64_t)a.num_sms * 3) return true;
     const int most = area > 128 * 128 ? 4 : area > 64 * 64 ? (rows ? 8 : 12) : rows ? (producer.skinny ? 7 : 16) : 24;
     return steps <= most && (area <= 64 * 64 || strips < (256 << 10));
   }

@@ -55,13 +55,19 @@ def test_small_products(M, N, K, BM, BN, rows, want):
 
 
 @pytest.mark.parametrize("M,N,K,BM,BN,ws,partial,inside", [
-    (2643, 1536, 257, 128, 128, 4, F32, True), (2643, 1536, 641, 128, 128, 8, F32, False),
+    # a row-major B (K a multiple of eight)
+    (2048, 2048, 128, 128, 128, 8, 2, True), (2048, 2048, 384, 128, 128, 8, 2, False), (2048, 2048, 512, 128, 128, 4, F32, True),
+    (704, 7616, 128, 256, 128, 4, F32, True), (704, 7616, 128, 256, 128, 4, 2, False), (4096, 2048, 256, 256, 128, 4, F32, False),
+    (3587, 448, 128, 256, 64, 4, 2, True), (3587, 448, 384, 256, 64, 4, 2, False), (3587, 448, 128, 256, 64, 8, 2, False),
+    # off the 16 bytes
+    (2580, 1000, 185, 256, 64, 8, 2, False), (2643, 1536, 257, 128, 128, 4, F32, True), (2643, 1536, 641, 128, 128, 8, F32, False),
     (2048, 2048, 321, 128, 128, 8, 2, True), (2048, 2048, 641, 128, 128, 8, 2, False),
     (2048, 2048, 641, 128, 128, 4, F32, True), (2048, 2048, 385, 128, 128, 8, F32, True),
     (1534, 3008, 321, 256, 128, 4, F32, True), (1534, 3008, 321, 256, 128, 4, 2, False), (4096, 2048, 321, 256, 128, 4, F32, False),
     (948, 7104, 193, 256, 256, 4, 2, False), (18, 6144, 129, 256, 64, 4, 2, True),
 ])
 def test_reduce_inside_the_program_or_behind_it(M, N, K, BM, BN, ws, partial, inside):
+    kw = ROWS(N) if K % 8 == 0 else {}
     name, _ = plan(M, N, K, BM, BN, ws=ws, epilogue=ops.EPI_ONE_SHOT, phase=ops.PHASE_FUSED, c=9 << 32, c_dtype=partial, stride_cm=N,
-                   stride_cn=1, stride_cm_global=N)
+                   stride_cn=1, stride_cm_global=N, **kw)
     assert name.endswith("+kernel+reduce") != inside, name
