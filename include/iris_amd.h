@@ -266,7 +266,9 @@ int iris_gemm_split_k(const iris_gemm_args* args, int* split_k);
  * no GEMM work): a tuning variant's name, that of a tile behind the table
  * ("..._rows": a row-major B; "..._gather_dma": operands along K at any alignment;
  * "..._gather": operands that lie across K otherwise, or fp32 at any alignment; fp32 tiles for a
- * longer K), or "few_rows_16xN" / "few_rows_32xN" / "cells_32x32", also with "_gather_dma" and (cells) "_rows", followed by "+stream_k", "+reduce" (the in-program reduce) or "+two_per_cu"
+ * longer K), or "few_rows_16xN" / "few_rows_32xN" / "cells_32x32", also with
+ * "_gather_dma" and (cells) "_rows" ("cells_16x32_rows" for up to 16 rows of A),
+ * followed by "+stream_k", "+reduce" (the in-program reduce) or "+two_per_cu"
  * (two programs a CU), and by "+two_tiles_each" / "+four_tiles_each" /
  * "+eight_tiles_each" where the launch computes a block of that many of the
  * caller's tiles as one (each tile keeps its own id and flag), and by

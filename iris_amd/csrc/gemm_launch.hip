@@ -277,11 +277,11 @@ bool plan_cells(const iris_gemm_args& a, int op, bool dma_ok, bool loose, bool b
   k.div_xcd = make_fast_div((uint32_t)a.num_xcds, (uint64_t)k.xcd_per * a.num_xcds + 1);
   plan->loose = loose;
   plan->b_rows = b_rows;
-  plan->skinny_lds = cells_lds_bytes();
+  plan->skinny_lds = cells_lds_bytes(rb);
   plan->skinny_grid = k.xcd_per * a.num_xcds;
   plan->skinny_grid_y = 1;
   plan->skinny_grid_z = parts;
-  plan->skinny_rb = 2;
+  plan->skinny_rb = rb;
   plan->skinny_cb = 2;
   k.split_k = 1;
   k.locks = a.locks;
@@ -1615,7 +1615,7 @@ extern "C" int iris_gemm_plan_name(const iris_gemm_args* args, char* buf, size_t
   Plan plan;
   hipError_t err = make_plan(*args, &plan);
   if (err != hipSuccess) return err;
-  const char* few = plan.skinny_cb == 2 ? "cells_32x32" : plan.skinny_rb == 2 ? "few_rows_32xN" : "few_rows_16xN";
+  const char* few = plan.skinny_cb == 2 ? (plan.skinny_rb == 2 ? "cells_32x32" : "cells_16x32") : plan.skinny_rb == 2 ? "few_rows_32xN" : "few_rows_16xN";
   std::snprintf(buf, len, "%s%s%s%s", plan.skinny ? few : plan.entry ? plan.entry->name : "", plan.loose ? "_gather_dma" : plan.b_rows ? "_rows" : "",
                 plan.entry && plan.k.stream_k                   ? "+stream_k"
                 : plan.entry && plan.in_program                 ? "+reduce"

@@ -72,13 +72,13 @@ constexpr int skinny_lds_bytes(int rb) { return skinny_a_bytes(rb) + SKINNY_WAVE
 // leaves in 16-byte stores.  The cells are dealt to the XCDs in consecutive runs (the shorter direction first), so that
 // each XCD's L2 fetches its share of the longer operand once.
 constexpr int CELL = 32;
-// LDS of a workgroup of RB x CB blocks
-constexpr int cells_lds_bytes() { return SKINNY_WAVES * SKINNY_UN * 4 * SKINNY_BLOCK_BYTES; }
+// LDS of a workgroup of RB x 2 blocks
+constexpr int cells_lds_bytes(int rb) { return SKINNY_WAVES * SKINNY_UN * (rb + 2) * SKINNY_BLOCK_BYTES; }
 
 // AROWS: rows of A in a block, 8 or 16.
 // RB: blocks of 16 rows a workgroup computes (1 for up to 32 rows; 2 up to 64
 // rows of a long K, and from 17 rows on where B is large).
-// CB: blocks of 16 columns, 1 or (with RB 2) 2.
+// CB: blocks of 16 columns, 1 or (cells: with RB 2, or a row-major B) 2.
 // LOOSE: operands along K at any alignment and of any K from eight on (see Loader in gemm_kernel.hpp): a chunk that K cuts is
 // fetched moved back to end there, and what it repeats is cleared in the fragments.  (us a pass, by the gathering tiles / so:
 // [1,8229] x [8229,3816] 29.0 / 15.5, [15,2293] x [2293,1344] 17.0 / 9.8, [2,29690] x [29690,336] 22.3 / 11.8, [25,137] x

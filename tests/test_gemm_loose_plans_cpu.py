@@ -42,8 +42,8 @@ def test_cells_that_share_k(M, N, K, BM, BN, cells):
     (73, 5824, 9281, 128, 128, False, ("128x128x64_w2x2_s4_f4_gather_dma", 5)),
     (569, 960, 3873, 256, 256, False, ("64x64x128_w2x2_s4_f4_gather_dma+parts_of_tiles", 1)),
     # cells with up to 16 rows of A
-    (5, 2432, 9536, 256, 256, True, ("cells_32x32_rows", 1)),
-    (2, 5696, 3840, 256, 128, True, ("cells_32x32_rows", 1)),
+    (5, 2432, 9536, 256, 256, True, ("cells_16x32_rows", 1)),
+    (2, 5696, 3840, 256, 128, True, ("cells_16x32_rows", 1)),
     (28, 4864, 7936, 64, 64, True, ("64x64x128_w2x2_s4_f4_rows", 3)),
     # a tile that is no more than half padding
     (4705, 128, 14912, 256, 256, True, ("256x128x64_w2x2_s3_f4_rows", 13)),

@@ -40,7 +40,8 @@ PARTS = "64x64x128_w2x2_s4_f4+parts_of_tiles"
 
 @pytest.mark.parametrize("M,N,K,BM,BN,want", [
     # a row-major weight: cells up to a K whose half lines no longer come in time, and for what 32 rows of them share
-    (1, 1376, 4096, 64, 64, ("cells_32x32_rows", 1)),
+    (1, 1376, 4096, 64, 64, ("cells_16x32_rows", 1)),
+    (16, 1376, 4096, 64, 64, ("cells_16x32_rows", 1)), (17, 1376, 4096, 64, 64, ("cells_32x32_rows", 1)),
     (27, 256, 28032, 256, 64, ("cells_32x32_rows", 1)),
     (128, 1376, 4096, 64, 64, ("cells_32x32_rows", 1)),
     (28, 4864, 7936, 64, 64, ("64x64x128_w2x2_s4_f4_rows", 3)),
