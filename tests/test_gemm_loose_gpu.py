@@ -196,13 +196,14 @@ def test_few_rows_and_cells(shmem, M, N, K, BM, BN, pad, shift, kernel, dtype, o
         assert flags.cpu().tolist() == [launch] * total + [0] and not locks.any()
 
 
-@pytest.mark.parametrize("M,N,K", [(5, 70, 1031), (70, 130, 517)])
-def test_fp32_few_rows(shmem, M, N, K):
+@pytest.mark.parametrize("M,N,K,name", [(5, 70, 1031, "few_rows_16xN_gather_dma"), (70, 130, 517, "few_rows_32xN_gather_dma")])
+def test_fp32_few_rows(shmem, M, N, K, name):
     A, B, a, b = operands(shmem, M, N, K, F32, 1, 1)
     cg = shmem.zeros((M, N), dtype=F32)
     flags = shmem.zeros((16,), dtype=torch.int32)
     locks = shmem.zeros((256,), dtype=torch.int32)
     args = (a, b, None, cg, flags, None, 0, 1, 256, 64, 64, 64, 2, ops.EPI_ALL_SCATTER)
+    assert ops.gemm_plan_name(*args, locks=locks, num_xcds=8) == name
     ops.gemm_launch(*args, locks=locks, num_xcds=8)
     torch.cuda.synchronize()
     check_close(cg, O.shard_gemm(A, B, F32), "fp32", block_rtol=1e-5)
