@@ -982,11 +982,11 @@ int blocks_by_count(const iris_gemm_args& a, int64_t tiles_n) {
 // where half of them suffice for the blocks and the caller's workspace has the slots; or the columns of tiles that block well
 // first and the rest as a launch of their own.  What blocks_by_count says, unless another is expected to be faster by more than
 // 5 % (2 % where it says the caller's tiles): the times above are not good for less, nor for as much on fewer programs than CUs,
-// which they were not taken on, so 8 % there.  (us, [8192,K] x [K,N] in 256 x 64 tiles, the caller's / 256 x 128 / 256 x 256: N 576,
+// which they were not taken on, so 10 % there.  (us, [8192,K] x [K,N] in 256 x 64 tiles, the caller's / 256 x 128 / 256 x 256: N 576,
 // K 1024 23 / 16 / 24; N 704, K 4128 98 / 53 / -; N 1152, K 12288 337 / 299 / 263; N 1344, K 4096 100 / 100 / 82.  6000 random calls,
 // on average over the fastest plan timed: by count alone 9 % for a weight along K and 14 to 17 % for others, so 0.3 %; slower than
 // by count by more than 3 %: 79 by the times alone, 45 so.  2000 calls on 16 to 248 programs, time by count / so 1.012 on average; slower
-// than by count by more than 3 % 10 at 5 %, 5 at 8 %.)  The plans are weighed first, and only the one that is taken is made.
+// than by count by more than 3 % 10 at 5 %, 4 at 10 %.)  The plans are weighed first, and only the one that is taken is made.
 bool plan_blocks(const iris_gemm_args& a, Plan* plan) {
   if (a.ab_dtype == IRIS_DTYPE_F32) return false;
   const int cus = current_cu_count();
@@ -1039,7 +1039,7 @@ bool plan_blocks(const iris_gemm_args& a, Plan* plan) {
   if (first == 0)
     list[0].us *= 0.98;
   else if (list[first].main_n < tiles_n || blocks(a, by_count).split == 1)
-    list[first].us *= a.num_sms < cus ? 0.92 : 0.95;
+    list[first].us *= a.num_sms < cus ? 0.9 : 0.95;
   // the least of them that there is a kernel for
   for (;;) {
     Candidate* c = &list[0];

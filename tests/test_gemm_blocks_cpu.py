@@ -43,4 +43,5 @@ def test_blocks(M, N, K, BM, BN, want):
 def test_fewer_programs_than_cus_leave_none_idle():
     assert plan(1024, 640, 256, 256, 64, num_sms=16) == (HALF + "+two_tiles_each", 1)
     assert plan(1024, 640, 256, 256, 64, ws=2, num_sms=16) == (HALF + "+two_tiles_each", 1)
+    assert plan(640, 392, 200, 128, 128, num_sms=8) == (HALF + "+two_tiles_each", 1)
     assert plan(1024, 640, 256, 256, 64) == ("128x64x64_w2x2_s4_f4+parts_of_tiles", 1)
