@@ -195,8 +195,8 @@ bool plan_few_rows(const iris_gemm_args& a, int op, bool dma_ok, bool loose, Pla
   const bool long_k = a.variant == 0 && !mid && rb == 2 && !f32 &&
                       (cells > cus ? a.K >= 8192 : !lines && a.M > 24 && a.K >= 20480 && b_bytes > (96 << 20));
   // Off the 16 bytes the L1 is the bound earlier, and the tiles no longer gather.  (us a pass, here / there: [9,12977] x
-  // [12977,4352] 52 / 46, [15,19393] x [19393,3392] 45 / 42, [24,449] x [449,5824] 11.6 / 10.5, [23,29889] x [29889,2368] 54 / 45,
-  // [36,26745] x [26745,1376] 42 / 31, fp32 [43,10433] x [10433,3136] 101 / 69, [109,2913] x [2913,7152] 95 / 79; but [1,23937] x
+  // [12977,4352] 46 / 35, [15,20993] x [20993,3392] 49 / 43, [24,449] x [449,5824] 11.3 / 7.1, [23,29889] x [29889,2368] 54 / 43,
+  // [36,26745] x [26745,1376] 42 / 26, fp32 [43,10433] x [10433,3136] 100 / 70, [115,10753] x [10753,6400] 341 / 177; but [1,23937] x
   // [23937,3584] 37 / 46, [24,15489] x [15489,1600] 16.7 / 18.3, [63,27009] x [27009,528] 23 / 29, fp32 [58,17025] x [17025,192] 18 / 20.)
   const bool off = loose && a.variant == 0;
   const bool off_f32 = off && f32 && (mid ? (cells >= 128 && a.K >= 32768) || (cells > cus && a.K >= 8192) || (cells > 4 * cus && a.K >= 1024)
@@ -258,10 +258,11 @@ bool plan_cells(const iris_gemm_args& a, int op, bool dma_ok, bool loose, bool b
   if (!ok) return false;
   int parts = 1;
   // (K of a row-major B is shared out for one row of cells only: [138,32000] x [32000,128] in twelve parts 24.4 us, 18.0 in tiles;
-  // not off the 16 bytes for more than four rows of cells of a long K: [152,29953] x [29953,320] in five 39, in tiles 27,
-  // [209,20041] x [20041,168] 26.6 / 21.9; but [119,17089] x [17089,384] 17.8 / 20.9, [273,16001] x [16001,192] 19.6 / 22.9)
+  // not off the 16 bytes for more than four rows of cells of a long K: [152,29953] x [29953,320] in five 39.5, in tiles 25.1,
+  // [209,20041] x [20041,168] 26.8 / 20.2; but [119,17089] x [17089,384] 17.8 / 20.9, [273,16001] x [16001,192] 19.6 / 22.9)
   const bool far = loose && a.ab_dtype != IRIS_DTYPE_F32 && m_cells > 4 && a.K >= 19000;
   if (a.split_k == 0 && a.partials && aligned16(a.partials) && a.locks && k.total_tiles + cells <= a.num_sms && (m_cells == 1 || !b_rows) && !far) {
+    // (0.6 us for 64 of K of a workgroup, 1.5 times that with a row-major B: its half lines)
     parts = few_rows_parts(cells, (a.K + 63) / 64, b_rows ? 0.9 : 0.6, (int64_t)a.N * a.K * 2);
     if (parts * cells * (CELL * CELL) > (int64_t)a.num_sms * a.partials_slot_elems) parts = 1;
   }
@@ -678,8 +679,8 @@ double cells_us(const iris_gemm_args& a, int64_t cells, int parts, const Operand
   const double mb = ((double)a.M + a.N) * a.K * 2e-6;
   // us for 64 of K, operands in whole lines / not: [512,512] 256 cells 0.090 / 0.13; [128,1376] 172 cells 0.083 / 0.11;
   // [200,512] 112 cells 0.048 / 0.066 as long as the L2s hold the operands, 0.07 / 0.08 beyond
-  // (a row-major B comes in half lines, from HBM at half the rate: [28,7936] x [7936,4864] 33.8, in tiles 23.5; with up to 16
-  // rows of A a cell fetches half of A)
+  // (a row-major B comes in half lines: 1.5 times the L1's time with the 32 rows of A beside it, and from HBM at half the rate;
+  // fitted with both in it.  [28,7936] x [7936,4864] 33.8, in tiles 23.5; with up to 16 rows of A a cell fetches half of A)
   const double lines = o.b_rows ? (a.M <= SKINNY_ROWS ? 1.08 : 1.8) : o.lines ? 1.0 : o.loose ? 2.1 : 1.45;
   const double step = 0.083 * (groups * 5 > cus * 4 ? 1.09 : groups * 2 <= cus && mb <= 30 ? 0.7 : 1.0) *
                       (o.f32 && lines < 1.65 ? 1.65 : lines);
@@ -1221,16 +1222,18 @@ hipError_t make_plan_body(const iris_gemm_args& a, Plan* plan, bool cells) {
   k.a_across = a_across;
   k.b_across = b_across;
   // A row-major B goes through the LDS-DMA too where its rows are whole aligned 16-byte chunks and all of it, K rows, lies
-  // within the 2 GiB window of a descriptor.  (us a pass gathered / so, row-major, operands from HBM: [2048,4096] x
-  // [4096,1376] 43.8 / 32.7, [2697,1936] x [1936,1600] 66.8 / 40.1, [50,2752] x [2752,7040] 27.1 / 16.2, [1232,29704] x
-  // [29704,512] 87.8 / 75.9, [42,320] x [320,3968] 11.8 / 9.4; the same weights along K take within 5 % of the latter.)
+  // within the 2 GiB window of a descriptor.  (us a pass gathered / so / the same weight along K, 256 x 64 tiles:
+  // [2048,4096] x [4096,1376] 81.6 / 34.2 / 34.5, [2697,1936] x [1936,1600] 77.9 / 30.9 / 32.6, [1232,29704] x [29704,512] 129 / 97 /
+  // 87; 64 x 64 [50,2752] x [2752,7040] 26.1 / 16.6 / 16.3; cells [42,320] x [320,3968] 8.7 / 6.2 / 6.1.  21 random calls in tiles take
+  // 0.87 to 1.12 of the time along K, 0.99 on average; 33 in cells 0.93 to 1.5, 1.15 on average, the more the longer K is.)
   const bool rows_ok = !dma_ok && unit == 1 && a.stride_ak == 1 && a.stride_am > 0 && (a.stride_am % 8) == 0 && (a.K % 8) == 0 &&
                        a.stride_bn == 1 && a.stride_bk > 0 && (a.stride_bk % 8) == 0 && (a.N % 8) == 0 && aligned16(a.a) &&
                        aligned16(a.b) && ((int64_t)256 * a.stride_am + a.K) * 2 < ((int64_t)1 << 31) &&
                        ((int64_t)(a.K > 128 ? a.K : 128) * a.stride_bk + 256) * 2 < ((int64_t)1 << 31);
   // Operands along K at any alignment and of any K from eight on: the same tiles, built to take them (LOAD_DMA_LOOSE; us a
-  // pass gathered / so: [1000,1500] x [1500,999] 18.3 / 17.0, [346,1849] x [1849,4544] 49 / 34, [2518,2911] x [2911,4744] 207 /
-  // 155; 50 random calls of a K that is no multiple of eight 1.11x, none slower).  Rows
+  // pass gathered / so / with one k less, aligned: 256 x 64 tiles [2048,4097] x [4097,1376] 60.1 / 42.8 / 34.5, [2871,4865] x
+  // [4865,5952] 409 / 266 / 187, 128 x 128 [3929,1153] x [1153,576] 22.3 / 18.5 / 13.4; 21 random calls in tiles take 1.12 to 1.9 of
+  // the aligned time, 1.3 on average, 37 in cells and few rows 1.07 to 1.4, 1.2 on average).  Rows
   // that overlap stay with the gathering tiles: past the edge, a chunk could straddle the end of the descriptor.
   const bool loose_ok = !dma_ok && a.stride_ak == unit && a.stride_bk == unit && a.K >= 8 && a.stride_am >= a.K &&
                         a.stride_bn >= a.K && ((int64_t)256 * a.stride_am + a.K + 8) * 2 < ((int64_t)1 << 31) &&

@@ -85,8 +85,9 @@ constexpr int cells_lds_bytes(int rb) { return SKINNY_WAVES * SKINNY_UN * (rb + 
 // [137,4864] and its reduce 17.2 / 16.8; 40 random calls of up to 32 rows 1.48x.)
 // BROWS (cells, 16-bit operands): a B whose rows are its k (row-major [K, N]), in whole aligned 16-byte chunks.  A block of B lies
 // in LDS as in memory, 64 k of 32 columns, and is transposed on its way to the MFMAs by ds_read_b64_tr_b16.  A row of 64
-// bytes is half a cache line, so that such a block costs the L1 twice what one along K does.  With up to 16 rows of A, RB is 1
-// ([4,1376] x [1376,4096] 8.0 -> 7.4 us, 27 random calls of 1 to 16 rows 1.08x, same bits; RB 2 fetched as many rows of A again,
+// bytes is half a cache line, so that such a block costs the L1 twice what one along K does, 1.5 times with a cell's 32 rows of
+// A beside it ([95,4224] x [4224,1280] along K 9.7 us, so 12.8: 1.6 times what is above a launch's fixed 4.5).  With up to 16
+// rows of A, RB is 1 ([4,1376] x [1376,4096] 8.0 -> 7.4 us, 27 random calls of 1 to 16 rows 1.08x, same bits; RB 2 fetched as many rows of A again,
 // and for up to eight three times as many, all out of range).
 template <int DT, int OP, int ODT, int AROWS, int RB = 1, int CB = 1, bool LOOSE = false, bool BROWS = false>
 __global__ __launch_bounds__(SKINNY_THREADS) __attribute__((amdgpu_waves_per_eu(2, 8))) void
