@@ -256,14 +256,16 @@ bool plan_cells(const iris_gemm_args& a, int op, bool dma_ok, bool loose, bool b
                   a.block_n % CELL == 0 && !a.mm_begin_timestamp && !a.mm_end_timestamp && (a.split_k == 0 || a.split_k == 1) &&
                   counters && (CELL * a.stride_am + a.K) * 2 < lim && (CELL * a.stride_bn + a.K) * 2 < lim;
   if (!ok) return false;
+  const int xcd_per = (int)((cells + a.num_xcds - 1) / a.num_xcds);
   int parts = 1;
-  // (K of a row-major B is shared out for one row of cells only: [138,32000] x [32000,128] in twelve parts 24.4 us, 18.0 in tiles;
-  // not off the 16 bytes for more than four rows of cells of a long K: [152,29953] x [29953,320] in five 39.5, in tiles 25.1,
-  // [209,20041] x [20041,168] 26.8 / 20.2; but [119,17089] x [17089,384] 17.8 / 20.9, [273,16001] x [16001,192] 19.6 / 22.9)
-  const bool far = loose && a.ab_dtype != IRIS_DTYPE_F32 && m_cells > 4 && a.K >= 19000;
-  if (a.split_k == 0 && a.partials && aligned16(a.partials) && a.locks && k.total_tiles + cells <= a.num_sms && (m_cells == 1 || !b_rows) && !far) {
+  // (K of a row-major B is shared out for one row of cells only: [138,32000] x [32000,128] in twelve parts 24.4 us, 18.0 in tiles)
+  if (a.split_k == 0 && a.partials && aligned16(a.partials) && a.locks && k.total_tiles + cells <= a.num_sms && (m_cells == 1 || !b_rows)) {
+    // An XCD takes xcd_per workgroups of each part: it is those that have to fit its CUs, not all parts' workgroups the device's.
+    // (us a pass with a second round on some XCDs, 35 workgroups on 32 CUs / so: off the 16 bytes [40,18929] x [18929,800] 25.3 /
+    // 18.4, [92,32385] x [32385,384] 33.7 / 25.2, row-major [20,26048] x [26048,576] 21.0 / 15.4, fp32 along K [171,21184] x
+    // [21184,960] 98.7 / 85.4; 137 random calls 1.21x, one slower than before cells took such operands.)
     // (0.6 us for 64 of K of a workgroup, 1.5 times that with a row-major B: its half lines)
-    parts = few_rows_parts(cells, (a.K + 63) / 64, b_rows ? 0.9 : 0.6, (int64_t)a.N * a.K * 2);
+    parts = few_rows_parts(xcd_per * a.num_xcds, (a.K + 63) / 64, b_rows ? 0.9 : 0.6, (int64_t)a.N * a.K * 2);
     if (parts * cells * (CELL * CELL) > (int64_t)a.num_sms * a.partials_slot_elems) parts = 1;
   }
   // (a row-major B with up to 16 rows of A: cells of 16 x 32, which fetch the half or the quarter of A that there is)
@@ -273,7 +275,7 @@ bool plan_cells(const iris_gemm_args& a, int op, bool dma_ok, bool loose, bool b
   k.cells = (int)cells;
   k.cells_by_row = a.M > a.N;
   k.cells_inner = (int)(k.cells_by_row ? n_cells : m_cells);
-  k.xcd_per = (int)((cells + a.num_xcds - 1) / a.num_xcds);
+  k.xcd_per = xcd_per;
   k.div_inner = make_fast_div((uint32_t)k.cells_inner, (uint64_t)cells + 1);
   k.div_xcd = make_fast_div((uint32_t)a.num_xcds, (uint64_t)k.xcd_per * a.num_xcds + 1);
   plan->loose = loose;

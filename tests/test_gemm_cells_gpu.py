@@ -89,3 +89,30 @@ def test_one_shot_and_atomics(shmem, dtype, part):
     check_close(shmem.on_rank(cg, ws - 1), O.one_shot_all_reduce(shards, part, dtype), "reduced")
     check_close(acc, O.shard_gemm(A, B, F32), "atomics")
     assert not locks.any()
+
+
+@pytest.mark.parametrize("M,N,K,dtype,kind,name", [
+    (92, 384, 32385, BF16, "loose", "cells_32x32_gather_dma"),     # 36 cells, five an XCD
+    (40, 800, 18929, F16, "loose", "cells_32x32_gather_dma"),      # 50, seven an XCD
+    (130, 160, 16384, BF16, "", "cells_32x32"),                    # 25
+    (140, 224, 6004, F32, "", "cells_32x32"),                      # 35
+    (27, 1120, 28032, BF16, "rows", "cells_32x32_rows"),           # 35 of a row-major B
+    (5, 576, 36032, BF16, "rows", "cells_16x32_rows"),             # 18
+])
+def test_parts_of_k_fit_the_cus_of_each_xcd(shmem, M, N, K, dtype, kind, name):
+    """A workgroup a CU: the parts of the cells that an XCD takes are all resident at once."""
+    A, B = make_ab(M, N, K, dtype)
+    a, b = place(shmem, A, False, 0, 0), place(shmem, B, False, 0, 0) if kind == "rows" else place(shmem, B.T, False, 0, 0).T
+    cg = shmem.zeros((M, N), dtype=dtype)
+    flags = shmem.zeros((ops.cdiv(M, 64) * ops.cdiv(N, 64),), dtype=torch.int32)
+    P, locks = shmem.full((256, 256 * 64), float("nan"), dtype=F32), shmem.zeros((256,), dtype=torch.int32)
+    args = (a, b, None, cg, flags, shmem.get_heap_bases(), 0, 1, 256, 64, 64, 64, 4, ops.EPI_ALL_SCATTER)
+    kw = dict(partials=P, locks=locks, num_xcds=8)
+    assert ops.gemm_plan_name(*args, **kw) == name
+    ops.gemm_launch(*args, **kw)
+    torch.cuda.synchronize()
+    check_close(cg, O.shard_gemm(A, B, dtype), name)
+    blocks = (1 if "16x32" in name else 2) * 2 * ops.cdiv(M, 32) * ops.cdiv(N, 32)  # of 16 x 16 sums, in register order
+    parts, rest = divmod(int((~P.view(-1, 256).isnan()).any(dim=1).sum()), blocks)
+    assert parts > 1 and rest == 0
+    assert parts * ops.cdiv(ops.cdiv(M, 32) * ops.cdiv(N, 32), 8) <= torch.cuda.get_device_properties(0).multi_processor_count // 8

@@ -26,8 +26,8 @@ def test_few_rows(M, N, K, BM, BN, dtype, few):
 
 
 @pytest.mark.parametrize("M,N,K,BM,BN,cells", [
-    # cells that share K: up to four rows of them, or up to some K
-    (152, 320, 29953, 128, 128, False), (209, 168, 20041, 64, 64, False), (268, 128, 19201, 64, 64, False),
+    # cells that share K
+    (152, 320, 29953, 128, 128, False), (209, 168, 20041, 64, 64, True), (268, 128, 19201, 64, 64, True),
     (119, 384, 17089, 128, 128, True), (66, 128, 32705, 128, 128, True), (273, 192, 16001, 128, 128, True),
 ])
 def test_cells_that_share_k(M, N, K, BM, BN, cells):
