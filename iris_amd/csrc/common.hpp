@@ -242,7 +242,7 @@ __device__ inline __amdgpu_buffer_rsrc_t tile_rsrc(const IRIS_GLOBAL char* base,
 // instruction after its write; nothing else in the kernels that load this way uses it.  dst, rs and at are the wave's.)
 // us a pass, the compiler's loads / these: a K-step of the 256 x 256 tile, whose waves fetch what they multiply, stood still
 // three times, [1816,34048] x [34048,6016] 1196 / 709, [8020,4224] x [4224,1472] 171 / 111, 46 random calls 1.24x; cells had one
-// set in flight for two, [14,4032] x [4032,192] 6.3 / 5.8; tiles with fetching waves waited for the tile before's stores, 1.01x.
+// set in flight for two, [14,4032] x [4032,192] 6.3 / 5.8; tiles with fetching waves waited for the tile before's stores, up to 1.02x.
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
 __device__ __attribute__((always_inline)) inline void lds_dma16(__amdgpu_buffer_rsrc_t rs, IRIS_LDS void* dst, uint32_t off, int at) {

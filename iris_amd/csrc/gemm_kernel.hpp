@@ -224,6 +224,11 @@ struct GemmCfg {
   static constexpr int NW = WM * WN, NT = NW * 64;  // the waves (threads) that multiply and store
   static constexpr int LW = LW_;
   static constexpr int NL = LW ? LW : NW;           // the waves that fetch
+  // The loads of a row-major B's tile by lds_dma16, for a wave that also transposes, and for a prologue behind another tile's
+  // stores.  Of the tiles with fetching waves those of 64 x 128 and 256 x 128 keep the compiler's, whose m0 costs an instruction less
+  // (time with lds_dma16 / with those, 560 random calls, K whole and shared out: 64 x 64 0.976, 0.986, 128 x 128 0.993, 0.987, 128 x 64
+  // 0.998, 256 x 64 0.995, 1.001, 256 x 128 0.999, 1.002 with [2048,4096] x [4096,1376] 1.009, 64 x 128 1.012).
+  static constexpr bool COUNTED_DMA = B_ROWS && (LW == 0 || CN != 128 || CM == 128);
   // TOUCH_: a build of the eight-wave 256 x 256 tile that touches lines of K-steps to come (see Loader::touch)
   static constexpr bool TOUCH = TOUCH_;
   static_assert(!TOUCH_ || (LOAD_ == LOAD_DMA && LW_ == 0 && WM_ * WN_ == 8 && CM_ == 256 && CN_ == 256), "the touching build's tile");
@@ -522,8 +527,10 @@ struct Loader {
         at_k = k * step_kb;
         if (!FULL && k0 + j * Cfg::NL * Cfg::B_RPB + rows_k(wave, lane) >= k_limit) off = 0x80000000u;
       }
-      lds_dma16(isA ? ra : rb, dst, off, at_k);
-      return;
+      if constexpr (Cfg::COUNTED_DMA) {
+        lds_dma16(isA ? ra : rb, dst, off, at_k);
+        return;
+      }
     }
     __builtin_amdgcn_raw_ptr_buffer_load_lds(isA ? ra : rb, (IRIS_LDS void*)dst, 16, off, at_k, 0, 0);
   }
