@@ -92,8 +92,10 @@ int iris_hip_arch_name(int device, char* buf, size_t len);
                               * peers).  In one program and tile by tile, as the reference kernel, where that is the
                               * faster form or the launch has fewer programs than the device has CUs; else as
                               * IRIS_PHASE_TWO_KERNELS.  Results and flags are the same. */
-#define IRIS_PHASE_TWO_KERNELS 7 /* both, as two kernels on the stream: the producer GEMM, then the reduce kernel
-                                  * (iris_one_shot_reduce_launch) behind it */
+#define IRIS_PHASE_TWO_KERNELS 7 /* both, no tile's reduce holding up another tile's product: the producer GEMM, then the
+                                  * reduce kernel (iris_one_shot_reduce_launch) behind it on the stream.  A product of few
+                                  * rows, or in cells, of up to 128 small tiles is one kernel that reduces as it stores and
+                                  * in which at most one workgroup a tile waits for the peers. */
 
 /* flag scopes */
 #define IRIS_SCOPE_AGENT 0  /* all "ranks" live on this GPU */
@@ -275,8 +277,8 @@ int iris_gemm_split_k(const iris_gemm_args* args, int* split_k);
  * "+last_round_in_N_parts" where a second launch shares K of the last round's
  * tiles out over the programs that round would leave idle (needs partials and
  * locks), by "+parts_of_tiles" where the caller's tiles are computed as several
- * smaller ones, and by "+kernel+reduce" where an IRIS_PHASE_FUSED launch reduces in
- * a kernel behind the producer rather than inside it. */
+ * smaller ones, and by "+kernel+reduce" where an IRIS_PHASE_FUSED launch runs as an
+ * IRIS_PHASE_TWO_KERNELS one. */
 int iris_gemm_plan_name(const iris_gemm_args* args, char* buf, size_t len);
 
 /* Name of tuning variant `variant` (1-based) of the kernel list used for

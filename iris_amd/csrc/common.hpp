@@ -335,10 +335,25 @@ __device__ inline void flag_add_relaxed(IRIS_GLOBAL int32_t* p, int v, bool sys)
 // Counts one of the groups that share a tile and returns how many had come before; the last one raises the tile's flag.
 // `release`: the flag is a release (IRIS_FLAG_SEM_RELEASE_ACQUIRE) and has to release what every group stored, not its
 // own group's stores alone, so each arrival releases and acquires at the flag's scope.
-__device__ inline int arrive(IRIS_GLOBAL int32_t* count, bool release, bool sys) {
-  if (!release) return __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  return sys ? __hip_atomic_fetch_add(count, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_SYSTEM)
-             : __hip_atomic_fetch_add(count, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+__device__ inline int arrive(IRIS_GLOBAL int32_t* count, bool release, bool sys, int as = 1) {
+  if (!release) return __hip_atomic_fetch_add(count, as, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return sys ? __hip_atomic_fetch_add(count, as, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_SYSTEM)
+             : __hip_atomic_fetch_add(count, as, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Acquires at the flags' scope (IRIS_FLAG_SEM_RELEASE_ACQUIRE).
+__device__ inline void acquire_at(bool sys) {
+  if (sys)
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "");
+  else
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+}
+
+// Load that is coherent at the flags' scope.
+template <typename T>
+__device__ inline T load_through(const IRIS_GLOBAL T* p, bool sys) {
+  return sys ? __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM)
+             : __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Store that is written through to the coherence point of the agent (or of

@@ -109,6 +109,10 @@ bool vec_ok(const void* base, int64_t stride_m, int64_t stride_n, int es) {
   return stride_n == 1 && aligned16(base) && ((stride_m * es) % 16) == 0;
 }
 
+// (the few-rows kernel's build that reduces) tiles of a launch, and bytes of all ranks' partials of a tile
+constexpr int REDUCE_MAX_TILES = 128;
+constexpr int64_t REDUCE_MAX_BYTES = 128 << 10;
+
 struct Plan {
   const GemmKernelEntry* entry = nullptr;
   GemmKArgs k{};
@@ -117,10 +121,12 @@ struct Plan {
   int parts = 0;         // the launch's tiles are parts of the caller's (plan_parts)
   int loose = 0;         // the few-rows kernel's build for operands at any alignment
   int b_rows = 0;        // ... for a row-major B (cells)
-  int two_kernels = 0;   // ... or, for such a launch too, producer and reduce as two kernels (reduce_in_program)
+  int two_kernels = 0;   // ... or, for such a launch too, what IRIS_PHASE_TWO_KERNELS would run (reduce_in_program)
   // the few-rows kernel instead of a table entry: workgroups along the columns, the rows and K
   GemmKernelFn skinny = nullptr;
   int skinny_grid = 0, skinny_grid_y = 1, skinny_grid_z = 1, skinny_lds = 0;
+  int reduces = 0;       // the few-rows kernel's build that reduces, too
+  int skinny_arows = 16;
   int skinny_rb = 1, skinny_cb = 1;  // blocks of 16 rows and of 16 columns a workgroup of the few-rows kernel takes
   // a second launch of the entry's split-K build behind the first: the tiles of the last round, K shared out
   // over the programs that round would leave idle
@@ -223,7 +229,7 @@ bool plan_few_rows(const iris_gemm_args& a, int op, bool dma_ok, bool loose, Pla
     const int64_t elems = cells * rb * (SKINNY_ROWS * SKINNY_COLS);  // of one part's sums
     if (parts * elems > (int64_t)a.num_sms * a.partials_slot_elems) parts = 1;
   }
-  plan->skinny = gemm_skinny_kernel_for(a.ab_dtype, op, a.M <= 8 ? 8 : 16, rb, 1, loose);
+  plan->skinny = gemm_skinny_kernel_for(a.ab_dtype, op, a.M <= 8 ? 8 : 16, rb, 1, loose, false, false);
   if (!plan->skinny) return false;
   plan->loose = loose;
   plan->skinny_lds = skinny_lds_bytes(rb);
@@ -231,6 +237,7 @@ bool plan_few_rows(const iris_gemm_args& a, int op, bool dma_ok, bool loose, Pla
   plan->skinny_grid_y = m_blocks;
   plan->skinny_grid_z = parts;
   plan->skinny_rb = rb;
+  plan->skinny_arows = a.M <= 8 ? 8 : 16;
   k.split_k = 1;
   k.locks = a.locks;
   k.partials = a.partials;
@@ -270,7 +277,7 @@ bool plan_cells(const iris_gemm_args& a, int op, bool dma_ok, bool loose, bool b
   }
   // (a row-major B with up to 16 rows of A: cells of 16 x 32, which fetch the half or the quarter of A that there is)
   const int rb = b_rows && a.M <= SKINNY_ROWS ? 1 : 2;
-  plan->skinny = gemm_skinny_kernel_for(a.ab_dtype, op, rb == 1 && a.M <= 8 ? 8 : 16, rb, 2, loose, b_rows);
+  plan->skinny = gemm_skinny_kernel_for(a.ab_dtype, op, rb == 1 && a.M <= 8 ? 8 : 16, rb, 2, loose, b_rows, false);
   if (!plan->skinny) return false;
   k.cells = (int)cells;
   k.cells_by_row = a.M > a.N;
@@ -285,6 +292,7 @@ bool plan_cells(const iris_gemm_args& a, int op, bool dma_ok, bool loose, bool b
   plan->skinny_grid_y = 1;
   plan->skinny_grid_z = parts;
   plan->skinny_rb = rb;
+  plan->skinny_arows = rb == 1 && a.M <= 8 ? 8 : 16;
   plan->skinny_cb = 2;
   k.split_k = 1;
   k.locks = a.locks;
@@ -1071,15 +1079,55 @@ bool plan_blocks(const iris_gemm_args& a, Plan* plan) {
   return false;
 }
 
+// Few rows and cells with a reduce behind them: the reduce in the same kernel (gemm_skinny.hpp, REDUCE), where a tile is small
+// enough for one workgroup to reduce it should its peers be late, and few enough workgroups may come to wait for theirs.
+// One workgroup has 32 KB of partials in flight, so a late tile of REDUCE_MAX_BYTES is four round trips to memory, about what a reduce
+// kernel's launch and chain take.  Waiting workgroups hold LDS that a peer on this device needs: REDUCE_MAX_TILES of them, of the
+// device's 256 (cells) to 768 places.  Not for a launch that shares the device with its peers' (fewer programs than CUs).
+bool reduce_in_few_rows(const iris_gemm_args& a, Plan* plan) {
+  GemmKArgs& k = plan->k;
+  if (!plan->skinny || !plan->fused_reduce || a.epilogue != IRIS_EPI_ONE_SHOT || a.world_size < 2) return false;
+  if (a.num_sms < current_cu_count() || !k.row_out || a.stride_cn_global != 1 || k.som < a.N || a.stride_cm_global < a.N) return false;
+  const int gdt = a.c_global_dtype, ies = dtype_size(a.c_dtype), oes = dtype_size(gdt);
+  if (gdt != IRIS_DTYPE_F32 && gdt != IRIS_DTYPE_F16 && gdt != IRIS_DTYPE_BF16) return false;
+  const int64_t lim = (int64_t)1 << 31, rows = a.block_m < a.M ? a.block_m : a.M, cols = a.block_n < a.N ? a.block_n : a.N;
+  if (((int64_t)a.block_m + 64) * k.som * ies >= lim || ((int64_t)a.block_m + 64) * a.stride_cm_global * oes >= lim) return false;
+  if (k.total_tiles > REDUCE_MAX_TILES || rows * cols * ies * a.world_size > REDUCE_MAX_BYTES) return false;
+  const GemmKernelFn fn = gemm_skinny_kernel_for(a.ab_dtype, a.c_dtype == IRIS_DTYPE_F32 ? OP_STORE32 : OP_STORE16, plan->skinny_arows,
+                                                 plan->skinny_rb, plan->skinny_cb, plan->loose != 0, plan->b_rows != 0, true);
+  if (!fn) return false;
+  plan->skinny = fn;
+  plan->fused_reduce = 0;
+  plan->reduces = 1;
+  k.cg = static_cast<char*>(a.c_global);
+  k.sgm = a.stride_cm_global;
+  k.sgn = a.stride_cn_global;
+  k.cg_dt = gdt;
+  k.fused_vec = k.vec_out && vec_ok(k.cg, k.sgm, k.sgn, oes) && a.block_n % (16 / ies) == 0 && (a.block_n * oes) % 16 == 0;
+  k.status = a.status;
+  k.timeout = a.spin_timeout_ticks ? a.spin_timeout_ticks : 200000000ull;  // 2 s at 100 MHz
+  return true;
+}
+
+hipError_t make_plan_tiles(const iris_gemm_args& a, Plan* plan);
+
 hipError_t make_plan_units(const iris_gemm_args& a, Plan* plan) {
+  const hipError_t err = make_plan_tiles(a, plan);
+  if (err == hipSuccess) reduce_in_few_rows(a, plan);
+  return err;
+}
+
+hipError_t make_plan_tiles(const iris_gemm_args& a, Plan* plan) {
   if (a.epilogue == IRIS_EPI_ONE_SHOT && a.phase == IRIS_PHASE_FUSED) {
     iris_gemm_args b = a;
     b.phase = IRIS_PHASE_TWO_KERNELS;
     Plan behind;
     if (a.split_k <= 1 && a.split_k != IRIS_GEMM_SPLIT_STREAM_K && make_plan_units(b, &behind) == hipSuccess &&
-        !reduce_in_program(a, behind)) {
+        (!reduce_in_program(a, behind) || (behind.reduces && !behind.loose && !behind.b_rows))) {
+      // (inside, few rows and cells of aligned operands are faster than the caller's tiles with their own reduce: us a pass, [125,384] x
+      // [384,1216] of 2, 64 x 64 tiles 9.9 / 8.8, [82,128] x [128,4120] of 8 11.3 / 10.8)
       *plan = behind;
-      plan->two_kernels = 1;
+      plan->two_kernels = !reduce_in_program(a, behind);
       return hipSuccess;
     }
   }
@@ -1648,9 +1696,9 @@ extern "C" int iris_gemm_plan_name(const iris_gemm_args* args, char* buf, size_t
     const size_t n = std::strlen(buf);
     std::snprintf(buf + n, len > n ? len - n : 0, "+parts_of_tiles");
   }
-  if (plan.two_kernels) {
+  if (plan.two_kernels || (plan.reduces && args->phase == IRIS_PHASE_FUSED)) {
     const size_t n = std::strlen(buf);
-    std::snprintf(buf + n, len > n ? len - n : 0, "+kernel+reduce");
+    std::snprintf(buf + n, len > n ? len - n : 0, plan.two_kernels ? "+kernel+reduce" : "+reduce");
   }
   return hipSuccess;
 }

@@ -75,6 +75,34 @@ constexpr int CELL = 32;
 // LDS of a workgroup of RB x 2 blocks
 constexpr int cells_lds_bytes(int rb) { return SKINNY_WAVES * SKINNY_UN * (rb + 2) * SKINNY_BLOCK_BYTES; }
 
+// (REDUCE) four columns of the result's row m, from column n on, written through like the reference's store (".wt").
+__device__ __attribute__((always_inline)) inline void store_result4(const GemmKArgs& p, int m, int n, f32x4 s) {
+  const bool f32 = p.cg_dt == IRIS_DTYPE_F32, bf16 = p.cg_dt == IRIS_DTYPE_BF16;
+  IRIS_GLOBAL char* d = (IRIS_GLOBAL char*)p.cg + ((int64_t)m * p.sgm + n) * (f32 ? 4 : 2);
+  const u32x4 wide = __builtin_bit_cast(u32x4, s);
+  const u32x2 half = bf16 ? u32x2{pack2<IRIS_DTYPE_BF16>(s[0], s[1]), pack2<IRIS_DTYPE_BF16>(s[2], s[3])}
+                          : u32x2{pack2<IRIS_DTYPE_F16>(s[0], s[1]), pack2<IRIS_DTYPE_F16>(s[2], s[3])};
+  if (n + 4 <= p.N) {
+    if (f32 && p.sys)
+      store16_any<AUX_SC0 | AUX_SC1>(d, wide);
+    else if (f32)
+      store16_any<AUX_SC1>(d, wide);
+    else if (p.sys)
+      store8_any<AUX_SC0 | AUX_SC1>(d, half);
+    else
+      store8_any<AUX_SC1>(d, half);
+    return;
+  }
+#pragma unroll
+  for (int e = 0; e < 3; ++e) {
+    if (n + e >= p.N) continue;
+    if (f32)
+      store_through((IRIS_GLOBAL unsigned int*)d + e, wide[e], p.sys != 0);
+    else
+      store_through((IRIS_GLOBAL unsigned short*)d + e, (unsigned short)(half[e / 2] >> (16 * (e & 1))), p.sys != 0);
+  }
+}
+
 // AROWS: rows of A in a block, 8 or 16.
 // RB: blocks of 16 rows a workgroup computes (1 for up to 32 rows; 2 up to 64
 // rows of a long K, and from 17 rows on where B is large).
@@ -89,7 +117,13 @@ constexpr int cells_lds_bytes(int rb) { return SKINNY_WAVES * SKINNY_UN * (rb + 
 // A beside it ([95,4224] x [4224,1280] along K 9.7 us, so 12.8: 1.6 times what is above a launch's fixed 4.5).  With up to 16
 // rows of A, RB is 1 ([4,1376] x [1376,4096] 8.0 -> 7.4 us, 27 random calls of 1 to 16 rows 1.08x, same bits; RB 2 fetched as many rows of A again,
 // and for up to eight three times as many, all out of range).
-template <int DT, int OP, int ODT, int AROWS, int RB = 1, int CB = 1, bool LOOSE = false, bool BROWS = false>
+// REDUCE (one-shot epilogue): the workgroup also reduces its block of C over all ranks.  Of its own rank's partial it needs
+// what it has just computed, so it waits for no other workgroup; the peers' strips, where their signal is there by the
+// last blocks of K, are fetched (wave w: rank w) under the last products and the exchange between the waves, and the sum is stored
+// behind the partial.  A reduce kernel behind the product cost its launch, its gap (0.84 us) and a chain of flag, bases,
+// partials and result of its own: [16,1376] x [1376,4096], 8 fp32 partials, fill of the flags included 13.5 -> 9.7 us; 64 random
+// calls of up to 300 rows whose reduce is inside 1.24x, none slower.
+template <int DT, int OP, int ODT, int AROWS, int RB = 1, int CB = 1, bool LOOSE = false, bool BROWS = false, bool REDUCE = false>
 __global__ __launch_bounds__(SKINNY_THREADS) __attribute__((amdgpu_waves_per_eu(2, 8))) void
 gemm_skinny_kernel(const GemmKArgs p) {
   constexpr bool ATOMIC = OP == OP_ATOMIC32 || OP == OP_ATOMIC16;
@@ -98,6 +132,7 @@ gemm_skinny_kernel(const GemmKArgs p) {
   static_assert(AROWS == 16 || (AROWS == 8 && RB == 1), "rows of a block of A");
   static_assert(RB == 1 || RB == 2, "blocks of rows per workgroup");
   static_assert(CB == 1 || (CB == 2 && ((RB == 2 && AROWS == 16) || BROWS)), "blocks of columns per workgroup");
+  static_assert(!REDUCE || !ATOMIC, "the one-shot epilogue stores");
   static_assert(!BROWS || (CB == 2 && !LOOSE && DT != IRIS_DTYPE_F32), "B by rows of k: cells of 16-bit operands");
   constexpr bool A_DMA = CB == 2;  // A in LDS, UN blocks a wave, like B
   constexpr int NB = RB * CB;
@@ -257,6 +292,47 @@ gemm_skinny_kernel(const GemmKArgs p) {
     asm volatile("" ::: "memory");  // (the blocks' loads stay in this order: the waits below count them)
   }
   touch_line(p.heap_bases);  // (read by the stores)
+  constexpr int ES = F32 ? 4 : 2;
+  // (REDUCE) the tile that the block belongs to, and its flag as it is now
+  int tile_id = 0, flag_now = 0;
+  // (REDUCE) this lane's columns of each block of rank r's partial, element by element where N ends inside the four
+  u32x4 strip[REDUCE ? NB : 1];
+  auto fetch_strips = [&](int r) __attribute__((always_inline)) {
+    const int cols = min(SKINNY_COLS * CB, p.N - n0);
+    IRIS_GLOBAL char* base = rank_ptr(p, p.out, r) + ((int64_t)m0 * p.som + n0) * ES;
+    const __amdgpu_buffer_rsrc_t rs =
+        __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, (int)((((int64_t)rows_a - 1) * p.som + cols) * ES), 0x00020000);
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      const int row = (b / CB) * 16 + lr, col = lq * (4 * CB) + 4 * (b % CB);
+      const uint32_t off = row < rows_a && col + 4 <= cols ? (uint32_t)(((int64_t)row * p.som + col) * ES) : DEAD_OFFSET;
+      if constexpr (F32) {
+        strip[b] = p.sys ? __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off, 0, AUX_SC0 | AUX_SC1)
+                         : __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off, 0, AUX_SC1);
+      } else {
+        const u32x2 x = p.sys ? __builtin_amdgcn_raw_buffer_load_b64(rs, (int)off, 0, AUX_SC0 | AUX_SC1)
+                              : __builtin_amdgcn_raw_buffer_load_b64(rs, (int)off, 0, AUX_SC1);
+        strip[b] = u32x4{x[0], x[1], 0u, 0u};
+      }
+      if (row < rows_a && col < cols && col + 4 > cols) {
+        const IRIS_GLOBAL char* at = base + ((int64_t)row * p.som + col) * ES;
+        strip[b] = u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int e = 0; e < 3; ++e) {
+          if (col + e >= cols) continue;
+          if constexpr (F32)
+            strip[b][e] = load_through((const IRIS_GLOBAL unsigned int*)at + e, p.sys != 0);
+          else
+            strip[b][e / 2] |= (unsigned int)load_through((const IRIS_GLOBAL unsigned short*)at + e, p.sys != 0) << (16 * (e & 1));
+        }
+      }
+    }
+  };
+  auto flag_of = [&]() __attribute__((always_inline)) { return (IRIS_GLOBAL int32_t*)(p.flags + tile_id); };
+  if constexpr (REDUCE) {
+    tile_id = tile_id_of(m0 / p.BM, n0 / p.BN, p.num_pid_m, p.num_pid_n, p.G);
+    flag_now = load_through(flag_of(), p.sys != 0);
+  }
   // A long range of K: as a block has been read its place takes the one UN further on, so that the fetches in
   // flight never run dry (B has landed in this wave's own region once the wave's counter says so: nobody else
   // reads or writes it).
@@ -274,6 +350,16 @@ gemm_skinny_kernel(const GemmKArgs p) {
   // the last blocks: the loads behind them are all on their way
   IRIS_WAIT_VMCNT(0);
   asm volatile("" ::: "memory");
+  // (REDUCE, K of one group) peers that are done: wave w fetches the strips of rank w, which arrive under the last products
+  // and the exchange behind them
+  bool peers_done = false;
+  if constexpr (REDUCE) {
+    peers_done = gridDim.z == 1 && __builtin_amdgcn_readfirstlane(flag_now) >= p.ws - 1;
+    if (peers_done) {
+      if (p.flag_mode & FLAG_RELEASE) acquire_at(p.sys != 0);
+      if (wave < p.ws && wave != p.cur_rank) fetch_strips(wave);
+    }
+  }
 #pragma unroll
   for (int u = 0; u < UN; ++u) multiply(u, b0 + SKINNY_WAVES * u);
   IRIS_WAIT_LGKMCNT0();
@@ -281,6 +367,10 @@ gemm_skinny_kernel(const GemmKArgs p) {
 
   // acc[i]: row m = i*16 + l%16 of the workgroup's rows, columns 4*(l/16) .. +3 (operands swapped, as in the
   // persistent kernel).  The waves' partial sums meet in LDS, [wave][block][lane].
+  // (REDUCE: a wave's own region of B, which it has read, takes its strips and whether it saw the flag)
+  if constexpr (REDUCE) {
+    if (lane == 0) *(IRIS_LDS int*)(wb + NB * 1024) = peers_done;
+  }
   __syncthreads();  // every wave is done with its blocks of A: the region becomes `red`
 #pragma unroll
   for (int i = 0; i < NB; ++i) red[(wave * NB + i) * 64 + lane] = acc[i];
@@ -303,6 +393,10 @@ gemm_skinny_kernel(const GemmKArgs p) {
     __syncthreads();
   }
 
+  if constexpr (REDUCE) {
+    const int seen = lane < SKINNY_WAVES ? *(IRIS_LDS int*)(wb + (lane - wave) * (UN * CB * SKINNY_BLOCK_BYTES) + NB * 1024) : 1;
+    if (peers_done && __ballot(seen == 0) != 0) peers_done = false;
+  }
   const bool split = gridDim.z > 1;
   if (split) {
     // K shared out over gridDim.z groups: each leaves its sum in `partials` (register order, 1 KiB a block), and
@@ -330,6 +424,7 @@ gemm_skinny_kernel(const GemmKArgs p) {
       asm volatile("" ::: "memory");
       IRIS_GLOBAL int32_t* cnt = (IRIS_GLOBAL int32_t*)(p.locks + p.total_tiles + cell);
       int last = 0;
+      if constexpr (REDUCE) flag_now = load_through(flag_of(), p.sys != 0);
       if (lane == 0) {
         last = __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (int)gridDim.z - 1;
         if (last) __hip_atomic_store(cnt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
@@ -356,15 +451,22 @@ gemm_skinny_kernel(const GemmKArgs p) {
 #pragma unroll
         for (int b = 0; b < NB; ++b) red[b * 64 + lane] = s[b];
       }
-      if (lane == 0) *is_last = last;
+      if (lane == 0) *is_last = last | (REDUCE && flag_now >= p.ws - 1 ? 2 : 0);
     }
     __syncthreads();
-    if (!*is_last) return;
+    const int found = *is_last;
+    if (!(found & 1)) return;
+    if constexpr (REDUCE) {
+      peers_done = (__builtin_amdgcn_readfirstlane(found) & 2) != 0;
+      if (peers_done) {
+        if (p.flag_mode & FLAG_RELEASE) acquire_at(p.sys != 0);
+        if (wave < p.ws && wave != p.cur_rank) fetch_strips(wave);
+      }
+    }
   }
 
   const int r_begin = p.dest_all ? 0 : p.cur_rank;
   const int r_end = p.dest_all ? p.ws : p.cur_rank + 1;
-  constexpr int ES = F32 ? 4 : 2;
   // four columns of a row, from column n on
   auto store4 = [&](IRIS_GLOBAL char* dst, int m, int n, f32x4 s) __attribute__((always_inline)) {
     if constexpr (ATOMIC) {
@@ -415,6 +517,68 @@ gemm_skinny_kernel(const GemmKArgs p) {
       }
     }
   };
+  if constexpr (REDUCE) {
+    // One-shot epilogue with the reduce inside (gemm_one_shot_all_reduce.py:197-271).  Wave i stores block i of the rows to
+    // this rank's partial; where the peers have signalled the tile, it adds all ranks' strips up, in rank order, and stores
+    // the result: what the workgroup needs of its own rank it holds, so it waits for nobody.
+    const int m = m0 + wave * 16 + lr, n = n0 + lq * (4 * CB);
+    const bool mine = wave < RB && m < p.M && n < p.N;
+    f32x4 own[CB], sum[CB];
+    if (mine) {
+#pragma unroll
+      for (int j = 0; j < CB; ++j) {
+        own[j] = red[(wave * CB + j) * 64 + lane];
+        if (NB == 1 && !split) {
+#pragma unroll
+          for (int w = 1; w < SKINNY_WAVES; ++w) own[j] += red[w * 64 + lane];  // wave order
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < CB; ++j) {
+        if (n + 4 * j < p.N) store4((IRIS_GLOBAL char*)p.out, m, n + 4 * j, own[j]);
+        if constexpr (!F32) {
+          // (what the partial holds is what is added)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) own[j][e] = from16<ODT>(to16<ODT>(own[j][e]));
+        }
+      }
+    }
+    if (peers_done) {
+      for (int r0 = 0;; r0 += SKINNY_WAVES) {
+        if (r0 + wave < p.ws && r0 + wave != p.cur_rank) {
+          if (r0 > 0) fetch_strips(r0 + wave);
+#pragma unroll
+          for (int b = 0; b < NB; ++b) {
+            f32x4 v = __builtin_bit_cast(f32x4, strip[b]);
+            if constexpr (!F32)
+#pragma unroll
+              for (int e = 0; e < 4; ++e) v[e] = from16<ODT>((unsigned short)(strip[b][e / 2] >> (16 * (e & 1))));
+            *reinterpret_cast<IRIS_LDS f32x4*>(wb + b * 1024 + lane * 16) = v;
+          }
+        }
+        __syncthreads();
+        if (mine) {
+          for (int q = 0; q < SKINNY_WAVES && r0 + q < p.ws; ++q)
+#pragma unroll
+            for (int j = 0; j < CB; ++j) {
+              const f32x4 v = r0 + q == p.cur_rank
+                                  ? own[j]
+                                  : *reinterpret_cast<const IRIS_LDS f32x4*>(wb + (q - wave) * (UN * CB * SKINNY_BLOCK_BYTES) +
+                                                                             (wave * CB + j) * 1024 + lane * 16);
+              const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+              sum[j] = (r0 + q == 0 ? zero : sum[j]) + v;
+            }
+        }
+        if (r0 + SKINNY_WAVES >= p.ws) break;
+        __syncthreads();  // the strips have been read
+      }
+      if (mine) {
+#pragma unroll
+        for (int j = 0; j < CB; ++j)
+          if (n + 4 * j < p.N) store_result4(p, m, n + 4 * j, sum[j]);
+      }
+    }
+  } else {
   // (rank, row block) pairs over the waves
   for (int it = wave; it < (r_end - r_begin) * RB; it += SKINNY_WAVES) {
     const int r = r_begin + it / RB, i = it % RB;
@@ -444,14 +608,61 @@ gemm_skinny_kernel(const GemmKArgs p) {
     for (int j = 0; j < CB; ++j)
       if (n + 4 * j < p.N) store4(dst, m, n + 4 * j, s[j]);
   }
+  }
   if (p.flag_mode == 0) return;
 
   // The stores were write-through at the flags' scope: once every wave has
   // seen its own complete, the group's part of the tile is visible there.
   IRIS_WAIT_VMCNT(0);
   __syncthreads();
+  const int pid_m = m0 / p.BM, pid_n = n0 / p.BN;
+  if constexpr (REDUCE) {
+    // Two counts in the tile's word: the workgroups that have stored, and those of them that have reduced.  The last to
+    // arrive signals the peers and, where all have reduced, consumes the flag (CAS(ws-1 -> 0), :220-234).  Else it waits for
+    // the flag and reduces the tile itself: one workgroup a tile waits, the others have made room for the peers' launches.
+    IRIS_LDS int* todo = (IRIS_LDS int*)lds;
+    Item it{};
+    it.lm0 = pid_m * p.BM;
+    it.ln0 = pid_n * p.BN;
+    it.m_end = min(p.M, it.lm0 + p.BM);
+    it.n_end = min(p.N, it.ln0 + p.BN);
+    if (wave == 0) {
+      constexpr int COLS = SKINNY_COLS * CB, ROWS = SKINNY_ROWS * RB;
+      const int parts = ((it.n_end - it.ln0 + COLS - 1) / COLS) * ((it.m_end - it.lm0 + ROWS - 1) / ROWS);
+      int stored = 1, reduced = peers_done ? 1 : 0;
+      if (parts > 1) {
+        IRIS_GLOBAL int32_t* cnt = (IRIS_GLOBAL int32_t*)(p.locks + tile_id);
+        int before = 0;
+        if (lane == 0) before = arrive(cnt, (p.flag_mode & FLAG_RELEASE) != 0, p.sys != 0, 1 + (reduced << 16));
+        before = __builtin_amdgcn_readfirstlane(before);
+        stored += before & 0xFFFF;
+        reduced += before >> 16;
+        if (stored == parts && lane == 0) __hip_atomic_store(cnt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
+      }
+      int wait = 0;
+      if (stored == parts) {
+        publish_tile(p, tile_id, lane);
+        if (reduced < parts)
+          wait = 1;
+        else if (lane == 0)
+          flag_add_relaxed(flag_of(), 1 - p.ws, p.sys != 0);
+      }
+      if (lane == 0) {
+        if (wait && wait_tile_flag(flag_of(), p.ws, p.sys != 0, p.timeout, p.status)) wait = 2;
+        *todo = wait;
+      }
+    }
+    __syncthreads();
+    if (*todo == 2) {
+      constexpr int IN_DT = F32 ? IRIS_DTYPE_F32 : ODT;
+      if (p.sys)
+        fused_reduce_tile<IN_DT, SKINNY_THREADS, 1, true>(p, it, tid);
+      else
+        fused_reduce_tile<IN_DT, SKINNY_THREADS, 1, false>(p, it, tid);
+    }
+    return;
+  }
   if (wave == 0) {
-    const int pid_m = m0 / p.BM, pid_n = n0 / p.BN;
     const int tile_id = tile_id_of(pid_m, pid_n, p.num_pid_m, p.num_pid_n, p.G);
     const int cols = min(p.N, (pid_n + 1) * p.BN) - pid_n * p.BN, rows = min(p.M, (pid_m + 1) * p.BM) - pid_m * p.BM;
     constexpr int COLS = SKINNY_COLS * CB;
@@ -471,6 +682,7 @@ gemm_skinny_kernel(const GemmKArgs p) {
 
 // The kernel for (operand type, store op, rows of A in a block, blocks of rows and of columns a workgroup), or null.
 // `loose`: for operands at any alignment.  `b_rows` (cells): for a row-major B.
-GemmKernelFn gemm_skinny_kernel_for(int dt, int op, int arows, int rb, int cb, bool loose, bool b_rows = false);
+// `reduce`: the build that also reduces (the one-shot epilogue).
+GemmKernelFn gemm_skinny_kernel_for(int dt, int op, int arows, int rb, int cb, bool loose, bool b_rows, bool reduce);
 
 }  // namespace iris_amd
