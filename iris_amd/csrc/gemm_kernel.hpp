@@ -47,6 +47,8 @@
 namespace iris_amd {
 
 constexpr int FLAG_MODE_MASK = 3, FLAG_RELEASE = 4;
+// GemmKArgs::sliced of a launch with fp32 atomics whose parts each add their own sums
+constexpr int SPLIT_DIRECT = 3;
 
 struct GemmKArgs {
   const char* a;
@@ -107,7 +109,7 @@ struct GemmKArgs {
   // runs the epilogue on them, so that no program does a whole tile's worth
   // of serial work; locks[first slot + 1] counts the parts that are done, and
   // the last one publishes the tile and re-arms both counters.
-  int sliced;  // 1: as above; 2 (two parts only): each part keeps the half of the waves it owns, see dump_half
+  int sliced;  // 1: as above; 2 (two parts only): each part keeps the half of the waves it owns, see dump_half; SPLIT_DIRECT
   float* partials;
   int32_t* locks;
   int64_t partial_stride;
@@ -1764,8 +1766,11 @@ __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKAr
       if (wave == 0) publish_tile<MERGED, Cfg::PARTS>(p, pending_tile, lane);
       pending_tile = -1;
     }
+    // (fp32 atomics) every part adds its own sum up where the tile's would go: no hand-over, nobody waits
+    constexpr bool DIRECT = SPLIT && OP == OP_ATOMIC32;
     if constexpr (SPLIT) {
-      if (ONE_ITEM || p.sliced) {
+      const bool direct = DIRECT && p.sliced == SPLIT_DIRECT;
+      if (!direct && (ONE_ITEM || p.sliced)) {
         // (One item per program: whatever this hand-over reads of the launch's arguments is read here, from the
         // argument block, through a pointer the compiler cannot see through; held in scalar registers from the
         // kernel's entry on, those arguments pushed fragments of the K loop out of the 128-accumulator tiles'
@@ -1853,6 +1858,7 @@ __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKAr
       }
       // (the tiles without the owner's way are only launched with the sliced one)
       if constexpr (Cfg::SPLIT_OWNER) {
+      if (!direct) {
       const KRange kr = k_range<Cfg, SPLIT>(p, sr, pid, c_item, nk);
       if (kr.part != 0) {
         // not the owner: leave the partial, raise the lock once every wave's
@@ -1877,12 +1883,14 @@ __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKAr
           for (int q = 1; q < parts; q += GROUP) add_partials<Cfg, GROUP>(p, acc, kr.slot, q, parts, tid);
       }
       }
+      }
     }
     // (The 128-accumulator tiles with fetching waves have no register to spare: what the stores read of the arguments is
     // read here, as in the split hand-over above, not held in spilled scalar registers across the K loop.  Atomics read
     // less and fit as they are: 8 x [4096,512] x [512,4096] 527 us, 530 with the arguments read late.)
-    constexpr bool LATE = !SPLIT && !FUSED && (OP == OP_STORE16 || OP == OP_STORE32) && Cfg::DMA && Cfg::LW != 0 &&
-                          Cfg::IM * Cfg::IN * 4 > 64;
+    constexpr bool LATE = (!SPLIT && !FUSED && (OP == OP_STORE16 || OP == OP_STORE32) && Cfg::DMA && Cfg::LW != 0 &&
+                           Cfg::IM * Cfg::IN * 4 > 64) ||
+                          (DIRECT && ONE_ITEM);
     typedef const __attribute__((address_space(4))) GemmKArgs* KernArgPtr;
     KernArgPtr late_args = (KernArgPtr)__builtin_amdgcn_kernarg_segment_ptr();
     if constexpr (LATE) asm volatile("" : "+s"(late_args));

@@ -1117,6 +1117,126 @@ hipError_t make_plan_units(const iris_gemm_args& a, Plan* plan) {
   return err;
 }
 
+// A launch with atomics has no flags, so nothing shows which tiles it ran in: any tile will do, not only one that divides the
+// caller's, and with fp32 atomics K may be shared out over programs that each add their own sums, with no hand-over and
+// nobody waiting.  (16-bit atomics would round every part's sum on its way in: they keep whole sums.)
+//
+// Times of such a launch in us: fixed + the first tile + the others, each as long as its K loop or its atomics (the chip adds
+// 331 G a second, a CU a 64 x 64 tile in 1.1 us) + the last tile's atomics; `step`: 64 units of K of a tile, dearer by the same
+// three things as BlockTime's.  Fitted to 6500 timings of 390 random calls ([33 .. 8192, 128 .. 36864] x [.., 128 .. 8192], 16-bit and
+// fp32, weights in rows of either direction and at any alignment, K in up to 16 parts), rms 11 % on a third kept apart.
+struct AtomicTime {
+  int cm, cn;
+  double tile, step, step_f32;  // (0: no such tile)
+};
+constexpr AtomicTime ATOMIC_TIMES[] = {
+    {64, 64, 0.78, 0.149, 0.512},  {128, 64, 1.51, 0.234, 0},  {64, 128, 1.98, 0.245, 0.934}, {128, 128, 5.14, 0.333, 1.773},
+    {256, 64, 4.46, 0.403, 1.832}, {256, 128, 10.3, 0.514, 0}, {128, 256, 9.20, 0.519, 0},
+};
+struct AtomicLaunch {
+  double streamed;  // how much of the operands comes from HBM
+  double each;      // us that the chip takes for all atomics of one part of K
+  double kind;      // of the loader
+  bool f32, lines;
+};
+double atomic_us(const iris_gemm_args& a, const AtomicTime& t, int parts, const AtomicLaunch& l) {
+  const int64_t items = ((int64_t)a.M + t.cm - 1) / t.cm * (((int64_t)a.N + t.cn - 1) / t.cn) * parts;
+  const int64_t rounds = (items + a.num_sms - 1) / a.num_sms, nk = ((int64_t)a.K + 63) / 64, steps = (nk + parts - 1) / parts;
+  const double busy = rounds > 1 ? 1.0 : (double)items / a.num_sms;
+  const double step = (l.f32 ? t.step_f32 * (1 + 0.043 * busy) : t.step * (1 + 0.148 * busy) * (1 + 0.399 * l.streamed)) *
+                      (l.lines ? 1.0 : 1.19) * l.kind;
+  const double loop = t.tile + steps * step, chip = 0.537 * l.each * parts / rounds, cu = 0.518 * t.cm * t.cn / 4096;
+  const double adds = chip > cu ? chip : cu, next = loop + 1.083 * adds;
+  return 6.82 + 1.09 * busy + loop + (rounds - 1) * (next > adds ? next : adds) + adds;
+}
+
+// K of an unsplit plan with fp32 atomics in `parts`, each of which adds its own sums.
+bool split_direct(const iris_gemm_args& a, int parts, Plan* plan) {
+  GemmKArgs& k = plan->k;
+  const GemmKernelEntry* e = plan->entry;
+  const int nk = (a.K + e->bk - 1) / e->bk;
+  if (e->op != OP_ATOMIC32 || !e->fn_split || k.split_k != 1 || k.stream_k || k.sub_m != 1 || k.sub_n != 1 || parts > nk ||
+      (int64_t)k.total_tiles * parts > a.num_sms)
+    return false;
+  k.num_sms = a.num_sms;
+  k.split_k = parts;
+  k.split_q = nk / parts;
+  k.split_r = nk % parts;
+  k.sliced = SPLIT_DIRECT;
+  launch_constants(a, *e, &k);
+  return true;
+}
+
+// Replaces the plan of a launch with atomics where another tile, or (fp32 atomics) another number of parts of K, is expected to be
+// faster by more than an eighth, a quarter where K is short and the atomics are most of the time; less the times above are not
+// good for.  (us, in the caller's tiles or what plan_small made of
+// them / so: [828,20672] x [20672,2688] in 256 x 64 tiles 208 / 109, 128 x 256 in three parts; [2023,22656] x [22656,192] in 256 x 128
+// 54 / 36; fp32 [904,1024] x [1024,4224] in 128 x 128 140 / 77, 64 x 128; fp32 [1171,456] x [456,258] 41 / 15; row-major
+// [494,9968] x [9968,4480] with 16-bit atomics in 64 x 64 98 / 68.  Of 353 random calls in tiles 96 change, 1.07x on average
+// over all of them; four slower by 4 to 7 %, all in more than four rounds of tiles, which are left out.)
+void plan_atomics(const iris_gemm_args& a, Plan* plan) {
+  const GemmKernelEntry* own = plan->entry;
+  if (a.epilogue != IRIS_EPI_ATOMIC_ADD || !own || plan->skinny || plan->k.stream_k) return;
+  if (a.variant != 0 || a.split_k != 0 || a.mm_begin_timestamp || a.mm_end_timestamp || a.num_sms != current_cu_count() || a.K <= 0) return;
+  const bool wide = a.c_global_dtype == IRIS_DTYPE_F32, handed = plan->k.split_k > 1;
+  if (!wide && handed) return;
+  AtomicLaunch l;
+  const double mb = ((double)a.M + a.N) * a.K * 2e-6;
+  l.streamed = mb < 50 ? 0 : mb > 150 ? 1 : (mb - 50) / 100;
+  l.each = (double)a.M * a.N * a.world_size / 331e3 * (wide ? 1.0 : 0.5);
+  l.kind = !own->dma ? 1.9 : own->loose ? 1.24 : 1.0;
+  l.f32 = a.ab_dtype == IRIS_DTYPE_F32;
+  l.lines = whole_lines(a);
+  constexpr int TILES = sizeof(ATOMIC_TIMES) / sizeof(ATOMIC_TIMES[0]);
+  double own_us = -1;
+  for (const AtomicTime& t : ATOMIC_TIMES)
+    if (t.cm == own->cm && t.cn == own->cn) {
+      // (a hand-over: 6 us, and the parts' sums are added up once)
+      AtomicLaunch whole = l;
+      whole.each /= plan->k.split_k;
+      own_us = atomic_us(a, t, plan->k.split_k, whole) + (handed ? 6 : 0);
+    }
+  if (own_us < 12) return;  // (another tile than these, or nothing to gain that the search would not cost)
+  double best_us[TILES];
+  int best_parts[TILES];
+  for (int i = 0; i < TILES; ++i) {
+    const AtomicTime& t = ATOMIC_TIMES[i];
+    best_us[i] = 1e30;
+    if (l.f32 && t.step_f32 == 0) continue;
+    const int64_t tiles = ((int64_t)a.M + t.cm - 1) / t.cm * (((int64_t)a.N + t.cn - 1) / t.cn);
+    if (tiles > 4 * (int64_t)a.num_sms) continue;
+    int most = wide ? (int)(a.num_sms / tiles) : 1;
+    if (most > 16) most = 16;
+    if (most > (a.K + 63) / 64 / 3) most = (a.K + 63) / 64 / 3;
+    for (int parts = 1; parts == 1 || parts <= most; parts += parts < 4 || parts + 2 > most ? 1 : 2) {
+      const double us = atomic_us(a, t, parts, l);
+      if (us < best_us[i]) best_us[i] = us, best_parts[i] = parts;
+    }
+  }
+  // the least of them that there is a kernel for
+  for (;;) {
+    int i = 0;
+    for (int j = 1; j < TILES; ++j)
+      if (best_us[j] < best_us[i]) i = j;
+    const AtomicTime& t = ATOMIC_TIMES[i];
+    if (best_us[i] > (a.K < 512 && !l.f32 ? 0.78 : 0.87) * own_us) return;
+    if (t.cm == own->cm && t.cn == own->cn && best_parts[i] == 1 && !handed) return;
+    iris_gemm_args b = a;
+    b.block_m = t.cm;
+    b.block_n = t.cn;
+    b.variant = IRIS_GEMM_VARIANT_PERSISTENT;
+    b.split_k = 1;
+    Plan free;
+    if (make_plan_body(b, &free) == hipSuccess && free.entry && free.entry->cm == t.cm && free.entry->cn == t.cn &&
+        (free.entry->dma || !own->dma) && (best_parts[i] == 1 || split_direct(b, best_parts[i], &free))) {
+      own_flags(&free);
+      *plan = std::move(free);
+      return;
+    }
+    best_us[i] = 1e30;
+  }
+}
+
 hipError_t make_plan_tiles(const iris_gemm_args& a, Plan* plan) {
   if (a.epilogue == IRIS_EPI_ONE_SHOT && a.phase == IRIS_PHASE_FUSED) {
     iris_gemm_args b = a;
@@ -1131,7 +1251,10 @@ hipError_t make_plan_tiles(const iris_gemm_args& a, Plan* plan) {
       return hipSuccess;
     }
   }
-  if (plan_small(a, plan)) return hipSuccess;
+  if (plan_small(a, plan)) {
+    plan_atomics(a, plan);
+    return hipSuccess;
+  }
   const bool plain = a.variant == 0 && a.split_k == 0 && !a.mm_begin_timestamp && !a.mm_end_timestamp &&
                      !(a.epilogue == IRIS_EPI_ONE_SHOT && a.phase != IRIS_PHASE_PRODUCE && a.phase != IRIS_PHASE_TWO_KERNELS) &&
                      a.epilogue != IRIS_EPI_ATOMIC_ADD && a.num_sms > 0 && (a.block_m == 128 || a.block_m == 256) &&
@@ -1139,7 +1262,10 @@ hipError_t make_plan_tiles(const iris_gemm_args& a, Plan* plan) {
   if (plain && plan_blocks(a, plan)) return hipSuccess;
   const hipError_t err = make_plan_body(a, plan);
   own_flags(plan);
-  if (err == hipSuccess) split_last_round(a, plan);
+  if (err == hipSuccess) {
+    split_last_round(a, plan);
+    plan_atomics(a, plan);
+  }
   return err;
 }
 
