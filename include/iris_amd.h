@@ -277,7 +277,8 @@ int iris_gemm_split_k(const iris_gemm_args* args, int* split_k);
  * "+last_round_in_N_parts" where a second launch shares K of the last round's
  * tiles out over the programs that round would leave idle (needs partials and
  * locks), by "+parts_of_tiles" where the caller's tiles are computed as several
- * smaller ones, and by "+kernel+reduce" where an IRIS_PHASE_FUSED launch runs as an
+ * smaller ones, by "+across_the_tiles" where it runs in tiles that need not divide
+ * them (partials and locks as above), and by "+kernel+reduce" where an IRIS_PHASE_FUSED launch runs as an
  * IRIS_PHASE_TWO_KERNELS one. */
 int iris_gemm_plan_name(const iris_gemm_args* args, char* buf, size_t len);
 

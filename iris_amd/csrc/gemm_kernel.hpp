@@ -155,16 +155,17 @@ struct GemmKArgs {
   int a_across, b_across;
   // rows of `out` are contiguous, at whatever alignment (vec_out: and 16-byte aligned)
   int row_out;
-  // part_m * part_n > 1 (tiles of up to 128 x 128): the launch's tiles are parts of the caller's, part_m x part_n to
-  // one, numbered over num_pid_m x num_pid_n; the parts of a caller's tile count their arrivals in
-  // tile_arrivals[its id] (all zero between launches), and the last one raises its flag
-  int part_m, part_n;
+  // cover_bm > 0: the launch's tiles (CM x CN each) lie across the caller's, cover_bm x cover_bn, of which there are
+  // flag_num_pid_m x flag_num_pid_n.  The tiles that share one of the caller's count their arrivals at it in a word of
+  // tile_arrivals (arrive_pack 0) or a byte of one (2), all zero between launches, and the last one raises its flag
+  int cover_bm, cover_bn, arrive_pack;
   int32_t* tile_arrivals;
   FastDiv div_xcd;  // num_xcds
   // (the few-rows kernel in cells of 32 x 32) `cells` of them, numbered in runs of cells_inner along the rows of C
   // (cells_by_row) or its columns; xcd_per consecutive ones to an XCD
   int cells, cells_inner, cells_by_row;
   FastDiv div_inner;
+  FastDiv div_cover_m, div_cover_n;  // cover_bm, cover_bn
 };
 
 template <int DT>
@@ -254,7 +255,7 @@ struct GemmCfg {
   // accumulators are dead once its partial is written.
   static constexpr bool SPLITK = PIPE && KSUB % 2 == 0 && IM * IN * 4 <= 128;
   static constexpr bool SPLIT_OWNER = SPLITK && IM * IN * 4 <= 64;
-  // The launcher may run the tile as a part of the caller's (see GemmKArgs::part_m).
+  // The launcher may run the tile across the caller's (see `covers`).
   static constexpr bool PARTS = CM <= 128 && CN <= 128 && LW != 0;
   // Waves per SIMD the register budget is sized for: 256 registers a wave.
   static constexpr int WPE = 2;
@@ -279,6 +280,11 @@ struct GemmCfg {
   static_assert(LDS_BYTES <= 160 * 1024, "LDS budget of one CU");
   static_assert(!B_ROWS || (DT != IRIS_DTYPE_F32 && IN <= 4 && CN % 64 == 0), "B by rows of k: 16-bit elements, wave tiles of at most 64 columns");
 };
+
+// Builds that may run launches whose tiles lie across the caller's (GemmKArgs::cover_bm).  (The unsplit 256 x 128 ones for a
+// row-major B and for any alignment, which spill as they are, would spill 8 bytes more.)
+template <class Cfg, bool SPLIT, bool MERGED>
+constexpr bool covers = Cfg::PARTS || (MERGED && !(Cfg::CM == 256 && Cfg::CN == 128 && !SPLIT && (Cfg::B_ROWS || Cfg::LOOSE)));
 
 // One compute tile of work.
 struct Item {
@@ -1174,54 +1180,86 @@ __device__ __attribute__((always_inline)) inline bool store_acc(const GemmKArgs&
 // Lane l takes ranks l, l + 64, ...: the ranks' heap bases come in with one
 // vector load and the increments leave together (one thread walking the ranks
 // waits for a scalar load per rank: 0.8 us for eight).
-// PARTS: the build may run launches whose tiles are parts of the caller's.
-template <bool MERGED = false, bool PARTS = false>
-__device__ __attribute__((always_inline)) inline void publish_tile(const GemmKArgs& p, int tile_id, int lane) {
+// COVER: the build may run launches whose tiles, CM x CN, lie across the caller's.
+template <bool MERGED = false, bool COVER = false, int CM = 1, int CN = 1>
+__device__ __attribute__((always_inline)) inline void publish_tile(const GemmKArgs& early, int tile_id, int lane) {
+  // (the arguments are read here, from the argument block: held in scalar registers across the K loop they would push others
+  // out.  The 256 x 128 tile, whose stores read theirs late already, spilled 17 registers so.)
+  typedef const __attribute__((address_space(4))) GemmKArgs* KernArgPtr;
+  KernArgPtr late_args = (KernArgPtr)__builtin_amdgcn_kernarg_segment_ptr();
+  constexpr bool LATE = COVER && !(MERGED && CM == 256 && CN == 128);
+  if constexpr (LATE) asm volatile("" : "+s"(late_args));
+  const GemmKArgs& p = LATE ? *(const GemmKArgs*)late_args : early;
   // the caller's tiles the launch's tile covers: itself, or (the MERGED builds, which only run launches whose
   // tiles are blocks of the caller's) merge_m x merge_n of them, fewer at the edges.  A build of its own: the
   // unmerged 256 x 256 kernel with these four scalars live across its K loop ran 4 % slower.
   constexpr bool merged = MERGED;
   int first = tile_id, rows = 1, cols = 1, pm0 = 0, pn0 = 0;
-  if constexpr (merged) {
-    const TileCoord t = tile_map_fast(tile_id, p.num_pid_m, p.num_pid_n, p.G, p.tile_divs);
-    pm0 = t.pid_m * p.merge_m;
-    pn0 = t.pid_n * p.merge_n + p.flag_pn_base;
-    rows = min(p.merge_m, p.flag_num_pid_m - pm0);
-    cols = min(p.merge_n, p.flag_num_pid_n - pn0);
-  }
-  if constexpr (PARTS) {
-    if (p.part_m * p.part_n > 1) {
+  bool across = false;
+  if constexpr (COVER) {
+    across = p.cover_bm > 0;
+    if (across) {
       const TileCoord t = tile_map_fast(tile_id, p.num_pid_m, p.num_pid_n, p.G, p.tile_divs);
-      const int pm = t.pid_m / p.part_m, pn = t.pid_n / p.part_n;
-      first = tile_id_of(pm, pn, p.flag_num_pid_m, p.flag_num_pid_n, p.G);
-      const int parts = min(p.part_m, p.num_pid_m - pm * p.part_m) * min(p.part_n, p.num_pid_n - pn * p.part_n);
-      // (the group's stores of the part have completed, written through: the part that counts last finds all of them.
-      // Flags that are releases need more than that, and launches with such flags are not run in parts: an arrival
-      // that can also release and acquire, here, cost the default launches 0.3 to 1 us, [823,1024] x [1024,1096] with 16-bit
-      // atomics 11.0 -> 12.0 a launch, by where it moved the compiler's scalar spills.)
-      IRIS_GLOBAL int32_t* cnt = (IRIS_GLOBAL int32_t*)(p.tile_arrivals + first);
-      int last = 0;
-      if (lane == 0) {
-        last = __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == parts - 1;
-        if (last) __hip_atomic_store(cnt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
-      }
-      if (!__builtin_amdgcn_readfirstlane(last)) return;
+      const int m0 = t.pid_m * CM, n0 = t.pid_n * CN;
+      pm0 = (int)fast_div((uint32_t)m0, p.div_cover_m);
+      pn0 = (int)fast_div((uint32_t)n0, p.div_cover_n);
+      rows = (int)fast_div((uint32_t)(min(p.M, m0 + CM) - 1), p.div_cover_m) - pm0 + 1;
+      cols = (int)fast_div((uint32_t)(min(p.N, n0 + CN) - 1), p.div_cover_n) - pn0 + 1;
+    }
+  }
+  if constexpr (merged) {
+    if (!across) {
+      const TileCoord t = tile_map_fast(tile_id, p.num_pid_m, p.num_pid_n, p.G, p.tile_divs);
+      pm0 = t.pid_m * p.merge_m;
+      pn0 = t.pid_n * p.merge_n + p.flag_pn_base;
+      rows = min(p.merge_m, p.flag_num_pid_m - pm0);
+      cols = min(p.merge_n, p.flag_num_pid_n - pn0);
     }
   }
   for (int i = 0; i < rows; ++i)
     for (int j = 0; j < cols; ++j) {
-      if constexpr (merged) first = tile_id_of(pm0 + i, pn0 + j, p.flag_num_pid_m, p.flag_num_pid_n, p.G);
+      IRIS_GLOBAL int32_t* word = nullptr;
+      int back = 0;
+      if (merged || (COVER && across)) first = tile_id_of(pm0 + i, pn0 + j, p.flag_num_pid_m, p.flag_num_pid_n, p.G);
+      if constexpr (COVER) {
+        if (across) {
+          // (the group's stores have completed, written through: the group that counts last finds all of them.
+          // Flags that are releases need more than that, and launches with such flags are not run so: an arrival
+          // that can also release and acquire, here, cost the default launches 0.3 to 1 us, [823,1024] x [1024,1096] with 16-bit
+          // atomics 11.0 -> 12.0 a launch, by where it moved the compiler's scalar spills.)
+          const int r0 = (pm0 + i) * p.cover_bm, r1 = min(p.M, r0 + p.cover_bm) - 1, c0 = (pn0 + j) * p.cover_bn, c1 = min(p.N, c0 + p.cover_bn) - 1;
+          const int parts = (int)((uint32_t)r1 / CM - (uint32_t)r0 / CM + 1) * (int)((uint32_t)c1 / CN - (uint32_t)c0 / CN + 1);
+          word = (IRIS_GLOBAL int32_t*)(p.tile_arrivals + (first >> p.arrive_pack));
+          const int shift = p.arrive_pack ? (first & 3) * 8 : 0, most = p.arrive_pack ? 0xFF : 0x7FFFFFFF;
+          int last = 0;
+          if (lane == 0) {
+            const uint32_t before = (uint32_t)__hip_atomic_fetch_add(word, 1 << shift, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            last = (int)(before >> shift & most) == parts - 1;
+          }
+          if (!__builtin_amdgcn_readfirstlane(last)) continue;
+          back = parts << shift;
+        }
+      }
       IRIS_GLOBAL int32_t* own = (IRIS_GLOBAL int32_t*)(p.flags + first);
       for (int r = lane; r < p.ws; r += 64) {
         if ((p.flag_mode & FLAG_MODE_MASK) == 2 && r == p.cur_rank) continue;
         IRIS_GLOBAL int32_t* f = own;
         if (r != p.cur_rank && p.heap_bases != nullptr)
-          f = translate(p.flags + first, p.heap_bases[p.cur_rank], p.heap_bases[r]);
+          f = translate(p.flags + first, ((const IRIS_GLOBAL uint64_t*)p.heap_bases)[p.cur_rank], ((const IRIS_GLOBAL uint64_t*)p.heap_bases)[r]);
         if (p.flag_mode & FLAG_RELEASE)
           flag_add_release(f, 1, p.sys != 0);  // gemm_one_shot_all_reduce.py:207-218 verbatim
         else
           flag_add_relaxed(f, 1, p.sys != 0);
       }
+      // the count back to zero for the next launch, behind the flags: in front of them the bases above, which return in
+      // order, waited for it (a word by a store: an atomic on the heap's memory takes 0.6 us longer)
+      if constexpr (COVER)
+        if (across && lane == 0) {
+          if (p.arrive_pack)
+            __hip_atomic_fetch_add(word, -back, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          else
+            __hip_atomic_store(word, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
     }
 }
 
@@ -1601,6 +1639,7 @@ enum WaveRole { ROLE_ANY, ROLE_WORKER, ROLE_FETCH_A, ROLE_FETCH_A_ACROSS, ROLE_F
 template <class Cfg, int OP, int ODT, bool SPLIT, bool FUSED, bool MERGED, int ROLE>
 __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKArgs& p) {
   static_assert(!MERGED || !FUSED, "blocks of the caller's tiles: no build with the reduce inside");
+  constexpr bool COVER = covers<Cfg, SPLIT, MERGED>;
   touch_args<sizeof(GemmKArgs)>();
   extern __shared__ __attribute__((aligned(1024))) char lds_raw[];
   IRIS_LDS char* lds = (IRIS_LDS char*)lds_raw;
@@ -1763,7 +1802,7 @@ __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKAr
       // a one-step tile: the previous tile has not been published yet
       IRIS_WAIT_VMCNT(0);
       __syncthreads();
-      if (wave == 0) publish_tile<MERGED, Cfg::PARTS>(p, pending_tile, lane);
+      if (wave == 0) publish_tile<MERGED, COVER, Cfg::CM, Cfg::CN>(p, pending_tile, lane);
       pending_tile = -1;
     }
     // (fp32 atomics) every part adds its own sum up where the tile's would go: no hand-over, nobody waits
@@ -1841,7 +1880,7 @@ __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKAr
           before = __builtin_amdgcn_readfirstlane(before);
           if (before == parts - 1) {
             // every slice is in memory: publish, and leave both counters at 0
-            if (p.flag_mode != 0) publish_tile<MERGED, Cfg::PARTS>(p, c_it.tile_id, lane);
+            if (p.flag_mode != 0) publish_tile<MERGED, COVER, Cfg::CM, Cfg::CN>(p, c_it.tile_id, lane);
             if (lane == 0) {
               flag_add_relaxed(done, -parts, false);
               flag_add_relaxed((IRIS_GLOBAL int32_t*)(p.locks + slot0), -parts, false);
@@ -1914,7 +1953,7 @@ __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKAr
         __syncthreads();
         int ok = 1;
         if (p.ws > 1) {
-          if (wave == 0) publish_tile<MERGED, Cfg::PARTS>(p, c_it.tile_id, lane);  // +1 on every other rank (:207-218)
+          if (wave == 0) publish_tile<MERGED, COVER, Cfg::CM, Cfg::CN>(p, c_it.tile_id, lane);  // +1 on every other rank (:207-218)
           if (tid == 0) {
             *slot = !peers_gone && wait_tile_flag((IRIS_GLOBAL int32_t*)(p.flags + c_it.tile_id), p.ws, p.sys != 0,
                                                   p.timeout, p.status)
@@ -1947,7 +1986,7 @@ __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKAr
       } else if (p.flag_mode != 0) {
         IRIS_WAIT_VMCNT(0);  // this wave's stores of the tile have completed
         __syncthreads();
-        if (wave == 0) publish_tile<MERGED, Cfg::PARTS>(p, c_it.tile_id, lane);
+        if (wave == 0) publish_tile<MERGED, COVER, Cfg::CM, Cfg::CN>(p, c_it.tile_id, lane);
       }
       if (p.ts_end && tid == 0)
         __hip_atomic_fetch_max((IRIS_GLOBAL unsigned long long*)(p.ts_end + c_it.tile_id),
@@ -2167,7 +2206,7 @@ __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKAr
         if constexpr (!LEAN) {
           if (pend >= 0) {
             if (skip == 0) {
-              if (wave == 0) publish_tile<MERGED, Cfg::PARTS>(p, pend, lane);
+              if (wave == 0) publish_tile<MERGED, COVER, Cfg::CM, Cfg::CN>(p, pend, lane);
               pending_tile = -1;
             } else {
               pending_skip = 0;
@@ -2364,7 +2403,7 @@ __device__ __attribute__((always_inline)) inline void gemm_program(const GemmKAr
   if (pending_tile >= 0) {
     IRIS_WAIT_VMCNT(0);
     __syncthreads();
-    if (wave == 0) publish_tile<MERGED, Cfg::PARTS>(p, pending_tile, lane);
+    if (wave == 0) publish_tile<MERGED, COVER, Cfg::CM, Cfg::CN>(p, pending_tile, lane);
   }
 }
 

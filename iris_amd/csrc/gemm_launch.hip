@@ -118,7 +118,8 @@ struct Plan {
   GemmKArgs k{};
   int fused_reduce = 0;  // ONE_SHOT, CONSUME on its own or IRIS_PHASE_TWO_KERNELS: follow with the reduce kernel
   int in_program = 0;    // ONE_SHOT, IRIS_PHASE_FUSED: the build of the kernel that reduces each tile itself
-  int parts = 0;         // the launch's tiles are parts of the caller's (plan_parts)
+  int one_per_cu = 0;    // (asked for) not two programs of a small tile a CU: they have no fetching waves, and no build that covers
+  int parts = 0;         // the launch's tiles lie across the caller's (plan_cover; 2: by plan_across)
   int loose = 0;         // the few-rows kernel's build for operands at any alignment
   int b_rows = 0;        // ... for a row-major B (cells)
   int two_kernels = 0;   // ... or, for such a launch too, what IRIS_PHASE_TWO_KERNELS would run (reduce_in_program)
@@ -702,26 +703,51 @@ double cells_us(const iris_gemm_args& a, int64_t cells, int parts, const Operand
          (o.atomic ? 0.4 : 0.0) + (k_time > 0 ? k_time : 0.0);
 }
 
-// The launch in parts of the caller's tiles, `cm` x `cn` each, every part with a program of its own in one round, K
-// shared out in split_k.  A caller's tile is the unit of a flag, not of work: the parts of a tile count their arrivals in
-// the caller's locks (`words` of them), and the last one raises its flag.
-bool plan_parts(const iris_gemm_args& a, int cm, int cn, int split_k, int64_t words, Plan* plan) {
+// Words of the caller's locks in which its `tiles` tiles count arrivals, one each (pack 0) or four to a word (2).
+int64_t arrival_words(int64_t tiles, int pack) { return pack ? (tiles + 3) / 4 : tiles; }
+
+// Whether tiles of cm x cn may lie across the caller's: a lane for each of the caller's that one of them touches, a byte for
+// their number in one of the caller's.
+bool can_cover(const iris_gemm_args& a, int cm, int cn) {
+  const int64_t touched = ((int64_t)(cm - 1) / a.block_m + 2) * ((cn - 1) / a.block_n + 2);
+  const int64_t parts = ((int64_t)(a.block_m - 1) / cm + 2) * ((a.block_n - 1) / cn + 2);
+  return touched <= 64 && parts <= 255;
+}
+
+// The launch in tiles of cm x cn, K shared out in split_k.  A caller's tile is the unit of a flag, not of work: the tiles that share
+// one of the caller's count their arrivals in the caller's locks (the last `words` of them), and the last one raises its flag.
+bool plan_cover(const iris_gemm_args& a, int cm, int cn, int split_k, int64_t words, int pack, Plan* plan) {
   iris_gemm_args b = a;
   b.block_m = cm;
   b.block_n = cn;
   b.variant = IRIS_GEMM_VARIANT_PERSISTENT;
   b.split_k = split_k;
+  // (slots of this tile's size, as many as the workspace holds)
+  const int64_t items = ((int64_t)a.M + cm - 1) / cm * (((int64_t)a.N + cn - 1) / cn) * split_k;
+  // (and the parts of a tile's K count in the locks, too)
+  if (words > a.num_sms || (split_k > 1 && items + words > a.num_sms)) return false;
+  if (split_k > 1 && a.partials && a.partials_slot_elems < (int64_t)cm * cn)
+    b.partials_slot_elems = (int64_t)a.num_sms * a.partials_slot_elems / items & ~(int64_t)3;
+  plan->one_per_cu = 1;
   if (make_plan_body(b, plan) != hipSuccess) return false;
   GemmKArgs& k = plan->k;
-  if (!plan->entry || plan->entry->cm != cm || plan->entry->cn != cn || k.sub_m != 1 || k.sub_n != 1 ||
-      plan->entry->fetch_waves == 0 || k.num_sms != a.num_sms)
+  if (!plan->entry || plan->entry->cm != cm || plan->entry->cn != cn || k.sub_m != 1 || k.sub_n != 1 || k.num_sms != a.num_sms ||
+      plan->in_program)
     return false;
   own_flags(plan);
   k.flag_num_pid_m = (a.M + a.block_m - 1) / a.block_m;
   k.flag_num_pid_n = (a.N + a.block_n - 1) / a.block_n;
   if (words > 0) {
-    k.part_m = a.block_m / cm;
-    k.part_n = a.block_n / cn;
+    const GemmKernelEntry* e = plan->entry;
+    const bool small = cm <= 128 && cn <= 128 && e->fetch_waves != 0;
+    if (!small && !(split_k > 1 ? e->fn_split_merged : e->fn_merged)) return false;
+    if (cm == 256 && cn == 128 && split_k == 1 && (e->b_rows || e->loose)) return false;  // (`covers`)
+    plan->remap_flags = small ? 0 : 1;
+    k.cover_bm = a.block_m;
+    k.cover_bn = a.block_n;
+    k.arrive_pack = pack;
+    k.div_cover_m = make_fast_div((uint32_t)a.block_m, (uint64_t)a.M);
+    k.div_cover_n = make_fast_div((uint32_t)a.block_n, (uint64_t)a.N);
     k.tile_arrivals = a.locks + (a.num_sms - words);
   }
   plan->parts = 1;
@@ -789,7 +815,7 @@ bool plan_small(const iris_gemm_args& a, Plan* plan) {
   double times[8];
   int count = 0;
   for (const auto& s : shapes) {
-    if (a.block_m % s[0] != 0 || a.block_n % s[1] != 0) continue;
+    if (a.block_m % s[0] != 0 || a.block_n % s[1] != 0 || !can_cover(a, s[0], s[1])) continue;
     const int64_t tiles = tiles_of(s[0], s[1]);
     if (tiles > a.num_sms) continue;
     if (s[0] == a.block_m && s[1] == a.block_n) break;  // (the caller's tile is the smallest that fits)
@@ -814,7 +840,7 @@ bool plan_small(const iris_gemm_args& a, Plan* plan) {
       if (times[i] < least && (best < 0 || times[i] < times[best])) best = i;
     if (best < 0) return found;
     Plan parts;
-    if (plan_parts(a, list[best].cm, list[best].cn, list[best].split_k, words, &parts)) {
+    if (plan_cover(a, list[best].cm, list[best].cn, list[best].split_k, words, 0, &parts)) {
       *plan = parts;
       return true;
     }
@@ -860,7 +886,7 @@ bool reduce_in_program(const iris_gemm_args& a, const Plan& producer) {
   if ((rows || loose) && producer.parts && tiles <= a.num_sms && k.vec_out && a.block_m * a.block_n <= 128 * 128 && steps <= 4 &&
       strips < (wide ? (256 << 10) + 1 : 256 << 10))
     return true;
-  if ((producer.skinny && producer.skinny_cb == 1) || producer.last_round || producer.rest || producer.parts) return false;
+  if ((producer.skinny && producer.skinny_cb == 1) || producer.last_round || producer.rest || producer.parts == 1) return false;
   // (cells: the caller's tiles inside, when they are as small as the parts they would be run in)
   if (producer.skinny && a.block_m * a.block_n > 64 * 64) return false;
   if (k.split_k > 1 || k.merge_m * k.merge_n > 1 || k.total_tiles > a.num_sms || !k.vec_out) return false;
@@ -1237,6 +1263,109 @@ void plan_atomics(const iris_gemm_args& a, Plan* plan) {
   }
 }
 
+// Times of a launch with flags in us, for tiles that need not divide the caller's: fixed + rounds of tiles + the other copies of the
+// output + the hand-over of a shared K, which grows with the partials that cross memory (MB) and with the parts; `step`: 64 units of
+// K of a tile, dearer as BlockTime's are.  Fitted to two thirds of 11000 timings of 600 random
+// calls ([33 .. 8192, 128 .. 36864] x [.., 128 .. 8192], 16-bit and fp32, weights in rows of either direction and at any alignment, up to eight
+// copies, operands changed from launch to launch), rms 13 % on the rest.
+struct AcrossTime {
+  int cm, cn;
+  double tile, step, step_f32;  // (0: no such tile)
+};
+constexpr AcrossTime ACROSS_TIMES[] = {
+    {64, 64, 2.55, 0.153, 0.486}, {128, 64, 2.99, 0.245, 0.000}, {64, 128, 2.72, 0.256, 0.913}, {128, 128, 3.63, 0.343, 1.701},
+    {256, 64, 3.75, 0.409, 0.000}, {256, 128, 5.07, 0.528, 0.000}, {256, 256, 6.20, 0.918, 0.000},
+};
+struct AcrossLaunch {
+  double streamed, kind;
+  int copies;  // of the output, in 16-bit elements
+  bool f32, lines;
+};
+double across_us(const iris_gemm_args& a, const AcrossTime& t, int parts, const AcrossLaunch& l) {
+  const int64_t items = ((int64_t)a.M + t.cm - 1) / t.cm * (((int64_t)a.N + t.cn - 1) / t.cn) * parts;
+  const int64_t rounds = (items + a.num_sms - 1) / a.num_sms, nk = ((int64_t)a.K + 63) / 64, steps = (nk + parts - 1) / parts;
+  const double busy = rounds > 1 ? 1.0 : (double)items / a.num_sms, area = (double)t.cm * t.cn / 4096;
+  const double step = (l.f32 ? t.step_f32 * (1 + 0.059 * busy) : t.step * (1 + 0.112 * busy) * (1 + 0.404 * l.streamed)) * (l.lines ? 1.0 : 1.223) * l.kind;
+  const double loop = t.tile + steps * step, store = area / parts * 0.377 * (l.copies - 1) * (busy > 0.37 ? busy : 0.37);
+  const double mb = items * area / 64, low = mb < 16 ? mb : 16;
+  const double hand = parts > 1 ? 3.210 + 0.417 * area + 0.114 * low + 0.092 * (mb - low) + 0.151 * parts : 0;
+  return 3.946 + 0.920 * busy + rounds * loop + store * (1 + (rounds - 1) * 0.67) + hand;
+}
+
+// Replaces the plan of a launch in tiles where tiles of another size, that lie across the caller's (plan_cover), are expected to be
+// faster by more than an eighth.  (us, the caller's tiles or what the plans above made of
+// them / so: fp32 [1972,448] x [448,696] in 256 x 256 tiles, whose 128 x 128 ones a program computes in turn, 136 / 25; [2152,22464] x
+// [22464,384] in 256 x 256 tiles 105 / 59; [668,16256] x [16256,960] in 256 x 64 55 / 41; [916,2240] x [2240,5184] in 256 x 256 46 / 29;
+// [108,27664] x [27664,4032] in 256 x 64 137 / 74.  Of 370 random calls in tiles 45 change, 1.024x on average over all of them; slower
+// by more than 3 %: two, by 5 %.  Small tiles two to a CU are not in the fit: only where K is long.)
+void plan_across(const iris_gemm_args& a, Plan* plan) {
+  const GemmKernelEntry* own = plan->entry;
+  if (!own || plan->skinny || plan->in_program || plan->last_round || plan->rest || plan->k.stream_k) return;
+  if (a.epilogue == IRIS_EPI_ATOMIC_ADD || a.variant != 0 || a.split_k != 0 || a.mm_begin_timestamp || a.mm_end_timestamp) return;
+  if (a.num_sms != current_cu_count() || a.K <= 0) return;
+  const bool flags = a.epilogue == IRIS_EPI_ALL_SCATTER ? a.notify != 0 : a.world_size > 1;
+  const int64_t own_tiles = flags ? ((int64_t)a.M + a.block_m - 1) / a.block_m * (((int64_t)a.N + a.block_n - 1) / a.block_n) : 0;
+  const int64_t least = arrival_words(own_tiles, 2);  // (words that the arrivals need)
+  if (flags && (!a.locks || least > a.num_sms || a.flag_sem == IRIS_FLAG_SEM_RELEASE_ACQUIRE)) return;
+  const bool scatter = a.epilogue == IRIS_EPI_ALL_SCATTER;
+  AcrossLaunch l;
+  const double mb = ((double)a.M + a.N) * a.K * 2e-6;
+  l.streamed = mb < 50 ? 0 : mb > 150 ? 1 : (mb - 50) / 100;
+  l.kind = !own->dma ? 1.368 : own->loose ? 1.177 : own->b_rows ? 1.023 : 1.0;
+  l.copies = (scatter ? a.world_size : 1) * ((scatter ? a.c_global_dtype : a.c_dtype) == IRIS_DTYPE_F32 ? 2 : 1);
+  l.f32 = a.ab_dtype == IRIS_DTYPE_F32;
+  l.lines = whole_lines(a);
+  constexpr int TILES = sizeof(ACROSS_TIMES) / sizeof(ACROSS_TIMES[0]);
+  double own_us = -1;
+  for (const AcrossTime& t : ACROSS_TIMES)
+    if (t.cm == own->cm && t.cn == own->cn && !(l.f32 && t.step_f32 == 0)) own_us = across_us(a, t, plan->k.split_k, l);
+  if (plan->k.num_sms != a.num_sms && a.K < 2048) return;
+  const int own_parts = plan->k.split_k;
+  // (what the times above are not good for: K in this many parts, and small tiles that share it, whose operands the L2s hold)
+  if (own_parts > 12 || (own_parts > 2 && own->cm * own->cn == 64 * 64)) return;
+  if (own_us < 12) return;  // (another tile than these, or nothing to gain that the search would not cost)
+  double best_us[TILES];
+  int best_parts[TILES];
+  const int64_t room = a.partials && a.locks && aligned16(a.partials) ? a.num_sms * a.partials_slot_elems : 0;
+  for (int i = 0; i < TILES; ++i) {
+    const AcrossTime& t = ACROSS_TIMES[i];
+    best_us[i] = 1e30;
+    if ((l.f32 && t.step_f32 == 0) || !can_cover(a, t.cm, t.cn)) continue;
+    const int64_t tiles = ((int64_t)a.M + t.cm - 1) / t.cm * (((int64_t)a.N + t.cn - 1) / t.cn), elems = tiles * t.cm * t.cn;
+    if (tiles > 4 * (int64_t)a.num_sms) continue;
+    int most = (int)((a.num_sms - least) / tiles);
+    if (most > 12) most = 12;
+    if (most > (a.K + 63) / 64 / 4) most = (a.K + 63) / 64 / 4;
+    for (int parts = 1; parts == 1 || parts <= most; parts += parts < 4 || parts + 2 > most ? 1 : 2) {
+      // (two parts of a tile of 128 accumulators hand half of it over each)
+      const bool half = parts == 2 && t.cm * t.cn >= 256 * 128;
+      // (K of a 128 x 128 tile stays shared out rather than the tile cut, as plan_small has it)
+      if (parts == 1 && own_parts > 1 && a.block_m < 256 && t.cm * t.cn < own->cm * own->cn) continue;
+      if (parts > 1 && elems * parts > room * (half ? 2 : 1)) break;
+      const double us = across_us(a, t, parts, l);
+      if (us < best_us[i]) best_us[i] = us, best_parts[i] = parts;
+    }
+  }
+  // the least of them that there is a kernel for
+  for (;;) {
+    int i = 0;
+    for (int j = 1; j < TILES; ++j)
+      if (best_us[j] < best_us[i]) i = j;
+    const AcrossTime& t = ACROSS_TIMES[i];
+    if (best_us[i] > 0.87 * own_us) return;
+    // (a word for each of the caller's tiles where they have room beside those of the parts of K)
+    const int64_t used = best_parts[i] > 1 ? ((int64_t)a.M + t.cm - 1) / t.cm * (((int64_t)a.N + t.cn - 1) / t.cn) * best_parts[i] : 0;
+    const int pack = used + own_tiles <= a.num_sms ? 0 : 2;
+    Plan across;
+    if (plan_cover(a, t.cm, t.cn, best_parts[i], arrival_words(own_tiles, pack), pack, &across) && across.k.split_k == best_parts[i] && (across.entry->dma || !own->dma)) {
+      across.parts = 2;
+      *plan = std::move(across);
+      return;
+    }
+    best_us[i] = 1e30;
+  }
+}
+
 hipError_t make_plan_tiles(const iris_gemm_args& a, Plan* plan) {
   if (a.epilogue == IRIS_EPI_ONE_SHOT && a.phase == IRIS_PHASE_FUSED) {
     iris_gemm_args b = a;
@@ -1253,18 +1382,23 @@ hipError_t make_plan_tiles(const iris_gemm_args& a, Plan* plan) {
   }
   if (plan_small(a, plan)) {
     plan_atomics(a, plan);
+    plan_across(a, plan);
     return hipSuccess;
   }
   const bool plain = a.variant == 0 && a.split_k == 0 && !a.mm_begin_timestamp && !a.mm_end_timestamp &&
                      !(a.epilogue == IRIS_EPI_ONE_SHOT && a.phase != IRIS_PHASE_PRODUCE && a.phase != IRIS_PHASE_TWO_KERNELS) &&
                      a.epilogue != IRIS_EPI_ATOMIC_ADD && a.num_sms > 0 && (a.block_m == 128 || a.block_m == 256) &&
                      (a.block_n == 64 || a.block_n == 128) && a.M >= 256;
-  if (plain && plan_blocks(a, plan)) return hipSuccess;
+  if (plain && plan_blocks(a, plan)) {
+    plan_across(a, plan);
+    return hipSuccess;
+  }
   const hipError_t err = make_plan_body(a, plan);
   own_flags(plan);
   if (err == hipSuccess) {
     split_last_round(a, plan);
     plan_atomics(a, plan);
+    plan_across(a, plan);
   }
   return err;
 }
@@ -1511,7 +1645,7 @@ hipError_t make_plan_body(const iris_gemm_args& a, Plan* plan, bool cells) {
   // the plain tile of the same shape: [512,1376] x [1376,4096] 20.6 -> 17.1 us.)
   const GemmKernelEntry* twin = a.variant > 0 ? nullptr : plain_twin(list, count, *pick);
   const bool two_ok = pick->fetch_waves == 0 || twin;
-  if (!plan->in_program && k.split_k == 1 && two_ok && (twin ? twin : pick)->lds_bytes * 2 <= 160 * 1024 &&
+  if (!plan->in_program && !plan->one_per_cu && k.split_k == 1 && two_ok && (twin ? twin : pick)->lds_bytes * 2 <= 160 * 1024 &&
       a.num_sms >= current_cu_count() && a.num_sms <= 2 * current_cu_count() && items >= 2 * (int64_t)a.num_sms &&
       !a.mm_begin_timestamp && !a.mm_end_timestamp) {
     k.num_sms = 2 * a.num_sms;
@@ -1744,7 +1878,7 @@ extern "C" int iris_gemm_launch_noalloc(const iris_gemm_args* args, void* stream
   // wait that timed out leaves one raised).  A fill kernel, not a memset, so
   // that the call can be recorded into a HIP graph.
   auto needs_locks = [](const Plan& q) {
-    return (q.skinny && (q.k.flag_mode != 0 || q.skinny_grid_z > 1)) || q.k.part_m * q.k.part_n > 1 || (q.entry && (q.k.split_k > 1 || q.k.stream_k || q.last_round));
+    return (q.skinny && (q.k.flag_mode != 0 || q.skinny_grid_z > 1)) || q.k.cover_bm > 0 || (q.entry && (q.k.split_k > 1 || q.k.stream_k || q.last_round));
   };
   const bool uses_locks = needs_locks(plan) || (plan.rest && needs_locks(*plan.rest));
   if (uses_locks) {
@@ -1820,7 +1954,7 @@ extern "C" int iris_gemm_plan_name(const iris_gemm_args* args, char* buf, size_t
   }
   if (plan.parts) {
     const size_t n = std::strlen(buf);
-    std::snprintf(buf + n, len > n ? len - n : 0, "+parts_of_tiles");
+    std::snprintf(buf + n, len > n ? len - n : 0, plan.parts == 2 ? "+across_the_tiles" : "+parts_of_tiles");
   }
   if (plan.two_kernels || (plan.reduces && args->phase == IRIS_PHASE_FUSED)) {
     const size_t n = std::strlen(buf);
