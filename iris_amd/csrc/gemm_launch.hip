@@ -1145,7 +1145,8 @@ hipError_t make_plan_units(const iris_gemm_args& a, Plan* plan) {
 
 // A launch with atomics has no flags, so nothing shows which tiles it ran in: any tile will do, not only one that divides the
 // caller's, and with fp32 atomics K may be shared out over programs that each add their own sums, with no hand-over and
-// nobody waiting.  (16-bit atomics would round every part's sum on its way in: they keep whole sums.)
+// nobody waiting.  (16-bit atomics would round every part's sum on its way in: they keep whole sums.  So do launches whose
+// ranks are other GPUs: each part's sums would cross the links, and the rate below is the one GPU's.)
 //
 // Times of such a launch in us: fixed + the first tile + the others, each as long as its K loop or its atomics (the chip adds
 // 331 G a second, a CU a 64 x 64 tile in 1.1 us) + the last tile's atomics; `step`: 64 units of K of a tile, dearer by the same
@@ -1205,7 +1206,8 @@ void plan_atomics(const iris_gemm_args& a, Plan* plan) {
   if (a.epilogue != IRIS_EPI_ATOMIC_ADD || !own || plan->skinny || plan->k.stream_k) return;
   if (a.variant != 0 || a.split_k != 0 || a.mm_begin_timestamp || a.mm_end_timestamp || a.num_sms != current_cu_count() || a.K <= 0) return;
   const bool wide = a.c_global_dtype == IRIS_DTYPE_F32, handed = plan->k.split_k > 1;
-  if (!wide && handed) return;
+  const bool parts_add = wide && (a.scope != IRIS_SCOPE_SYSTEM || a.world_size <= 1);
+  if (!parts_add && handed) return;
   AtomicLaunch l;
   const double mb = ((double)a.M + a.N) * a.K * 2e-6;
   l.streamed = mb < 50 ? 0 : mb > 150 ? 1 : (mb - 50) / 100;
@@ -1231,7 +1233,7 @@ void plan_atomics(const iris_gemm_args& a, Plan* plan) {
     if (l.f32 && t.step_f32 == 0) continue;
     const int64_t tiles = ((int64_t)a.M + t.cm - 1) / t.cm * (((int64_t)a.N + t.cn - 1) / t.cn);
     if (tiles > 4 * (int64_t)a.num_sms) continue;
-    int most = wide ? (int)(a.num_sms / tiles) : 1;
+    int most = parts_add ? (int)(a.num_sms / tiles) : 1;
     if (most > 16) most = 16;
     if (most > (a.K + 63) / 64 / 3) most = (a.K + 63) / 64 / 3;
     for (int parts = 1; parts == 1 || parts <= most; parts += parts < 4 || parts + 2 > most ? 1 : 2) {

@@ -143,3 +143,12 @@ def test_where_operands_that_are_gathered_inside_are_reduced(M, N, K, BM, BN, ws
     name, _ = plan(M, N, K, BM, BN, ws=ws, epilogue=ops.EPI_ONE_SHOT, phase=ops.PHASE_FUSED, c=9 << 32, stride_cm=N, stride_cn=1,
                    stride_cm_global=N, **kw)
     assert name.endswith("+kernel+reduce") != inside, name
+
+
+@pytest.mark.parametrize("M,N,K,BM,BN", [(828, 2688, 20672, 256, 64), (2023, 192, 22656, 256, 128)])
+def test_atomics_to_other_gpus_add_whole_sums(M, N, K, BM, BN):
+    """Parts of K that each add their own sums would send all of them over the links; ranks of one GPU take them.  (Without
+    a workspace K is not shared out in any other way.)"""
+    kw = dict(epilogue=ops.EPI_ATOMIC_ADD, c_global_dtype=F32, ws=2, partials=0, locks=0)
+    assert plan(M, N, K, BM, BN, **kw)[1] > 1
+    assert plan(M, N, K, BM, BN, scope=ops.SCOPE_SYSTEM, **kw)[1] == 1
