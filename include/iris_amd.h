@@ -94,8 +94,10 @@ int iris_hip_arch_name(int device, char* buf, size_t len);
                               * IRIS_PHASE_TWO_KERNELS.  Results and flags are the same. */
 #define IRIS_PHASE_TWO_KERNELS 7 /* both, no tile's reduce holding up another tile's product: the producer GEMM, then the
                                   * reduce kernel (iris_one_shot_reduce_launch) behind it on the stream.  A product of few
-                                  * rows, or in cells, of up to 128 small tiles is one kernel that reduces as it stores and
-                                  * in which at most one workgroup a tile waits for the peers. */
+                                  * rows, or in cells, of up to 128 small tiles is one kernel that reduces as it stores.  In
+                                  * it at most 7 / (world_size - 1) workgroups of a shader engine wait for the peers at a
+                                  * time, so that all ranks but one, waiting on this device, leave that one a CU of each
+                                  * engine; more than eight ranks: two kernels (iris_gemm_launch_kernels says which). */
 
 /* flag scopes */
 #define IRIS_SCOPE_AGENT 0  /* all "ranks" live on this GPU */
@@ -281,6 +283,11 @@ int iris_gemm_split_k(const iris_gemm_args* args, int* split_k);
  * them (partials and locks as above), and by "+kernel+reduce" where an IRIS_PHASE_FUSED launch runs as an
  * IRIS_PHASE_TWO_KERNELS one. */
 int iris_gemm_plan_name(const iris_gemm_args* args, char* buf, size_t len);
+
+/* What `iris_gemm_launch` would put on the stream for `args`: the number of kernels (one where a launch with a reduce reduces
+ * inside its product's kernel, two where a reduce kernel follows), and the most workgroups of the product's kernel that wait
+ * for other ranks' flags at a time, holding their LDS (0 where the product waits for nobody).  Either pointer may be NULL. */
+int iris_gemm_launch_kernels(const iris_gemm_args* args, int* kernels, int* waiting);
 
 /* Name of tuning variant `variant` (1-based) of the kernel list used for
  * (ab_dtype, fp32 output?, atomic?); hipErrorInvalidValue past the end. */

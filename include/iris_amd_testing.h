@@ -75,6 +75,14 @@ int iris_rma_selftest_launch(int32_t op, int32_t dtype, int32_t sem, int32_t sco
                              const uint64_t* heap_bases, int32_t cur_rank, int32_t num_ranks, int32_t block_size,
                              void* stream);
 
+/*
+ * Which workgroups wait for late peers (late_tiles.hpp): the word that an XCD's workgroups share, after one has come upon
+ * the late tile `tile` where `most` may wait, and after one is done with its own and takes the tile left last, whose own
+ * word holds `link`.
+ */
+int32_t iris_late_join_host(int32_t word, int32_t most, int32_t tile);
+int32_t iris_late_next_host(int32_t word, int32_t link);
+
 #ifdef __cplusplus
 }
 #endif

@@ -145,6 +145,7 @@ SIGNATURES = {
     "iris_gemm_split_k": (_I, [ctypes.POINTER(GemmArgs), ctypes.POINTER(_I)]),
     "iris_gemm_variant_name": (_I, [_I, _I, _I, _I, ctypes.c_char_p, ctypes.c_size_t]),
     "iris_gemm_plan_name": (_I, [ctypes.POINTER(GemmArgs), ctypes.c_char_p, ctypes.c_size_t]),
+    "iris_gemm_launch_kernels": (_I, [ctypes.POINTER(GemmArgs), ctypes.POINTER(_I), ctypes.POINTER(_I)]),
     "iris_one_shot_reduce_launch": (_I, [ctypes.POINTER(ReduceArgs), _P]),
     "iris_signal_tiles_launch": (_I, [_P, _P, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32,
                                       ctypes.c_int32, _P]),
@@ -160,6 +161,8 @@ SIGNATURES = {
 ALLOCATOR_SYMBOLS = ("finegrained_hipMalloc", "finegrained_hipFree")
 # every symbol include/iris_amd_testing.h declares for libiris_amd_testing.so
 TESTING_SIGNATURES = {
+    "iris_late_join_host": (ctypes.c_int32, [ctypes.c_int32] * 3),
+    "iris_late_next_host": (ctypes.c_int32, [ctypes.c_int32] * 2),
     "iris_mfma_probe_launch": (_I, [_P, _P, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, _P]),
     "iris_store_probe_launch": (_I, [_P, _P, _P, ctypes.c_uint64] + [ctypes.c_int32] * 5 + [_P]),
     "iris_rma_selftest_launch": (_I, [ctypes.c_int32] * 4 + [_P, _P, _P] + [ctypes.c_int32] * 3 + [_P]),

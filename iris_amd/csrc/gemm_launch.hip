@@ -1106,10 +1106,13 @@ bool plan_blocks(const iris_gemm_args& a, Plan* plan) {
 }
 
 // Few rows and cells with a reduce behind them: the reduce in the same kernel (gemm_skinny.hpp, REDUCE), where a tile is small
-// enough for one workgroup to reduce it should its peers be late, and few enough workgroups may come to wait for theirs.
+// enough for one workgroup to reduce it should its peers be late, and there are few enough tiles for that.
 // One workgroup has 32 KB of partials in flight, so a late tile of REDUCE_MAX_BYTES is four round trips to memory, about what a reduce
-// kernel's launch and chain take.  Waiting workgroups hold LDS that a peer on this device needs: REDUCE_MAX_TILES of them, of the
-// device's 256 (cells) to 768 places.  Not for a launch that shares the device with its peers' (fewer programs than CUs).
+// kernel's launch and chain take.  Waiting workgroups hold LDS that a peer on this device needs: late_tiles.hpp says how many of
+// them wait at a time, of however many ranks; the others leave their tiles to those, up to REDUCE_MAX_TILES (of eight ranks one
+// on a shader engine waits, on 32: four tiles one after the other).  The words for that, one an engine, are the last of the
+// caller's locks.  Up to eight ranks (a wave each fetches their strips), of which late_most has one wait.  Not for
+// a launch that shares the device with its peers' by its number of programs (fewer than CUs).
 bool reduce_in_few_rows(const iris_gemm_args& a, Plan* plan) {
   GemmKArgs& k = plan->k;
   if (!plan->skinny || !plan->fused_reduce || a.epilogue != IRIS_EPI_ONE_SHOT || a.world_size < 2) return false;
@@ -1122,6 +1125,13 @@ bool reduce_in_few_rows(const iris_gemm_args& a, Plan* plan) {
   const GemmKernelFn fn = gemm_skinny_kernel_for(a.ab_dtype, a.c_dtype == IRIS_DTYPE_F32 ? OP_STORE32 : OP_STORE16, plan->skinny_arows,
                                                  plan->skinny_rb, plan->skinny_cb, plan->loose != 0, plan->b_rows != 0, true);
   if (!fn) return false;
+  const int most = late_most(a.world_size);
+  if (most < 1 || a.world_size > SKINNY_WAVES) return false;
+  if (k.total_tiles > most) {
+    const int64_t counters = k.total_tiles + (plan->skinny_grid_z > 1 ? (int64_t)plan->skinny_grid * plan->skinny_grid_y : 0);
+    if (!a.locks || counters + LATE_ENGINES > a.num_sms) return false;
+    k.tile_arrivals = a.locks + (a.num_sms - LATE_ENGINES);
+  }
   plan->skinny = fn;
   plan->fused_reduce = 0;
   plan->reduces = 1;
@@ -1961,6 +1971,23 @@ extern "C" int iris_gemm_plan_name(const iris_gemm_args* args, char* buf, size_t
   if (plan.two_kernels || (plan.reduces && args->phase == IRIS_PHASE_FUSED)) {
     const size_t n = std::strlen(buf);
     std::snprintf(buf + n, len > n ? len - n : 0, plan.two_kernels ? "+kernel+reduce" : "+reduce");
+  }
+  return hipSuccess;
+}
+
+extern "C" int iris_gemm_launch_kernels(const iris_gemm_args* args, int* kernels, int* waiting) {
+  if (!args) return hipErrorInvalidValue;
+  Plan plan;
+  const hipError_t err = make_plan(*args, &plan);
+  if (err != hipSuccess) return err;
+  auto count = [](const Plan& q) { return q.skinny ? 1 : q.entry ? (q.last_round ? 2 : 1) : 0; };
+  // (a reduce of nothing is no kernel)
+  const bool behind = plan.fused_reduce && args->M > 0 && args->N > 0;
+  if (kernels) *kernels = count(plan) + (plan.rest ? count(*plan.rest) : 0) + (behind ? 1 : 0);
+  if (waiting) {
+    const int on_all_engines = LATE_ENGINES * late_most(args->world_size);
+    const int most = plan.reduces ? on_all_engines : plan.in_program && plan.entry && args->world_size > 1 ? plan.k.num_sms : 0;
+    *waiting = most < plan.k.total_tiles ? most : plan.k.total_tiles;
   }
   return hipSuccess;
 }

@@ -43,6 +43,7 @@
 #pragma once
 
 #include "gemm_registry.hpp"
+#include "late_tiles.hpp"
 
 namespace iris_amd {
 
@@ -100,6 +101,52 @@ __device__ __attribute__((always_inline)) inline void store_result4(const GemmKA
       store_through((IRIS_GLOBAL unsigned int*)d + e, wide[e], p.sys != 0);
     else
       store_through((IRIS_GLOBAL unsigned short*)d + e, (unsigned short)(half[e / 2] >> (16 * (e & 1))), p.sys != 0);
+  }
+}
+
+// The word of the shader engine that this workgroup runs on (late_tiles.hpp).
+__device__ inline IRIS_GLOBAL int32_t* late_word(const GemmKArgs& p) {
+  // (hwreg(HW_REG_HW_ID, 13, 3) and hwreg(HW_REG_XCC_ID, 0, 4))
+  const int engine = __builtin_amdgcn_s_getreg(4 | 13 << 6 | (3 - 1) << 11), xcd = __builtin_amdgcn_s_getreg(20 | (4 - 1) << 11);
+  return (IRIS_GLOBAL int32_t*)(p.tile_arrivals + ((xcd << 2 | (engine & 3)) & (LATE_ENGINES - 1)));
+}
+
+// Compare-and-swap that orders what this workgroup and the one it meets here have stored: `word` as it was.
+__device__ inline int32_t late_swap(IRIS_GLOBAL int32_t* at, int32_t word, int32_t to) {
+  __hip_atomic_compare_exchange_strong(at, &word, to, __ATOMIC_ACQ_REL, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
+  return word;
+}
+
+// One lane, for a tile whose peers are late: whether this workgroup waits for it (else one that waits already takes it).
+__device__ inline bool late_tile_enter(const GemmKArgs& p, int tile) {
+  if (p.tile_arrivals == nullptr) return true;  // (as many as may wait have a tile each)
+  IRIS_GLOBAL int32_t *at = late_word(p), *link = (IRIS_GLOBAL int32_t*)(p.locks + tile);
+  const int most = late_most(p.ws);
+  int32_t word = __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  for (;;) {
+    const bool waits = late_waits(word, most);
+    if (!waits) __hip_atomic_store(link, late_left(word), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int32_t seen = late_swap(at, word, late_join(word, most, tile));
+    if (seen == word) return waits;
+    word = seen;
+    if (!waits) __hip_atomic_store(link, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
+// One lane, done with a late tile: the next one (plus one), or zero.
+__device__ inline int late_tile_next(const GemmKArgs& p) {
+  IRIS_GLOBAL int32_t* at = late_word(p);
+  int32_t word = __hip_atomic_load(at, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
+  for (;;) {
+    const int tile = late_left(word);
+    IRIS_GLOBAL int32_t* link = (IRIS_GLOBAL int32_t*)(p.locks + (tile ? tile - 1 : 0));
+    const int32_t before = tile ? __hip_atomic_load(link, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+    const int32_t seen = late_swap(at, word, late_next(word, before));
+    if (seen == word) {
+      if (tile) __hip_atomic_store(link, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
+      return tile;
+    }
+    word = seen;
   }
 }
 
@@ -543,36 +590,28 @@ gemm_skinny_kernel(const GemmKArgs p) {
         }
       }
     }
-    if (peers_done) {
-      for (int r0 = 0;; r0 += SKINNY_WAVES) {
-        if (r0 + wave < p.ws && r0 + wave != p.cur_rank) {
-          if (r0 > 0) fetch_strips(r0 + wave);
+    if (peers_done) {  // (up to eight ranks, a wave each)
+      if (wave < p.ws && wave != p.cur_rank) {
 #pragma unroll
-          for (int b = 0; b < NB; ++b) {
-            f32x4 v = __builtin_bit_cast(f32x4, strip[b]);
-            if constexpr (!F32)
+        for (int b = 0; b < NB; ++b) {
+          f32x4 v = __builtin_bit_cast(f32x4, strip[b]);
+          if constexpr (!F32)
 #pragma unroll
-              for (int e = 0; e < 4; ++e) v[e] = from16<ODT>((unsigned short)(strip[b][e / 2] >> (16 * (e & 1))));
-            *reinterpret_cast<IRIS_LDS f32x4*>(wb + b * 1024 + lane * 16) = v;
-          }
+            for (int e = 0; e < 4; ++e) v[e] = from16<ODT>((unsigned short)(strip[b][e / 2] >> (16 * (e & 1))));
+          *reinterpret_cast<IRIS_LDS f32x4*>(wb + b * 1024 + lane * 16) = v;
         }
-        __syncthreads();
-        if (mine) {
-          for (int q = 0; q < SKINNY_WAVES && r0 + q < p.ws; ++q)
-#pragma unroll
-            for (int j = 0; j < CB; ++j) {
-              const f32x4 v = r0 + q == p.cur_rank
-                                  ? own[j]
-                                  : *reinterpret_cast<const IRIS_LDS f32x4*>(wb + (q - wave) * (UN * CB * SKINNY_BLOCK_BYTES) +
-                                                                             (wave * CB + j) * 1024 + lane * 16);
-              const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-              sum[j] = (r0 + q == 0 ? zero : sum[j]) + v;
-            }
-        }
-        if (r0 + SKINNY_WAVES >= p.ws) break;
-        __syncthreads();  // the strips have been read
       }
+      __syncthreads();
       if (mine) {
+        for (int q = 0; q < p.ws; ++q)
+#pragma unroll
+          for (int j = 0; j < CB; ++j) {
+            const f32x4 v = q == p.cur_rank ? own[j]
+                                            : *reinterpret_cast<const IRIS_LDS f32x4*>(wb + (q - wave) * (UN * CB * SKINNY_BLOCK_BYTES) +
+                                                                                       (wave * CB + j) * 1024 + lane * 16);
+            const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+            sum[j] = (q == 0 ? zero : sum[j]) + v;
+          }
 #pragma unroll
         for (int j = 0; j < CB; ++j)
           if (n + 4 * j < p.N) store_result4(p, m, n + 4 * j, sum[j]);
@@ -619,16 +658,12 @@ gemm_skinny_kernel(const GemmKArgs p) {
   if constexpr (REDUCE) {
     // Two counts in the tile's word: the workgroups that have stored, and those of them that have reduced.  The last to
     // arrive signals the peers and, where all have reduced, consumes the flag (CAS(ws-1 -> 0), :220-234).  Else it waits for
-    // the flag and reduces the tile itself: one workgroup a tile waits, the others have made room for the peers' launches.
+    // the flag and reduces the tile itself, or leaves the tile to one that waits already (late_tiles.hpp).
     IRIS_LDS int* todo = (IRIS_LDS int*)lds;
-    Item it{};
-    it.lm0 = pid_m * p.BM;
-    it.ln0 = pid_n * p.BN;
-    it.m_end = min(p.M, it.lm0 + p.BM);
-    it.n_end = min(p.N, it.ln0 + p.BN);
     if (wave == 0) {
       constexpr int COLS = SKINNY_COLS * CB, ROWS = SKINNY_ROWS * RB;
-      const int parts = ((it.n_end - it.ln0 + COLS - 1) / COLS) * ((it.m_end - it.lm0 + ROWS - 1) / ROWS);
+      const int cols = min(p.N, (pid_n + 1) * p.BN) - pid_n * p.BN, rows = min(p.M, (pid_m + 1) * p.BM) - pid_m * p.BM;
+      const int parts = ((cols + COLS - 1) / COLS) * ((rows + ROWS - 1) / ROWS);
       int stored = 1, reduced = peers_done ? 1 : 0;
       if (parts > 1) {
         IRIS_GLOBAL int32_t* cnt = (IRIS_GLOBAL int32_t*)(p.locks + tile_id);
@@ -639,26 +674,50 @@ gemm_skinny_kernel(const GemmKArgs p) {
         reduced += before >> 16;
         if (stored == parts && lane == 0) __hip_atomic_store(cnt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
       }
-      int wait = 0;
+      int late = 0;
       if (stored == parts) {
         publish_tile(p, tile_id, lane);
-        if (reduced < parts)
-          wait = 1;
-        else if (lane == 0)
-          flag_add_relaxed(flag_of(), 1 - p.ws, p.sys != 0);
+        if (lane == 0) {
+          if (reduced < parts)
+            late = late_tile_enter(p, tile_id) ? tile_id + 1 : 0;
+          else
+            flag_add_relaxed(flag_of(), 1 - p.ws, p.sys != 0);
+        }
       }
-      if (lane == 0) {
-        if (wait && wait_tile_flag(flag_of(), p.ws, p.sys != 0, p.timeout, p.status)) wait = 2;
-        *todo = wait;
-      }
+      if (lane == 0) *todo = late;
     }
     __syncthreads();
-    if (*todo == 2) {
-      constexpr int IN_DT = F32 ? IRIS_DTYPE_F32 : ODT;
-      if (p.sys)
-        fused_reduce_tile<IN_DT, SKINNY_THREADS, 1, true>(p, it, tid);
-      else
-        fused_reduce_tile<IN_DT, SKINNY_THREADS, 1, false>(p, it, tid);
+    // (the arguments are read here, from the argument block: held in scalar registers up to here they push others out)
+    typedef const __attribute__((address_space(4))) GemmKArgs* KernArgPtr;
+    KernArgPtr late_args = (KernArgPtr)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(late_args));
+    const GemmKArgs& q = *(const GemmKArgs*)late_args;
+    bool gone = false;  // (a peer that has not come within the bound: what it has not signalled is not waited for again)
+    for (int late = __builtin_amdgcn_readfirstlane(*todo); late != 0;) {
+      __syncthreads();  // (`todo` has been read)
+      if (tid == 0)
+        *todo = wait_tile_flag((IRIS_GLOBAL int32_t*)(q.flags + late - 1), q.ws, q.sys != 0, gone ? 0 : q.timeout, q.status);
+      __syncthreads();
+      if (__builtin_amdgcn_readfirstlane(*todo)) {
+        const TileCoord t = tile_map(late - 1, q.num_pid_m, q.num_pid_n, q.G);
+        Item it{};
+        it.lm0 = t.pid_m * q.BM;
+        it.ln0 = t.pid_n * q.BN;
+        it.m_end = min(q.M, it.lm0 + q.BM);
+        it.n_end = min(q.N, it.ln0 + q.BN);
+        constexpr int IN_DT = F32 ? IRIS_DTYPE_F32 : ODT;
+        if (q.sys)
+          fused_reduce_tile<IN_DT, SKINNY_THREADS, 1, true>(q, it, tid);
+        else
+          fused_reduce_tile<IN_DT, SKINNY_THREADS, 1, false>(q, it, tid);
+      } else {
+        gone = true;
+      }
+      if (q.tile_arrivals == nullptr) break;
+      __syncthreads();
+      if (tid == 0) *todo = late_tile_next(q);
+      __syncthreads();
+      late = __builtin_amdgcn_readfirstlane(*todo);
     }
     return;
   }
