@@ -887,6 +887,11 @@ bool reduce_in_program(const iris_gemm_args& a, const Plan& producer) {
       strips < (wide ? (256 << 10) + 1 : 256 << 10))
     return true;
   if ((producer.skinny && producer.skinny_cb == 1) || producer.last_round || producer.rest || producer.parts == 1) return false;
+  // (a producer that runs faster across the caller's tiles: inside, those are back, in a round for every num_sms of them.  us a pass,
+  // inside / behind: 30 random calls of more tiles than programs 1.22x, [1330,552] x [552,3560] of 4, 64 x 128 tiles 46.4 / 35.4; one
+  // round of 256 x 256 tiles [2550,344] x [344,2376] of 8 58.8 / 39.6, fp32 in 128 x 128 [418,256] x [256,760] 30.2 / 22.4, 256 x 64
+  // 1.09x; of 128 x 64, fp32 [748,256] x [256,1504] of 4 23.0 / 27.1, row-major [580,227] x [227,2880] 16.9 / 22.3, 24 calls 0.92x)
+  if (producer.parts == 2 && (tiles > a.num_sms || a.block_m * a.block_n > 128 * 64)) return false;
   // (cells: the caller's tiles inside, when they are as small as the parts they would be run in)
   if (producer.skinny && a.block_m * a.block_n > 64 * 64) return false;
   if (k.split_k > 1 || k.merge_m * k.merge_n > 1 || k.total_tiles > a.num_sms || !k.vec_out) return false;

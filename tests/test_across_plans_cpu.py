@@ -1,0 +1,29 @@
+"""Launches whose tiles need not divide the caller's: which calls are planned so, and what is planned around them."""
+
+import pytest
+
+from iris_amd import ops
+from test_gemm_plans_cpu import BF16, F32, plan
+
+F16 = 1
+
+
+def one_shot(M, N, K, BM, BN, dtype, ws, phase, partial, **kw):
+    return plan(M, N, K, BM, BN, dtype, ws, epilogue=ops.EPI_ONE_SHOT, phase=phase, c=9 << 32, c_dtype=partial, stride_cm=N, stride_cn=1,
+                stride_cm_global=N, **kw)[0]
+
+
+@pytest.mark.parametrize("M,N,K,BM,BN,dtype,ws,partial,inside", [
+    # more of the caller's tiles than programs: never inside, in however few tiles the producer runs
+    (1219, 1016, 1168, 64, 64, BF16, 2, BF16, False), (1219, 1016, 1168, 64, 64, BF16, 8, BF16, False),
+    (1911, 2120, 472, 128, 64, BF16, 8, BF16, False), (2084, 2684, 72, 64, 128, BF16, 2, F32, False),
+    # one round of large ones
+    (2550, 2376, 344, 256, 256, BF16, 8, BF16, False), (418, 760, 256, 128, 128, F32, 2, F32, False),
+    # ... and of small ones
+    (748, 1504, 256, 128, 64, F32, 4, F32, True), (580, 2880, 227, 128, 64, BF16, 4, BF16, True),
+])
+def test_the_reduce_of_a_producer_in_other_tiles(M, N, K, BM, BN, dtype, ws, partial, inside):
+    rows = dict(stride_bk=N, stride_bn=1) if K == 227 else {}
+    assert "+across_the_tiles" in one_shot(M, N, K, BM, BN, dtype, ws, ops.PHASE_TWO_KERNELS, partial, **rows)
+    name = one_shot(M, N, K, BM, BN, dtype, ws, ops.PHASE_FUSED, partial, **rows)
+    assert name.endswith("+reduce") and name.endswith("+across_the_tiles+kernel+reduce") != inside
