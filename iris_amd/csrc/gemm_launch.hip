@@ -1389,9 +1389,10 @@ hipError_t make_plan_tiles(const iris_gemm_args& a, Plan* plan) {
     b.phase = IRIS_PHASE_TWO_KERNELS;
     Plan behind;
     if (a.split_k <= 1 && a.split_k != IRIS_GEMM_SPLIT_STREAM_K && make_plan_units(b, &behind) == hipSuccess &&
-        (!reduce_in_program(a, behind) || (behind.reduces && !behind.loose && !behind.b_rows))) {
+        (!reduce_in_program(a, behind) || (behind.reduces && !behind.loose && !behind.b_rows && a.variant == 0))) {
       // (inside, few rows and cells of aligned operands are faster than the caller's tiles with their own reduce: us a pass, [125,384] x
-      // [384,1216] of 2, 64 x 64 tiles 9.9 / 8.8, [82,128] x [128,4120] of 8 11.3 / 10.8)
+      // [384,1216] of 2, 64 x 64 tiles 9.9 / 8.8, [82,128] x [128,4120] of 8 11.3 / 10.8.  A variant that was asked for is not among
+      // the programs that reduce, or is one of them.)
       *plan = behind;
       plan->two_kernels = !reduce_in_program(a, behind);
       return hipSuccess;

@@ -1,9 +1,11 @@
 """Launches whose tiles need not divide the caller's: which calls are planned so, and what is planned around them."""
 
+import ctypes
+
 import pytest
 
-from iris_amd import ops
-from test_gemm_plans_cpu import BF16, F32, plan
+from iris_amd import _native, ops
+from test_gemm_plans_cpu import BF16, F32, plan, plan_args
 
 F16 = 1
 
@@ -27,3 +29,14 @@ def test_the_reduce_of_a_producer_in_other_tiles(M, N, K, BM, BN, dtype, ws, par
     assert "+across_the_tiles" in one_shot(M, N, K, BM, BN, dtype, ws, ops.PHASE_TWO_KERNELS, partial, **rows)
     name = one_shot(M, N, K, BM, BN, dtype, ws, ops.PHASE_FUSED, partial, **rows)
     assert name.endswith("+reduce") and name.endswith("+across_the_tiles+kernel+reduce") != inside
+
+
+@pytest.mark.parametrize("M,N,K,BM,BN,dtype", [(16, 4096, 1376, 64, 64, BF16), (46, 128, 22784, 64, 64, F16), (53, 1344, 1008, 128, 128, F32)])
+def test_the_few_rows_kernel_by_name_is_no_program_that_also_reduces(M, N, K, BM, BN, dtype):
+    """IRIS_PHASE_FUSED with IRIS_GEMM_VARIANT_FEW_ROWS is refused, whatever the launcher itself would choose for the call."""
+    args = plan_args(M, N, K, BM, BN, dtype, 4, epilogue=ops.EPI_ONE_SHOT, phase=ops.PHASE_FUSED, c=9 << 32, c_dtype=dtype, stride_cm=N,
+                     stride_cn=1, stride_cm_global=N, variant=ops.VARIANT_FEW_ROWS)
+    name = ctypes.create_string_buffer(256)
+    assert _native.lib().iris_gemm_plan_name(ctypes.byref(args), name, 256) == _native.HIP_ERROR_INVALID_VALUE
+    args.phase = ops.PHASE_TWO_KERNELS
+    assert _native.lib().iris_gemm_plan_name(ctypes.byref(args), name, 256) == 0 and name.value.startswith(b"few_rows")
