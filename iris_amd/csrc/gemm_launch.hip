@@ -1118,6 +1118,12 @@ bool plan_blocks(const iris_gemm_args& a, Plan* plan) {
 // on a shader engine waits, on 32: four tiles one after the other).  The words for that, one an engine, are the last of the
 // caller's locks.  Up to eight ranks (a wave each fetches their strips), of which late_most has one wait.  Not for
 // a launch that shares the device with its peers' by its number of programs (fewer than CUs).
+// Only for a result that shares no memory with what the kernel reads or stores besides: behind the product, one in the operands'
+// or the partials' own buffer is as good as any other.
+bool overlap(const void* p, int64_t p_bytes, const void* q, int64_t q_bytes) {
+  const uintptr_t x = reinterpret_cast<uintptr_t>(p), y = reinterpret_cast<uintptr_t>(q);
+  return x < y + (uint64_t)q_bytes && y < x + (uint64_t)p_bytes;
+}
 bool reduce_in_few_rows(const iris_gemm_args& a, Plan* plan) {
   GemmKArgs& k = plan->k;
   if (!plan->skinny || !plan->fused_reduce || a.epilogue != IRIS_EPI_ONE_SHOT || a.world_size < 2) return false;
@@ -1127,6 +1133,13 @@ bool reduce_in_few_rows(const iris_gemm_args& a, Plan* plan) {
   const int64_t lim = (int64_t)1 << 31, rows = a.block_m < a.M ? a.block_m : a.M, cols = a.block_n < a.N ? a.block_n : a.N;
   if (((int64_t)a.block_m + 64) * k.som * ies >= lim || ((int64_t)a.block_m + 64) * a.stride_cm_global * oes >= lim) return false;
   if (k.total_tiles > REDUCE_MAX_TILES || rows * cols * ies * a.world_size > REDUCE_MAX_BYTES) return false;
+  // (operands of fp32: K and strides in 16-bit units, make_plan)
+  const int unit = a.ab_dtype == IRIS_DTYPE_F32 ? 2 : 1;
+  const int64_t result = ((a.M - 1) * a.stride_cm_global + a.N) * oes, last_k = a.K / unit - 1;
+  if (overlap(a.c_global, result, a.a, ((a.M - 1) * a.stride_am + last_k * a.stride_ak + unit) * 2) ||
+      overlap(a.c_global, result, a.b, (last_k * a.stride_bk + (a.N - 1) * a.stride_bn + unit) * 2) ||
+      overlap(a.c_global, result, a.c, ((a.M - 1) * a.stride_cm + a.N) * ies))
+    return false;
   const GemmKernelFn fn = gemm_skinny_kernel_for(a.ab_dtype, a.c_dtype == IRIS_DTYPE_F32 ? OP_STORE32 : OP_STORE16, plan->skinny_arows,
                                                  plan->skinny_rb, plan->skinny_cb, plan->loose != 0, plan->b_rows != 0, true);
   if (!fn) return false;

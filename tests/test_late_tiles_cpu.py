@@ -12,11 +12,11 @@ from test_gemm_plans_cpu import BF16, F32, plan_args
 ENGINES, CUS = 32, 8  # and the CUs of an engine
 
 
-def kernels(M, N, K, BM, BN, ws, phase=ops.PHASE_TWO_KERNELS, **kw):
+def kernels(M, N, K, BM, BN, ws, phase=ops.PHASE_TWO_KERNELS, dtype=BF16, **kw):
     """(kernels, workgroups that wait at a time) of a one-shot launch"""
     kw = dict(dict(epilogue=ops.EPI_ONE_SHOT, phase=phase, c=9 << 32, stride_cm=N, stride_cn=1, stride_cm_global=N), **kw)
     n, waiting = ctypes.c_int(-1), ctypes.c_int(-1)
-    args = plan_args(M, N, K, BM, BN, ws=ws, **kw)
+    args = plan_args(M, N, K, BM, BN, dtype, ws, **kw)
     assert _native.lib().iris_gemm_launch_kernels(ctypes.byref(args), ctypes.byref(n), ctypes.byref(waiting)) == 0
     return n.value, waiting.value
 
@@ -116,3 +116,21 @@ def test_every_tile_that_is_left_is_taken_once(most, seed):
         steps += 1
         assert steps < 200000
     assert sorted(done) == list(range(tiles)) and word == [0] and not any(links)
+
+
+@pytest.mark.parametrize("dtype", [BF16, F32])
+def test_a_result_that_overlaps_what_the_product_reads_is_stored_behind_it(dtype):
+    """The activations' buffer, the weights' or this rank's partials taken again for the result."""
+    M, N, K, es = 16, 1024, 512, 2 if dtype == BF16 else 4
+    a, b, c = 1 << 32, 2 << 32, 9 << 32
+    ends = {a: M * K * es, b: N * K * es, c: M * N * es}
+    result = M * N * es
+    call = lambda at: kernels(M, N, K, 64, 64, 4, dtype=dtype, c_global=at)[0]  # noqa: E731
+    for phase in (ops.PHASE_TWO_KERNELS, ops.PHASE_FUSED):
+        assert kernels(M, N, K, 64, 64, 4, phase, dtype=dtype)[0] == 1
+    for begin, size in ends.items():
+        assert call(begin - result) == 1 and call(begin + size) == 1  # beside it
+        assert call(begin) == 2 and call(begin - result + 16) == 2 and call(begin + size - 16) == 2
+    # a row-major weight, and operands that are a part of wider ones
+    assert kernels(M, N, K, 64, 64, 4, stride_bk=N, stride_bn=1, c_global=b + N * K * 2 - 16)[0] == 2
+    assert kernels(M, N, K, 64, 64, 4, row=4096, c_global=a + 15 * 4096 * 2)[0] == 2

@@ -7,6 +7,8 @@ import pytest
 import torch
 
 from iris_amd import ops
+from oracle import iris_oracle as O
+from parity import check_close
 from test_few_rows_reduce_gpu import BF16, F32, Ranks
 from test_late_tiles_cpu import kernels
 
@@ -121,3 +123,23 @@ def test_three_ranks_side_by_side(shmem, streams, M, N, ks, rows):
         torch.cuda.synchronize()
         for r in range(ws):
             job.check(r)
+
+
+@pytest.mark.parametrize("phase", [ops.PHASE_TWO_KERNELS, ops.PHASE_FUSED])
+@pytest.mark.parametrize("over", ["activations", "weights", "partials"])
+def test_a_result_in_a_buffer_that_the_product_reads(shmem, over, phase):
+    M, N, ks, ws = 16, 1024, 1024, 4
+    job = Ranks(shmem, M, N, ks, 64, 64, ws, BF16, BF16, BF16)
+    on = shmem.on_rank
+    for r in range(1, ws):
+        job.launch(r, ops.PHASE_PRODUCE)
+    torch.cuda.synchronize()
+    # rank 0's operands by themselves, its result on top of one of them
+    a, b = job.args[0][0].contiguous(), job.args[0][1].T.contiguous().T
+    out = {"activations": a.view(M, N), "weights": b.T[:M, :].view(M, N), "partials": on(job.part, 0)}[over]
+    want_part = torch.stack([O.shard_gemm(*job.shards[0], BF16)] + [on(job.part, r).cpu() for r in range(1, ws)])
+    args = (a, b, on(job.part, 0), out) + job.args[0][4:]
+    ops.gemm_launch(*args, phase=phase, status=job.status, partials=job.P[0], locks=job.locks[0], num_xcds=8)
+    torch.cuda.synchronize()
+    assert int(job.status.item()) == 0 and not on(job.flags, 0).any()
+    check_close(out, O.one_shot_reduce(want_part, BF16), over)
