@@ -703,6 +703,11 @@ double cells_us(const iris_gemm_args& a, int64_t cells, int parts, const Operand
          (o.atomic ? 0.4 : 0.0) + (k_time > 0 ? k_time : 0.0);
 }
 
+// Whether `e` fetches the operands by the loader of `own`, or by a faster one: the DMA, the gathering loads, single elements.
+bool no_slower_loader(const GemmKernelEntry& e, const GemmKernelEntry& own) {
+  return e.dma || (!own.dma && (e.gather || !own.gather));
+}
+
 // Words of the caller's locks in which its `tiles` tiles count arrivals, one each (pack 0) or four to a word (2).
 int64_t arrival_words(int64_t tiles, int pack) { return pack ? (tiles + 3) / 4 : tiles; }
 
@@ -840,7 +845,8 @@ bool plan_small(const iris_gemm_args& a, Plan* plan) {
       if (times[i] < least && (best < 0 || times[i] < times[best])) best = i;
     if (best < 0) return found;
     Plan parts;
-    if (plan_cover(a, list[best].cm, list[best].cn, list[best].split_k, words, 0, &parts)) {
+    if (plan_cover(a, list[best].cm, list[best].cn, list[best].split_k, words, 0, &parts) &&
+        no_slower_loader(*parts.entry, *whole.entry)) {
       *plan = parts;
       return true;
     }
@@ -1284,7 +1290,7 @@ void plan_atomics(const iris_gemm_args& a, Plan* plan) {
     b.split_k = 1;
     Plan free;
     if (make_plan_body(b, &free) == hipSuccess && free.entry && free.entry->cm == t.cm && free.entry->cn == t.cn &&
-        (free.entry->dma || !own->dma) && (best_parts[i] == 1 || split_direct(b, best_parts[i], &free))) {
+        no_slower_loader(*free.entry, *own) && (best_parts[i] == 1 || split_direct(b, best_parts[i], &free))) {
       own_flags(&free);
       *plan = std::move(free);
       return;
@@ -1387,7 +1393,7 @@ void plan_across(const iris_gemm_args& a, Plan* plan) {
     const int64_t used = best_parts[i] > 1 ? ((int64_t)a.M + t.cm - 1) / t.cm * (((int64_t)a.N + t.cn - 1) / t.cn) * best_parts[i] : 0;
     const int pack = used + own_tiles <= a.num_sms ? 0 : 2;
     Plan across;
-    if (plan_cover(a, t.cm, t.cn, best_parts[i], arrival_words(own_tiles, pack), pack, &across) && across.k.split_k == best_parts[i] && (across.entry->dma || !own->dma)) {
+    if (plan_cover(a, t.cm, t.cn, best_parts[i], arrival_words(own_tiles, pack), pack, &across) && across.k.split_k == best_parts[i] && no_slower_loader(*across.entry, *own)) {
       across.parts = 2;
       *plan = std::move(across);
       return;

@@ -1,6 +1,7 @@
 """Launches whose tiles need not divide the caller's: which calls are planned so, and what is planned around them."""
 
 import ctypes
+import random
 
 import pytest
 
@@ -40,3 +41,30 @@ def test_the_few_rows_kernel_by_name_is_no_program_that_also_reduces(M, N, K, BM
     assert _native.lib().iris_gemm_plan_name(ctypes.byref(args), name, 256) == _native.HIP_ERROR_INVALID_VALUE
     args.phase = ops.PHASE_TWO_KERNELS
     assert _native.lib().iris_gemm_plan_name(ctypes.byref(args), name, 256) == 0 and name.value.startswith(b"few_rows")
+
+
+@pytest.mark.parametrize("M,N,K,BM,BN,kw", [
+    (1764, 940, 401, 256, 64, dict(epilogue=ops.EPI_ATOMIC_ADD, stride_cm_global=940)),
+    (2000, 829, 349, 256, 128, dict(epilogue=ops.EPI_ATOMIC_ADD, stride_cm_global=829, stride_bk=829, stride_bn=1, partials=0, locks=0)),
+    (5197, 322, 320, 128, 128, dict(epilogue=ops.EPI_ONE_SHOT, phase=ops.PHASE_PRODUCE, c=9 << 32, stride_cm=322, stride_cn=1, stride_bk=322,
+                                    stride_bn=1, partials=0, locks=0)),
+])
+def test_operands_that_are_gathered_are_not_left_to_the_loader_of_single_elements(M, N, K, BM, BN, kw):
+    """There is no gathering 64 x 64 tile for fp32 of a short K."""
+    assert "_gather" in plan(M, N, K, BM, BN, F32, **kw)[0]
+
+
+def test_no_tile_that_loads_single_elements_for_one_that_does_not():
+    rng, seen = random.Random(5), 0
+    for _ in range(6000):
+        M, N, K = (int(2 ** rng.uniform(0, 13)) for _ in range(3))
+        BM, BN = rng.choice([(64, 64), (128, 128), (256, 64), (256, 128)])
+        kw = rng.choice([dict(epilogue=ops.EPI_ATOMIC_ADD, stride_cm_global=N), dict(),
+                         dict(epilogue=ops.EPI_ONE_SHOT, phase=ops.PHASE_PRODUCE, c=9 << 32, stride_cm=N, stride_cn=1)])
+        if rng.random() < 0.6:
+            kw = dict(kw, stride_bk=N, stride_bn=1)
+        own = plan(M, N, K, BM, BN, F32, variant=ops.VARIANT_PERSISTENT, **kw)[0]
+        if "generic" not in own:
+            assert "generic" not in plan(M, N, K, BM, BN, F32, **kw)[0], (M, N, K, BM, BN, kw, own)
+            seen += "_gather" in own
+    assert seen > 100
