@@ -711,12 +711,14 @@ bool no_slower_loader(const GemmKernelEntry& e, const GemmKernelEntry& own) {
 // Words of the caller's locks in which its `tiles` tiles count arrivals, one each (pack 0) or four to a word (2).
 int64_t arrival_words(int64_t tiles, int pack) { return pack ? (tiles + 3) / 4 : tiles; }
 
-// Whether tiles of cm x cn may lie across the caller's: a lane for each of the caller's that one of them touches, a byte for
-// their number in one of the caller's.
-bool can_cover(const iris_gemm_args& a, int cm, int cn) {
+// Whether tiles of cm x cn may lie across the caller's, whose arrivals are counted in words (pack 0) or bytes (2): no more of
+// them to one of the caller's than a byte counts, and no more of the caller's to one of them than its publication, which takes
+// them one after another, walks in MOST_TOUCHED round trips of an atomic.
+constexpr int MOST_TOUCHED = 64;
+bool can_cover(const iris_gemm_args& a, int cm, int cn, int pack) {
   const int64_t touched = ((int64_t)(cm - 1) / a.block_m + 2) * ((cn - 1) / a.block_n + 2);
   const int64_t parts = ((int64_t)(a.block_m - 1) / cm + 2) * ((a.block_n - 1) / cn + 2);
-  return touched <= 64 && parts <= 255;
+  return touched <= MOST_TOUCHED && (pack == 0 || parts <= 255);
 }
 
 // The launch in tiles of cm x cn, K shared out in split_k.  A caller's tile is the unit of a flag, not of work: the tiles that share
@@ -820,7 +822,7 @@ bool plan_small(const iris_gemm_args& a, Plan* plan) {
   double times[8];
   int count = 0;
   for (const auto& s : shapes) {
-    if (a.block_m % s[0] != 0 || a.block_n % s[1] != 0 || !can_cover(a, s[0], s[1])) continue;
+    if (a.block_m % s[0] != 0 || a.block_n % s[1] != 0 || !can_cover(a, s[0], s[1], 0)) continue;
     const int64_t tiles = tiles_of(s[0], s[1]);
     if (tiles > a.num_sms) continue;
     if (s[0] == a.block_m && s[1] == a.block_n) break;  // (the caller's tile is the smallest that fits)
@@ -1366,7 +1368,7 @@ void plan_across(const iris_gemm_args& a, Plan* plan) {
   for (int i = 0; i < TILES; ++i) {
     const AcrossTime& t = ACROSS_TIMES[i];
     best_us[i] = 1e30;
-    if ((l.f32 && t.step_f32 == 0) || !can_cover(a, t.cm, t.cn)) continue;
+    if ((l.f32 && t.step_f32 == 0) || !can_cover(a, t.cm, t.cn, 0)) continue;
     const int64_t tiles = ((int64_t)a.M + t.cm - 1) / t.cm * (((int64_t)a.N + t.cn - 1) / t.cn), elems = tiles * t.cm * t.cn;
     if (tiles > 4 * (int64_t)a.num_sms) continue;
     int most = (int)((a.num_sms - least) / tiles);
@@ -1393,7 +1395,7 @@ void plan_across(const iris_gemm_args& a, Plan* plan) {
     const int64_t used = best_parts[i] > 1 ? ((int64_t)a.M + t.cm - 1) / t.cm * (((int64_t)a.N + t.cn - 1) / t.cn) * best_parts[i] : 0;
     const int pack = used + own_tiles <= a.num_sms ? 0 : 2;
     Plan across;
-    if (plan_cover(a, t.cm, t.cn, best_parts[i], arrival_words(own_tiles, pack), pack, &across) && across.k.split_k == best_parts[i] && no_slower_loader(*across.entry, *own)) {
+    if (can_cover(a, t.cm, t.cn, pack) && plan_cover(a, t.cm, t.cn, best_parts[i], arrival_words(own_tiles, pack), pack, &across) && across.k.split_k == best_parts[i] && no_slower_loader(*across.entry, *own)) {
       across.parts = 2;
       *plan = std::move(across);
       return;

@@ -68,3 +68,12 @@ def test_no_tile_that_loads_single_elements_for_one_that_does_not():
             assert "generic" not in plan(M, N, K, BM, BN, F32, **kw)[0], (M, N, K, BM, BN, kw, own)
             seen += "_gather" in own
     assert seen > 100
+
+
+@pytest.mark.parametrize("M,N,K,dtype,kw", [
+    (966, 992, 2288, F16, {}), (108, 5288, 1505, BF16, {}),
+    (59, 7648, 488, BF16, dict(epilogue=ops.EPI_ATOMIC_ADD, stride_cm_global=7648)),
+])
+def test_a_word_counts_the_parts_of_a_large_tile(M, N, K, dtype, kw):
+    """Parts of the caller's tiles count in a word each, so that a tile may have any number of them."""
+    assert plan(M, N, K, 1024, 1024, dtype, **kw)[0].startswith("64x64") and "+parts_of_tiles" in plan(M, N, K, 1024, 1024, dtype, **kw)[0]
