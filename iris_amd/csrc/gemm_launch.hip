@@ -1199,18 +1199,22 @@ constexpr AtomicTime ATOMIC_TIMES[] = {
 struct AtomicLaunch {
   double streamed;  // how much of the operands comes from HBM
   double each;      // us that the chip takes for all atomics of one part of K
+  double contend;   // ... by which it takes longer for each part that adds to the same sums
   double kind;      // of the loader
   bool f32, lines;
 };
-double atomic_us(const iris_gemm_args& a, const AtomicTime& t, int parts, const AtomicLaunch& l) {
+// (`last_parts`: K of the last round's tiles in as many, as split_last_round leaves them, at 20 us for their launch and hand-over.)
+double atomic_us(const iris_gemm_args& a, const AtomicTime& t, int parts, const AtomicLaunch& l, int last_parts = 1) {
   const int64_t items = ((int64_t)a.M + t.cm - 1) / t.cm * (((int64_t)a.N + t.cn - 1) / t.cn) * parts;
   const int64_t rounds = (items + a.num_sms - 1) / a.num_sms, nk = ((int64_t)a.K + 63) / 64, steps = (nk + parts - 1) / parts;
   const double busy = rounds > 1 ? 1.0 : (double)items / a.num_sms;
   const double step = (l.f32 ? t.step_f32 * (1 + 0.043 * busy) : t.step * (1 + 0.148 * busy) * (1 + 0.399 * l.streamed)) *
                       (l.lines ? 1.0 : 1.19) * l.kind;
-  const double loop = t.tile + steps * step, chip = 0.537 * l.each * parts / rounds, cu = 0.518 * t.cm * t.cn / 4096;
+  const double loop = t.tile + steps * step, cu = 0.518 * t.cm * t.cn / 4096;
+  const double chip = 0.537 * l.each * parts / rounds * (1 + l.contend * (parts - 1));
   const double adds = chip > cu ? chip : cu, next = loop + 1.083 * adds;
-  return 6.82 + 1.09 * busy + loop + (rounds - 1) * (next > adds ? next : adds) + adds;
+  const double spared = last_parts > 1 ? steps * step * (1 - 1.0 / last_parts) - 20 : 0;
+  return 6.82 + 1.09 * busy + loop + (rounds - 1) * (next > adds ? next : adds) + adds - (spared > 0 ? spared : 0);
 }
 
 // K of an unsplit plan with fp32 atomics in `parts`, each of which adds its own sums.
@@ -1236,18 +1240,23 @@ bool split_direct(const iris_gemm_args& a, int parts, Plan* plan) {
 // them / so: [828,20672] x [20672,2688] in 256 x 64 tiles 208 / 109, 128 x 256 in three parts; [2023,22656] x [22656,192] in 256 x 128
 // 54 / 36; fp32 [904,1024] x [1024,4224] in 128 x 128 140 / 77, 64 x 128; fp32 [1171,456] x [456,258] 41 / 15; row-major
 // [494,9968] x [9968,4480] with 16-bit atomics in 64 x 64 98 / 68.  Of 353 random calls in tiles 96 change, 1.07x on average
-// over all of them; four slower by 4 to 7 %, all in more than four rounds of tiles, which are left out.)
+// over all of them; four slower by 4 to 7 %, all in more than four rounds of tiles, which are left out.  Of 320 random calls of up
+// to eight copies that a plan without the last two of these rules changes, 55 take another for them: those 55 are 0.93 of
+// the caller's tiles without and 0.89 with them, 18 and 3 of them slower by more than 3 %, 1.57x and 1.08x at most.)
 void plan_atomics(const iris_gemm_args& a, Plan* plan) {
   const GemmKernelEntry* own = plan->entry;
   if (a.epilogue != IRIS_EPI_ATOMIC_ADD || !own || plan->skinny || plan->k.stream_k) return;
   if (a.variant != 0 || a.split_k != 0 || a.mm_begin_timestamp || a.mm_end_timestamp || a.num_sms != current_cu_count() || a.K <= 0) return;
   const bool wide = a.c_global_dtype == IRIS_DTYPE_F32, handed = plan->k.split_k > 1;
-  const bool parts_add = wide && (a.scope != IRIS_SCOPE_SYSTEM || a.world_size <= 1);
+  // (To more than two copies, parts that hand over add their own slices of a tile to each, which is faster than all of it: of
+  // 23 random calls of four and eight 0.95x so, [39,3816] x [3816,287] of eight 18 us and 28.)
+  const bool parts_add = wide && (a.scope != IRIS_SCOPE_SYSTEM || a.world_size <= 1) && !(handed && a.world_size > 2);
   if (!parts_add && handed) return;
   AtomicLaunch l;
   const double mb = ((double)a.M + a.N) * a.K * 2e-6;
   l.streamed = mb < 50 ? 0 : mb > 150 ? 1 : (mb - 50) / 100;
   l.each = (double)a.M * a.N * a.world_size / 331e3 * (wide ? 1.0 : 0.5);
+  l.contend = a.world_size > 2 ? 0.15 : 0;
   l.kind = !own->dma ? 1.9 : own->loose ? 1.24 : 1.0;
   l.f32 = a.ab_dtype == IRIS_DTYPE_F32;
   l.lines = whole_lines(a);
@@ -1258,7 +1267,8 @@ void plan_atomics(const iris_gemm_args& a, Plan* plan) {
       // (a hand-over: 6 us, and the parts' sums are added up once)
       AtomicLaunch whole = l;
       whole.each /= plan->k.split_k;
-      own_us = atomic_us(a, t, plan->k.split_k, whole) + (handed ? 6 : 0);
+      whole.contend = 0;
+      own_us = atomic_us(a, t, plan->k.split_k, whole, plan->last_round ? plan->k_last.split_k : 1) + (handed ? 6 : 0);
     }
   if (own_us < 12) return;  // (another tile than these, or nothing to gain that the search would not cost)
   double best_us[TILES];

@@ -77,3 +77,19 @@ def test_no_tile_that_loads_single_elements_for_one_that_does_not():
 def test_a_word_counts_the_parts_of_a_large_tile(M, N, K, dtype, kw):
     """Parts of the caller's tiles count in a word each, so that a tile may have any number of them."""
     assert plan(M, N, K, 1024, 1024, dtype, **kw)[0].startswith("64x64") and "+parts_of_tiles" in plan(M, N, K, 1024, 1024, dtype, **kw)[0]
+
+
+@pytest.mark.parametrize("M,N,K,BM,BN,dtype,ws,kw,want", [
+    # parts that hand over, to four and eight copies
+    (39, 287, 3816, 128, 128, F32, 8, dict(stride_bk=287, stride_bn=1), ("64x64x64_w2x2_gather_fp32+parts_of_tiles", 16)),
+    (92, 192, 28736, 256, 64, BF16, 8, dict(stride_bk=192, stride_bn=1), ("64x64x128_w2x2_s4_f4_rows+parts_of_tiles", 16)),
+    (895, 671, 2685, 64, 64, F32, 4, dict(stride_bk=671, stride_bn=1), ("64x64x64_w2x2_gather_fp32", 1)),
+    # a last round whose K is shared out
+    (4035, 1145, 18287, 128, 128, BF16, 4, dict(c_global_dtype=BF16), ("128x128x64_w2x2_s4_f4_gather_dma+last_round_in_8_parts", 1)),
+    # ... and what other tiles and parts that add their own sums are for
+    (828, 2688, 20672, 256, 64, BF16, 1, {}, ("128x256x64_w1x4_s3_f4", 3)),
+    (4088, 131, 35880, 64, 128, F16, 4, {}, ("128x128x64_w2x2_s4_f4", 4)),
+    (1104, 1126, 11095, 64, 64, BF16, 1, {}, ("128x128x64_w2x2_s4_f4_gather_dma", 3)),
+])
+def test_atomics(M, N, K, BM, BN, dtype, ws, kw, want):
+    assert plan(M, N, K, BM, BN, dtype, ws, **dict(dict(epilogue=ops.EPI_ATOMIC_ADD, c_global_dtype=F32, stride_cm_global=N), **kw)) == want
