@@ -1927,7 +1927,8 @@ extern "C" int iris_gemm_launch_noalloc(const iris_gemm_args* args, void* stream
   // wait that timed out leaves one raised).  A fill kernel, not a memset, so
   // that the call can be recorded into a HIP graph.
   auto needs_locks = [](const Plan& q) {
-    return (q.skinny && (q.k.flag_mode != 0 || q.skinny_grid_z > 1)) || q.k.cover_bm > 0 || (q.entry && (q.k.split_k > 1 || q.k.stream_k || q.last_round));
+    const bool handed = q.k.split_k > 1 && q.k.sliced != SPLIT_DIRECT;
+    return (q.skinny && (q.k.flag_mode != 0 || q.skinny_grid_z > 1)) || q.k.cover_bm > 0 || (q.entry && (handed || q.k.stream_k || q.last_round));
   };
   const bool uses_locks = needs_locks(plan) || (plan.rest && needs_locks(*plan.rest));
   if (uses_locks) {
