@@ -82,6 +82,10 @@ int iris_hip_arch_name(int device, char* buf, size_t len);
 
 /* epilogues of the persistent shard GEMM */
 #define IRIS_EPI_ALL_SCATTER 0 /* examples/07_gemm_all_scatter/gemm_all_scatter.py:209-251 */
+/* With fp32 atomics on one device (IRIS_SCOPE_AGENT, or one rank) the launcher may share K out over programs that each
+ * add their own sums to c_global (split_k 0; iris_gemm_split_k says how many): an element is then added in that many
+ * roundings at the magnitude c_global holds, in no fixed order, and the last bits of launches with equal inputs may
+ * differ.  split_k 1 asks for one sum an element, the same bits from every launch in stream order. */
 #define IRIS_EPI_ATOMIC_ADD 1  /* examples/08_gemm_atomics_all_reduce/gemm_atomics_all_reduce.py:206-248 */
 #define IRIS_EPI_ONE_SHOT 2    /* examples/09_gemm_one_shot_all_reduce/gemm_one_shot_all_reduce.py:197-271 */
 

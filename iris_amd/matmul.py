@@ -72,6 +72,7 @@ def make_matmul(epilogue: int, name: str):
         status = None            # optional int32 device word for flag-wait timeouts
         spin_timeout_ticks = 0
         split_k = 0  # 0: the launcher decides, 1: never split K, n: exactly n parts
+        # (fp32 atomics, 0: parts of K may each add their sums, in no fixed order; 1: one sum an element, the same bits each time)
 
         @staticmethod
         def set_debug(debug: bool):

@@ -4,6 +4,7 @@ import pytest
 import torch
 
 from iris_amd import ops
+from iris_amd.matmul import matmul_atomics_all_reduce
 from oracle import iris_oracle as O
 from parity import check_close, make_ab
 from test_gemm_gather_gpu import place
@@ -37,3 +38,30 @@ def test_parts_that_hand_nothing_over_need_no_locks_cleared(shmem):
     names = kernels_of(lambda: ops.gemm_launch(*args, num_xcds=8, noalloc=True))
     assert len(names) == 1 and "gemm" in names[0], names
     check_close(c, O.shard_gemm(A, B, F32))
+
+
+@pytest.mark.parametrize("M,N,K", [(266, 1152, 6248), (965, 1296, 4504)])
+def test_one_sum_an_element_on_request(shmem, M, N, K):
+    """split_k 1: what C held and the whole sum, rounded once, in every run; without it K of these is in parts."""
+    A, B, c, args = product(shmem, M, N, K)
+    P, locks = torch.zeros((256, 64 * 64), device="cuda"), torch.zeros((256,), dtype=torch.int32, device="cuda")
+    assert ops.gemm_split_k(*args, num_xcds=8, partials=P, locks=locks) > 1
+    assert ops.gemm_split_k(*args, num_xcds=8, partials=P, locks=locks, split_k=1) == 1
+
+    def sums(held):
+        c.fill_(held)
+        matmul_atomics_all_reduce.apply(args[0], args[1], None, c, None, P, locks, None, 0, 1, 256, 64, 64, 64, 4, "True", 2, 8, 0, 16, 2,
+                                        args[5], 256)
+        torch.cuda.synchronize()
+        return c.clone()
+
+    matmul_atomics_all_reduce.set_debug(False)
+    matmul_atomics_all_reduce.split_k = 1
+    try:
+        whole = sums(0.0)
+        for held in (0.0, 1000.0, -0.37, 1000.0):
+            assert torch.equal(sums(held), whole + held)
+    finally:
+        matmul_atomics_all_reduce.split_k = 0
+    check_close(whole, O.shard_gemm(A, B, F32))
+    check_close(sums(0.0), O.shard_gemm(A, B, F32), "in parts")
