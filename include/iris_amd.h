@@ -285,7 +285,7 @@ int iris_gemm_split_k(const iris_gemm_args* args, int* split_k);
  * locks), by "+parts_of_tiles" where the caller's tiles are computed as several
  * smaller ones, by "+across_the_tiles" where it runs in tiles that need not divide
  * them (partials and locks as above), and by "+kernel+reduce" where an IRIS_PHASE_FUSED launch runs as an
- * IRIS_PHASE_TWO_KERNELS one. */
+ * IRIS_PHASE_TWO_KERNELS one.  The name is the product's: iris_gemm_launch_kernels says whether a reduce kernel follows. */
 int iris_gemm_plan_name(const iris_gemm_args* args, char* buf, size_t len);
 
 /* What `iris_gemm_launch` would put on the stream for `args`: the number of kernels (one where a launch with a reduce reduces

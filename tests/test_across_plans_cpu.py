@@ -93,3 +93,14 @@ def test_a_word_counts_the_parts_of_a_large_tile(M, N, K, dtype, kw):
 ])
 def test_atomics(M, N, K, BM, BN, dtype, ws, kw, want):
     assert plan(M, N, K, BM, BN, dtype, ws, **dict(dict(epilogue=ops.EPI_ATOMIC_ADD, c_global_dtype=F32, stride_cm_global=N), **kw)) == want
+
+
+@pytest.mark.parametrize("kw", [dict(mm_begin_timestamp=10 << 32, mm_end_timestamp=11 << 32), dict(mm_end_timestamp=11 << 32), dict(split_k=1),
+                                dict(split_k=2), dict(variant=ops.VARIANT_PERSISTENT), dict(num_sms=248)])
+def test_what_is_asked_for_keeps_the_callers_tiles(kw):
+    """Timestamps are the caller's tiles' own; parts, a variant and fewer programs than CUs are the caller's choice."""
+    atomics = dict(epilogue=ops.EPI_ATOMIC_ADD, c_global_dtype=F32, stride_cm_global=1296)
+    assert plan(965, 1296, 4504, 128, 128, F16, **atomics)[0].startswith("256x64x64")
+    assert plan(965, 1296, 4504, 128, 128, F16, **dict(atomics, **kw))[0].startswith("128x128x64")
+    assert "+across_the_tiles" in plan(1911, 2120, 472, 256, 64)[0]
+    assert "across" not in plan(1911, 2120, 472, 256, 64, **kw)[0]
