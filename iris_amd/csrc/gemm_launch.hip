@@ -1328,13 +1328,14 @@ struct AcrossLaunch {
   double streamed, kind;
   int copies;  // of the output, in 16-bit elements
   bool f32, lines;
+  int off;  // copies of rows that 16-byte stores don't fit, or end inside one (the times above know only the others)
 };
-double across_us(const iris_gemm_args& a, const AcrossTime& t, int parts, const AcrossLaunch& l) {
+double across_us(const iris_gemm_args& a, const AcrossTime& t, int parts, const AcrossLaunch& l, bool off = false) {
   const int64_t items = ((int64_t)a.M + t.cm - 1) / t.cm * (((int64_t)a.N + t.cn - 1) / t.cn) * parts;
   const int64_t rounds = (items + a.num_sms - 1) / a.num_sms, nk = ((int64_t)a.K + 63) / 64, steps = (nk + parts - 1) / parts;
   const double busy = rounds > 1 ? 1.0 : (double)items / a.num_sms, area = (double)t.cm * t.cn / 4096;
   const double step = (l.f32 ? t.step_f32 * (1 + 0.059 * busy) : t.step * (1 + 0.112 * busy) * (1 + 0.404 * l.streamed)) * (l.lines ? 1.0 : 1.223) * l.kind;
-  const double loop = t.tile + steps * step, store = area / parts * 0.377 * (l.copies - 1) * (busy > 0.37 ? busy : 0.37);
+  const double loop = t.tile + steps * step, store = area / parts * (0.377 * (l.copies - 1) + (off ? 1 + l.off : 0)) * (busy > 0.37 ? busy : 0.37);
   const double mb = items * area / 64, low = mb < 16 ? mb : 16;
   const double hand = parts > 1 ? 3.210 + 0.417 * area + 0.114 * low + 0.092 * (mb - low) + 0.151 * parts : 0;
   return 3.946 + 0.920 * busy + rounds * loop + store * (1 + (rounds - 1) * 0.67) + hand;
@@ -1372,6 +1373,14 @@ void plan_across(const iris_gemm_args& a, Plan* plan) {
   // (what the times above are not good for: K in this many parts, and small tiles that share it, whose operands the L2s hold)
   if (own_parts > 12 || (own_parts > 2 && own->cm * own->cn == 64 * 64)) return;
   if (own_us < 12) return;  // (another tile than these, or nothing to gain that the search would not cost)
+  // (one or two K-steps: the stores are most of it, and other tiles than the caller's are 0.99 of the time over 17 random calls,
+  // 1.44 at most)
+  if (a.K <= 128 && own->dma && plan->k.merge_m * plan->k.merge_n == 1) return;
+  const int es = dtype_size(scatter ? a.c_global_dtype : a.c_dtype);
+  l.off = !plan->k.vec_out || (int64_t)a.N * es % 16 != 0 ? (scatter ? a.world_size : 1) : 0;
+  const AcrossTime* own_time = nullptr;
+  for (const AcrossTime& t : ACROSS_TIMES)
+    if (t.cm == own->cm && t.cn == own->cn) own_time = &t;
   double best_us[TILES];
   int best_parts[TILES];
   const int64_t room = a.partials && a.locks && aligned16(a.partials) ? a.num_sms * a.partials_slot_elems : 0;
@@ -1401,6 +1410,12 @@ void plan_across(const iris_gemm_args& a, Plan* plan) {
       if (best_us[j] < best_us[i]) i = j;
     const AcrossTime& t = ACROSS_TIMES[i];
     if (best_us[i] > 0.87 * own_us) return;
+    // (us a pass, the caller's tiles / so, without this: [1034,64] x [64,2135] to eight 31 / 42, [753,467] x [467,3183] 45 / 58; of 541
+    // random calls that were planned so 27 keep theirs for it and the line of K above, 1.04x slower so on average)
+    if (l.off && across_us(a, t, best_parts[i], l, true) > 0.95 * across_us(a, *own_time, own_parts, l, true)) {
+      best_us[i] = 1e30;
+      continue;
+    }
     // (a word for each of the caller's tiles where they have room beside those of the parts of K)
     const int64_t used = best_parts[i] > 1 ? ((int64_t)a.M + t.cm - 1) / t.cm * (((int64_t)a.N + t.cn - 1) / t.cn) * best_parts[i] : 0;
     const int pack = used + own_tiles <= a.num_sms ? 0 : 2;

@@ -19,7 +19,7 @@ def one_shot(M, N, K, BM, BN, dtype, ws, phase, partial, **kw):
 @pytest.mark.parametrize("M,N,K,BM,BN,dtype,ws,partial,inside", [
     # more of the caller's tiles than programs: never inside, in however few tiles the producer runs
     (1219, 1016, 1168, 64, 64, BF16, 2, BF16, False), (1219, 1016, 1168, 64, 64, BF16, 8, BF16, False),
-    (1911, 2120, 472, 128, 64, BF16, 8, BF16, False), (2084, 2684, 72, 64, 128, BF16, 2, F32, False),
+    (1911, 2120, 472, 128, 64, BF16, 8, BF16, False), (1330, 3560, 552, 64, 128, BF16, 4, BF16, False),
     # one round of large ones
     (2550, 2376, 344, 256, 256, BF16, 8, BF16, False), (418, 760, 256, 128, 128, F32, 2, F32, False),
     # ... and of small ones
@@ -105,3 +105,15 @@ def test_what_is_asked_for_keeps_the_callers_tiles(kw):
     assert "+across_the_tiles" in plan(1911, 2120, 472, 256, 64)[0]
     if kw.get("split_k") != 2:  # (the caller's tiles are more than half the programs: no two parts of them)
         assert "across" not in plan(1911, 2120, 472, 256, 64, **kw)[0]
+
+
+@pytest.mark.parametrize("M,N,K,BM,BN,dtype,ws,across", [
+    # one or two K-steps, in the caller's tiles and in blocks of them
+    (1034, 2135, 64, 64, 128, F16, 8, False), (2654, 1920, 128, 256, 256, F16, 8, False), (290, 5765, 64, 128, 64, BF16, 8, True),
+    # rows of an odd length, to eight copies and to one
+    (6500, 679, 320, 64, 128, BF16, 8, False), (2011, 2523, 186, 64, 128, BF16, 1, False), (1911, 2121, 472, 256, 64, BF16, 1, True),
+    (1911, 2120, 472, 256, 64, BF16, 8, True),
+])
+def test_where_the_stores_are_most_of_it(M, N, K, BM, BN, dtype, ws, across):
+    row = K + 1 if K == 186 else K
+    assert ("+across_the_tiles" in plan(M, N, K, BM, BN, dtype, ws, row=row)[0]) == across
