@@ -603,15 +603,18 @@ gemm_skinny_kernel(const GemmKArgs p) {
       }
       __syncthreads();
       if (mine) {
-        for (int q = 0; q < p.ws; ++q)
 #pragma unroll
-          for (int j = 0; j < CB; ++j) {
-            const f32x4 v = q == p.cur_rank ? own[j]
-                                            : *reinterpret_cast<const IRIS_LDS f32x4*>(wb + (q - wave) * (UN * CB * SKINNY_BLOCK_BYTES) +
-                                                                                       (wave * CB + j) * 1024 + lane * 16);
-            const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-            sum[j] = (q == 0 ? zero : sum[j]) + v;
-          }
+        for (int j = 0; j < CB; ++j) {
+          f32x4 v[SKINNY_WAVES];  // (all on their way before the first is added)
+#pragma unroll
+          for (int q = 0; q < SKINNY_WAVES; ++q)
+            v[q] = *reinterpret_cast<const IRIS_LDS f32x4*>(wb + (q - wave) * (UN * CB * SKINNY_BLOCK_BYTES) + (wave * CB + j) * 1024 +
+                                                            lane * 16);
+          sum[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int q = 0; q < SKINNY_WAVES; ++q)
+            if (q < p.ws) sum[j] += q == p.cur_rank ? own[j] : v[q];
+        }
 #pragma unroll
         for (int j = 0; j < CB; ++j)
           if (n + 4 * j < p.N) store_result4(p, m, n + 4 * j, sum[j]);
@@ -652,18 +655,22 @@ gemm_skinny_kernel(const GemmKArgs p) {
 
   // The stores were write-through at the flags' scope: once every wave has
   // seen its own complete, the group's part of the tile is visible there.
+  const int pid_m = m0 / p.BM, pid_n = n0 / p.BN;
+  int parts = 0;  // (REDUCE) workgroups that share the tile, counted while the stores complete
+  if constexpr (REDUCE) {
+    constexpr int COLS = SKINNY_COLS * CB, ROWS = SKINNY_ROWS * RB;
+    const int cols = min(p.N, (pid_n + 1) * p.BN) - pid_n * p.BN, rows = min(p.M, (pid_m + 1) * p.BM) - pid_m * p.BM;
+    parts = ((cols + COLS - 1) / COLS) * ((rows + ROWS - 1) / ROWS);
+    asm volatile("" : "+s"(parts));
+  }
   IRIS_WAIT_VMCNT(0);
   __syncthreads();
-  const int pid_m = m0 / p.BM, pid_n = n0 / p.BN;
   if constexpr (REDUCE) {
     // Two counts in the tile's word: the workgroups that have stored, and those of them that have reduced.  The last to
     // arrive signals the peers and, where all have reduced, consumes the flag (CAS(ws-1 -> 0), :220-234).  Else it waits for
     // the flag and reduces the tile itself, or leaves the tile to one that waits already (late_tiles.hpp).
     IRIS_LDS int* todo = (IRIS_LDS int*)lds;
     if (wave == 0) {
-      constexpr int COLS = SKINNY_COLS * CB, ROWS = SKINNY_ROWS * RB;
-      const int cols = min(p.N, (pid_n + 1) * p.BN) - pid_n * p.BN, rows = min(p.M, (pid_m + 1) * p.BM) - pid_m * p.BM;
-      const int parts = ((cols + COLS - 1) / COLS) * ((rows + ROWS - 1) / ROWS);
       int stored = 1, reduced = peers_done ? 1 : 0;
       if (parts > 1) {
         IRIS_GLOBAL int32_t* cnt = (IRIS_GLOBAL int32_t*)(p.locks + tile_id);
@@ -678,7 +685,7 @@ gemm_skinny_kernel(const GemmKArgs p) {
       if (stored == parts) {
         publish_tile(p, tile_id, lane);
         if (lane == 0) {
-          if (reduced < parts)
+          if (__builtin_expect(reduced < parts, 0))
             late = late_tile_enter(p, tile_id) ? tile_id + 1 : 0;
           else
             flag_add_relaxed(flag_of(), 1 - p.ws, p.sys != 0);
@@ -693,7 +700,7 @@ gemm_skinny_kernel(const GemmKArgs p) {
     asm volatile("" : "+s"(late_args));
     const GemmKArgs& q = *(const GemmKArgs*)late_args;
     bool gone = false;  // (a peer that has not come within the bound: what it has not signalled is not waited for again)
-    for (int late = __builtin_amdgcn_readfirstlane(*todo); late != 0;) {
+    for (int late = __builtin_amdgcn_readfirstlane(*todo); __builtin_expect(late != 0, 0);) {
       __syncthreads();  // (`todo` has been read)
       if (tid == 0)
         *todo = wait_tile_flag((IRIS_GLOBAL int32_t*)(q.flags + late - 1), q.ws, q.sys != 0, gone ? 0 : q.timeout, q.status);
