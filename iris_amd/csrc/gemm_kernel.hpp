@@ -159,6 +159,7 @@ struct GemmKArgs {
   // flag_num_pid_m x flag_num_pid_n.  The tiles that share one of the caller's count their arrivals at it in a word of
   // tile_arrivals (arrive_pack 0) or a byte of one (2), all zero between launches, and the last one raises its flag
   int cover_bm, cover_bn, arrive_pack;
+  // (the few-rows kernel that reduces: a word for each shader engine, late_tiles.hpp, or null where tiles are too few to need them)
   int32_t* tile_arrivals;
   FastDiv div_xcd;  // num_xcds
   // (the few-rows kernel in cells of 32 x 32) `cells` of them, numbered in runs of cells_inner along the rows of C

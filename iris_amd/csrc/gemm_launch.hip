@@ -690,7 +690,7 @@ double cells_us(const iris_gemm_args& a, int64_t cells, int parts, const Operand
   const double mb = ((double)a.M + a.N) * a.K * 2e-6;
   // us for 64 of K, operands in whole lines / not: [512,512] 256 cells 0.090 / 0.13; [128,1376] 172 cells 0.083 / 0.11;
   // [200,512] 112 cells 0.048 / 0.066 as long as the L2s hold the operands, 0.07 / 0.08 beyond
-  // (a row-major B comes in half lines: 1.5 times the L1's time with the 32 rows of A beside it, and from HBM at half the rate;
+  // (a row-major B comes in half lines: 1.5 times the requests' time with the 32 rows of A beside it, and from HBM at half the rate;
   // fitted with both in it.  [28,7936] x [7936,4864] 33.8, in tiles 23.5; with up to 16 rows of A a cell fetches half of A)
   const double lines = o.b_rows ? (a.M <= SKINNY_ROWS ? 1.08 : 1.8) : o.lines ? 1.0 : o.loose ? 2.1 : 1.45;
   const double step = 0.083 * (groups * 5 > cus * 4 ? 1.09 : groups * 2 <= cus && mb <= 30 ? 0.7 : 1.0) *

@@ -67,8 +67,10 @@ constexpr int skinny_lds_bytes(int rb) { return skinny_a_bytes(rb) + SKINNY_WAVE
 // persistent kernel's tiles are too few to fill the chip or too short to pay for its fixed costs (its prologue, hand-over
 // and flag take 3 us more than this kernel's; sharing K out over programs 4 to 6 us).  Here the eight waves share K
 // inside the workgroup.  A comes in like B, by LDS-DMA, two blocks a wave in flight: 8 KiB a block of K, 128 KiB a
-// workgroup, one workgroup a CU.  It is bound by the CU's L1: 0.08 us for every 64 of K, 0.09 on
-// all CUs at once ([512,512], 256 workgroups: 9.0 us at K = 1024, 61 at 36864), where 64 bytes a clock would be 0.053.
+// workgroup, one workgroup a CU.  64 of K take 0.08 us, 0.09 on all CUs at once ([512,512], 256 workgroups: 9.0 us at K =
+// 1024, 61 at 36864), and 0.048 with 112 workgroups whose operands the L2s hold.  No one unit bounds it: at [128,1376], 172 workgroups,
+// a CU's L1 takes 0.73 accesses of 64 bytes a clock, an XCD's L2 gives 2.4 TB/s, half of what its channels can, and 23 % of
+// its requests miss it (operands changed from launch to launch; counters at K = 4096 and 8192).
 // A lane's columns are eight in a row: the block j of a row of 32 columns takes columns 8q + 4j .. + 3, so that a row
 // leaves in 16-byte stores.  The cells are dealt to the XCDs in consecutive runs (the shorter direction first), so that
 // each XCD's L2 fetches its share of the longer operand once.
@@ -168,8 +170,9 @@ __device__ inline int late_tile_next(const GemmKArgs& p) {
 // what it has just computed, so it waits for no other workgroup; the peers' strips, where their signal is there by the
 // last blocks of K, are fetched (wave w: rank w) under the last products and the exchange between the waves, and the sum is stored
 // behind the partial.  A reduce kernel behind the product cost its launch, its gap (0.84 us) and a chain of flag, bases,
-// partials and result of its own: [16,1376] x [1376,4096], 8 fp32 partials, fill of the flags included 13.5 -> 9.7 us; 64 random
-// calls of up to 300 rows whose reduce is inside 1.24x, none slower.
+// partials and result of its own: [16,1376] x [1376,4096], 8 fp32 partials, fill of the flags included 13.2 -> 9.5 us; 64 random
+// calls of up to 300 rows whose reduce is inside 1.24x, none slower.  Up to eight ranks, a wave each; where peers are late, few
+// workgroups wait (late_tiles.hpp).
 template <int DT, int OP, int ODT, int AROWS, int RB = 1, int CB = 1, bool LOOSE = false, bool BROWS = false, bool REDUCE = false>
 __global__ __launch_bounds__(SKINNY_THREADS) __attribute__((amdgpu_waves_per_eu(2, 8))) void
 gemm_skinny_kernel(const GemmKArgs p) {
