@@ -143,3 +143,34 @@ def test_a_result_in_a_buffer_that_the_product_reads(shmem, over, phase):
     torch.cuda.synchronize()
     assert int(job.status.item()) == 0 and not on(job.flags, 0).any()
     check_close(out, O.one_shot_reduce(want_part, BF16), over)
+
+
+def test_replays_of_a_graph(shmem):
+    """A pass recorded once and replayed with eager work between: tiles that are signalled, and some that are not within the bound."""
+    ws, M, N, ks = 8, 16, 4096, 1376
+    job = Ranks(shmem, M, N, ks, 64, 64, ws, BF16, F32, BF16)
+    on = shmem.on_rank
+    for r in range(1, ws):
+        job.launch(r, ops.PHASE_PRODUCE)
+    want, late = torch.full((job.total,), ws - 1, dtype=torch.int32, device="cuda"), torch.arange(job.total, device="cuda") % 4 == 2
+
+    def one_pass():
+        on(job.flags, 0).copy_(want)
+        job.launch(0, ops.PHASE_TWO_KERNELS, spin_timeout_ticks=2000)
+
+    one_pass()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        one_pass()
+    for replay in range(6):
+        want.copy_(torch.where(late, ws - 2, ws - 1) if replay % 2 else torch.full_like(want, ws - 1))
+        job.status.zero_()
+        on(job.out, 0).fill_(-7)
+        graph.replay()
+        torch.cuda.synchronize()
+        if replay % 2 == 0:
+            job.check(0)
+        else:
+            assert int(job.status.item()) == 1 and not any(x.any() for x in job.locks)
+            assert torch.equal(on(job.flags, 0), torch.where(late, ws - 2, 0).to(torch.int32))
