@@ -207,7 +207,8 @@ typedef struct iris_gemm_args {
    * the programs of a launch meet.  Parts of a shared K hand over there; where a
    * tile is computed by several workgroups (the few-rows kernel, cells of 32 x 32,
    * parts of the caller's tiles), they count their arrivals there, and the last one
-   * raises the tile's flag, whether K is shared or not.  So a launch of any shape
+   * raises the tile's flag, whether K is shared or not; a launch that reduces as it
+   * stores lists its late tiles there.  So a launch of any shape
    * may write them, and both buffers belong to ONE launch at a time: launches that
    * can run at the same time (other streams, other ranks of the device) need
    * buffers of their own, or NULL, without which no such plan is taken. */

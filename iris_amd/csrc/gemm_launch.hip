@@ -1118,6 +1118,12 @@ bool plan_blocks(const iris_gemm_args& a, Plan* plan) {
   return false;
 }
 
+// Whether `p_bytes` from p on and `q_bytes` from q on share any.
+bool overlap(const void* p, int64_t p_bytes, const void* q, int64_t q_bytes) {
+  const uintptr_t x = reinterpret_cast<uintptr_t>(p), y = reinterpret_cast<uintptr_t>(q);
+  return x < y + (uint64_t)q_bytes && y < x + (uint64_t)p_bytes;
+}
+
 // Few rows and cells with a reduce behind them: the reduce in the same kernel (gemm_skinny.hpp, REDUCE), where a tile is small
 // enough for one workgroup to reduce it should its peers be late, and there are few enough tiles for that.
 // One workgroup has 32 KB of partials in flight, so a late tile of REDUCE_MAX_BYTES is four round trips to memory, about what a reduce
@@ -1128,10 +1134,6 @@ bool plan_blocks(const iris_gemm_args& a, Plan* plan) {
 // a launch that shares the device with its peers' by its number of programs (fewer than CUs).
 // Only for a result that shares no memory with what the kernel reads or stores besides: behind the product, one in the operands'
 // or the partials' own buffer is as good as any other.
-bool overlap(const void* p, int64_t p_bytes, const void* q, int64_t q_bytes) {
-  const uintptr_t x = reinterpret_cast<uintptr_t>(p), y = reinterpret_cast<uintptr_t>(q);
-  return x < y + (uint64_t)q_bytes && y < x + (uint64_t)p_bytes;
-}
 bool reduce_in_few_rows(const iris_gemm_args& a, Plan* plan) {
   GemmKArgs& k = plan->k;
   if (!plan->skinny || !plan->fused_reduce || a.epilogue != IRIS_EPI_ONE_SHOT || a.world_size < 2) return false;
@@ -1240,9 +1242,9 @@ bool split_direct(const iris_gemm_args& a, int parts, Plan* plan) {
 // them / so: [828,20672] x [20672,2688] in 256 x 64 tiles 208 / 109, 128 x 256 in three parts; [2023,22656] x [22656,192] in 256 x 128
 // 54 / 36; fp32 [904,1024] x [1024,4224] in 128 x 128 140 / 77, 64 x 128; fp32 [1171,456] x [456,258] 41 / 15; row-major
 // [494,9968] x [9968,4480] with 16-bit atomics in 64 x 64 98 / 68.  Of 353 random calls in tiles 96 change, 1.07x on average
-// over all of them; four slower by 4 to 7 %, all in more than four rounds of tiles, which are left out.  Of 320 random calls of up
-// to eight copies that a plan without the last two of these rules changes, 55 take another for them: those 55 are 0.93 of
-// the caller's tiles without and 0.89 with them, 18 and 3 of them slower by more than 3 %, 1.57x and 1.08x at most.)
+// over all of them; four slower by 4 to 7 %, all in more than four rounds of tiles, which are left out.  The rules on
+// more than two copies and on a last round whose K is shared out change the plans of 55 of 320 random calls of up to eight copies:
+// 0.93 of the time in the caller's tiles without them, 18 of the 55 slower by more than 3 %, and 0.89 with them, three slower.)
 void plan_atomics(const iris_gemm_args& a, Plan* plan) {
   const GemmKernelEntry* own = plan->entry;
   if (a.epilogue != IRIS_EPI_ATOMIC_ADD || !own || plan->skinny || plan->k.stream_k) return;
